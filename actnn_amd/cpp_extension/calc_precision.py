@@ -44,7 +44,13 @@ def calc_precision_dp(A, C, max_b, target, states):
     return b_vec, p_vec
 
 
-DEVICE_MAX_CANDIDATES = 8192
+DEVICE_MAX_CANDIDATES = 8192               # calc_precision_device
+ALLOCATE_MAX_CANDIDATES = 1 << 20          # allocate_bits_device: items, and items * (start width - 1)
+
+
+def allocation_fits(N, initial_bits):
+    """True when allocate_bits_device (and the one-call sequences built on it) take the batch."""
+    return 1 <= int(initial_bits) <= 8 and N * max(int(initial_bits) - 1, 1) <= ALLOCATE_MAX_CANDIDATES
 
 
 def device_allocation_fits(N, initial_bits):

@@ -96,13 +96,7 @@ extern "C" int actnn_bits_prefix(const int32_t* bits, int32_t* prefix, int64_t N
 extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
                                           int mult_per_sample, float* sensitivity, int32_t* bits,
                                           int32_t* prefix, int64_t N, int64_t G, int initial_bits,
-                                          int64_t target, int dtype, void* stream) {
-  int rc = actnn_range_sqr(mn, mx, sensitivity, N, G, factor, mult, mult_per_sample, dtype, stream);
-  if (rc != ACTNN_OK) return rc;
-  rc = actnn_calc_precision_device(sensitivity, bits, N, initial_bits, target, stream);
-  if (rc != ACTNN_OK) return rc;
-  return actnn_bits_prefix(bits, prefix, N, stream);
-}
+                                          int64_t target, int dtype, void* stream);
 
 // One crossing of the language boundary for a layer's whole forward-side sequence: the calls below
 // on one stream, arguments as theirs.  Nothing is launched unless the arguments of the first step

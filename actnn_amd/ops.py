@@ -391,9 +391,13 @@ def _fused_grad_weight_ok(quantized, shape, go):
 class linear(Function):
     @staticmethod
     def forward(ctx, input, weight, bias=None, scheme=None):
-        started = start_quantize(input, scheme)
-        output = F.linear(input, weight, bias)
-        quantized = finish_saved(started, input)
+        quantized = quantize_on_device(input, scheme)
+        if quantized is not None:
+            output = F.linear(input, weight, bias)
+        else:
+            started = start_quantize(input, scheme)
+            output = F.linear(input, weight, bias)
+            quantized = finish_saved(started, input)
         empty_cache(config.empty_cache_threshold)
         ctx.scheme = scheme
         ctx.saved = quantized, weight, bias

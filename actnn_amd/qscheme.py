@@ -145,7 +145,7 @@ def allocate_bits_on_device(mn, mx, N, num_pixels, factor, mult, initial_bits, a
 
 
 def allocate_on_device(N, initial_bits):
-    return config.device_allocation and ext_calc_precision.device_allocation_fits(N, initial_bits)
+    return config.device_allocation and ext_calc_precision.allocation_fits(N, initial_bits)
 
 
 class AllocationArgs:

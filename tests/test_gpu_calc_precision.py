@@ -111,6 +111,24 @@ def test_allocation_in_one_call_from_dirty_buffers(N):
         assert torch.equal(bits, first)
 
 
+@pytest.mark.parametrize("N,initial", [(146, 8), (147, 8), (1024, 2), (1170, 8), (1171, 8), (9362, 8), (9363, 8), (16385, 3),
+                                       (40000, 8)])
+@pytest.mark.parametrize("coarse", [False, True])
+def test_allocation_of_large_batches_equals_the_host_routine(N, initial, coarse):
+    """Around the switches of the allocation kernel (256 / 1024 threads, candidates in registers, items in
+    LDS); coarse sensitivities make ties of which only some are taken."""
+    g = torch.Generator().manual_seed(N)
+    mx = torch.exp(torch.randn(N, generator=g))
+    if coarse:
+        mx = mx.round(decimals=1)
+    mx = mx.to(DEV)
+    for target in (int(2.3 * N), N + 1, initial * N - 1):
+        sens, bits, prefix = ext_cp.allocate_bits_device(torch.zeros_like(mx), mx, N, 1.0, None, initial, target)
+        exp = _host(sens.cpu(), initial, target)
+        assert np.array_equal(bits.cpu().numpy(), exp.numpy())
+        assert torch.equal(prefix[1:], torch.cumsum(bits, 0).to(torch.int32)) and int(prefix[0]) == 0
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("known", [False, True])
 def test_quantise_an_activation_in_one_call_equals_the_three_calls(dtype, known):
