@@ -53,6 +53,30 @@ def test_library_matches_oracle(lib, seed):
     assert np.array_equal(_lib_calc(lib, b0, C, w, target), cp.calc_precision(b0, C, w, target))
 
 
+@pytest.mark.parametrize("kind", ["lognormal", "coarse", "zeros", "denormal", "one_bit_start", "infinite", "over_budget"])
+def test_library_selection_and_heap_match_oracle(lib, kind):
+    # start widths and weights of every kind; the last four hold items that only the heap takes, or
+    # a budget outside what the widths span
+    rng = np.random.default_rng(7)
+    N = 257
+    C = rng.lognormal(0, 3, N).astype(np.float32)
+    w = rng.integers(1, 200000, N).astype(np.int32)
+    b0 = rng.integers(2, 9, N).astype(np.int32)
+    if kind == "coarse":
+        C, w = np.round(C), np.full(N, 3, np.int32)
+    elif kind == "zeros":
+        C[::2] = 0.0
+    elif kind == "denormal":
+        C = (C * 1e-40).astype(np.float32)
+    elif kind == "one_bit_start":
+        b0[5] = 1
+    elif kind == "infinite":
+        C[3] = np.inf
+    full = float((b0.astype(np.float64) * w).sum())
+    for share in (0.9, 0.5, 0.3) if kind != "over_budget" else (1.0, 1.5):
+        assert np.array_equal(_lib_calc(lib, b0, C, w, share * full), cp.calc_precision(b0, C, w, share * full))
+
+
 def test_library_known_answer_and_errors(lib):
     b = _lib_calc(lib, np.full(256, 8), np.zeros(256), np.ones(256), 512)
     assert (b[:36] == 8).all() and b[36] == 5 and (b[37:] == 1).all()
