@@ -14,6 +14,8 @@
 // needs (a contiguous span of the plane) into LDS with 16-byte loads, and then works out of LDS,
 // so HBM sees each input byte once and all global accesses are coalesced.  Planes too wide for
 // the LDS budget fall back to direct global loads.
+#include <type_traits>
+
 #include "device_utils.h"
 
 namespace actnn {
@@ -226,31 +228,31 @@ template <> ACTNN_DEV float lds_value<bf16_t>(const bf16_t* p, int i) { return b
 // Geometry presets: with PRESET != 0 the window parameters are compile-time constants (loops
 // unroll, divisions become shifts); PRESET 0 reads them from the argument.
 //   1: 3x3 stride 2 pad 1 (ResNet stem)   2: 2x2 stride 2 pad 0   3: 3x3 stride 1 pad 1
+//   4: 3x3 stride 2 pad 0
 template <int PRESET> struct Win {
   int KH, KW, SH, SW, PH, PW;
   __device__ __forceinline__ explicit Win(const PoolGeom& g)
-      : KH(PRESET == 1 || PRESET == 3 ? 3 : PRESET == 2 ? 2 : g.KH),
-        KW(PRESET == 1 || PRESET == 3 ? 3 : PRESET == 2 ? 2 : g.KW),
-        SH(PRESET == 1 || PRESET == 2 ? 2 : PRESET == 3 ? 1 : g.SH),
-        SW(PRESET == 1 || PRESET == 2 ? 2 : PRESET == 3 ? 1 : g.SW),
-        PH(PRESET == 1 || PRESET == 3 ? 1 : PRESET == 2 ? 0 : g.PH),
-        PW(PRESET == 1 || PRESET == 3 ? 1 : PRESET == 2 ? 0 : g.PW) {}
+      : KH(PRESET == 0 ? g.KH : PRESET == 2 ? 2 : 3), KW(PRESET == 0 ? g.KW : PRESET == 2 ? 2 : 3),
+        SH(PRESET == 0 ? g.SH : PRESET == 3 ? 1 : 2), SW(PRESET == 0 ? g.SW : PRESET == 3 ? 1 : 2),
+        PH(PRESET == 0 ? g.PH : PRESET == 1 || PRESET == 3 ? 1 : 0),
+        PW(PRESET == 0 ? g.PW : PRESET == 1 || PRESET == 3 ? 1 : 0) {}
 };
 
 inline int preset_of(const PoolGeom& g) {
   if (g.KH == 3 && g.KW == 3 && g.SH == 2 && g.SW == 2 && g.PH == 1 && g.PW == 1) return 1;
   if (g.KH == 2 && g.KW == 2 && g.SH == 2 && g.SW == 2 && g.PH == 0 && g.PW == 0) return 2;
   if (g.KH == 3 && g.KW == 3 && g.SH == 1 && g.SW == 1 && g.PH == 1 && g.PW == 1) return 3;
+  if (g.KH == 3 && g.KW == 3 && g.SH == 2 && g.SW == 2 && g.PH == 0 && g.PW == 0) return 4;
   return 0;
 }
 
-template <typename T, int PRESET, bool NIB>      // NIB: Wo even, so the two outputs of a byte sit in one row
+template <typename T, bool NIB>                  // NIB: Wo even, so the two outputs of a byte sit in one row
 __global__ __launch_bounds__(kThreads) void max_pool2d_forward_lds_kernel(
     const T* __restrict__ x, T* __restrict__ y, int8_t* __restrict__ idx, int64_t total_in,
     PoolGeom g, int rows_per_band, int bands) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* s_in = reinterpret_cast<T*>(smem);
-  const Win<PRESET> k(g);
+  const Win<0> k(g);
   const int64_t nc = blockIdx.x / bands;
   const int ho0 = (int)(blockIdx.x % bands) * rows_per_band;
   const int rows_out = g.Ho - ho0 < rows_per_band ? g.Ho - ho0 : rows_per_band;
@@ -296,7 +298,7 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_forward_lds_kernel(
   }
 }
 
-template <typename T, int PRESET, bool NIB>
+template <typename T, bool NIB>
 __global__ __launch_bounds__(kThreads) void max_pool2d_backward_lds_kernel(
     const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin,
     int64_t total_out, PoolGeom g, int rows_per_band, int bands, int max_out_rows) {
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_lds_kernel(
   // [grad_output rows | index rows], each with room for the alignment shift
   T* s_g = reinterpret_cast<T*>(smem);
   int8_t* s_i = reinterpret_cast<int8_t*>(smem + (((size_t)max_out_rows * g.Wo + 16) * sizeof(T) + 15) / 16 * 16);
-  const Win<PRESET> k(g);
+  const Win<0> k(g);
   const int64_t nc = blockIdx.x / bands;
   const int h0 = (int)(blockIdx.x % bands) * rows_per_band;
   const int rows_in = g.H - h0 < rows_per_band ? g.H - h0 : rows_per_band;
@@ -354,8 +356,307 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_lds_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Stride-2 fast path (3x3 pad 1 and 2x2 pad 0 with W % 8 == 0, Wo == W / 2, Ho == H / 2): the
-// shapes of every stem / VGG-style pooling layer.  A thread produces 4 adjacent outputs from three
+// The preset windows over planes of any size: rows that start anywhere, odd widths, and (two indices
+// per byte) bytes whose two outputs lie in different rows.  No LDS: consecutive threads take
+// consecutive outputs (forward) or cells of consecutive input pixels (backward) of the flattened
+// tensor, so every load of a wave is a run of a few lines that the next load of the window finds in
+// L1.  What the LDS-tiled kernels lost on these shapes was not traffic but instructions: 64-bit
+// divisions, loops with run-time bounds and one load in flight.  Here positions come from
+// multiply-high divisions, all loads of a window are issued before the first comparison, and a
+// thread owns the pixels that share windows: 2x2 of them (stride 2, backward) or 4 of a column (stride 1).  Measured on f32 [64,96,55,55], 3x3 stride 2: forward 40 -> 22 us, backward
+// 116 -> 18 us; bf16 [256,256,13,13], 2x2 stride 2: 73 -> 11 and 111 -> 10 us; 3x3 stride 1 on f32
+// [64,64,112,112]: 170 -> 102 and 236 -> 94 us.
+struct DirectGeom {
+  uint32_t count;                         // threads with work
+  uint32_t cols, per_plane;               // cells (outputs) of a row and of a plane
+  FastDiv by_plane, by_cols;
+};
+struct DirectAt { uint32_t id, plane, row, col; };
+ACTNN_DEV DirectAt direct_at(const DirectGeom& q, uint32_t block) {
+  DirectAt a;
+  a.id = block * kThreads + threadIdx.x;
+  a.plane = q.by_plane.div(a.id);
+  const uint32_t r = a.id - a.plane * q.per_plane;
+  a.row = q.by_cols.div(r);
+  a.col = r - a.row * q.cols;
+  return a;
+}
+// (neighbouring blocks read the same rows: a run of them stays on one XCD)
+ACTNN_DEV uint32_t direct_block() {
+  return (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+}
+// false when the tensor is too large for 32-bit element numbers
+inline bool direct_geometry(int64_t planes, int64_t rows, int64_t cols, DirectGeom& q) {
+  const int64_t count = planes * rows * cols;
+  if (count > 0x7fffff00LL) return false;
+  q.count = (uint32_t)count;
+  q.cols = (uint32_t)cols;
+  q.per_plane = (uint32_t)(rows * cols);
+  q.by_plane = FastDiv(q.per_plane);
+  q.by_cols = FastDiv(q.cols);
+  return true;
+}
+inline dim3 direct_grid(const DirectGeom& q) { return dim3(xcd_grid(((int64_t)q.count + kThreads - 1) / kThreads)); }
+
+template <typename T, int PRESET, bool NIB>
+__global__ __launch_bounds__(kThreads) void max_pool2d_forward_direct_kernel(
+    const T* __restrict__ x, T* __restrict__ y, int8_t* __restrict__ idx, DirectGeom q, PoolGeom g) {
+  constexpr int K = PRESET == 2 ? 2 : 3;
+  const Win<PRESET> k(g);
+  const DirectAt at = direct_at(q, direct_block());
+  const bool live = at.id < q.count;
+  int index = 0;
+  if (live) {
+    const float init = Conv<T>::round(-1e10f);          // as the reference, .cu:656
+    const T* plane = x + (uint64_t)at.plane * (uint32_t)(g.H * g.W);
+    const int i0 = (int)at.row * k.SH - k.PH, j0 = (int)at.col * k.SW - k.PW;
+    // a position outside the plane reads the nearest one inside and counts as the start value, which
+    // never wins the strict compare
+    int col[K];
+    bool col_in[K];
+#pragma unroll
+    for (int b = 0; b < K; ++b) {
+      const int j = j0 + b;
+      col_in[b] = k.PW == 0 || (uint32_t)j < (uint32_t)g.W;
+      col[b] = k.PW == 0 ? j : (j < 0 ? 0 : j < g.W ? j : g.W - 1);
+    }
+    float c[K * K];
+#pragma unroll
+    for (int a = 0; a < K; ++a) {
+      const int i = i0 + a;
+      const bool row_in = k.PH == 0 || (uint32_t)i < (uint32_t)g.H;
+      const uint32_t row = (uint32_t)(k.PH == 0 ? i : (i < 0 ? 0 : i < g.H ? i : g.H - 1)) * (uint32_t)g.W;
+#pragma unroll
+      for (int b = 0; b < K; ++b) {
+        const float v = Conv<T>::load(plane, row + (uint32_t)col[b]);
+        c[a * K + b] = row_in && col_in[b] ? v : init;
+      }
+    }
+    float v = init;
+#pragma unroll
+    for (int p = 0; p < K * K; ++p)
+      if (c[p] > v) {
+        v = c[p];
+        index = p;
+      }
+    Conv<T>::store(y, at.id, v);
+    if (!NIB) idx[at.id] = (int8_t)index;
+  }
+  if (NIB) {
+    // the even thread writes the byte of outputs id and id + 1 (0 for an output past the end)
+    const int next = lane_xor<1>(index);
+    if (live && !(at.id & 1)) idx[at.id >> 1] = (int8_t)(index | (next << 4));
+  }
+}
+
+// One and two adjacent elements stored at any element-aligned address.  NT: past the caches, for
+// results that would not stay there anyway (stream_results).
+typedef uint32_t u32x2_e4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32_e2 __attribute__((aligned(2)));
+template <bool NT> ACTNN_DEV void store_one(float* p, float v) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <bool NT> ACTNN_DEV void store_half_word(void* p, uint32_t w) {
+  if (NT) __builtin_nontemporal_store((uint16_t)w, static_cast<uint16_t*>(p));
+  else *static_cast<uint16_t*>(p) = (uint16_t)w;
+}
+template <bool NT> ACTNN_DEV void store_one(__half* p, float v) { store_half_word<NT>(p, float_to_half_bits(v)); }
+template <bool NT> ACTNN_DEV void store_one(bf16_t* p, float v) { store_half_word<NT>(p, float_to_bf16_bits(v)); }
+template <bool NT> ACTNN_DEV void store_two(float* p, const float (&v)[2]) {
+  const u32x2_e4 w = {as_uint(v[0]), as_uint(v[1])};
+  if (NT) __builtin_nontemporal_store(w, reinterpret_cast<u32x2_e4*>(p));
+  else *reinterpret_cast<u32x2_e4*>(p) = w;
+}
+template <bool NT> ACTNN_DEV void store_word_e2(void* p, uint32_t w) {
+  if (NT) __builtin_nontemporal_store(w, static_cast<u32_e2*>(p));
+  else *static_cast<u32_e2*>(p) = w;
+}
+template <bool NT> ACTNN_DEV void store_two(__half* p, const float (&v)[2]) {
+  store_word_e2<NT>(p, float_to_half_bits(v[0]) | (float_to_half_bits(v[1]) << 16));
+}
+template <bool NT> ACTNN_DEV void store_two(bf16_t* p, const float (&v)[2]) { store_word_e2<NT>(p, pack_bf16x2(v[0], v[1])); }
+
+// The windows that reach rows 2a and 2a + 1 of a stride-2 pool are rows a + kFirst .. a + kFirst + kCount - 1
+// of windows; row 2a + rr sits at row rr + P - 2j of window a + j.
+template <int K, int P> struct CellWindows {
+  static constexpr int kCount = K == 3 ? 2 : 1;
+  static constexpr int kFirst = K == 3 && P == 0 ? -1 : 0;
+};
+
+template <typename T, int K, int P, bool NIB, bool NT>
+__global__ __launch_bounds__(kThreads) void max_pool2d_backward_direct_s2_kernel(
+    const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, DirectGeom q, PoolGeom g) {
+  using CW = CellWindows<K, P>;
+  constexpr int NWIN = CW::kCount, J0 = CW::kFirst;
+  const DirectAt at = direct_at(q, direct_block());
+  if (at.id >= q.count) return;
+  const uint32_t obase = at.plane * (uint32_t)(g.Ho * g.Wo);
+  float gv[NWIN][NWIN];
+  int iv[NWIN][NWIN];
+#pragma unroll
+  for (int j = 0; j < NWIN; ++j) {
+    const int ho = (int)at.row + J0 + j;
+    const bool row_in = (uint32_t)ho < (uint32_t)g.Ho;
+    const uint32_t row = obase + (uint32_t)(row_in ? ho : 0) * (uint32_t)g.Wo;
+#pragma unroll
+    for (int t = 0; t < NWIN; ++t) {
+      const int wo = (int)at.col + J0 + t;
+      const bool in = row_in && (uint32_t)wo < (uint32_t)g.Wo;
+      const uint32_t o = row + (uint32_t)(in ? wo : 0);
+      gv[j][t] = Conv<T>::load(gout, o);
+      const int i = read_index<NIB>(idx, o);
+      iv[j][t] = in ? i : -1;                            // matches no position of a window
+    }
+  }
+  float out[2][2];
+#pragma unroll
+  for (int rr = 0; rr < 2; ++rr)
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NWIN; ++j) {
+        const int kh = rr + P - 2 * (J0 + j);
+        if (kh < 0 || kh >= K) continue;
+#pragma unroll
+        for (int t = 0; t < NWIN; ++t) {
+          const int kw = cc + P - 2 * (J0 + t);
+          if (kw < 0 || kw >= K) continue;
+          acc += iv[j][t] == kh * K + kw ? gv[j][t] : 0.0f;
+        }
+      }
+      out[rr][cc] = acc;
+    }
+  T* cell = gin + (uint64_t)at.plane * (uint32_t)(g.H * g.W) + 2 * at.row * (uint32_t)g.W + 2 * at.col;
+  const bool two_cols = 2 * at.col + 1 < (uint32_t)g.W;
+#pragma unroll
+  for (int rr = 0; rr < 2; ++rr) {
+    if (2 * at.row + rr >= (uint32_t)g.H) break;
+    if (two_cols) store_two<NT>(cell + rr * g.W, out[rr]);
+    else store_one<NT>(cell + rr * g.W, out[rr][0]);
+  }
+}
+
+// 3x3 stride 1 pad 1: neighbouring windows share two thirds of their pixels, so a thread owns kStrip
+// pixels (outputs) of one column - lanes still take consecutive columns - and loads the kStrip + 2
+// rows around them once.
+constexpr int kStrip = 4;
+
+template <typename T, bool NIB, bool NT>
+__global__ __launch_bounds__(kThreads) void max_pool2d_backward_direct_s1_kernel(
+    const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, DirectGeom q, PoolGeom g) {
+  const DirectAt at = direct_at(q, direct_block());      // rows of strips, columns of pixels
+  if (at.id >= q.count) return;
+  const uint32_t plane = at.plane * (uint32_t)(g.H * g.W);       // (Ho = H, Wo = W)
+  const int h0 = kStrip * (int)at.row, w = (int)at.col;
+  float acc[kStrip];
+#pragma unroll
+  for (int r = 0; r < kStrip; ++r) acc[r] = 0.0f;
+  // (row by row of windows: every pixel adds its windows in row-major order)
+#pragma unroll
+  for (int j = -1; j <= kStrip; ++j) {
+    const int ho = h0 + j;
+    const bool row_in = (uint32_t)ho < (uint32_t)g.H;
+    const uint32_t row = plane + (uint32_t)(row_in ? ho : 0) * (uint32_t)g.W;
+    float gv[3];
+    int iv[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {                        // window column w - 1 + t sees the pixel at kw = 2 - t
+      const int wo = w - 1 + t;
+      const bool in = row_in && (uint32_t)wo < (uint32_t)g.W;
+      const uint32_t o = row + (uint32_t)(in ? wo : 0);
+      gv[t] = Conv<T>::load(gout, o);
+      const int i = read_index<NIB>(idx, o);
+      iv[t] = in ? i : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < kStrip; ++r) {
+      const int kh = r - j + 1;                          // of pixel h0 + r in the windows of row ho
+      if (kh < 0 || kh > 2) continue;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) acc[r] += iv[t] == kh * 3 + 2 - t ? gv[t] : 0.0f;
+    }
+  }
+  T* out = gin + plane + (uint32_t)h0 * (uint32_t)g.W + (uint32_t)w;
+#pragma unroll
+  for (int r = 0; r < kStrip; ++r)
+    if (h0 + r < g.H) store_one<NT>(out + r * g.W, acc[r]);
+}
+
+// The same on the way forward.  A row of three pixels is reduced once for the three windows that
+// read it (first strict maximum and its column), a window then takes the first strict maximum of its
+// three rows: the row-major scan.  With two indices per byte W is even, so that the two outputs of a
+// byte are held by neighbouring lanes.
+template <typename T, bool NIB>
+__global__ __launch_bounds__(kThreads) void max_pool2d_forward_direct_s1_kernel(
+    const T* __restrict__ x, T* __restrict__ y, int8_t* __restrict__ idx, DirectGeom q, PoolGeom g) {
+  const DirectAt at = direct_at(q, direct_block());
+  const bool live = at.id < q.count;
+  const uint32_t plane = at.plane * (uint32_t)(g.H * g.W);
+  const int h0 = kStrip * (int)at.row, w = (int)at.col;
+  const float init = Conv<T>::round(-1e10f);             // as the reference, .cu:656
+  float best[kStrip];
+  int index[kStrip];
+#pragma unroll
+  for (int r = 0; r < kStrip; ++r) {
+    best[r] = init;
+    index[r] = 0;
+  }
+  if (live) {
+#pragma unroll
+    for (int j = -1; j <= kStrip; ++j) {
+      const int i = h0 + j;
+      const bool row_in = (uint32_t)i < (uint32_t)g.H;
+      const uint32_t row = plane + (uint32_t)(row_in ? i : 0) * (uint32_t)g.W;
+      float c[3];
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        const int col = w - 1 + b;
+        const bool in = row_in && (uint32_t)col < (uint32_t)g.W;
+        const float v = Conv<T>::load(x, row + (uint32_t)(in ? col : 0));
+        c[b] = in ? v : init;
+      }
+      float m = init;
+      int at_col = 0;
+#pragma unroll
+      for (int b = 0; b < 3; ++b)
+        if (c[b] > m) {
+          m = c[b];
+          at_col = b;
+        }
+#pragma unroll
+      for (int r = 0; r < kStrip; ++r) {
+        const int a = j - r + 1;                         // row of the window of output h0 + r
+        if (a < 0 || a > 2) continue;
+        if (m > best[r]) {
+          best[r] = m;
+          index[r] = 3 * a + at_col;
+        }
+      }
+    }
+  }
+  const uint32_t out = plane + (uint32_t)h0 * (uint32_t)g.W + (uint32_t)w;
+#pragma unroll
+  for (int r = 0; r < kStrip; ++r) {
+    const bool here = live && h0 + r < g.H;
+    const uint32_t o = out + (uint32_t)(r * g.W);
+    if (here) Conv<T>::store(y, o, best[r]);
+    if (NIB) {
+      const int next = lane_xor<1>(index[r]);            // (w and the lane have the same parity)
+      if (here && !(w & 1)) idx[o >> 1] = (int8_t)(index[r] | (next << 4));
+    } else if (here) {
+      idx[o] = (int8_t)index[r];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Stride-2 fast path, forward of the 16-bit types and backward of all (3x3 pad 1 and 2x2 pad 0 with W % 8 == 0, Wo == W / 2,
+// Ho == H / 2): the shapes of every stem / VGG-style pooling layer.  (bf16 [64,64,112,112], 3x3: forward
+// 28 us, backward 26 us, against 59 and 38 us of the direct kernels on [64,64,114,114].  For fp32, whose
+// elements are loads of a whole dword, the direct forward is the faster one - 67 against 69 us, 2x2 40
+// against 63 us - and the backward pass keeps this one: 46 against 69 us.)  A thread produces 4 adjacent outputs from three
 // 16-byte LDS reads (forward) or 8 adjacent inputs of two rows from a handful of LDS reads
 // (backward), compares against compile-time window positions, and writes 8/16-byte pieces that are
 // contiguous across the wave.  Padding is handled by data, not by branches: the row above the
@@ -567,7 +868,7 @@ template <typename T, bool NIB>
 int launch_fwd(const void* x, void* y, int8_t* idx, int64_t total, const PoolGeom& g, hipStream_t s) {
   const int64_t planes = total / ((int64_t)g.Ho * g.Wo);
   auto need = [&](int rows) { return ((size_t)((rows - 1) * g.SH + g.KH) * g.W + 16) * sizeof(T); };
-  if (const int k = s2_kernel_of(g); k != 0 && aligned16(x) && aligned16(y) && aligned16(idx)) {
+  if (const int k = sizeof(T) == 2 ? s2_kernel_of(g) : 0; k != 0 && aligned16(x) && aligned16(y) && aligned16(idx)) {
     const int rb = pick_band(g.Ho, g.Wo / 4, kFwdS2Threads, kFwdS2Passes, need);
     const int bands = rb > 0 ? (g.Ho + rb - 1) / rb : 0;
     if (rb > 0 && planes * bands <= 0x7fffffffLL) {
@@ -579,20 +880,35 @@ int launch_fwd(const void* x, void* y, int8_t* idx, int64_t total, const PoolGeo
       ACTNN_RETURN_LAUNCH_STATUS();
     }
   }
+  const int preset = preset_of(g);
+  // (without padding the direct kernel looks at no bounds: every window must lie inside the plane)
+  const bool whole = g.PH > 0 || ((g.Ho - 1) * (int64_t)g.SH + g.KH <= g.H && (g.Wo - 1) * (int64_t)g.SW + g.KW <= g.W);
+  DirectGeom q;
+  if (preset != 0 && whole && planes * g.H * g.W <= 0x7fffffffLL && direct_geometry(planes, g.Ho, g.Wo, q)) {
+    const dim3 grid = direct_grid(q), blk(kThreads);
+    const T* xi = static_cast<const T*>(x);
+    T* yo = static_cast<T*>(y);
+    switch (preset) {
+      case 1: max_pool2d_forward_direct_kernel<T, 1, NIB><<<grid, blk, 0, s>>>(xi, yo, idx, q, g); break;
+      case 2: max_pool2d_forward_direct_kernel<T, 2, NIB><<<grid, blk, 0, s>>>(xi, yo, idx, q, g); break;
+      case 3:
+        // (an odd width has bytes that hold the last output of a row and the first of the next)
+        if ((!NIB || g.W % 2 == 0) && g.Ho == g.H && g.Wo == g.W && direct_geometry(planes, (g.H + kStrip - 1) / kStrip, g.W, q))
+          max_pool2d_forward_direct_s1_kernel<T, NIB><<<direct_grid(q), blk, 0, s>>>(xi, yo, idx, q, g);
+        else
+          max_pool2d_forward_direct_kernel<T, 3, NIB><<<grid, blk, 0, s>>>(xi, yo, idx, q, g);
+        break;
+      default: max_pool2d_forward_direct_kernel<T, 4, NIB><<<grid, blk, 0, s>>>(xi, yo, idx, q, g); break;
+    }
+    ACTNN_RETURN_LAUNCH_STATUS();
+  }
   const int rb = pick_rows(g.Ho, g.Wo, 1024, need);
   if (rb > 0 && aligned16(x) && (!NIB || g.Wo % 2 == 0)) {
     const int bands = (g.Ho + rb - 1) / rb;
     if (planes * bands <= 0x7fffffffLL) {
       const dim3 grid((unsigned)(planes * bands)), blk(kThreads);
-      const T* xi = static_cast<const T*>(x);
-      T* yo = static_cast<T*>(y);
-      const int64_t tin = planes * g.H * g.W;
-      switch (preset_of(g)) {
-        case 1: max_pool2d_forward_lds_kernel<T, 1, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, tin, g, rb, bands); break;
-        case 2: max_pool2d_forward_lds_kernel<T, 2, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, tin, g, rb, bands); break;
-        case 3: max_pool2d_forward_lds_kernel<T, 3, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, tin, g, rb, bands); break;
-        default: max_pool2d_forward_lds_kernel<T, 0, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, tin, g, rb, bands); break;
-      }
+      max_pool2d_forward_lds_kernel<T, NIB><<<grid, blk, need(rb), s>>>(
+          static_cast<const T*>(x), static_cast<T*>(y), idx, planes * g.H * g.W, g, rb, bands);
       ACTNN_RETURN_LAUNCH_STATUS();
     }
   }
@@ -631,21 +947,34 @@ int launch_bwd(const void* gout, const int8_t* idx, void* gin, int64_t total, co
       ACTNN_RETURN_LAUNCH_STATUS();
     }
   }
+  const int preset = preset_of(g);
+  DirectGeom q;
+  const bool s1 = preset == 3;                           // threads: kStrip pixels of a column, or 2x2 pixels
+  if (preset != 0 && (!s1 || (g.Ho == g.H && g.Wo == g.W)) && total <= 0x7fffffffLL && planes * g.Ho * g.Wo <= 0x7fffffffLL &&
+      direct_geometry(planes, s1 ? (g.H + kStrip - 1) / kStrip : (g.H + 1) / 2, s1 ? g.W : (g.W + 1) / 2, q)) {
+    const dim3 grid = direct_grid(q), blk(kThreads);
+    const T* go = static_cast<const T*>(gout);
+    T* gi = static_cast<T*>(gin);
+    auto launch = [&](auto nt) {
+      constexpr bool NT = decltype(nt)::value;
+      switch (preset) {
+        case 1: max_pool2d_backward_direct_s2_kernel<T, 3, 1, NIB, NT><<<grid, blk, 0, s>>>(go, idx, gi, q, g); break;
+        case 2: max_pool2d_backward_direct_s2_kernel<T, 2, 0, NIB, NT><<<grid, blk, 0, s>>>(go, idx, gi, q, g); break;
+        case 3: max_pool2d_backward_direct_s1_kernel<T, NIB, NT><<<grid, blk, 0, s>>>(go, idx, gi, q, g); break;
+        default: max_pool2d_backward_direct_s2_kernel<T, 3, 0, NIB, NT><<<grid, blk, 0, s>>>(go, idx, gi, q, g); break;
+      }
+    };
+    if (stream_results(total * (int64_t)sizeof(T))) launch(std::true_type());
+    else launch(std::false_type());
+    ACTNN_RETURN_LAUNCH_STATUS();
+  }
   const int rb = pick_rows(g.H, g.W, 2048, need);
   if (rb > 0 && aligned16(gout) && aligned16(idx)) {
     const int bands = (g.H + rb - 1) / rb;
     if (planes * bands <= 0x7fffffffLL) {
       const dim3 grid((unsigned)(planes * bands)), blk(kThreads);
-      const T* go = static_cast<const T*>(gout);
-      T* gi = static_cast<T*>(gin);
-      const int64_t tout = planes * g.Ho * g.Wo;
-      const int orows = out_rows(rb);
-      switch (preset_of(g)) {
-        case 1: max_pool2d_backward_lds_kernel<T, 1, NIB><<<grid, blk, need(rb), s>>>(go, idx, gi, tout, g, rb, bands, orows); break;
-        case 2: max_pool2d_backward_lds_kernel<T, 2, NIB><<<grid, blk, need(rb), s>>>(go, idx, gi, tout, g, rb, bands, orows); break;
-        case 3: max_pool2d_backward_lds_kernel<T, 3, NIB><<<grid, blk, need(rb), s>>>(go, idx, gi, tout, g, rb, bands, orows); break;
-        default: max_pool2d_backward_lds_kernel<T, 0, NIB><<<grid, blk, need(rb), s>>>(go, idx, gi, tout, g, rb, bands, orows); break;
-      }
+      max_pool2d_backward_lds_kernel<T, NIB><<<grid, blk, need(rb), s>>>(
+          static_cast<const T*>(gout), idx, static_cast<T*>(gin), planes * g.Ho * g.Wo, g, rb, bands, out_rows(rb));
       ACTNN_RETURN_LAUNCH_STATUS();
     }
   }
@@ -794,7 +1123,8 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_forward_cl_window_kernel(
       const T* base = img + ((int64_t)(a - k.PH) * g.W + (b - k.PW)) * (int64_t)C;
       // pixels that no other window reads (every pixel of a 2x2 stride-2 window, the centre of a 3x3
       // stride-2 one) are streamed; the others are read again by the neighbours and stay cached
-      const bool once = PRESET == 2 || (PRESET == 1 && a == 1 && b == 1);   // (constant after unrolling)
+      // (constant after unrolling; without padding the pixel at 1, 1 is the centre as well)
+      const bool once = PRESET == 2 || ((PRESET == 1 || PRESET == 4) && a == 1 && b == 1);
       raw[a * KW + b] = inside ? (once ? load16_nt(base + lane) : load16(base + lane)) : u32x4{fill, fill, fill, fill};
     }
   float best[E];
@@ -860,23 +1190,24 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_kernel(
   narrow_chunk<T, E>(gin + pix * C + c, acc);
 }
 
-// Backward for the stride-2 windows of the stem / VGG-style layers (3x3 pad 1 and 2x2 pad 0, H and W
-// even): a thread owns the 2x2 block of input pixels (2a.., 2b..) of one chunk of channels.  The windows
-// that reach the block are (a..a+1) x (b..b+1) (3x3) or (a, b) alone (2x2): one (gradient, index) load
-// per input pixel where the general kernel needs 2.25 (3x3).  Every pixel adds its windows in the
+// Backward for the stride-2 windows (3x3 pad 1 or 0, 2x2 pad 0; planes of any size, EVEN: H = 2 Ho and
+// W = 2 Wo): a thread owns the 2x2 block of input pixels (2a.., 2b..) of one chunk of channels.  The
+// windows that reach the block are 2x2 of them (3x3) or one (2x2): one (gradient, index) load per
+// input pixel where the general kernel needs 2.25 (3x3).  Every pixel adds its windows in the
 // general kernel's order (rows, then columns), hence the same bits.  grad_in is written once and
 // not read: streamed stores (measured 0.104 -> 0.079 ms on f16 [256,64,112,112]).
-template <typename T, int K, int P, bool NIB>
+template <typename T, int K, int P, bool NIB, bool EVEN>
 __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
     const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, ClGeom q, PoolGeom g) {
   constexpr int E = PoolChunk<T>::kElems;
-  constexpr int NWIN = K == 3 ? 2 : 1;
+  using CW = CellWindows<K, P>;
+  constexpr int NWIN = CW::kCount, J0 = CW::kFirst;
   constexpr uint64_t kNone = ~uint64_t(0);             // fields that match no window position (K * K < 15)
   const ClAt at = cl_at(q);                            // rows and columns of windows
   if (!at.live) return;
   const uint32_t C = q.cpp * E;
-  const int64_t image_o = (int64_t)at.n * q.per_image * E;
-  const uint32_t lane_o = at.i * E;                    // window (row, col) of this chunk inside the image
+  const int64_t image_o = (int64_t)at.n * g.Ho * g.Wo * C;
+  const uint32_t lane_o = (at.row * (uint32_t)g.Wo + at.col) * C + at.chunk * E;   // window (row, col) of this chunk in the image
   const T* gimg = gout + image_o;
   const int8_t* iimg = idx + IndexFields<NIB>::byte_of(image_o);
   u32x4 raw[NWIN][NWIN];
@@ -885,8 +1216,8 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
   for (int j = 0; j < NWIN; ++j)
 #pragma unroll
     for (int t = 0; t < NWIN; ++t) {
-      const bool inside = at.row + j < (uint32_t)g.Ho && at.col + t < (uint32_t)g.Wo;
-      const int64_t step = ((int64_t)j * g.Wo + t) * C;              // uniform
+      const bool inside = at.row + (J0 + j) < (uint32_t)g.Ho && at.col + (J0 + t) < (uint32_t)g.Wo;   // (-1 wraps)
+      const int64_t step = ((int64_t)(J0 + j) * g.Wo + (J0 + t)) * C;              // uniform
       raw[j][t] = inside ? load16(gimg + step + lane_o) : u32x4{0, 0, 0, 0};
       fields[j][t] = inside ? IndexFields<NIB>::template load<E>(iimg + IndexFields<NIB>::byte_of(step), (int64_t)lane_o) : kNone;
     }
@@ -903,14 +1234,14 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
     for (int t = 0; t < NWIN; ++t) {
       float v[E];
       raw_widen_chunk<T, E>(raw[j][t], v);
-      // input row 2a + rr sits at window row kh = rr + P - 2j of window row a + j; columns alike
+      // input row 2a + rr sits at window row kh = rr + P - 2 (J0 + j) of window row a + J0 + j; columns alike
 #pragma unroll
       for (int rr = 0; rr < 2; ++rr) {
-        const int kh = rr + P - 2 * j;
+        const int kh = rr + P - 2 * (J0 + j);
         if (kh < 0 || kh >= K) continue;
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc) {
-          const int kw = cc + P - 2 * t;
+          const int kw = cc + P - 2 * (J0 + t);
           if (kw < 0 || kw >= K) continue;
 #pragma unroll
           for (int e = 0; e < E; ++e)
@@ -925,7 +1256,44 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
   for (int rr = 0; rr < 2; ++rr)
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc)
-      narrow_chunk_nt<T, E>(out + ((int64_t)rr * g.W + cc) * C + lane_in, acc[rr][cc]);
+      if (EVEN || (2 * at.row + rr < (uint32_t)g.H && 2 * at.col + cc < (uint32_t)g.W))
+        narrow_chunk_nt<T, E>(out + ((int64_t)rr * g.W + cc) * C + lane_in, acc[rr][cc]);
+}
+
+// Backward for 3x3 stride 1 pad 1: one pixel per thread, the loads of its nine windows issued together.
+template <typename T, bool NIB>
+__global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s1_kernel(
+    const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, ClGeom q, PoolGeom g) {
+  constexpr int E = PoolChunk<T>::kElems;
+  const ClAt at = cl_at(q);
+  if (!at.live) return;
+  const uint32_t C = q.cpp * E;
+  const int64_t image = (int64_t)at.n * g.H * g.W * C;         // (Ho = H, Wo = W)
+  const uint32_t lane = at.i * E;
+  const T* gimg = gout + image;
+  const int8_t* iimg = idx + IndexFields<NIB>::byte_of(image);
+  u32x4 raw[9];
+  uint64_t fields[9];
+#pragma unroll
+  for (int p = 0; p < 9; ++p) {                                // window (row - 1 + j, col - 1 + t) sees the pixel at (2 - j, 2 - t)
+    const int j = p / 3, t = p % 3;
+    const bool inside = at.row + (j - 1) < (uint32_t)g.H && at.col + (t - 1) < (uint32_t)g.W;
+    const int64_t step = ((int64_t)(j - 1) * g.W + (t - 1)) * C;
+    raw[p] = inside ? load16(gimg + step + lane) : u32x4{0, 0, 0, 0};
+    fields[p] = inside ? IndexFields<NIB>::template load<E>(iimg + IndexFields<NIB>::byte_of(step), (int64_t)lane) : ~uint64_t(0);
+  }
+  float acc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = 0.0f;
+#pragma unroll
+  for (int p = 0; p < 9; ++p) {
+    float v[E];
+    raw_widen_chunk<T, E>(raw[p], v);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (IndexFields<NIB>::get(fields[p], e) == 8 - p) acc[e] += v[e];
+  }
+  narrow_chunk_nt<T, E>(gin + image + lane, acc);
 }
 
 // thread positions for rows x cols pixels per image; false when an image is too large for 32-bit offsets
@@ -972,19 +1340,25 @@ int launch_cl(bool forward, const void* a, const int8_t* idx_in, int8_t* idx_out
       switch (p) {
         case 1: max_pool2d_forward_cl_window_kernel<T, 1, NIB><<<grid, blk, 0, s>>>(xi, yo, idx_out, q, g); break;
         case 2: max_pool2d_forward_cl_window_kernel<T, 2, NIB><<<grid, blk, 0, s>>>(xi, yo, idx_out, q, g); break;
-        default: max_pool2d_forward_cl_window_kernel<T, 3, NIB><<<grid, blk, 0, s>>>(xi, yo, idx_out, q, g); break;
+        case 3: max_pool2d_forward_cl_window_kernel<T, 3, NIB><<<grid, blk, 0, s>>>(xi, yo, idx_out, q, g); break;
+        default: max_pool2d_forward_cl_window_kernel<T, 4, NIB><<<grid, blk, 0, s>>>(xi, yo, idx_out, q, g); break;
       }
     } else {
       max_pool2d_forward_cl_kernel<T, NIB><<<dim3(xcd_grid(blocks)), dim3(kThreads), 0, s>>>(xi, yo, idx_out, chunks, cpp, C, g);
     }
-  } else if ((p == 1 || p == 2) && g.H == 2 * g.Ho && g.W == 2 * g.Wo && cl_geometry(N, g.Ho, g.Wo, cpp, image_elems, q)) {
+  } else if (p == 3 && g.Ho == g.H && g.Wo == g.W && cl_geometry(N, g.H, g.W, cpp, image_elems, q)) {
+    max_pool2d_backward_cl_s1_kernel<T, NIB><<<dim3(xcd_grid(q.blocks)), dim3(kThreads), 0, s>>>(
+        static_cast<const T*>(a), idx_in, static_cast<T*>(out), q, g);
+  } else if (p != 0 && p != 3 && cl_geometry(N, (g.H + 1) / 2, (g.W + 1) / 2, cpp, image_elems, q)) {
     const dim3 grid(xcd_grid(q.blocks)), blk(kThreads);
-    if (p == 1)
-      max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB><<<grid, blk, 0, s>>>(
-          static_cast<const T*>(a), idx_in, static_cast<T*>(out), q, g);
-    else
-      max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB><<<grid, blk, 0, s>>>(
-          static_cast<const T*>(a), idx_in, static_cast<T*>(out), q, g);
+    const T* go = static_cast<const T*>(a);
+    T* gi = static_cast<T*>(out);
+    const bool even = g.H == 2 * g.Ho && g.W == 2 * g.Wo;
+    if (p == 1 && even) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, true><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    else if (p == 1) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    else if (p == 2 && even) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, true><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    else if (p == 2) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    else max_pool2d_backward_cl_s2_kernel<T, 3, 0, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
   } else {
     max_pool2d_backward_cl_kernel<T, NIB><<<dim3(xcd_grid(blocks)), dim3(kThreads), 0, s>>>(
         static_cast<const T*>(a), idx_in, static_cast<T*>(out), chunks, cpp, C, g);

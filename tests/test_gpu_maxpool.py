@@ -215,3 +215,39 @@ def test_channels_last_stride2_backward_adds_in_the_order_of_the_default_layout(
     tol = 1e-5 if dtype == torch.float32 else 2e-2
     # torch picks the first maximum too, so the sums hold the same terms
     assert torch.allclose(gin_cl.float(), xr.grad.float(), atol=tol, rtol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("k,s,p", [((3, 3), (2, 2), (1, 1)), ((3, 3), (2, 2), (0, 0)), ((2, 2), (2, 2), (0, 0)),
+                                   ((3, 3), (1, 1), (1, 1))])
+@pytest.mark.parametrize("shape", [(1, 16, 3, 3), (2, 8, 4, 6), (2, 8, 5, 4), (1, 24, 9, 13), (3, 16, 13, 6), (1, 8, 16, 65)])
+@pytest.mark.parametrize("channels_last", [False, True])
+@pytest.mark.parametrize("nibble", [False, True])
+def test_preset_windows_on_planes_of_any_size(dtype, k, s, p, shape, channels_last, nibble):
+    """Edges of the direct kernels: odd extents, windows that end inside the plane, strips of 4 rows with a
+    remainder, bytes that hold outputs of two rows.  Integers with ties: exact against the oracle."""
+    x = torch.randint(-2, 3, shape, generator=torch.Generator().manual_seed(sum(shape))).to(dtype)
+    out_o, idx_o = pool.max_pool2d_forward(x.float().numpy(), k, s, p)
+    g = torch.randint(-3, 4, out_o.shape, generator=torch.Generator().manual_seed(1)).to(dtype)
+    gin_o = pool.max_pool2d_backward(g.float().numpy(), idx_o, shape, k, s, p)
+    fmt = torch.channels_last if channels_last else torch.contiguous_format
+    y, idx = ext_q.max_pool2d_forward(x.to(DEV).contiguous(memory_format=fmt), k, s, p, (1, 1), nibble)
+    assert np.array_equal(y.float().cpu().numpy(), out_o)
+    if not nibble:
+        assert np.array_equal(idx.cpu().numpy(), idx_o)
+    cl = ext_q.pool_takes_channels_last(x.to(DEV).contiguous(memory_format=fmt))
+    gin = ext_q.max_pool2d_backward(g.to(DEV).contiguous(memory_format=fmt), idx, shape, k, s, p, cl)
+    assert np.array_equal(gin.float().cpu().numpy(), gin_o)
+
+
+@pytest.mark.parametrize("k,s,p", [((3, 3), (2, 2), (0, 0)), ((3, 3), (1, 1), (1, 1))])
+def test_large_results_are_streamed_and_equal(k, s, p):
+    # above 128 MB the backward pass stores past the caches: the same values as in pieces below that
+    x = torch.randn(48, 64, 105, 105, device=DEV)
+    y, idx = ext_q.max_pool2d_forward(x, k, s, p, (1, 1))
+    g = torch.randn_like(y)
+    whole = ext_q.max_pool2d_backward(g, idx, x.shape, k, s, p)
+    assert whole.numel() * 4 > 128 << 20
+    for i in range(0, 48, 16):
+        part = ext_q.max_pool2d_backward(g[i:i + 16], idx[i:i + 16], x[i:i + 16].shape, k, s, p)
+        assert torch.equal(part, whole[i:i + 16])
