@@ -4,8 +4,7 @@
 // t = 16*j + k of a block is bit j of the block's word k (16 int32 words per block).  Lane j
 // of a 32-lane half-wave therefore owns 16 contiguous elements; two blocks fill a 32-bit
 // register per lane and one 32x32 bit transpose leaves the 32 mask words of the two blocks in
-// lanes 0..31, stored as one contiguous 128-byte run.  A 256-thread block covers 16 mask
-// blocks (8192 elements).
+// lanes 0..31, stored as one contiguous 128-byte run.
 #include "device_utils.h"
 
 namespace actnn {
@@ -13,21 +12,19 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaskBlock = 512;
-constexpr int kMaskBlocksPerBlock = (kThreads / 32) * 2;   // 16
 
 enum class Op { kRelu, kDropout };
 
-// Forward.  OP selects the keep rule: x > 0 (ReLU) or Philox r16 >= threshold (Dropout).
+// The tensor's last n < 2048 elements (their mask blocks, fully materialised), by one block.
+// OP selects the keep rule: x > 0 (ReLU) or Philox r16 >= threshold (Dropout); elem_offset: index of
+// x[0] in the tensor.
 template <typename T, Op OP>
-__global__ __launch_bounds__(kThreads) void mask_forward_kernel(const T* __restrict__ x,
-                                                                T* __restrict__ y,
-                                                                int32_t* __restrict__ mask, int64_t n,
-                                                                int64_t n_mask_blocks, uint32_t thr,
-                                                                float keep_div, uint64_t seed,
-                                                                uint64_t offset, int64_t elem_offset,
-                                                                const T* __restrict__ add = nullptr) {
+ACTNN_DEV void mask_forward_rest(const T* __restrict__ x, T* __restrict__ y, int32_t* __restrict__ mask, int64_t n,
+                                 uint32_t thr, float keep_div, uint64_t seed, uint64_t offset,
+                                 int64_t elem_offset, const T* __restrict__ add) {
   const uint32_t lane = threadIdx.x & 31;
-  const int64_t mb0 = (int64_t)blockIdx.x * kMaskBlocksPerBlock + (threadIdx.x >> 5) * 2;
+  const int64_t mb0 = (threadIdx.x >> 5) * 2;
+  const int64_t n_mask_blocks = (n + kMaskBlock - 1) / kMaskBlock;
   uint32_t acc = 0;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
@@ -90,13 +87,11 @@ __global__ __launch_bounds__(kThreads) void mask_forward_kernel(const T* __restr
 }
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void mask_backward_kernel(const T* __restrict__ gout,
-                                                                 const int32_t* __restrict__ mask,
-                                                                 T* __restrict__ gin, int64_t n,
-                                                                 int64_t n_mask_blocks, float keep_div,
-                                                                 bool divide, const T* __restrict__ acc = nullptr) {
+ACTNN_DEV void mask_backward_rest(const T* __restrict__ gout, const int32_t* __restrict__ mask, T* __restrict__ gin,
+                                  int64_t n, float keep_div, bool divide, const T* __restrict__ acc) {
   const uint32_t lane = threadIdx.x & 31;
-  const int64_t mb0 = (int64_t)blockIdx.x * kMaskBlocksPerBlock + (threadIdx.x >> 5) * 2;
+  const int64_t mb0 = (threadIdx.x >> 5) * 2;
+  const int64_t n_mask_blocks = (n + kMaskBlock - 1) / kMaskBlock;
   uint32_t w = 0;
   if (mb0 + (lane >> 4) < n_mask_blocks) w = (uint32_t)mask[mb0 * 16 + lane];
   const uint32_t rows = transpose32(w, lane);       // bits 16*r + k: keep flag of element 16*lane + k of block r
@@ -142,31 +137,33 @@ __global__ __launch_bounds__(kThreads) void mask_backward_kernel(const T* __rest
 }
 
 // ---------------------------------------------------------------------------------------------
-// 16-bit element types: whole-line streaming variant.  A wave handles 4 mask blocks (2048
-// elements) with four wave-wide 16-byte non-temporal loads and stores, so that HBM sees only whole
-// cache lines.  Lane l then holds elements 8l..8l+7 of each block, i.e. half of the 16 elements a
-// mask row belongs to: lane pairs swap their 8-bit halves (one DPP move) so that the even lanes
-// hold the rows of blocks A|B and the odd lanes those of C|D, two interleaved 32x32 bit
-// transposes turn rows into mask words, and the 64 words leave as one 256-byte store.
-constexpr int kTileElems = 4 * kMaskBlock;        // elements per wave and iteration
+// Whole-line streaming.  A wave handles 4 mask blocks (2048 elements) with wave-wide 16-byte loads and
+// stores, so that every instruction covers whole cache lines (a lane that owned the 16 contiguous
+// elements of a mask row came back to its line four times in fp32).  What is left of the tensor (< 2048
+// elements) is the last block's, in the same launch.  Bound by memory: fp32 [256, 100352] 34 us forward and
+// 34 us backward (6 TB/s; 54 and 54 us with a lane per mask row), bf16 [362, 122467] 31 + 30 us (37 + 36 us with
+// the remainder in a launch of its own).
+constexpr int kTileElems = 4 * kMaskBlock;        // elements per wave
 constexpr int kTilesPerBlock = kThreads / 64;
+
+struct RestArgs {                                 // the last block's part
+  int64_t tiles;                                  // whole tiles before it
+  int64_t tile_blocks;                            // blocks that hold them
+  int rest;                                       // elements behind them (0: there is no such block)
+};
 
 // MINMAX: also write the minimum and maximum of every group of 256 consecutive outputs (the lower
 // and upper 32 lanes of each load own one group each) - what actnn_minimax returns for the output
 // viewed as rows of 256, for a consumer that quantises it next.
 // ADD: the rule is applied to x + add, rounded to T as the tensor addition it replaces rounds it
 // (the closing `relu(out + identity)` of a residual block in one pass over the two operands).
-template <typename T, Op OP, bool MINMAX = false, bool ADD = false>
-__global__ __launch_bounds__(kThreads) void mask_forward16_kernel(const T* __restrict__ x, T* __restrict__ y,
-                                                                  int32_t* __restrict__ mask, int64_t tiles,
-                                                                  uint32_t thr, float keep_div,
-                                                                  uint64_t seed, uint64_t offset,
-                                                                  T* __restrict__ mn = nullptr,
-                                                                  T* __restrict__ mx = nullptr,
-                                                                  const T* __restrict__ add = nullptr) {
+// 16-bit element types: lane l holds elements 8l..8l+7 of each block, i.e. half of the 16 elements a
+// mask row belongs to (rows_to_word).
+template <typename T, Op OP, bool MINMAX, bool ADD>
+ACTNN_DEV void mask_forward_tile(const T* __restrict__ x, T* __restrict__ y, int32_t* __restrict__ mask, int64_t tile,
+                                 uint32_t thr, float keep_div, uint64_t seed, uint64_t offset,
+                                 T* __restrict__ mn, T* __restrict__ mx, const T* __restrict__ add) {
   const uint32_t lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
-  if (tile >= tiles) return;                       // whole waves leave together
   const int64_t e0 = tile * kTileElems + lane * 8;
   float v[4][8];
 #pragma unroll
@@ -217,18 +214,146 @@ __global__ __launch_bounds__(kThreads) void mask_forward16_kernel(const T* __res
   mask[tile * 64 + (lane & 1u) * 32 + (lane >> 1)] = (int32_t)w;
 }
 
+// fp32: a wave-wide load is half a mask block, lane l elements 4l..4l+3, so the quad Q = l / 4 holds mask
+// row Q (first half of a block) or 16 + Q (second half) and lane l its bits 4 (l & 3) .. + 3.  The four
+// lanes of a quad hand each other their nibbles - each ends with the two 16-bit rows of one half u = bit
+// 1 of its index and of the blocks 2h, 2h + 1, h = bit 0 of its index - and the two interleaved 32x32 bit
+// transposes (the matrices of the even and of the odd lanes) run over the remaining lane bits: row
+// bit 4 is lane bit 1, row bits 3..0 are lane bits 5..2.
+ACTNN_DEV uint32_t transpose32_quads(uint32_t x, uint32_t lane) {
+  auto stage = [&](uint32_t p, int s, uint32_t m, bool hi) {
+    const uint32_t u = __builtin_amdgcn_alignbit(p, p, hi ? s : 32 - s);
+    const uint32_t sel = hi ? m : ~m;
+    x = (x & sel) | (u & ~sel);
+  };
+  stage(lane_xor<2>(x), 16, 0xFFFF0000u, (lane & 2u) != 0);
+  stage((uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane ^ 32u) << 2), (int)x), 8, 0xFF00FF00u, (lane & 32u) != 0);
+  stage(lane_xor<16>(x), 4, 0xF0F0F0F0u, (lane & 16u) != 0);
+  stage(lane_xor<8>(x), 2, 0xCCCCCCCCu, (lane & 8u) != 0);
+  stage(lane_xor<4>(x), 1, 0xAAAAAAAAu, (lane & 4u) != 0);
+  return x;
+}
+// where the lane's word lies in the tile's 64: word p % 16 of block 2h + p / 16, p as the lane bits say
+ACTNN_DEV uint32_t quads_word_at(uint32_t lane) {
+  const uint32_t p = ((lane & 2u) << 3) | ((lane & 32u) >> 2) | ((lane & 16u) >> 2) | ((lane & 8u) >> 2) | ((lane & 4u) >> 2);
+  return (lane & 1u) * 32 + p;
+}
+// nib[i]: the lane's four keep bits of half block i (blocks i / 2, halves i & 1) -> its mask word
+ACTNN_DEV uint32_t nibbles_to_word(const uint32_t (&nib)[8], uint32_t lane) {
+  const int sh = 4 * (int)(lane & 3u);
+  uint32_t pair[2][2];                             // [h][u]: bits of blocks 2h | 2h + 1 of half u
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) pair[h][u] = (nib[4 * h + u] | (nib[4 * h + 2 + u] << 16)) << sh;
+  const bool h = lane & 1u, u = lane & 2u;
+  uint32_t half[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) half[k] = (h ? pair[1][k] : pair[0][k]) | lane_xor<1>(h ? pair[0][k] : pair[1][k]);
+  const uint32_t row = (u ? half[1] : half[0]) | lane_xor<2>(u ? half[0] : half[1]);
+  return transpose32_quads(row, lane);
+}
+// inverse
+ACTNN_DEV void word_to_nibbles(uint32_t w, uint32_t lane, uint32_t (&nib)[8]) {
+  const int row = (int)transpose32_quads(w, lane);
+  const int sh = 4 * (int)(lane & 3u);
+  uint32_t quad[4];                                // rows of the quad's lanes: [2u + h]
+  quad[0] = (uint32_t)__builtin_amdgcn_update_dpp(0, row, 0x00, 0xF, 0xF, true);
+  quad[1] = (uint32_t)__builtin_amdgcn_update_dpp(0, row, 0x55, 0xF, 0xF, true);
+  quad[2] = (uint32_t)__builtin_amdgcn_update_dpp(0, row, 0xAA, 0xF, 0xF, true);
+  quad[3] = (uint32_t)__builtin_amdgcn_update_dpp(0, row, 0xFF, 0xF, 0xF, true);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) nib[i] = (quad[2 * (i & 1) + (i >> 2)] >> (16 * ((i >> 1) & 1) + sh)) & 0xfu;
+}
+
+ACTNN_DEV void store_result(float* p, u32x4 v, bool stream) {
+  if (stream) store16_nt(p, v);
+  else store16(p, v);
+}
+
+template <Op OP, bool ADD>
+ACTNN_DEV void mask_forward_tile32(const float* __restrict__ x, float* __restrict__ y, int32_t* __restrict__ mask,
+                                   int64_t tile, uint32_t thr, float keep_div, uint64_t seed, uint64_t offset,
+                                   const float* __restrict__ add, bool stream) {
+  const uint32_t lane = threadIdx.x & 63;
+  const int64_t e0 = tile * kTileElems + lane * 4;
+  u32x4 v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = load16_nt(x + e0 + i * 256);
+  if (ADD) {
+    u32x4 a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = load16_nt(add + e0 + i * 256);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[i][k] = as_uint(as_float(v[i][k]) + as_float(a[i][k]));
+  }
+  uint32_t nib[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    uint32_t na[2], nb[2];                         // draws of half blocks i and i + 1, two to a word
+    if (OP == Op::kDropout) {
+      // lanes 2j and 2j + 1 hold the halves of one octet: the even lane evaluates the octet of half
+      // block i, the odd lane that of half block i + 1, and they hand each other the words they do not use
+      const bool odd = lane & 1u;
+      const Philox4 r = philox_at((uint64_t)((e0 + (i + (odd ? 1 : 0)) * 256) >> 3), seed, offset);
+      const uint32_t nx = lane_xor<1>(r.x), ny = lane_xor<1>(r.y), nz = lane_xor<1>(r.z), nw = lane_xor<1>(r.w);
+      na[0] = odd ? nz : r.x;
+      na[1] = odd ? nw : r.y;
+      nb[0] = odd ? r.z : nx;
+      nb[1] = odd ? r.w : ny;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      nib[i + q] = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float f = as_float(v[i + q][k]);
+        bool keep;
+        if (OP == Op::kRelu) {
+          keep = f > 0.0f;
+          v[i + q][k] = keep ? as_uint(f) : 0u;
+        } else {
+          keep = (((q ? nb : na)[k >> 1] >> (16 * (k & 1))) & 0xffffu) >= thr;
+          v[i + q][k] = keep ? as_uint(f / keep_div) : 0u;
+        }
+        nib[i + q] |= (uint32_t)keep << k;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) store_result(y + e0 + i * 256, v[i], stream);
+  mask[tile * 64 + quads_word_at(lane)] = (int32_t)nibbles_to_word(nib, lane);
+}
+
+template <typename T, Op OP, bool MINMAX = false, bool ADD = false>
+__global__ __launch_bounds__(kThreads) void mask_forward_kernel(const T* __restrict__ x, T* __restrict__ y,
+                                                                int32_t* __restrict__ mask, RestArgs part,
+                                                                uint32_t thr, float keep_div, uint64_t seed,
+                                                                uint64_t offset, bool stream,
+                                                                T* __restrict__ mn = nullptr,
+                                                                T* __restrict__ mx = nullptr,
+                                                                const T* __restrict__ add = nullptr) {
+  if ((int64_t)blockIdx.x >= part.tile_blocks) {
+    const int64_t done = part.tiles * kTileElems;
+    mask_forward_rest<T, OP>(x + done, y + done, mask + done / 32, part.rest, thr, keep_div, seed, offset, done,
+                             ADD ? add + done : nullptr);
+    return;
+  }
+  const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
+  if (tile >= part.tiles) return;                  // whole waves leave together
+  if constexpr (sizeof(T) == 4) mask_forward_tile32<OP, ADD>(x, y, mask, tile, thr, keep_div, seed, offset, add, stream);
+  else mask_forward_tile<T, OP, MINMAX, ADD>(x, y, mask, tile, thr, keep_div, seed, offset, mn, mx, add);
+}
+
 // ACC: gin = acc + masked gradient (rounded to T as the tensor addition of the two rounds it): the
 // gradient that arrives at a residual block's input over the skip connection, masked and added to the
 // one from the block's first convolution in one pass.
-template <typename T, bool ACC = false>
-__global__ __launch_bounds__(kThreads) void mask_backward16_kernel(const T* __restrict__ gout,
-                                                                   const int32_t* __restrict__ mask,
-                                                                   T* __restrict__ gin, int64_t tiles,
-                                                                   float keep_div, bool divide,
-                                                                   const T* __restrict__ acc = nullptr) {
+template <typename T, bool ACC>
+ACTNN_DEV void mask_backward_tile(const T* __restrict__ gout, const int32_t* __restrict__ mask, T* __restrict__ gin,
+                                  int64_t tile, float keep_div, bool divide, const T* __restrict__ acc) {
   const uint32_t lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
-  if (tile >= tiles) return;
   const int64_t e0 = tile * kTileElems + lane * 8;
   float v[4][8];
 #pragma unroll
@@ -252,36 +377,78 @@ __global__ __launch_bounds__(kThreads) void mask_backward16_kernel(const T* __re
   }
 }
 
+template <bool ACC>
+ACTNN_DEV void mask_backward_tile32(const float* __restrict__ gout, const int32_t* __restrict__ mask,
+                                    float* __restrict__ gin, int64_t tile, float keep_div, bool divide,
+                                    const float* __restrict__ acc, bool stream) {
+  const uint32_t lane = threadIdx.x & 63;
+  const int64_t e0 = tile * kTileElems + lane * 4;
+  const uint32_t word = (uint32_t)mask[tile * 64 + quads_word_at(lane)];
+  u32x4 v[8], a[ACC ? 8 : 1];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = load16_nt(gout + e0 + i * 256);
+  if (ACC) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[ACC ? i : 0] = load16_nt(acc + e0 + i * 256);
+  }
+  uint32_t nib[8];
+  word_to_nibbles(word, lane, nib);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float f = as_float(v[i][k]);
+      const bool keep = (nib[i] >> k) & 1u;
+      const float g = keep ? (divide ? f / keep_div : f) : 0.0f;
+      v[i][k] = as_uint(ACC ? as_float(a[ACC ? i : 0][k]) + g : g);
+    }
+    store_result(gin + e0 + i * 256, v[i], stream);
+  }
+}
+
+template <typename T, bool ACC = false>
+__global__ __launch_bounds__(kThreads) void mask_backward_kernel(const T* __restrict__ gout,
+                                                                 const int32_t* __restrict__ mask,
+                                                                 T* __restrict__ gin, RestArgs part,
+                                                                 float keep_div, bool divide, bool stream,
+                                                                 const T* __restrict__ acc = nullptr) {
+  if ((int64_t)blockIdx.x >= part.tile_blocks) {
+    const int64_t done = part.tiles * kTileElems;
+    mask_backward_rest<T>(gout + done, mask + done / 32, gin + done, part.rest, keep_div, divide,
+                          ACC ? acc + done : nullptr);
+    return;
+  }
+  const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
+  if (tile >= part.tiles) return;
+  if constexpr (sizeof(T) == 4) mask_backward_tile32<ACC>(gout, mask, gin, tile, keep_div, divide, acc, stream);
+  else mask_backward_tile<T, ACC>(gout, mask, gin, tile, keep_div, divide, acc);
+}
+
+// -> blocks of the launch, 0 when there are too many for a grid
+inline int64_t split_tensor(int64_t n, RestArgs& part) {
+  part.tiles = n / kTileElems;
+  part.tile_blocks = (part.tiles + kTilesPerBlock - 1) / kTilesPerBlock;
+  part.rest = (int)(n - part.tiles * kTileElems);
+  const int64_t blocks = part.tile_blocks + (part.rest > 0 ? 1 : 0);
+  return blocks > 0x7fffffffLL ? 0 : blocks;
+}
+
 template <typename T, Op OP>
 int launch_forward(const void* x, void* y, int32_t* mask, int64_t n, uint32_t thr, float keep_div,
                    uint64_t seed, uint64_t offset, hipStream_t s, const void* add = nullptr) {
   const T* xi = static_cast<const T*>(x);
   const T* ai = static_cast<const T*>(add);
   T* yo = static_cast<T*>(y);
-  int64_t done = 0;                               // elements handled by the whole-line kernel
-  if (sizeof(T) == 2) {
-    const int64_t tiles = n / kTileElems;
-    const int64_t tblocks = (tiles + kTilesPerBlock - 1) / kTilesPerBlock;
-    if (tblocks > 0x7fffffffLL) return ACTNN_EINVAL;
-    if (tiles > 0) {
-      if (ai)
-        mask_forward16_kernel<T, OP, false, true><<<dim3((unsigned)tblocks), dim3(kThreads), 0, s>>>(
-            xi, yo, mask, tiles, thr, keep_div, seed, offset, nullptr, nullptr, ai);
-      else
-        mask_forward16_kernel<T, OP><<<dim3((unsigned)tblocks), dim3(kThreads), 0, s>>>(
-            xi, yo, mask, tiles, thr, keep_div, seed, offset);
-    }
-    done = tiles * kTileElems;
-  }
-  const int64_t rest = n - done;
-  if (rest > 0) {
-    const int64_t nmb = (rest + kMaskBlock - 1) / kMaskBlock;
-    const int64_t blocks = (nmb + kMaskBlocksPerBlock - 1) / kMaskBlocksPerBlock;
-    if (blocks > 0x7fffffffLL) return ACTNN_EINVAL;
-    mask_forward_kernel<T, OP><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
-        xi + done, yo + done, mask + done / 32, rest, nmb, thr, keep_div, seed, offset, done,
-        ai ? ai + done : nullptr);
-  }
+  RestArgs part;
+  const int64_t blocks = split_tensor(n, part);
+  if (blocks == 0) return ACTNN_EINVAL;
+  const bool stream = stream_results(n * (int64_t)sizeof(T));
+  const dim3 grid((unsigned)blocks), blk(kThreads);
+  if (OP == Op::kRelu && ai)
+    mask_forward_kernel<T, Op::kRelu, false, true><<<grid, blk, 0, s>>>(xi, yo, mask, part, thr, keep_div, seed, offset,
+                                                                        stream, nullptr, nullptr, ai);
+  else
+    mask_forward_kernel<T, OP><<<grid, blk, 0, s>>>(xi, yo, mask, part, thr, keep_div, seed, offset, stream);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -291,29 +458,13 @@ int launch_backward(const void* gout, const int32_t* mask, void* gin, int64_t n,
   const T* go = static_cast<const T*>(gout);
   const T* ac = static_cast<const T*>(acc);
   T* gi = static_cast<T*>(gin);
-  int64_t done = 0;
-  if (sizeof(T) == 2) {
-    const int64_t tiles = n / kTileElems;
-    const int64_t tblocks = (tiles + kTilesPerBlock - 1) / kTilesPerBlock;
-    if (tblocks > 0x7fffffffLL) return ACTNN_EINVAL;
-    if (tiles > 0) {
-      if (ac)
-        mask_backward16_kernel<T, true><<<dim3((unsigned)tblocks), dim3(kThreads), 0, s>>>(go, mask, gi, tiles,
-                                                                                           keep_div, divide, ac);
-      else
-        mask_backward16_kernel<T><<<dim3((unsigned)tblocks), dim3(kThreads), 0, s>>>(go, mask, gi, tiles,
-                                                                                     keep_div, divide);
-    }
-    done = tiles * kTileElems;
-  }
-  const int64_t rest = n - done;
-  if (rest > 0) {
-    const int64_t nmb = (rest + kMaskBlock - 1) / kMaskBlock;
-    const int64_t blocks = (nmb + kMaskBlocksPerBlock - 1) / kMaskBlocksPerBlock;
-    if (blocks > 0x7fffffffLL) return ACTNN_EINVAL;
-    mask_backward_kernel<T><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
-        go + done, mask + done / 32, gi + done, rest, nmb, keep_div, divide, ac ? ac + done : nullptr);
-  }
+  RestArgs part;
+  const int64_t blocks = split_tensor(n, part);
+  if (blocks == 0) return ACTNN_EINVAL;
+  const bool stream = stream_results(n * (int64_t)sizeof(T));
+  const dim3 grid((unsigned)blocks), blk(kThreads);
+  if (ac) mask_backward_kernel<T, true><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide, stream, ac);
+  else mask_backward_kernel<T><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide, stream);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -371,18 +522,18 @@ extern "C" int actnn_relu_forward_minmax(const void* x, void* y, int32_t* mask, 
   if (n == 0) return ACTNN_OK;
   if (!x || !y || !mask || !mn || !mx) return ACTNN_EINVAL;
   if (!aligned16(x) || !aligned16(y)) return ACTNN_EALIGN;
-  const int64_t tiles = n / kTileElems;
-  const int64_t blocks = (tiles + kTilesPerBlock - 1) / kTilesPerBlock;
-  if (blocks > 0x7fffffffLL) return ACTNN_EINVAL;
+  RestArgs part;
+  const int64_t blocks = split_tensor(n, part);
+  if (blocks == 0) return ACTNN_EINVAL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)blocks), blk(kThreads);
   if (dtype == ACTNN_F16)
-    mask_forward16_kernel<__half, Op::kRelu, true><<<grid, blk, 0, s>>>(
-        static_cast<const __half*>(x), static_cast<__half*>(y), mask, tiles, 0u, 1.0f, 0, 0,
+    mask_forward_kernel<__half, Op::kRelu, true><<<grid, blk, 0, s>>>(
+        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0, true,
         static_cast<__half*>(mn), static_cast<__half*>(mx));
   else
-    mask_forward16_kernel<bf16_t, Op::kRelu, true><<<grid, blk, 0, s>>>(
-        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, tiles, 0u, 1.0f, 0, 0,
+    mask_forward_kernel<bf16_t, Op::kRelu, true><<<grid, blk, 0, s>>>(
+        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0, true,
         static_cast<bf16_t*>(mn), static_cast<bf16_t*>(mx));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
@@ -398,18 +549,18 @@ extern "C" int actnn_relu_add_forward(const void* x, const void* residual, void*
   if (n == 0) return ACTNN_OK;
   if (!x || !y || !mask) return ACTNN_EINVAL;
   if (!aligned16(x) || !aligned16(residual) || !aligned16(y)) return ACTNN_EALIGN;
-  const int64_t tiles = n / kTileElems;
-  const int64_t blocks = (tiles + kTilesPerBlock - 1) / kTilesPerBlock;
-  if (blocks > 0x7fffffffLL) return ACTNN_EINVAL;
+  RestArgs part;
+  const int64_t blocks = split_tensor(n, part);
+  if (blocks == 0) return ACTNN_EINVAL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)blocks), blk(kThreads);
   if (dtype == ACTNN_F16)
-    mask_forward16_kernel<__half, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
-        static_cast<const __half*>(x), static_cast<__half*>(y), mask, tiles, 0u, 1.0f, 0, 0,
+    mask_forward_kernel<__half, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
+        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0, true,
         static_cast<__half*>(mn), static_cast<__half*>(mx), static_cast<const __half*>(residual));
   else
-    mask_forward16_kernel<bf16_t, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
-        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, tiles, 0u, 1.0f, 0, 0,
+    mask_forward_kernel<bf16_t, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
+        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0, true,
         static_cast<bf16_t*>(mn), static_cast<bf16_t*>(mx), static_cast<const bf16_t*>(residual));
   ACTNN_RETURN_LAUNCH_STATUS();
 }

@@ -192,3 +192,27 @@ def test_relu_of_a_sum_rejects_bad_arguments():
     assert lib.actnn_relu_add_forward(*args(mn=mn.data_ptr(), mx=mn.data_ptr(), dtype=0)) != 0
     assert lib.actnn_relu_add_forward(*args(n=0)) == 0
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 511, 2047, 2048, 2049, 8191, 8192, 8193, 5 * 2048 + 513, 41 * 2048 + 1])
+def test_whole_tiles_and_remainder(dtype, n):
+    """A tensor is whole 2048-element tiles (four to a block) and a remainder of the same launch: both
+    operators, with the second operand, against torch bit for bit, the masks against the layout."""
+    torch.manual_seed(n)
+    x, r, g = (torch.randn(n).to(dtype) for _ in range(3))
+    x[::7] = 0.0
+    y, mask = ext_q.relu_add_forward(x.to(DEV), r.to(DEV))
+    total = x + r
+    keep = total > 0
+    assert torch.equal(y.cpu(), F.relu(total))
+    assert np.array_equal(mask.cpu().numpy(), layouts.mask_words(keep.numpy()))
+    masked = torch.where(keep, g, torch.zeros_like(g))
+    assert torch.equal(ext_q.relu_backward(g.to(DEV), mask).cpu(), masked)
+    assert torch.equal(ext_q.relu_backward_add(g.to(DEV), mask, x.to(DEV)).cpu(), x + masked)
+    torch.cuda.manual_seed(n)
+    offset = torch.cuda.default_generators[0].get_offset()
+    yd, md = ext_q.dropout_forward(x.to(DEV), 0.5)
+    drawn = philox.noise16(np.arange(n, dtype=np.uint64), n, offset) >= np.uint32(32768)
+    assert torch.equal(yd.cpu(), torch.where(torch.from_numpy(drawn), x * 2, torch.zeros_like(x)))   # / 0.5 is exact
+    assert np.array_equal(md.cpu().numpy(), layouts.mask_words(drawn))
