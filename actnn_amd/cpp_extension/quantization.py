@@ -225,6 +225,58 @@ def unpack_single_precision(data, bits, scale, min, N, num_groups, group_size):
 
 
 # ------------------------------------------------------------------------------------------
+# rows of any length in groups of 256, the last group padded with zeros
+# ------------------------------------------------------------------------------------------
+def quantize_rows_fixed(rows, bits, known_minmax, store_dtype):
+    """Contiguous [N, F] -> (packed, scale, mn), scale and mn [N, G, 1] in `store_dtype` (the rows' dtype, or
+    bfloat16 for fp32 rows): group_min_max and pack_single_precision of the zero-padded rows, and the
+    compact storage, from one read of the rows.  `known_minmax`: (mn, mx) [N * G] of whole groups."""
+    N, F = rows.shape
+    G = (F + 255) // 256
+    dev = rows.device
+    packed = torch.empty(single_packed_bytes(N, G, 256, bits), dtype=torch.int8, device=dev)
+    scale = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
+    mn_ptr = mx_ptr = None
+    if known_minmax is None:
+        mn = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
+    else:
+        rows = g.aligned(rows)
+        known_mn, known_mx = known_minmax
+        mn_ptr, mx_ptr = known_mn.data_ptr(), known_mx.data_ptr()
+        mn = known_mn.view(N, G, 1) if store_dtype == known_mn.dtype \
+            else torch.empty(N, G, 1, dtype=store_dtype, device=dev)
+    seed, offset = g.philox_args(dev)
+    with g.on_device(dev):
+        check(g.lib().actnn_quantize_fixed(
+            rows.data_ptr(), mn_ptr, mx_ptr, bits, scale.data_ptr(),
+            None if mn_ptr is not None and mn.data_ptr() == mn_ptr else mn.data_ptr(), packed.data_ptr(), seed, offset,
+            N, F, g.DTYPE_CODE[rows.dtype], g.DTYPE_CODE[store_dtype], g.stream_ptr(dev)), "quantize_fixed")
+    return packed, scale, mn
+
+
+def unpack_rows_fixed(packed, bits, scale, mn, N, F, dtype):
+    """Inverse of quantize_rows_fixed: [N, F] of `dtype`, nothing materialised for the padding."""
+    g.check_typed(packed, "data", torch.int8, 1)
+    g.check_float(scale, "scale", 3)
+    g.check_float(mn, "min", 3)
+    if 8 % bits != 0:
+        raise RuntimeError("unpack_single_precision: 8 % bits must be 0")          # .cu:375
+    if mn.dtype != scale.dtype:
+        raise RuntimeError("The type of min is not correct!")
+    G = (F + 255) // 256
+    if scale.numel() != N * G or mn.numel() != N * G:
+        raise RuntimeError("unpack_single_precision: shape mismatch")
+    if packed.numel() < single_packed_bytes(N, G, 256, bits) - 1:
+        raise RuntimeError("unpack_single_precision: packed stream is too short")
+    out = torch.empty(N, F, dtype=dtype, device=packed.device)
+    with g.on_device(packed.device):
+        check(g.lib().actnn_unpack_single_rows(
+            packed.data_ptr(), bits, scale.data_ptr(), mn.data_ptr(), out.data_ptr(), N, F, g.DTYPE_CODE[dtype],
+            g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)), "unpack_single_precision")
+    return out
+
+
+# ------------------------------------------------------------------------------------------
 # fused QLinear weight gradient (no counterpart among the reference's operators: it replaces
 # dequantize + grad_output.t().mm(input) of linear.backward, actnn/actnn/ops.py:407-421)
 # ------------------------------------------------------------------------------------------

@@ -160,6 +160,57 @@ template <typename T> ACTNN_DEV void raw8_zero(Raw8<T>& r) {
   r.a = (u32x4){0, 0, 0, 0};
   if constexpr (sizeof(T) == 4) r.b = (u32x4){0, 0, 0, 0};
 }
+// Rows of any length: 16 bytes at an address that is only a multiple of the element, and the first
+// `valid` of 8 elements (the others 0).  Global memory takes 16-byte accesses at any address; a lane that
+// straddles two lines costs a second one, where copying the rows to aligned ones cost two passes.
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+ACTNN_DEV u32x4 load16_any(const float* p) { return *reinterpret_cast<const u32x4_a4*>(p); }
+ACTNN_DEV u32x4 load16_any(const __half* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+ACTNN_DEV u32x4 load16_any(const bf16_t* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+ACTNN_DEV void store16_any(float* p, u32x4 v) { *reinterpret_cast<u32x4_a4*>(p) = v; }
+ACTNN_DEV void store16_any(__half* p, u32x4 v) { *reinterpret_cast<u32x4_a2*>(p) = v; }
+ACTNN_DEV void store16_any(bf16_t* p, u32x4 v) { *reinterpret_cast<u32x4_a2*>(p) = v; }
+// the elements of one 16-byte vector that lie in the row
+template <typename T> ACTNN_DEV u32x4 load16_part(const T* p, int valid) {
+  constexpr int E = 16 / sizeof(T);
+  u32x4 u = (u32x4){0, 0, 0, 0};
+  if (valid >= E) {
+    u = load16_any(p);
+  } else if (valid > 0) {
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < E - 1; ++k) {
+      if (k >= valid) continue;
+      if constexpr (sizeof(T) == 4) w[k] = reinterpret_cast<const uint32_t*>(p)[k];
+      else w[k / 2] |= (uint32_t)reinterpret_cast<const uint16_t*>(p)[k] << (16 * (k & 1));
+    }
+    u = (u32x4){w[0], w[1], w[2], w[3]};
+  }
+  return u;
+}
+template <typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
+  constexpr int E = 16 / sizeof(T);
+  if (valid >= E) {
+    store16_any(p, v);
+  } else if (valid > 0) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < E - 1; ++k) {
+      if (k >= valid) continue;
+      if constexpr (sizeof(T) == 4) reinterpret_cast<uint32_t*>(p)[k] = w[k];
+      else reinterpret_cast<uint16_t*>(p)[k] = (uint16_t)(w[k / 2] >> (16 * (k & 1)));
+    }
+  }
+}
+ACTNN_DEV void raw8_load_part(const float* p, int valid, Raw8<float>& r) {
+  r.a = load16_part(p, valid);
+  r.b = load16_part(p + 4, valid - 4);
+}
+ACTNN_DEV void raw8_load_part(const __half* p, int valid, Raw8<__half>& r) { r.a = load16_part(p, valid); }
+ACTNN_DEV void raw8_load_part(const bf16_t* p, int valid, Raw8<bf16_t>& r) { r.a = load16_part(p, valid); }
+// how many elements of a row of F lie at `at` and behind (capped: only small counts matter)
+ACTNN_DEV int part_of_row(int64_t F, int64_t at) { return F - at < 1024 ? (int)(F - at) : 1024; }
 ACTNN_DEV void raw8_widen(const Raw8<float>& r, float (&v)[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) { v[i] = as_float(r.a[i]); v[4 + i] = as_float(r.b[i]); }
@@ -222,6 +273,18 @@ ACTNN_DEV void store8(bf16_t* p, const float (&v)[8]) {
   store16(p, (u32x4){w[0], w[1], w[2], w[3]});
 }
 
+ACTNN_DEV u32x4 words_of8(const __half*, const float (&v)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = float_to_half_bits(v[2 * i]) | (float_to_half_bits(v[2 * i + 1]) << 16);
+  return (u32x4){w[0], w[1], w[2], w[3]};
+}
+ACTNN_DEV u32x4 words_of8(const bf16_t*, const float (&v)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+  return (u32x4){w[0], w[1], w[2], w[3]};
+}
 ACTNN_DEV void store8_nt(float* p, const float (&v)[8]) { store8(p, v); }  // fp32: 32 bytes per lane, plain
 ACTNN_DEV void store8_nt(__half* p, const float (&v)[8]) {
   uint32_t w[4];

@@ -19,6 +19,7 @@ namespace actnn {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kFixedGs = 256;           // group size of the one-pass kernel and of rows of any length
 
 template <typename T, bool DET>
 __global__ __launch_bounds__(kThreads) void scale_single_kernel(const T* __restrict__ mn,
@@ -39,7 +40,7 @@ __global__ __launch_bounds__(kThreads) void scale_single_kernel(const T* __restr
 // no 64-bit divisions per thread (they cost more instructions than the quantisation of the thread's
 // elements: 4-bit pack of bf16 [512,256,56,56] 0.198 -> 0.180 ms, unpack 0.173 -> 0.155 ms).
 struct SingleGeom {
-  int64_t N, G;
+  int64_t N, G, F;                 // F: elements a row of the tensor has (G * gs, or fewer: the last group is padded)
   int gs, chunks, chunk_shift;     // chunk_shift < 0: chunks is not a power of two
   int64_t rows;                    // ceil(N / (8 / bits))
   uint32_t per_row;                // G * chunks
@@ -141,7 +142,9 @@ __global__ __launch_bounds__(kThreads) void pack_single_kernel(
   }
 }
 
-template <typename T, int BITS>
+// ROWS: rows of any length at any address (the elements past a row's end are not written); their lines are
+// shared between waves, so the stores go through the cache.
+template <typename T, int BITS, bool ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_single_kernel(
     const int8_t* __restrict__ packed, const T* __restrict__ scale, const T* __restrict__ mn,
     T* __restrict__ out, SingleGeom q) {
@@ -166,16 +169,18 @@ __global__ __launch_bounds__(kThreads) void unpack_single_kernel(
           const uint32_t word = k < 4 ? w.x : w.y;
           v[k] = dq((word >> (8 * (k & 3) + ni * BITS)) & kMask);
         }
-        store8_nt(out + gi * gs + d0, v);
+        if constexpr (ROWS) store16_part(out + n * q.F + g * gs + d0, words_of8(out, v), part_of_row(q.F, g * gs + d0));
+        else store8_nt(out + gi * gs + d0, v);
       }
     }
   }
 }
 
 // ---------------------------------------------------------------------------- fp32 unpack: 4 elements per lane
-template <int BITS>
+// S: the type the scales and minima are stored in (bfloat16 in the compact form of an fp32 activation).
+template <typename S, int BITS, bool ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_single_f32_kernel(
-    const int8_t* __restrict__ packed, const float* __restrict__ scale, const float* __restrict__ mn,
+    const int8_t* __restrict__ packed, const S* __restrict__ scale, const S* __restrict__ mn,
     float* __restrict__ out, SingleGeom q) {
   constexpr int WPT = 8 / BITS;
   constexpr uint32_t kMask = (1u << BITS) - 1u;
@@ -191,11 +196,12 @@ __global__ __launch_bounds__(kThreads) void unpack_single_f32_kernel(
       const int64_t n = no * WPT + ni;
       if (n < N) {
         const int64_t gi = n * G + g;
-        const Dequant<float> dq(scale[gi], mn[gi]);
+        const Dequant<float> dq(Conv<S>::load(scale, gi), Conv<S>::load(mn, gi));
         u32x4 v;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = as_uint(dq((w >> (8 * k + ni * BITS)) & kMask));
-        store16_nt(out + gi * gs + d0, v);
+        if constexpr (ROWS) store16_part(out + n * q.F + g * gs + d0, v, part_of_row(q.F, g * gs + d0));
+        else store16_nt(out + gi * gs + d0, v);
       }
     }
   }
@@ -207,6 +213,7 @@ bool single_geometry(int64_t N, int64_t G, int64_t gs, int bits, int elems, Sing
   const int wpt = 8 / bits;
   q.N = N;
   q.G = G;
+  q.F = G * gs;
   q.gs = (int)gs;
   q.chunks = (int)(gs / elems);
   q.chunk_shift = -1;
@@ -239,10 +246,145 @@ int launch_pack_bits(int bits, const T* data, const T* mn, const T* scale, int8_
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
+// ---------------------------------------------------------------------------- groups of 256 in one pass
+// Minimum and maximum, scale and codes of every group from one read of the tensor: at one width for all
+// nothing but the group itself is needed for its codes.  32 lanes own the group of 8/BITS samples (at least
+// four, for loads in flight), a lane 8 consecutive elements of each; the lanes fold their minima and maxima,
+// each takes over the scale (a double division) of one of the samples and hands it to the others.
+// Bound by the read: minimax, scale and pack as kernels of their own took 20.7 + 3.0 + 28.9 us at 4 bits on
+// bf16 [256, 200704]; with this one, packing and unpacking took 46.5 instead of 69.6 us.
+// KNOWN: the ranges come from another kernel.  ROWS: rows of F elements at any address, the last group
+// padded with zeros.  S: type of the scales and minima written (mn_out may be null if KNOWN).
+template <typename T, typename S, int BITS, bool KNOWN, bool ROWS>
+__global__ __launch_bounds__(kThreads) void quantize_fixed_kernel(
+    const T* __restrict__ data, const T* __restrict__ mn_in, const T* __restrict__ mx_in, S* __restrict__ scale,
+    S* __restrict__ mn_out, int8_t* __restrict__ packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F,
+    int64_t G, int64_t rows) {
+  constexpr int WPT = 8 / BITS;
+  constexpr int U = WPT >= 4 ? 1 : 4 / WPT;              // rows of the stream a thread handles at a time
+  constexpr int SPT = U * WPT;                           // samples
+  constexpr float kUnit = (float)(1u << (32 - BITS - Noise<T>::kBits));
+  const int lane = threadIdx.x & 31;
+  const int half = threadIdx.x & 32;
+  const int64_t g = (int64_t)blockIdx.x * (kThreads / 32) + (threadIdx.x >> 5);
+  const bool live = g < G;                               // (lanes stay with the others: they exchange data)
+  const int64_t d0 = g * kFixedGs + lane * 8;
+  const int valid = ROWS && live ? part_of_row(F, d0) : 8;
+  for (int64_t no0 = (int64_t)blockIdx.y * U; no0 < rows; no0 += (int64_t)gridDim.y * U) {
+    const int64_t n0 = no0 * WPT;
+    Raw8<T> raw[SPT];
+#pragma unroll
+    for (int s = 0; s < SPT; ++s) {
+      raw8_zero(raw[s]);
+      if (live && n0 + s < N) {
+        if constexpr (ROWS) raw8_load_part(data + (n0 + s) * F + d0, valid, raw[s]);
+        else raw8_load_nt(data + (n0 + s) * F + d0, raw[s]);
+      }
+    }
+    // this lane's share of the scales: the sample lane % SPT
+    const int own = lane & (SPT - 1);
+    const int64_t gi = (n0 + own) * G + g;
+    const bool mine = live && n0 + own < N;
+    float lo = 0.0f, hi = 0.0f;
+    if constexpr (KNOWN) {
+      if (mine) {
+        lo = Conv<T>::load(mn_in, gi);
+        hi = Conv<T>::load(mx_in, gi);
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SPT; ++s) {
+        float v[8], l, h;
+        raw8_widen(raw[s], v);
+        minmax_of<8>(v, l, h);
+        lanes_minmax<2>(l, h);                           // the last lanes of each half hold the group's
+        l = as_float((uint32_t)__builtin_amdgcn_ds_swizzle((int)as_uint(l), 0x3E0));   // lane 31 of the half
+        h = as_float((uint32_t)__builtin_amdgcn_ds_swizzle((int)as_uint(h), 0x3E0));
+        lo = own == s ? l : lo;
+        hi = own == s ? h : hi;
+      }
+      lo = min_f32(INFINITY, lo);                        // (a group of NaNs only, as minimax leaves it)
+      hi = max_f32(-INFINITY, hi);
+    }
+    float mul, sub;
+    const float sc = GroupQuant<T, false>::prepare(lo, hi, BITS, mul, sub);
+    if (mine && lane < SPT) {
+      Conv<S>::store(scale, gi, sc);
+      if (mn_out) Conv<S>::store(mn_out, gi, lo);
+    }
+    uint32_t rw[SPT][Noise<T>::kWords];
+    const uint64_t o0 = (uint64_t)(n0 * G + g) * 32 + lane, per_sample = (uint64_t)G * 32;
+#pragma unroll
+    for (int s = 0; s < SPT; s += 2)                     // (the neighbouring lane holds the neighbouring octet)
+      Noise<T>::octets(o0 + s * per_sample, o0 + (s + 1) * per_sample, seed, offset, rw[s], rw[s + 1]);
+    float m[SPT], b[SPT];
+#pragma unroll
+    for (int s = 0; s < SPT; ++s) {
+      m[s] = as_float((uint32_t)__builtin_amdgcn_ds_bpermute((half + s) << 2, (int)as_uint(mul)));
+      b[s] = as_float((uint32_t)__builtin_amdgcn_ds_bpermute((half + s) << 2, (int)as_uint(sub)));
+      if (n0 + s >= N) m[s] = b[s] = 0.0f;               // samples past the end of the batch: code 0
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      CodeShifter<BITS, false> lo4, hi4;                 // last byte first, last sample first within a byte
+      float v[WPT][8];
+#pragma unroll
+      for (int ni = 0; ni < WPT; ++ni) raw8_widen(raw[u * WPT + ni], v[ni]);
+#pragma unroll
+      for (int k = 3; k >= 0; --k) {
+#pragma unroll
+        for (int ni = WPT - 1; ni >= 0; --ni) {
+          const int s = u * WPT + ni;
+          lo4.push(RngFixed<T>::word(v[ni][k], Noise<T>::at(rw[s], k), m[s], b[s], kUnit));
+          hi4.push(RngFixed<T>::word(v[ni][k + 4], Noise<T>::at(rw[s], k + 4), m[s], b[s], kUnit));
+        }
+      }
+      if (live && no0 + u < rows)
+        *reinterpret_cast<uint2*>(packed + (no0 + u) * G * kFixedGs + d0) = make_uint2(lo4.lo, hi4.lo);
+    }
+  }
+}
+
+template <typename T, typename S, bool KNOWN, bool ROWS>
+int launch_fixed_bits(const void* data, const void* mn_in, const void* mx_in, int bits, void* scale, void* mn_out,
+                      int8_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F, hipStream_t s) {
+  const int64_t G = (F + kFixedGs - 1) / kFixedGs, wpt = 8 / bits, rows = (N + wpt - 1) / wpt;
+  const int64_t bx = (G + kThreads / 32 - 1) / (kThreads / 32), by = wpt >= 4 ? rows : (rows * wpt + 3) / 4;
+  if (bx > 0x7fffffffLL) return ACTNN_EINVAL;
+  const dim3 grid((unsigned)bx, (unsigned)(by < 65535 ? by : 65535)), blk(kThreads);
+  const T* d = static_cast<const T*>(data);
+  const T* lo = static_cast<const T*>(mn_in);
+  const T* hi = static_cast<const T*>(mx_in);
+  S* sc = static_cast<S*>(scale);
+  S* m = static_cast<S*>(mn_out);
+  switch (bits) {
+#define ACTNN_CASE(B_)                                                                              \
+  case B_:                                                                                          \
+    quantize_fixed_kernel<T, S, B_, KNOWN, ROWS>                                                    \
+        <<<grid, blk, 0, s>>>(d, lo, hi, sc, m, packed, seed, offset, N, F, G, rows);               \
+    break;
+    ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(4) ACTNN_CASE(8)
+#undef ACTNN_CASE
+    default: return ACTNN_EBITS;
+  }
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
+template <typename T, typename S>
+int launch_fixed(const void* data, const void* mn_in, const void* mx_in, int bits, void* scale, void* mn_out,
+                 int8_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F, hipStream_t s) {
+  if (mn_in) return launch_fixed_bits<T, S, true, false>(data, mn_in, mx_in, bits, scale, mn_out, packed, seed, offset, N, F, s);
+  if (F % kFixedGs == 0 && aligned16(data))
+    return launch_fixed_bits<T, S, false, false>(data, mn_in, mx_in, bits, scale, mn_out, packed, seed, offset, N, F, s);
+  return launch_fixed_bits<T, S, false, true>(data, mn_in, mx_in, bits, scale, mn_out, packed, seed, offset, N, F, s);
+}
+
 template <typename T>
 int launch_pack(const void* data, const void* mn, const void* mx, int bits, void* scale,
                 int8_t* packed, const void* noise, uint64_t seed, uint64_t offset, int64_t N,
                 int64_t G, int64_t gs, hipStream_t s) {
+  if (!noise && gs == kFixedGs)
+    return launch_fixed<T, T>(data, mn, mx, bits, scale, nullptr, packed, seed, offset, N, G * gs, s);
   const int64_t count = N * G;
   const int64_t sblocks = (count + kThreads - 1) / kThreads;
   if (sblocks > 0x7fffffffLL) return ACTNN_EINVAL;
@@ -260,38 +402,38 @@ int launch_pack(const void* data, const void* mn, const void* mx, int bits, void
                                     offset, N, G, (int)gs, s);
 }
 
-template <typename T>
+// F: elements a row of `out` has; below G * gs (or with `out` not 16-byte aligned) the ROWS kernels.
+template <typename T, typename S, bool ROWS>
 int launch_unpack(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
-                  int64_t N, int64_t G, int64_t gs, hipStream_t s) {
+                  int64_t N, int64_t G, int64_t gs, int64_t F, hipStream_t s) {
   SingleGeom q;
   dim3 grid;
   const dim3 blk(kThreads);
-  if constexpr (sizeof(T) == 4) {
-    if (gs % 4 != 0 || !single_geometry(N, G, gs, bits, 4, q, grid)) return ACTNN_EINVAL;
-    const float* sc4 = static_cast<const float*>(scale);
-    const float* lo4 = static_cast<const float*>(mn);
-    float* o4 = static_cast<float*>(out);
-    switch (bits) {
-      case 1: unpack_single_f32_kernel<1><<<grid, blk, 0, s>>>(packed, sc4, lo4, o4, q); break;
-      case 2: unpack_single_f32_kernel<2><<<grid, blk, 0, s>>>(packed, sc4, lo4, o4, q); break;
-      case 4: unpack_single_f32_kernel<4><<<grid, blk, 0, s>>>(packed, sc4, lo4, o4, q); break;
-      case 8: unpack_single_f32_kernel<8><<<grid, blk, 0, s>>>(packed, sc4, lo4, o4, q); break;
-      default: return ACTNN_EBITS;
-    }
-    ACTNN_RETURN_LAUNCH_STATUS();
-  }
-  if (!single_geometry(N, G, gs, bits, 8, q, grid)) return ACTNN_EINVAL;
-  const T* sc = static_cast<const T*>(scale);
-  const T* lo = static_cast<const T*>(mn);
+  constexpr int kElems = sizeof(T) == 4 ? 4 : 8;
+  if (gs % kElems != 0 || !single_geometry(N, G, gs, bits, kElems, q, grid)) return ACTNN_EINVAL;
+  q.F = F;
+  const S* sc = static_cast<const S*>(scale);
+  const S* lo = static_cast<const S*>(mn);
   T* o = static_cast<T*>(out);
   switch (bits) {
-    case 1: unpack_single_kernel<T, 1><<<grid, blk, 0, s>>>(packed, sc, lo, o, q); break;
-    case 2: unpack_single_kernel<T, 2><<<grid, blk, 0, s>>>(packed, sc, lo, o, q); break;
-    case 4: unpack_single_kernel<T, 4><<<grid, blk, 0, s>>>(packed, sc, lo, o, q); break;
-    case 8: unpack_single_kernel<T, 8><<<grid, blk, 0, s>>>(packed, sc, lo, o, q); break;
+#define ACTNN_CASE(B_)                                                                                       \
+  case B_:                                                                                                   \
+    if constexpr (sizeof(T) == 4) unpack_single_f32_kernel<S, B_, ROWS><<<grid, blk, 0, s>>>(packed, sc, lo, o, q); \
+    else unpack_single_kernel<T, B_, ROWS><<<grid, blk, 0, s>>>(packed, sc, lo, o, q);                       \
+    break;
+    ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(4) ACTNN_CASE(8)
+#undef ACTNN_CASE
     default: return ACTNN_EBITS;
   }
   ACTNN_RETURN_LAUNCH_STATUS();
+}
+
+template <typename T, typename S>
+int launch_unpack_rows(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
+                       int64_t N, int64_t F, hipStream_t s) {
+  const int64_t G = (F + kFixedGs - 1) / kFixedGs;
+  if (F == G * kFixedGs) return launch_unpack<T, S, false>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
+  return launch_unpack<T, S, true>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
 }
 
 inline bool single_bits_ok(int bits) { return bits == 1 || bits == 2 || bits == 4 || bits == 8; }
@@ -331,9 +473,51 @@ extern "C" int actnn_unpack_single(const int8_t* packed, int bits, const void* s
   if (!aligned16(out) || (reinterpret_cast<uintptr_t>(packed) & 7u) != 0) return ACTNN_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
-    case ACTNN_F32: return launch_unpack<float>(packed, bits, scale, mn, out, N, G, gs, s);
-    case ACTNN_F16: return launch_unpack<__half>(packed, bits, scale, mn, out, N, G, gs, s);
-    case ACTNN_BF16: return launch_unpack<bf16_t>(packed, bits, scale, mn, out, N, G, gs, s);
+    case ACTNN_F32: return launch_unpack<float, float, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    case ACTNN_F16: return launch_unpack<__half, __half, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    case ACTNN_BF16: return launch_unpack<bf16_t, bf16_t, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
+extern "C" int actnn_quantize_fixed(const void* data, const void* mn_known, const void* mx_known, int bits,
+                                    void* scale, void* mn, int8_t* packed, uint64_t seed, uint64_t offset,
+                                    int64_t N, int64_t F, int dtype, int store_dtype, void* stream) {
+  using namespace actnn;
+  if (!single_bits_ok(bits)) return ACTNN_EBITS;
+  if (N < 0 || F < 0) return ACTNN_EINVAL;
+  if (N == 0 || F == 0) return ACTNN_OK;
+  if (!data || !scale || !packed || (!mn_known != !mx_known) || (!mn_known && !mn)) return ACTNN_EINVAL;
+  if (mn_known && F % kFixedGs != 0) return ACTNN_EINVAL;
+  if ((mn_known && !aligned16(data)) || (reinterpret_cast<uintptr_t>(packed) & 7u) != 0) return ACTNN_EALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == ACTNN_F32 && store_dtype == ACTNN_BF16)
+    return launch_fixed<float, bf16_t>(data, mn_known, mx_known, bits, scale, mn, packed, seed, offset, N, F, s);
+  if (dtype != store_dtype) return ACTNN_EDTYPE;
+  switch (dtype) {
+    case ACTNN_F32: return launch_fixed<float, float>(data, mn_known, mx_known, bits, scale, mn, packed, seed, offset, N, F, s);
+    case ACTNN_F16: return launch_fixed<__half, __half>(data, mn_known, mx_known, bits, scale, mn, packed, seed, offset, N, F, s);
+    case ACTNN_BF16: return launch_fixed<bf16_t, bf16_t>(data, mn_known, mx_known, bits, scale, mn, packed, seed, offset, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
+extern "C" int actnn_unpack_single_rows(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
+                                        int64_t N, int64_t F, int dtype, int store_dtype, void* stream) {
+  using namespace actnn;
+  if (!single_bits_ok(bits)) return ACTNN_EBITS;
+  if (N < 0 || F < 0) return ACTNN_EINVAL;
+  if (N == 0 || F == 0) return ACTNN_OK;
+  if (!packed || !scale || !mn || !out) return ACTNN_EINVAL;
+  if (!aligned16(out) || (reinterpret_cast<uintptr_t>(packed) & 7u) != 0) return ACTNN_EALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == ACTNN_F32 && store_dtype == ACTNN_BF16)
+    return launch_unpack_rows<float, bf16_t>(packed, bits, scale, mn, out, N, F, s);
+  if (dtype != store_dtype) return ACTNN_EDTYPE;
+  switch (dtype) {
+    case ACTNN_F32: return launch_unpack_rows<float, float>(packed, bits, scale, mn, out, N, F, s);
+    case ACTNN_F16: return launch_unpack_rows<__half, __half>(packed, bits, scale, mn, out, N, F, s);
+    case ACTNN_BF16: return launch_unpack_rows<bf16_t, bf16_t>(packed, bits, scale, mn, out, N, F, s);
     default: return ACTNN_EDTYPE;
   }
 }

@@ -84,10 +84,48 @@ def start_quantize(input, scheme, known_minmax=None):
         return ("raw", input)
     if scheme:
         return ("scheme", input.dtype, scheme, scheme.start_quantization_bits(input, known_minmax))
+    saved = _quantize_fixed(input, known_minmax)
+    if saved is not None:
+        return ("packed", saved)
     return ("fixed", input.dtype, no_scheme_compute_quantization_bits(input, known_minmax))
 
 
+def _rows_on_device(input):
+    """The activation as contiguous [N, features] rows in the order of its memory when it is one the
+    row kernels take (a GPU tensor of a supported dtype that is not empty), else None."""
+    if not (input.is_cuda and input.dtype in ext_quantization.g.DTYPE_CODE and input.dim() >= 2 and input.numel() > 0):
+        return None
+    return memory_order(input).reshape(input.shape[0], -1).contiguous()
+
+
+def _stored_dtype(dtype):
+    """Scale and minimum of an fp32 activation are kept as bfloat16 (ops.py:115-116)."""
+    return torch.bfloat16 if dtype == torch.float32 else dtype
+
+
+def _quantize_fixed(input, known_minmax):
+    """The saved tuple of an activation at one width for all, from one pass over it: at a fixed width a
+    group's codes need nothing but the group.  None when the general path has to do it (nothing has
+    been launched then): simulation, swapped streams, other group sizes, widths that do not divide 8."""
+    bits = config.activation_compression_bits[0]
+    if not (config.stochastic and not config.simulate and not config.swap and config.group_size == 256
+            and type(bits) is int and bits in (1, 2, 4, 8)):
+        return None
+    rows = _rows_on_device(input)
+    if rows is None:
+        return None
+    if known_minmax is not None:
+        mn, mx = known_minmax
+        if not (mn.dtype == input.dtype and mx.dtype == input.dtype and mn.numel() * 256 == input.numel()
+                and mx.numel() == mn.numel() and rows.shape[1] % 256 == 0 and mn.is_contiguous() and mx.is_contiguous()):
+            return None
+    packed, scale, q_min = ext_quantization.quantize_rows_fixed(rows, bits, known_minmax, _stored_dtype(input.dtype))
+    return packed, bits, scale, q_min
+
+
 def finish_quantize(started):
+    if started[0] == "packed":
+        return started[1]
     if started[0] == "raw":
         input = started[1]
         return (swap_to_cpu(input) if config.swap else input), None, None, None
@@ -108,13 +146,20 @@ def dequantize_activation(quantized, q_input_shape):
         ret = quantized[0]
         return swap_to_device(ret) if config.swap else ret
     q_input, q_bits, q_scale, q_min = quantized
-    if q_scale.dtype == torch.bfloat16 and _stored_as_bf16(q_input_shape, quantized):
-        q_scale = q_scale.to(torch.float32)
-        q_min = q_min.to(torch.float32)
-    out = dequantize_and_unpack(q_input, q_input_shape, q_bits, q_scale, q_min)
+    widen = q_scale.dtype == torch.bfloat16 and _stored_as_bf16(q_input_shape, quantized)
     N = q_input_shape[0]
     features = math.prod(q_input_shape[1:])
-    out = out.view(N, -1)[:, :features]
+    if (type(q_bits) is int and q_bits in (1, 2, 4, 8) and config.group_size == 256 and not config.simulate
+            and N * features > 0):
+        data = swap_to_device(q_input) if config.swap else q_input
+        out = ext_quantization.unpack_rows_fixed(data, q_bits, q_scale, q_min, N, features,
+                                                 torch.float32 if widen else q_scale.dtype)
+    else:
+        if widen:
+            q_scale = q_scale.to(torch.float32)
+            q_min = q_min.to(torch.float32)
+        out = dequantize_and_unpack(q_input, q_input_shape, q_bits, q_scale, q_min)
+        out = out.view(N, -1)[:, :features]
     memory_format = getattr(quantized, "memory_format", None)
     if memory_format is not None:
         # saved in channels-last order: rebuild [N, ..., C] and hand out the channels-last view

@@ -106,6 +106,24 @@ int actnn_unpack_single(const int8_t* packed, int bits, const void* scale, const
                         void* out, int64_t N, int64_t G, int64_t gs, int dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------
+ * Rows of any length at one width: data is [N, F], contiguous, at any element address; a row is cut
+ * into G = ceil(F / 256) groups of 256, the last one padded with zeros.
+ *   actnn_quantize_fixed: minimum, maximum, scale and codes of every group in one pass: the stream
+ *     actnn_minimax and actnn_pack_single give for the padded rows.  mn_known / mx_known: [N * G]
+ *     ranges another kernel has produced (then F % 256 == 0 and data 16-byte aligned; mn may be null),
+ *     or both null.  scale and mn, [N * G], are written in store_dtype: the dtype of data, or bfloat16
+ *     for fp32 data (the form in which ops.py:115-116 keeps them).
+ *   actnn_unpack_single_rows: the inverse; out is [N, F] in dtype, 16-byte aligned.
+ * Replaces qscheme.py:59-74 / ops.py:77-118 and ops.py:121-139 at a fixed width.
+ * ------------------------------------------------------------------------------- */
+int actnn_quantize_fixed(const void* data, const void* mn_known, const void* mx_known, int bits, void* scale,
+                         void* mn, int8_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F, int dtype,
+                         int store_dtype, void* stream);
+int actnn_unpack_single_rows(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
+                             int64_t N, int64_t F, int dtype, int store_dtype, void* stream);
+
+
+/* ---------------------------------------------------------------------------------
  * ReLU with a 1-bit mask.  mask holds 16 int32 words per block of 512 elements,
  * i.e. ceil(n / 512) * 16 words (equal to the reference's ceil(n / 32) whenever
  * n % 512 == 0; the reference's tail block writes past its shorter allocation).

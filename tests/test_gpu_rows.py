@@ -1,0 +1,90 @@
+"""Rows of any length (not whole groups of 256, any element address): the row kernels against the
+composition of minimax, pack and unpack on the zero-padded rows, which the oracle tests pin."""
+import pytest
+import torch
+
+from actnn_amd import ops
+from actnn_amd.conf import config
+from actnn_amd.cpp_extension import minimax as ext_minimax
+from actnn_amd.cpp_extension import quantization as ext_q
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.float16, torch.bfloat16]
+SHAPES = [(1, 1), (2, 7), (5, 255), (3, 256), (4, 257), (9, 2049), (2, 4093), (65, 300), (7, 512)]
+
+
+def _rows(N, F, dtype, shift, seed):
+    """[N, F] whose first element lies `shift` elements behind an allocation's start."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    flat = torch.randn(N * F + shift, generator=gen, device="cuda") * 3 + 1
+    return flat.to(dtype)[shift:].view(N, F)
+
+
+def _padded(x):
+    N, F = x.shape
+    G = (F + 255) // 256
+    return torch.cat([x, torch.zeros(N, G * 256 - F, dtype=x.dtype, device=x.device)], 1).view(N, G, 256)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+def test_fixed_width_rows_equal_the_padded_composition(dtype, bits):
+    for i, (N, F) in enumerate(SHAPES):
+        for shift in (0, 1):
+            x = _rows(N, F, dtype, shift, 17 * i + shift)
+            groups = _padded(x)
+            G = groups.shape[1]
+            mn, mx = ext_minimax.minimax(groups.view(-1, 256))
+            mn, mx = mn.view(N, G, 1), mx.view(N, G, 1)
+            torch.manual_seed(i)
+            want, want_scale = ext_q.pack_single_precision(groups, mn, mx, bits, True)
+            store = ops._stored_dtype(dtype)
+            want_scale, want_mn = want_scale.to(store), mn.to(store)
+            torch.manual_seed(i)
+            packed, scale, low = ext_q.quantize_rows_fixed(x, bits, None, store)
+            used = packed.numel() - 1                            # the last byte belongs to no element
+            assert torch.equal(packed[:used], want[:used]), (N, F, shift)
+            assert torch.equal(scale, want_scale) and torch.equal(low, want_mn), (N, F, shift)
+            back = ext_q.unpack_rows_fixed(packed, bits, scale, low, N, F, dtype)
+            full = ext_q.unpack_single_precision(want, bits, want_scale.to(dtype), want_mn.to(dtype), N, G, 256)
+            assert torch.equal(back, full.view(N, -1)[:, :F]), (N, F, shift)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_fixed_width_rows_with_known_ranges(dtype):
+    x = _rows(6, 1024, dtype, 0, 3)
+    mn, mx = ext_minimax.minimax(x.view(-1, 256))
+    store = ops._stored_dtype(dtype)
+    torch.manual_seed(5)
+    want = ext_q.quantize_rows_fixed(x, 4, None, store)
+    torch.manual_seed(5)
+    got = ext_q.quantize_rows_fixed(x, 4, (mn, mx), store)
+    assert torch.equal(got[0][:-1], want[0][:-1]) and torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_special_values_survive_the_one_pass(dtype, channels_last):
+    """Constant groups, infinities and NaNs: as the general path (taken for a noisy group size switch) leaves them."""
+    config.reset()
+    config.activation_compression_bits = [4]
+    try:
+        x = torch.randn(3, 8, 13, 7, device="cuda").to(dtype)
+        x[0] = 2.5
+        x[1, :, :2] = float("nan")
+        x[2, 0, 0, 0] = float("inf")
+        if channels_last:
+            x = x.contiguous(memory_format=torch.channels_last)
+        torch.manual_seed(1)
+        saved = ops.quantize_saved(x, None)
+        torch.manual_seed(1)
+        groups, bits, mn, mx = ops.no_scheme_compute_quantization_bits(x)
+        want, scale = ext_q.pack_single_precision(groups, mn, mx, bits, True)
+        store = ops._stored_dtype(dtype)
+        assert torch.equal(saved[0][:-1], want[:-1])
+        assert torch.equal(saved[2].nan_to_num(7.0), scale.to(store).nan_to_num(7.0))
+        assert torch.equal(saved[3].nan_to_num(7.0), mn.to(store).nan_to_num(7.0))
+        assert ops.dequantize_activation(saved, x.shape).stride() == x.stride()
+    finally:
+        config.reset()
