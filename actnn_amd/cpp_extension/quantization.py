@@ -105,34 +105,60 @@ def pack_mixed_precision(data, min, max, bits, stochastic, *, noise=None):
 
 def quantize_activation_device(rows, N, known_minmax, alloc):
     """[min/max of every group] -> widths on the device -> pack, in one call: what minimax,
-    allocate_bits_device and pack_mixed_precision do one after the other for `rows` (contiguous
-    [N * G, 256] view of the activation).  `known_minmax`: (mn, mx) [N * G] in the rows' dtype when
-    another kernel has produced them, else None.  `alloc`: the scheme's AllocationArgs.
+    allocate_bits_device and pack_mixed_precision do one after the other for `rows`, a contiguous
+    view of the activation's N samples, the last group of each padded with zeros.  `known_minmax`: (mn, mx) [N * G]
+    of whole groups in the rows' dtype when another kernel has produced them, else None.  `alloc`: the
+    scheme's AllocationArgs, whose `store_dtype` says what scale and mn come back in.
     -> (packed, bits with sum and prefix attached, scale [N, G, 1], mn [N * G])."""
     from .backward_func import _mult_args
     dev, dtype = rows.device, rows.dtype
-    G = rows.shape[0] // N
-    rows = g.aligned(rows)
+    store_dtype = alloc.store_dtype or dtype
+    F = rows.numel() // N
+    G = (F + 255) // 256
     if known_minmax is None:
         mn = torch.empty(N * G, dtype=dtype, device=dev)
         mx = torch.empty(N * G, dtype=dtype, device=dev)
     else:
         mn, mx = known_minmax
+    stored = mn if store_dtype == dtype else torch.empty(N * G, dtype=store_dtype, device=dev)
     sens = alloc.sens_out if alloc.sens_out is not None else torch.empty(N, dtype=torch.float32, device=dev)
     bits = torch.empty(N, dtype=torch.int32, device=dev)
     prefix = torch.empty(N + 1, dtype=torch.int32, device=dev)
     packed = torch.empty(alloc.total * G * 8, dtype=torch.int32, device=dev)
-    scale = torch.empty(N, G, 1, dtype=dtype, device=dev)
+    scale = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
     mult, mult_ptr, per_sample = _mult_args(alloc.mult, N, dev)           # (`mult` held until the launch)
     seed, offset = g.philox_args(dev)
     with g.on_device(dev):
-        check(g.lib().actnn_quantize_activation(
+        check(g.lib().actnn_quantize_rows(
             rows.data_ptr(), mn.data_ptr(), mx.data_ptr(), int(known_minmax is not None), alloc.factor, mult_ptr,
             per_sample, sens.data_ptr(), bits.data_ptr(), prefix.data_ptr(), alloc.initial, alloc.target,
-            scale.data_ptr(), packed.data_ptr(), seed, offset, N, G, g.DTYPE_CODE[dtype], g.stream_ptr(dev)),
-            "quantize_activation")
+            scale.data_ptr(), stored.data_ptr(), packed.data_ptr(), seed, offset, N, F, g.DTYPE_CODE[dtype],
+            g.DTYPE_CODE[store_dtype], g.stream_ptr(dev)), "quantize_activation")
     attach_bits_total(bits, alloc.total, prefix)
-    return packed, bits, scale, mn
+    return packed, bits, scale, stored
+
+
+def unpack_rows_mixed(packed, bits, scale, mn, N, F, dtype):
+    """The [N, F] rows of quantize_activation_device in `dtype`, nothing materialised for the padding."""
+    g.check_typed(packed, "data", torch.int32, 1)
+    g.check_typed(bits, "bits", torch.int32, 1)
+    g.check_float(scale, "scale", 3)
+    g.check_float(mn, "min", 3)
+    G = (F + 255) // 256
+    if mn.dtype != scale.dtype:
+        raise RuntimeError("The type of min is not correct!")
+    if scale.numel() != N * G or mn.numel() != N * G or bits.numel() != N:
+        raise RuntimeError("unpack_mixed_precision: shape mismatch")
+    total, prefix = _bits_info(bits)
+    if packed.numel() < total * G * 8:
+        raise RuntimeError("unpack_mixed_precision: packed stream is too short")
+    out = torch.empty(N, F, dtype=dtype, device=packed.device)
+    with g.on_device(packed.device):
+        check(g.lib().actnn_unpack_mixed_rows(
+            packed.data_ptr(), bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(), mn.data_ptr(), out.data_ptr(),
+            N, F, g.DTYPE_CODE[dtype], g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)),
+            "unpack_mixed_precision")
+    return out
 
 
 def unpack_mixed_precision(data, bits, scale, min, N, num_groups, group_size):

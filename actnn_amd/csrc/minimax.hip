@@ -19,8 +19,8 @@ constexpr int kRowsPerLaneGroup = 8;          // rows per lane group and block (
 template <typename T> struct Vec16;           // running min/max over one 16-byte vector of T
 template <> struct Vec16<float> {
   static constexpr int kElems = 4;
-  static ACTNN_DEV void minmax(const float* p, float& lo, float& hi) {
-    const u32x4 u = load16_nt(p);
+  static ACTNN_DEV void minmax(const float* p, float& lo, float& hi) { minmax(load16_nt(p), lo, hi); }
+  static ACTNN_DEV void minmax(u32x4 u, float& lo, float& hi) {
     const float a = as_float(u.x), b = as_float(u.y), c = as_float(u.z), d = as_float(u.w);
     lo = min3_f32(min3_f32(lo, a, b), c, d);
     hi = max3_f32(max3_f32(hi, a, b), c, d);
@@ -28,8 +28,8 @@ template <> struct Vec16<float> {
 };
 template <> struct Vec16<__half> {
   static constexpr int kElems = 8;
-  static ACTNN_DEV void minmax(const __half* p, float& lo, float& hi) {
-    const u32x4 u = load16_nt(p);
+  static ACTNN_DEV void minmax(const __half* p, float& lo, float& hi) { minmax(load16_nt(p), lo, hi); }
+  static ACTNN_DEV void minmax(u32x4 u, float& lo, float& hi) {
     const uint32_t w[4] = {u.x, u.y, u.z, u.w};
     float v[8];
 #pragma unroll
@@ -45,8 +45,8 @@ template <> struct Vec16<__half> {
 };
 template <> struct Vec16<bf16_t> {
   static constexpr int kElems = 8;
-  static ACTNN_DEV void minmax(const bf16_t* p, float& lo, float& hi) {
-    const u32x4 u = load16_nt(p);
+  static ACTNN_DEV void minmax(const bf16_t* p, float& lo, float& hi) { minmax(load16_nt(p), lo, hi); }
+  static ACTNN_DEV void minmax(u32x4 u, float& lo, float& hi) {
     const uint32_t w[4] = {u.x, u.y, u.z, u.w};
     float v[8];
 #pragma unroll
@@ -158,6 +158,54 @@ int launch_minimax(const void* data, void* mn, void* mx, int64_t M, int64_t D, h
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
+// Groups of 256 of rows of F elements at any address, the last group of a row padded with zeros (which count).
+// As the vector path: 64 lanes (fp32) or 32 lanes own a group with one 16-byte load each, eight groups a lane
+// in flight.  Copying the rows to padded ones first was two passes of its own (fp32 [32, 309123]: 16 us of the
+// 100 that packing and unpacking took, 49 now).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void minimax_rows_kernel(const T* __restrict__ data, T* __restrict__ mn,
+                                                                T* __restrict__ mx, uint32_t M, int64_t F,
+                                                                FastDiv groups) {
+  constexpr int E = 16 / sizeof(T);
+  constexpr int LPR = 256 / E;
+  constexpr int kSlots = kThreads / LPR;
+  constexpr int R = kRowsPerLaneGroup;
+  const int sub = threadIdx.x % LPR;
+  const uint32_t row0 = blockIdx.x * (kSlots * R) + threadIdx.x / LPR;
+  u32x4 u[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t row = row0 + r * kSlots;
+    u[r] = (u32x4){0, 0, 0, 0};
+    if (row < M) {
+      const uint32_t n = groups.div(row);
+      const int64_t at = (int64_t)(row - n * groups.d) * 256 + sub * E;
+      u[r] = load16_part(data + n * F + at, part_of_row(F, at));
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float lo = INFINITY, hi = -INFINITY;
+    Vec16<T>::minmax(u[r], lo, hi);
+    lanes_minmax<LPR / 16>(lo, hi);
+    const uint32_t row = row0 + r * kSlots;
+    if (sub == LPR - 1 && row < M) {
+      Conv<T>::store(mn, row, lo);
+      Conv<T>::store(mx, row, hi);
+    }
+  }
+}
+
+template <typename T>
+int launch_minimax_rows(const void* data, void* mn, void* mx, int64_t N, int64_t F, hipStream_t s) {
+  constexpr int kRows = kThreads / (256 * (int)sizeof(T) / 16) * kRowsPerLaneGroup;
+  const int64_t G = (F + 255) / 256, M = N * G;
+  if (M > 0x7fffffffLL - kRows) return ACTNN_EINVAL;
+  minimax_rows_kernel<T><<<dim3((unsigned)((M + kRows - 1) / kRows)), dim3(kThreads), 0, s>>>(
+      static_cast<const T*>(data), static_cast<T*>(mn), static_cast<T*>(mx), (uint32_t)M, F, FastDiv((uint32_t)G));
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
 // Squared L2 norm of every sample (the gradient statistic of the bit allocation, qscheme.py:47-55):
 // part[n * B + b] = sum of squares over slice b of row n, fp32, in a fixed order; the caller adds
 // the B slices.  Rows are read with 16-byte non-temporal loads; 16-bit types use the dot-product
@@ -214,6 +262,17 @@ __global__ __launch_bounds__(kThreads) void sample_sqnorm_kernel(const T* __rest
 }
 
 }  // namespace
+
+// minimum and maximum of the groups of [N, F] rows (actnn_quantize_rows has checked the arguments)
+int minimax_rows(const void* data, void* mn, void* mx, int64_t N, int64_t F, int dtype, hipStream_t s) {
+  switch (dtype) {
+    case ACTNN_F32: return launch_minimax_rows<float>(data, mn, mx, N, F, s);
+    case ACTNN_F16: return launch_minimax_rows<__half>(data, mn, mx, N, F, s);
+    case ACTNN_BF16: return launch_minimax_rows<bf16_t>(data, mn, mx, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
 }  // namespace actnn
 
 extern "C" int actnn_minimax(const void* data, void* mn, void* mx, int64_t M, int64_t D, int dtype,

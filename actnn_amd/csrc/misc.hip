@@ -121,10 +121,6 @@ extern "C" int actnn_batch_norm_forward_apply_relu(const void* x, void* y, const
                                                    const void* residual, int64_t N, int64_t C, int64_t HW,
                                                    int dtype, int channels_last, void* stream);
 extern "C" int actnn_minimax(const void* data, void* mn, void* mx, int64_t M, int64_t D, int dtype, void* stream);
-extern "C" int actnn_pack_mixed(const void* data, const void* mn, const void* mx, const int32_t* bits,
-                                const int32_t* prefix, void* scale, int32_t* packed, const void* noise,
-                                uint64_t seed, uint64_t offset, int64_t N, int64_t G, int64_t gs, int dtype,
-                                void* stream);
 
 extern "C" int actnn_batch_norm_forward_quantize(
     const void* x, const float* weight, const float* bias, float* running_mean, float* running_var, void* y,
@@ -158,23 +154,49 @@ extern "C" int actnn_batch_norm_forward_quantize(
                                         seed, offset, N, C, HW, dtype, channels_last, stream);
 }
 
-extern "C" int actnn_quantize_activation(const void* data, void* mn, void* mx, int minmax_known, float factor,
-                                         const float* mult, int mult_per_sample, float* sensitivity,
-                                         int32_t* bits, int32_t* prefix, int initial_bits, int64_t target,
-                                         void* scale, int32_t* packed, uint64_t seed, uint64_t offset, int64_t N,
-                                         int64_t G, int dtype, void* stream) {
+namespace actnn {
+int minimax_rows(const void* data, void* mn, void* mx, int64_t N, int64_t F, int dtype, hipStream_t s);
+int pack_mixed_rows(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
+                    void* scale, void* mn_out, int32_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F,
+                    int dtype, int store_dtype, hipStream_t s);
+}  // namespace actnn
+
+extern "C" int actnn_quantize_rows(const void* data, void* mn, void* mx, int minmax_known, float factor,
+                                   const float* mult, int mult_per_sample, float* sensitivity, int32_t* bits,
+                                   int32_t* prefix, int initial_bits, int64_t target, void* scale, void* mn_stored,
+                                   int32_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F, int dtype,
+                                   int store_dtype, void* stream) {
+  using namespace actnn;
   if (!data || !mn || !mx || !bits || !prefix || !scale || !packed || !sensitivity) return ACTNN_EINVAL;
-  if (N <= 0 || G <= 0) return ACTNN_EINVAL;
+  if (N <= 0 || F <= 0 || (minmax_known && F % 256 != 0)) return ACTNN_EINVAL;
+  if (dtype < ACTNN_F32 || dtype > ACTNN_BF16) return ACTNN_EDTYPE;
+  if (dtype != store_dtype && (dtype != ACTNN_F32 || store_dtype != ACTNN_BF16)) return ACTNN_EDTYPE;
+  if (dtype != store_dtype && !mn_stored) return ACTNN_EINVAL;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t G = (F + 255) / 256;
   int rc = ACTNN_OK;
   if (!minmax_known) {
-    rc = actnn_minimax(data, mn, mx, N * G, 256, dtype, stream);
+    rc = F % 256 == 0 && aligned16(data) ? actnn_minimax(data, mn, mx, N * G, 256, dtype, stream)
+                                         : minimax_rows(data, mn, mx, N, F, dtype, s);
     if (rc != ACTNN_OK) return rc;
   }
   rc = actnn_allocate_bits_device(mn, mx, factor, mult, mult_per_sample, sensitivity, bits, prefix, N, G,
                                   initial_bits, target, dtype, stream);
   if (rc != ACTNN_OK) return rc;
-  return actnn_pack_mixed(data, mn, mx, bits, prefix, scale, packed, nullptr, seed, offset, N, G, 256, dtype,
-                          stream);
+  return pack_mixed_rows(data, mn, mx, bits, prefix, scale, mn_stored, packed, seed, offset, N, F, dtype,
+                         store_dtype, s);
+}
+
+extern "C" int actnn_quantize_activation(const void* data, void* mn, void* mx, int minmax_known, float factor,
+                                         const float* mult, int mult_per_sample, float* sensitivity,
+                                         int32_t* bits, int32_t* prefix, int initial_bits, int64_t target,
+                                         void* scale, int32_t* packed, uint64_t seed, uint64_t offset, int64_t N,
+                                         int64_t G, int dtype, void* stream) {
+  if (N <= 0 || G <= 0) return ACTNN_EINVAL;
+  if (data && !actnn::aligned16(data)) return ACTNN_EALIGN;
+  return actnn_quantize_rows(data, mn, mx, minmax_known, factor, mult, mult_per_sample, sensitivity, bits, prefix,
+                             initial_bits, target, scale, nullptr, packed, seed, offset, N, G * 256, dtype, dtype,
+                             stream);
 }
 
 extern "C" const char* actnn_strerror(int code) {

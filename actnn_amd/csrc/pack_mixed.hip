@@ -51,8 +51,10 @@ template <int BITS, int GPH> struct Tile {
 // (measured 6.9 instead of 5.3 TB/s, and no dirty lines are left for the next kernel to wait on).
 // Only lanes of one wave exchange data, so no block barrier is needed: LDS operations of a wave
 // complete in order.  (The same staging for the fp32 loads of pack was measured slower.)
-template <int GPH, typename TL>
-ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int groups_valid,
+// ROWS: `out` is a row of F elements at any address and elem_base an offset in it; its lines are shared with
+// other waves, so the stores go through the cache.
+template <int GPH, typename TL, bool ROWS>
+ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t F, int groups_valid,
                              u32x4* __restrict__ slab, const float (&v)[GPH][8]) {
   const int wl = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
@@ -76,7 +78,9 @@ ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int gro
   for (int i = 0; i < 2 * GPH; ++i) {
     const int gl = TL::group_of(2 * w + i / GPH, i % GPH);
     if (gl < groups_valid) {
-      store16_nt(out + elem_base + (int64_t)gl * kGs + wl * 4, slab[i * 64 + wl]);
+      const int64_t at = elem_base + (int64_t)gl * kGs + wl * 4;
+      if constexpr (ROWS) store16_part(out + at, slab[i * 64 + wl], part_of_row(F, at));
+      else store16_nt(out + at, slab[i * 64 + wl]);
     }
   }
 }
@@ -90,8 +94,9 @@ template <> struct IsBf16<bf16_t> { static constexpr bool value = true; };
 // Issue the loads of this lane's elements (and noise in deterministic mode) for its GPH groups.
 // The elements stay as loaded until their group is packed (16-bit types: 4 registers per group
 // rather than 8), which keeps the kernel within the registers of 8 waves per SIMD.
-template <typename T, bool DET, int GPH>
-ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noise, int64_t elem_base,
+// ROWS: `data` is a row of F elements at any address and elem_base an offset in it.
+template <typename T, bool DET, int GPH, bool ROWS>
+ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noise, int64_t elem_base, int64_t F,
                            int groups_valid, Raw8<T> (&v)[GPH], Raw8<T> (&nz)[DET ? GPH : 1]) {
   using TL = Tile<1, GPH>;
   const uint32_t lane = threadIdx.x & 31;
@@ -101,7 +106,8 @@ ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noi
     const int gl = TL::group_of(hw, q);
     if (gl < groups_valid) {
       const int64_t e = elem_base + (int64_t)gl * kGs + lane * 8;
-      raw8_load_nt(data + e, v[q]);      // non-temporal for 16-bit types only (one instruction per line)
+      if constexpr (ROWS) raw8_load_part(data + e, part_of_row(F, e), v[q]);
+      else raw8_load_nt(data + e, v[q]); // non-temporal for 16-bit types only (one instruction per line)
       if (DET) raw8_load_nt(noise + e, nz[DET ? q : 0]);
     } else {
       raw8_zero(v[q]);
@@ -175,12 +181,14 @@ ACTNN_DEV void pack_groups(const Raw8<T> (&raw)[Gph<T>::kPack], const Raw8<T> (&
   }
 }
 
-template <typename T, bool DET>
+// ROWS: rows of F elements at any address, the last group padded with zeros.  S: the type the scales are
+// written in; where it is not the tensor's own (bfloat16 for fp32), the minima are written in it as well.
+template <typename T, typename S, bool DET, bool ROWS>
 __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
     const T* __restrict__ data, const T* __restrict__ mn, const T* __restrict__ mx,
-    const int32_t* __restrict__ bits, const int32_t* __restrict__ prefix, T* __restrict__ scale,
-    int32_t* __restrict__ packed, const T* __restrict__ noise, uint64_t seed, uint64_t offset,
-    int64_t G, int blocks_per_sample) {
+    const int32_t* __restrict__ bits, const int32_t* __restrict__ prefix, S* __restrict__ scale,
+    S* __restrict__ mn_out, int32_t* __restrict__ packed, const T* __restrict__ noise, uint64_t seed,
+    uint64_t offset, int64_t F, int64_t G, int blocks_per_sample) {
   constexpr int GPH = Gph<T>::kPack;
   constexpr int kGroupsPerBlock = kHalfWaves * GPH;
   __shared__ float s_mul[kGroupsPerBlock];
@@ -200,7 +208,16 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
   // picks its 32 bytes out of LDS.
   constexpr bool kViaLds = sizeof(T) == 4 && !DET;
   __shared__ __align__(16) uint8_t s_stage[kViaLds ? kGroupsPerBlock * kGs * 4 : 16];
-  if constexpr (kViaLds) {
+  u32x4 st[kViaLds && ROWS ? 2 * GPH : 1];                       // ROWS: by way of registers, at any address
+  if constexpr (kViaLds && ROWS) {
+#pragma unroll
+    for (int i = 0; i < 2 * GPH; ++i) {
+      const int gl = (threadIdx.x >> 6) * 2 * GPH + i;
+      const int64_t at = (gb + gl) * kGs + (threadIdx.x & 63) * 4;
+      st[i] = (u32x4){0, 0, 0, 0};
+      if (gl < groups_valid) st[i] = load16_part(data + n * F + at, part_of_row(F, at));
+    }
+  } else if constexpr (kViaLds) {
     const int wave = threadIdx.x >> 6;
     const uint32_t wl = threadIdx.x & 63;
 #pragma unroll
@@ -210,7 +227,8 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
         load_to_lds16_nt(data + elem_base + (int64_t)gl * kGs + wl * 4, s_stage + gl * (kGs * 4));
     }
   } else {
-    load_groups<T, DET, GPH>(data, noise, elem_base, groups_valid, v, nz);
+    if constexpr (ROWS) load_groups<T, DET, GPH, true>(data + n * F, noise, gb * kGs, F, groups_valid, v, nz);
+    else load_groups<T, DET, GPH, false>(data, noise, elem_base, F, groups_valid, v, nz);
   }
 
   const int b = bits[n];
@@ -218,15 +236,22 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
     float mul = 0.0f, sub = 0.0f;
     if ((int)threadIdx.x < groups_valid) {
       const int64_t gi = n * G + gb + threadIdx.x;
-      const float sc = GroupQuant<T, DET>::prepare(Conv<T>::load(mn, gi), Conv<T>::load(mx, gi), b, mul, sub);
-      Conv<T>::store(scale, gi, sc);
+      const float lo = Conv<T>::load(mn, gi);
+      const float sc = GroupQuant<T, DET>::prepare(lo, Conv<T>::load(mx, gi), b, mul, sub);
+      Conv<S>::store(scale, gi, sc);
+      if constexpr (sizeof(S) != sizeof(T)) Conv<S>::store(mn_out, gi, lo);
     }
     s_mul[threadIdx.x] = mul;
     s_sub[threadIdx.x] = sub;
   }
+  if constexpr (kViaLds && ROWS) {
+#pragma unroll
+    for (int i = 0; i < 2 * GPH; ++i)
+      *reinterpret_cast<u32x4*>(s_stage + ((threadIdx.x >> 6) * 2 * GPH + i) * (kGs * 4) + (threadIdx.x & 63) * 16) = st[i];
+  }
   __syncthreads();
   if constexpr (kViaLds) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's own groups have landed
+    if constexpr (!ROWS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's own groups have landed
     const uint32_t lane = threadIdx.x & 31;
     const int hw = threadIdx.x >> 5;
 #pragma unroll
@@ -256,9 +281,10 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
 }
 
 // ---------------------------------------------------------------------------- unpack (gs = 256)
-template <typename T, int BITS>
+// ROWS: `out` is a row of F elements at any address and elem_base an offset in it.
+template <typename T, int BITS, bool ROWS>
 ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__ out,
-                             int64_t elem_base, int64_t word_base, int groups_valid,
+                             int64_t elem_base, int64_t F, int64_t word_base, int groups_valid,
                              float* s_scale, float* s_min, float my_scale, float my_min, u32x4* slab) {
   constexpr int kGroupsPerHalf = Gph<T>::kUnpack;
   constexpr bool kStage = IsF32<T>::value;
@@ -326,7 +352,9 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
             const uint32_t sel = (c0 * 0x0202u + 0x0100u) | ((c1 * 0x0202u + 0x0100u) << 16);
             outw[j] = __builtin_amdgcn_perm(lut_hi, lut_lo, sel);
           }
-          store16_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, outw);
+          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
+          if constexpr (ROWS) store16_part(out + at, outw, part_of_row(F, at));
+          else store16_nt(out + at, outw);
           continue;
         }
         float v[8];
@@ -335,6 +363,9 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
         if constexpr (kStage) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) vs[kStage ? q0 + r : 0][k] = v[k];
+        } else if constexpr (ROWS) {
+          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
+          store16_part(out + at, words_of8(out, v), part_of_row(F, at));
         } else {
           store8_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, v);
         }
@@ -342,14 +373,15 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
     }
   }
   if constexpr (kStage)
-    stage_out_f32<kGroupsPerHalf, TL>(reinterpret_cast<float*>(out), elem_base, groups_valid, slab, vs);
+    stage_out_f32<kGroupsPerHalf, TL, ROWS>(reinterpret_cast<float*>(out), elem_base, F, groups_valid, slab, vs);
 }
 
-template <typename T>
+// S: the type the scales and minima are stored in.
+template <typename T, typename S, bool ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
     const int32_t* __restrict__ packed, const int32_t* __restrict__ bits,
-    const int32_t* __restrict__ prefix, const T* __restrict__ scale, const T* __restrict__ mn,
-    T* __restrict__ out, int64_t G, int blocks_per_sample) {
+    const int32_t* __restrict__ prefix, const S* __restrict__ scale, const S* __restrict__ mn,
+    T* __restrict__ out, int64_t F, int64_t G, int blocks_per_sample) {
   constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kUnpack;
   __shared__ float s_scale[kGroupsPerBlock];
   __shared__ float s_min[kGroupsPerBlock];
@@ -363,16 +395,17 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   float my_scale = 0.0f, my_min = 0.0f;
   if ((int)threadIdx.x < groups_valid) {
     const int64_t gi = n * G + gb + threadIdx.x;
-    my_scale = Conv<T>::load(scale, gi);
-    my_min = Conv<T>::load(mn, gi);
+    my_scale = Conv<S>::load(scale, gi);
+    my_min = Conv<S>::load(mn, gi);
   }
-  const int64_t elem_base = (n * G + gb) * kGs;
+  const int64_t elem_base = ROWS ? gb * kGs : (n * G + gb) * kGs;
+  if constexpr (ROWS) out += n * F;
   const int64_t word_base = (int64_t)prefix[n] * G * 8 + gb * 8 * b;
   switch (b) {
 #define ACTNN_CASE(B_)                                                                          \
   case B_:                                                                                      \
-    unpack_groups<T, B_>(packed, out, elem_base, word_base, groups_valid, s_scale, s_min,       \
-                         my_scale, my_min, slab);                                               \
+    unpack_groups<T, B_, ROWS>(packed, out, elem_base, F, word_base, groups_valid, s_scale,     \
+                               s_min, my_scale, my_min, slab);                                  \
     break;
     ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(3) ACTNN_CASE(4)
     ACTNN_CASE(5) ACTNN_CASE(6) ACTNN_CASE(7) ACTNN_CASE(8)
@@ -485,6 +518,49 @@ __global__ __launch_bounds__(1024) void bits_prefix_kernel(const int32_t* __rest
   }
 }
 
+template <typename T, typename S, bool DET, bool ROWS>
+int launch_pack_groups(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
+                       void* scale, void* mn_out, int32_t* packed, const void* noise, uint64_t seed, uint64_t offset,
+                       int64_t N, int64_t F, hipStream_t s) {
+  constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kPack;
+  const int64_t G = (F + kGs - 1) / kGs;
+  const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
+  if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
+  pack_mixed_kernel<T, S, DET, ROWS><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
+      static_cast<const T*>(data), static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
+      static_cast<S*>(scale), static_cast<S*>(mn_out), packed, static_cast<const T*>(noise), seed, offset, F, G, (int)bps);
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
+template <typename T, typename S, bool ROWS>
+int launch_unpack_groups(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
+                         const void* mn, void* out, int64_t N, int64_t F, hipStream_t s) {
+  constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kUnpack;
+  const int64_t G = (F + kGs - 1) / kGs;
+  const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
+  if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
+  unpack_mixed_kernel<T, S, ROWS><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
+      packed, bits, prefix, static_cast<const S*>(scale), static_cast<const S*>(mn), static_cast<T*>(out), F, G, (int)bps);
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
+// whole groups at an aligned address take the kernels without the row ends
+template <typename T, typename S>
+int launch_pack_rows(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
+                     void* scale, void* mn_out, int32_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F,
+                     hipStream_t s) {
+  if (F % kGs == 0 && aligned16(data))
+    return launch_pack_groups<T, S, false, false>(data, mn, mx, bits, prefix, scale, mn_out, packed, nullptr, seed, offset, N, F, s);
+  return launch_pack_groups<T, S, false, true>(data, mn, mx, bits, prefix, scale, mn_out, packed, nullptr, seed, offset, N, F, s);
+}
+
+template <typename T, typename S>
+int launch_unpack_rows(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
+                       const void* mn, void* out, int64_t N, int64_t F, hipStream_t s) {
+  if (F % kGs == 0) return launch_unpack_groups<T, S, false>(packed, bits, prefix, scale, mn, out, N, F, s);
+  return launch_unpack_groups<T, S, true>(packed, bits, prefix, scale, mn, out, N, F, s);
+}
+
 template <typename T>
 int launch_pack(const void* data, const void* mn, const void* mx, const int32_t* bits,
                 const int32_t* prefix, void* scale, int32_t* packed, const void* noise,
@@ -492,18 +568,9 @@ int launch_pack(const void* data, const void* mn, const void* mx, const int32_t*
   const T* d = static_cast<const T*>(data);
   const T* nz = static_cast<const T*>(noise);
   if (gs == kGs) {
-    constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kPack;
-    const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
-    if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
-    const dim3 grid((unsigned)(N * bps));
     if (noise)
-      pack_mixed_kernel<T, true><<<grid, dim3(kThreads), 0, s>>>(
-          d, static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
-          static_cast<T*>(scale), packed, nz, seed, offset, G, (int)bps);
-    else
-      pack_mixed_kernel<T, false><<<grid, dim3(kThreads), 0, s>>>(
-          d, static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
-          static_cast<T*>(scale), packed, nz, seed, offset, G, (int)bps);
+      return launch_pack_groups<T, T, true, false>(data, mn, mx, bits, prefix, scale, nullptr, packed, noise, seed, offset, N, G * kGs, s);
+    return launch_pack_groups<T, T, false, false>(data, mn, mx, bits, prefix, scale, nullptr, packed, noise, seed, offset, N, G * kGs, s);
   } else {
     if (N * G > 0x7fffffffLL) return ACTNN_EINVAL;
     const dim3 grid((unsigned)(N * G));
@@ -524,12 +591,7 @@ int launch_unpack(const int32_t* packed, const int32_t* bits, const int32_t* pre
                   const void* scale, const void* mn, void* out, int64_t N, int64_t G, int64_t gs,
                   hipStream_t s) {
   if (gs == kGs) {
-    constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kUnpack;
-    const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
-    if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
-    unpack_mixed_kernel<T><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
-        packed, bits, prefix, static_cast<const T*>(scale), static_cast<const T*>(mn),
-        static_cast<T*>(out), G, (int)bps);
+    return launch_unpack_groups<T, T, false>(packed, bits, prefix, scale, mn, out, N, G * kGs, s);
   } else {
     if (N * G > 0x7fffffffLL) return ACTNN_EINVAL;
     unpack_mixed_generic_kernel<T><<<dim3((unsigned)(N * G)), dim3(kThreads), 0, s>>>(
@@ -540,7 +602,44 @@ int launch_unpack(const int32_t* packed, const int32_t* bits, const int32_t* pre
 }
 
 }  // namespace
+
+// pack of [N, F] rows with the scales (and, for bfloat16 of fp32 rows, the minima) written in store_dtype
+// (actnn_quantize_rows has checked the arguments)
+int pack_mixed_rows(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
+                    void* scale, void* mn_out, int32_t* packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F,
+                    int dtype, int store_dtype, hipStream_t s) {
+  if (dtype == ACTNN_F32 && store_dtype == ACTNN_BF16)
+    return launch_pack_rows<float, bf16_t>(data, mn, mx, bits, prefix, scale, mn_out, packed, seed, offset, N, F, s);
+  if (dtype != store_dtype) return ACTNN_EDTYPE;
+  switch (dtype) {
+    case ACTNN_F32: return launch_pack_rows<float, float>(data, mn, mx, bits, prefix, scale, mn_out, packed, seed, offset, N, F, s);
+    case ACTNN_F16: return launch_pack_rows<__half, __half>(data, mn, mx, bits, prefix, scale, mn_out, packed, seed, offset, N, F, s);
+    case ACTNN_BF16: return launch_pack_rows<bf16_t, bf16_t>(data, mn, mx, bits, prefix, scale, mn_out, packed, seed, offset, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
 }  // namespace actnn
+
+extern "C" int actnn_unpack_mixed_rows(const int32_t* packed, const int32_t* bits, const int32_t* prefix,
+                                       const void* scale, const void* mn, void* out, int64_t N, int64_t F, int dtype,
+                                       int store_dtype, void* stream) {
+  using namespace actnn;
+  if (N < 0 || F < 0) return ACTNN_EINVAL;
+  if (N == 0 || F == 0) return ACTNN_OK;
+  if (!packed || !bits || !prefix || !scale || !mn || !out) return ACTNN_EINVAL;
+  if (!aligned16(out)) return ACTNN_EALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == ACTNN_F32 && store_dtype == ACTNN_BF16)
+    return launch_unpack_rows<float, bf16_t>(packed, bits, prefix, scale, mn, out, N, F, s);
+  if (dtype != store_dtype) return ACTNN_EDTYPE;
+  switch (dtype) {
+    case ACTNN_F32: return launch_unpack_rows<float, float>(packed, bits, prefix, scale, mn, out, N, F, s);
+    case ACTNN_F16: return launch_unpack_rows<__half, __half>(packed, bits, prefix, scale, mn, out, N, F, s);
+    case ACTNN_BF16: return launch_unpack_rows<bf16_t, bf16_t>(packed, bits, prefix, scale, mn, out, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
 
 extern "C" int actnn_bits_prefix(const int32_t* bits, int32_t* prefix, int64_t N, void* stream) {
   using namespace actnn;

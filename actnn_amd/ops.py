@@ -82,11 +82,11 @@ def start_quantize(input, scheme, known_minmax=None):
     `known_minmax`: per-group (mn, mx) of `input` when another kernel has produced them already."""
     if not config.compress_activation:
         return ("raw", input)
-    if scheme:
-        return ("scheme", input.dtype, scheme, scheme.start_quantization_bits(input, known_minmax))
-    saved = _quantize_fixed(input, known_minmax)
+    saved = quantize_on_device(input, scheme, known_minmax) if scheme else _quantize_fixed(input, known_minmax)
     if saved is not None:
         return ("packed", saved)
+    if scheme:
+        return ("scheme", input.dtype, scheme, scheme.start_quantization_bits(input, known_minmax))
     return ("fixed", input.dtype, no_scheme_compute_quantization_bits(input, known_minmax))
 
 
@@ -149,11 +149,12 @@ def dequantize_activation(quantized, q_input_shape):
     widen = q_scale.dtype == torch.bfloat16 and _stored_as_bf16(q_input_shape, quantized)
     N = q_input_shape[0]
     features = math.prod(q_input_shape[1:])
-    if (type(q_bits) is int and q_bits in (1, 2, 4, 8) and config.group_size == 256 and not config.simulate
+    mixed = isinstance(q_bits, torch.Tensor)
+    if ((mixed or type(q_bits) is int and q_bits in (1, 2, 4, 8)) and config.group_size == 256 and not config.simulate
             and N * features > 0):
         data = swap_to_device(q_input) if config.swap else q_input
-        out = ext_quantization.unpack_rows_fixed(data, q_bits, q_scale, q_min, N, features,
-                                                 torch.float32 if widen else q_scale.dtype)
+        unpack = ext_quantization.unpack_rows_mixed if mixed else ext_quantization.unpack_rows_fixed
+        out = unpack(data, q_bits, q_scale, q_min, N, features, torch.float32 if widen else q_scale.dtype)
     else:
         if widen:
             q_scale = q_scale.to(torch.float32)
@@ -188,36 +189,31 @@ def quantize_saved(input, scheme):
 
 def quantize_on_device(input, scheme, known_minmax=None):
     """start_quantize + finish_saved behind one library call, for the case the layers meet at every
-    step: a scheme whose widths are made on the device, whole groups of 256, per-group ranges,
-    in-kernel stochastic rounding, nothing swapped.  -> the saved tuple, or None when the case is
+    step: a scheme whose widths are made on the device, groups of 256, per-group ranges, in-kernel stochastic rounding, nothing swapped.  -> the saved tuple, or None when the case is
     another one (the caller then takes the two halves; nothing has been launched).  Same kernels on
     the same generator state: the result is the two halves' bit for bit."""
     if not (scheme and config.fused_quantize and config.compress_activation and config.pergroup
             and config.stochastic and not config.simulate and not config.swap and config.group_size == 256):
         return None
-    if not (input.is_cuda and input.dtype in ext_quantization.g.DTYPE_CODE and input.dim() >= 2):
+    rows = _rows_on_device(input)
+    if rows is None:
         return None
-    N = input.shape[0]
-    fmt = channels_last_format(input)
-    flat = (input.permute(0, *range(2, input.dim()), 1) if fmt is not None else input).reshape(N, -1)
-    features = flat.shape[1]
-    if N == 0 or features == 0 or features % 256 != 0 or not flat.is_contiguous():
-        return None
+    N, features = rows.shape
     if known_minmax is not None:
         mn, mx = known_minmax
         if not (mn.dtype == input.dtype and mx.dtype == input.dtype and mn.numel() * 256 == input.numel()
-                and mx.numel() == mn.numel() and mn.is_contiguous() and mx.is_contiguous()):
+                and mx.numel() == mn.numel() and features % 256 == 0 and mn.is_contiguous() and mx.is_contiguous()):
             known_minmax = None
+        else:
+            rows = ext_quantization.g.aligned(rows)
     alloc = scheme.allocation_arguments(N, features // input.shape[1], input.device)
     if alloc is None:
         return None
-    q_input, q_bits, q_scale, mn = ext_quantization.quantize_activation_device(
-        flat.view(-1, 256), N, known_minmax, alloc)
+    alloc.store_dtype = _stored_dtype(input.dtype)
+    q_input, q_bits, q_scale, q_min = ext_quantization.quantize_activation_device(
+        rows.view(-1, 256) if features % 256 == 0 else rows, N, known_minmax, alloc)
     scheme.adopt_device_bits(q_bits, features, alloc)
-    q_min = mn.view(N, -1, 1)
-    if input.dtype == torch.float32:
-        q_scale, q_min = q_scale.to(torch.bfloat16), q_min.to(torch.bfloat16)
-    return _mark_saved(_Quantized((q_input, q_bits, q_scale, q_min)), input)
+    return _mark_saved(_Quantized((q_input, q_bits, q_scale, q_min.view(N, -1, 1))), input)
 
 
 def _mark_saved(q, input):
@@ -227,7 +223,8 @@ def _mark_saved(q, input):
 
 
 def finish_saved(started, input):
-    return _mark_saved(_Quantized(finish_quantize(started)), input)
+    saved = finish_quantize(started)
+    return saved if isinstance(saved, _Quantized) else _mark_saved(_Quantized(saved), input)
 
 
 # ------------------------------------------------------------------------------------------
@@ -245,13 +242,9 @@ def _conv_forward(ctx, forward_op, input, weight, bias, stride, padding, dilatio
     if known_minmax is not None and (known_minmax[0].dtype != input.dtype
                                      or known_minmax[0].numel() * config.group_size != input.numel()):
         known_minmax = None                  # e.g. the input was cast on its way here
-    quantized = quantize_on_device(input, scheme, known_minmax)
-    if quantized is not None:
-        output = forward_op(input, weight, bias, stride, padding, dilation, groups)
-    else:
-        started = start_quantize(input, scheme, known_minmax)
-        output = forward_op(input, weight, bias, stride, padding, dilation, groups)
-        quantized = finish_saved(started, input)
+    started = start_quantize(input, scheme, known_minmax)
+    output = forward_op(input, weight, bias, stride, padding, dilation, groups)
+    quantized = finish_saved(started, input)
     ctx.scheme = scheme
     ctx.saved = quantized, weight, bias
     ctx.other_args = (input.shape, stride, padding, dilation, groups)
@@ -436,13 +429,9 @@ def _fused_grad_weight_ok(quantized, shape, go):
 class linear(Function):
     @staticmethod
     def forward(ctx, input, weight, bias=None, scheme=None):
-        quantized = quantize_on_device(input, scheme)
-        if quantized is not None:
-            output = F.linear(input, weight, bias)
-        else:
-            started = start_quantize(input, scheme)
-            output = F.linear(input, weight, bias)
-            quantized = finish_saved(started, input)
+        started = start_quantize(input, scheme)
+        output = F.linear(input, weight, bias)
+        quantized = finish_saved(started, input)
         empty_cache(config.empty_cache_threshold)
         ctx.scheme = scheme
         ctx.saved = quantized, weight, bias

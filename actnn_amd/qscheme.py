@@ -152,9 +152,10 @@ class AllocationArgs:
     """What the allocation kernels need for one layer's input (allocate_bits_on_device's arguments,
     resolved): `factor` and `mult` of the sensitivity, start width and target sum of the widths,
     the sum the widths will have (fixed by the budget, so the stream can be sized without a look
-    at them), where the sensitivities go (a row of the step's pool, or None) and what the scheme
-    keeps to read them back."""
-    __slots__ = ("factor", "mult", "initial", "target", "total", "sens_out", "pending")
+    at them), where the sensitivities go (a row of the step's pool, or None), what the scheme
+    keeps to read them back, and the dtype in which scale and minimum are kept (None: the
+    activation's own)."""
+    __slots__ = ("factor", "mult", "initial", "target", "total", "sens_out", "pending", "store_dtype")
 
     def __init__(self, N, factor, mult, initial_bits, avg_bits, sens_out=None, pending=None):
         self.factor = float(factor)
@@ -165,6 +166,7 @@ class AllocationArgs:
         self.total = N * self.initial - taken
         self.sens_out = sens_out
         self.pending = pending
+        self.store_dtype = None
 
 
 class _LazyHost:

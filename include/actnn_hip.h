@@ -88,6 +88,11 @@ int actnn_pack_mixed(const void* data, const void* mn, const void* mx, const int
 int actnn_unpack_mixed(const int32_t* packed, const int32_t* bits, const int32_t* prefix,
                        const void* scale, const void* mn, void* out, int64_t N, int64_t G,
                        int64_t gs, int dtype, void* stream);
+/* The same for the [N, F] rows of actnn_quantize_rows: out [N, F] in dtype, 16-byte aligned; scale and
+ * mn, [N * ceil(F / 256)], in store_dtype (bfloat16 or the dtype itself for fp32, else the dtype). */
+int actnn_unpack_mixed_rows(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
+                            const void* mn, void* out, int64_t N, int64_t F, int dtype, int store_dtype,
+                            void* stream);
 
 /* ---------------------------------------------------------------------------------
  * pack_single_precision: one bit width (1, 2, 4 or 8) for the whole tensor; 8/bits
@@ -282,6 +287,10 @@ int actnn_batch_norm_forward_apply_relu(const void* x, void* y, const void* work
  *       -> actnn_batch_norm_forward_apply_relu;
  *   actnn_quantize_activation = [actnn_minimax of data as rows of 256 unless minmax_known]
  *       -> actnn_allocate_bits_device -> actnn_pack_mixed (gs = 256, in-kernel Philox mode).
+ *   actnn_quantize_rows = the same for [N, F] rows of any length at any element address, cut into
+ *       G = ceil(F / 256) groups with the last one padded with zeros (minmax_known: F % 256 == 0);
+ *       scale is written in store_dtype - the dtype of data, or bfloat16 for fp32 data, and then
+ *       mn_stored (else unused) receives the minima in it.
  * Every output pointer is required. */
 int actnn_batch_norm_forward_quantize(
     const void* x, const float* weight, const float* bias, float* running_mean, float* running_var, void* y,
@@ -294,6 +303,10 @@ int actnn_quantize_activation(const void* data, void* mn, void* mx, int minmax_k
                               const float* mult, int mult_per_sample, float* sensitivity, int32_t* bits,
                               int32_t* prefix, int initial_bits, int64_t target, void* scale, int32_t* packed,
                               uint64_t seed, uint64_t offset, int64_t N, int64_t G, int dtype, void* stream);
+int actnn_quantize_rows(const void* data, void* mn, void* mx, int minmax_known, float factor, const float* mult,
+                        int mult_per_sample, float* sensitivity, int32_t* bits, int32_t* prefix, int initial_bits,
+                        int64_t target, void* scale, void* mn_stored, int32_t* packed, uint64_t seed,
+                        uint64_t offset, int64_t N, int64_t F, int dtype, int store_dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------
  * Fused QLinear weight gradient: grad_w[O, I] = grad_out[M, O]^T @ dequant(x)[M, I] where x is

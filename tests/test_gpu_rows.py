@@ -3,7 +3,7 @@ composition of minimax, pack and unpack on the zero-padded rows, which the oracl
 import pytest
 import torch
 
-from actnn_amd import ops
+from actnn_amd import ops, qscheme
 from actnn_amd.conf import config
 from actnn_amd.cpp_extension import minimax as ext_minimax
 from actnn_amd.cpp_extension import quantization as ext_q
@@ -88,3 +88,28 @@ def test_special_values_survive_the_one_pass(dtype, channels_last):
         assert ops.dequantize_activation(saved, x.shape).stride() == x.stride()
     finally:
         config.reset()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("initial,avg", [(8, 2.0), (8, 3.7), (2, 1.3)])
+def test_rows_at_widths_of_their_own_equal_the_padded_composition(dtype, initial, avg):
+    for i, (N, F) in enumerate(SHAPES):
+        for shift in (0, 1):
+            x = _rows(N, F, dtype, shift, 31 * i + shift)
+            groups = _padded(x)
+            G = groups.shape[1]
+            mn, mx = ext_minimax.minimax(groups.view(-1, 256))
+            C, bits = qscheme.allocate_bits_on_device(mn, mx, N, F, 1.0, None, initial, avg)
+            mn, mx = mn.view(N, G, 1), mx.view(N, G, 1)
+            torch.manual_seed(i)
+            want, want_scale = ext_q.pack_mixed_precision(groups, mn, mx, bits, True)
+            alloc = qscheme.AllocationArgs(N, 256 / F, None, initial, avg)
+            alloc.store_dtype = store = ops._stored_dtype(dtype)
+            torch.manual_seed(i)
+            packed, bits2, scale, low = ext_q.quantize_activation_device(x, N, None, alloc)
+            assert torch.equal(bits2, bits) and torch.equal(packed, want), (N, F, shift)
+            want_scale, want_mn = want_scale.to(store), mn.to(store)
+            assert torch.equal(scale, want_scale) and torch.equal(low.view(N, G, 1), want_mn), (N, F, shift)
+            back = ext_q.unpack_rows_mixed(packed, bits2, scale, low.view(N, G, 1), N, F, dtype)
+            full = ext_q.unpack_mixed_precision(want, bits, want_scale.to(dtype), want_mn.to(dtype), N, G, 256)
+            assert torch.equal(back, full.view(N, -1)[:, :F]), (N, F, shift)
