@@ -648,16 +648,20 @@ class batch_norm(Function):
         return _batch_norm_backward(ctx, grad_output) + (None,)
 
 
-def _batch_norm_backward(ctx, grad_output, relu_mask=None):
+def _batch_norm_backward(ctx, grad_output, relu_mask=None, keep_masked=None):
     """`relu_mask`: the mask of a ReLU the batch norm's output went through (batch_norm_relu);
     `grad_output` is then the gradient of the ReLU's output, masked by the batch-norm passes as they
-    read it where they can, else by the ReLU's own backward pass first."""
+    read it where they can, else by the ReLU's own backward pass first.  `keep_masked`: a list that
+    receives the masked gradient (a tensor of its own)."""
     quantized, weight, running_mean, running_var, save_mean, save_var, training, eps, reserve = ctx.saved
 
     def relu_backward_first(grad):
         fmt = getattr(quantized, "memory_format", None)
         grad = ext_quantization.relu_backward(memory_order(grad.contiguous(memory_format=fmt)), relu_mask)
-        return logical_order(grad, fmt)
+        grad = logical_order(grad, fmt)
+        if keep_masked is not None:
+            keep_masked.append(grad)
+        return grad
 
     if (training and config.compress_activation and not config.simulate
             and config.group_size == 256 and config.fused_bn_backward):
@@ -673,9 +677,12 @@ def _batch_norm_backward(ctx, grad_output, relu_mask=None):
             # (batch_norm_relu exists only for shapes whose passes take the mask)
             if relu_mask is not None and not config.fused_bn_relu_backward:
                 grad_output, relu_mask = relu_backward_first(grad_output), None
+            masked = torch.empty_like(grad_output) if relu_mask is not None and keep_masked is not None else None
             grads = ext_backward_func.hip_batch_norm_backward_packed(
                 ctx.other_args, quantized, grad_output, weight, save_mean, save_var,
-                sumsq=_leaves_grad_sqnorm(), relu_mask=relu_mask)
+                sumsq=_leaves_grad_sqnorm(), relu_mask=relu_mask, masked=masked)
+            if masked is not None:
+                keep_masked.append(masked)
             del quantized, ctx.saved
             if ctx.scheme:
                 ctx.scheme.if_allocate_perlayer()
@@ -764,11 +771,10 @@ class batch_norm_add_relu(Function):
             # and this batch norm masks what it reads itself
             grads = _batch_norm_backward(ctx, grad_output, relu_mask=mask)
             return (grads[0], None) + grads[1:] + (None, None)
-        # the masked gradient is the residual's gradient, so it is written once and the batch norm reads it
-        grad = logical_order(ext_quantization.relu_backward(
-            memory_order(grad_output.contiguous(memory_format=fmt)), mask), fmt)
-        grads = _batch_norm_backward(ctx, grad)
-        return (grads[0], grad) + grads[1:] + (None, None)
+        # the masked gradient is the residual's gradient: the batch norm's first pass writes it as it masks
+        masked = [] if ctx.needs_input_grad[1] else None
+        grads = _batch_norm_backward(ctx, grad_output, relu_mask=mask, keep_masked=masked)
+        return (grads[0], masked[0] if masked else None) + grads[1:] + (None, None)
 
 
 class SkipGradient:

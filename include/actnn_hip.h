@@ -475,6 +475,16 @@ int actnn_batch_norm_backward_packed_relu(const int32_t* packed, const int32_t* 
                                           int64_t workspace_bytes, float* sumsq, int64_t sumsq_entries,
                                           int64_t N, int64_t C, int64_t HW, int dtype, int channels_last,
                                           void* stream);
+/* The same with the masked gradient - the gradient of a residual that was added before the ReLU -
+ * written to `masked` (laid out like grad_out, 16-byte aligned; null: not written). */
+int actnn_batch_norm_backward_packed_add_relu(const int32_t* packed, const int32_t* bits, const int32_t* prefix,
+                                          const void* scale, const void* mn, const void* grad_out,
+                                          const int32_t* relu_mask, void* masked, const float* weight,
+                                          const float* save_mean, const float* save_invstd, void* dx,
+                                          float* dweight, float* dbias, void* workspace,
+                                          int64_t workspace_bytes, float* sumsq, int64_t sumsq_entries,
+                                          int64_t N, int64_t C, int64_t HW, int dtype, int channels_last,
+                                          void* stream);
 
 /* Plain device-to-device streaming copy of `bytes` bytes (16-byte aligned pointers and
  * size); used by the benchmark to calibrate bandwidth counters.  No reference counterpart. */
