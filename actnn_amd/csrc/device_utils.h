@@ -171,23 +171,40 @@ ACTNN_DEV u32x4 load16_any(const bf16_t* p) { return *reinterpret_cast<const u32
 ACTNN_DEV void store16_any(float* p, u32x4 v) { *reinterpret_cast<u32x4_a4*>(p) = v; }
 ACTNN_DEV void store16_any(__half* p, u32x4 v) { *reinterpret_cast<u32x4_a2*>(p) = v; }
 ACTNN_DEV void store16_any(bf16_t* p, u32x4 v) { *reinterpret_cast<u32x4_a2*>(p) = v; }
-// the elements of one 16-byte vector that lie in the row
-template <typename T> ACTNN_DEV u32x4 load16_part(const T* p, int valid) {
+// One 16-byte vector of a row, of which only the first `valid` elements lie in it (the others count as 0).  The
+// load is never guarded: it reads what follows the row, or ends with the tensor (`last`: its last 16
+// bytes; a tensor holds at least that much), and row_vector_ends() drops what does not belong.  With guarded
+// loads each vector waited for the one before and the addresses filled the registers (f32 [32, 309123]
+// minimum and maximum: 18.6 us, 9.3 like this).
+struct RowVector { u32x4 v; int ends; };               // ends: elements that count, 256 * elements to shift out below
+template <typename T> ACTNN_DEV RowVector load16_row(const T* p, int valid, const T* last) {
   constexpr int E = 16 / sizeof(T);
-  u32x4 u = (u32x4){0, 0, 0, 0};
-  if (valid >= E) {
-    u = load16_any(p);
-  } else if (valid > 0) {
-    uint32_t w[4] = {0, 0, 0, 0};
+  const int64_t over = p - last;
+  RowVector r;
+  r.v = load16_any(over > 0 ? last : p);
+  r.ends = valid >= E ? E : valid <= 0 ? 0 : over > 0 ? valid | (int)over << 8 : valid;
+  return r;
+}
+template <typename T> ACTNN_DEV u32x4 row_vector_ends(const RowVector& r) {
+  constexpr int E = 16 / sizeof(T);
+  if (r.ends == E) return r.v;
+  uint32_t w[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
+  for (int i = r.ends >> 8; i > 0; --i) {
+    if constexpr (sizeof(T) == 4) {
+      w[0] = w[1]; w[1] = w[2]; w[2] = w[3];
+    } else {
 #pragma unroll
-    for (int k = 0; k < E - 1; ++k) {
-      if (k >= valid) continue;
-      if constexpr (sizeof(T) == 4) w[k] = reinterpret_cast<const uint32_t*>(p)[k];
-      else w[k / 2] |= (uint32_t)reinterpret_cast<const uint16_t*>(p)[k] << (16 * (k & 1));
+      for (int k = 0; k < 3; ++k) w[k] = __builtin_amdgcn_alignbit(w[k + 1], w[k], 16);
+      w[3] >>= 16;
     }
-    u = (u32x4){w[0], w[1], w[2], w[3]};
   }
-  return u;
+  const int count = r.ends & 255;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (sizeof(T) == 4) w[k] = k < count ? w[k] : 0u;
+    else w[k] = 2 * k >= count ? 0u : 2 * k + 1 == count ? w[k] & 0xffffu : w[k];
+  }
+  return (u32x4){w[0], w[1], w[2], w[3]};
 }
 template <typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
   constexpr int E = 16 / sizeof(T);
@@ -203,12 +220,6 @@ template <typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
     }
   }
 }
-ACTNN_DEV void raw8_load_part(const float* p, int valid, Raw8<float>& r) {
-  r.a = load16_part(p, valid);
-  r.b = load16_part(p + 4, valid - 4);
-}
-ACTNN_DEV void raw8_load_part(const __half* p, int valid, Raw8<__half>& r) { r.a = load16_part(p, valid); }
-ACTNN_DEV void raw8_load_part(const bf16_t* p, int valid, Raw8<bf16_t>& r) { r.a = load16_part(p, valid); }
 // how many elements of a row of F lie at `at` and behind (capped: only small counts matter)
 ACTNN_DEV int part_of_row(int64_t F, int64_t at) { return F - at < 1024 ? (int)(F - at) : 1024; }
 ACTNN_DEV void raw8_widen(const Raw8<float>& r, float (&v)[8]) {

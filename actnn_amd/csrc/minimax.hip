@@ -160,33 +160,29 @@ int launch_minimax(const void* data, void* mn, void* mx, int64_t M, int64_t D, h
 
 // Groups of 256 of rows of F elements at any address, the last group of a row padded with zeros (which count).
 // As the vector path: 64 lanes (fp32) or 32 lanes own a group with one 16-byte load each, eight groups a lane
-// in flight.  Copying the rows to padded ones first was two passes of its own (fp32 [32, 309123]: 16 us of the
-// 100 that packing and unpacking took, 49 now).
+// in flight.  Copying the rows to padded ones first was two passes of its own (fp32 [32, 309123]: 16.0 + 8.3 us
+// for the copy and its minimax, 9.3 now).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void minimax_rows_kernel(const T* __restrict__ data, T* __restrict__ mn,
                                                                 T* __restrict__ mx, uint32_t M, int64_t F,
-                                                                FastDiv groups) {
+                                                                FastDiv groups, const T* last) {
   constexpr int E = 16 / sizeof(T);
   constexpr int LPR = 256 / E;
   constexpr int kSlots = kThreads / LPR;
   constexpr int R = kRowsPerLaneGroup;
   const int sub = threadIdx.x % LPR;
   const uint32_t row0 = blockIdx.x * (kSlots * R) + threadIdx.x / LPR;
-  u32x4 u[R];
+  RowVector u[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const uint32_t row = row0 + r * kSlots;
-    u[r] = (u32x4){0, 0, 0, 0};
-    if (row < M) {
-      const uint32_t n = groups.div(row);
-      const int64_t at = (int64_t)(row - n * groups.d) * 256 + sub * E;
-      u[r] = load16_part(data + n * F + at, part_of_row(F, at));
-    }
+    const uint32_t row = row0 + r * kSlots, n = groups.div(row);
+    const int64_t at = (int64_t)(row - n * groups.d) * 256 + sub * E;
+    u[r] = load16_row(data + n * F + at, row < M ? part_of_row(F, at) : 0, last);
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     float lo = INFINITY, hi = -INFINITY;
-    Vec16<T>::minmax(u[r], lo, hi);
+    Vec16<T>::minmax(row_vector_ends<T>(u[r]), lo, hi);
     lanes_minmax<LPR / 16>(lo, hi);
     const uint32_t row = row0 + r * kSlots;
     if (sub == LPR - 1 && row < M) {
@@ -201,8 +197,9 @@ int launch_minimax_rows(const void* data, void* mn, void* mx, int64_t N, int64_t
   constexpr int kRows = kThreads / (256 * (int)sizeof(T) / 16) * kRowsPerLaneGroup;
   const int64_t G = (F + 255) / 256, M = N * G;
   if (M > 0x7fffffffLL - kRows) return ACTNN_EINVAL;
+  const T* d = static_cast<const T*>(data);
   minimax_rows_kernel<T><<<dim3((unsigned)((M + kRows - 1) / kRows)), dim3(kThreads), 0, s>>>(
-      static_cast<const T*>(data), static_cast<T*>(mn), static_cast<T*>(mx), (uint32_t)M, F, FastDiv((uint32_t)G));
+      d, static_cast<T*>(mn), static_cast<T*>(mx), (uint32_t)M, F, FastDiv((uint32_t)G), d + N * F - 16 / sizeof(T));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 

@@ -168,7 +168,7 @@ extern "C" int actnn_quantize_rows(const void* data, void* mn, void* mx, int min
                                    int store_dtype, void* stream) {
   using namespace actnn;
   if (!data || !mn || !mx || !bits || !prefix || !scale || !packed || !sensitivity) return ACTNN_EINVAL;
-  if (N <= 0 || F <= 0 || (minmax_known && F % 256 != 0)) return ACTNN_EINVAL;
+  if (N <= 0 || F <= 0 || N * F < 8 || (minmax_known && F % 256 != 0)) return ACTNN_EINVAL;   // (8: one 16-byte vector)
   if (dtype < ACTNN_F32 || dtype > ACTNN_BF16) return ACTNN_EDTYPE;
   if (dtype != store_dtype && (dtype != ACTNN_F32 || store_dtype != ACTNN_BF16)) return ACTNN_EDTYPE;
   if (dtype != store_dtype && !mn_stored) return ACTNN_EINVAL;

@@ -94,9 +94,8 @@ template <> struct IsBf16<bf16_t> { static constexpr bool value = true; };
 // Issue the loads of this lane's elements (and noise in deterministic mode) for its GPH groups.
 // The elements stay as loaded until their group is packed (16-bit types: 4 registers per group
 // rather than 8), which keeps the kernel within the registers of 8 waves per SIMD.
-// ROWS: `data` is a row of F elements at any address and elem_base an offset in it.
-template <typename T, bool DET, int GPH, bool ROWS>
-ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noise, int64_t elem_base, int64_t F,
+template <typename T, bool DET, int GPH>
+ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noise, int64_t elem_base,
                            int groups_valid, Raw8<T> (&v)[GPH], Raw8<T> (&nz)[DET ? GPH : 1]) {
   using TL = Tile<1, GPH>;
   const uint32_t lane = threadIdx.x & 31;
@@ -106,8 +105,7 @@ ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noi
     const int gl = TL::group_of(hw, q);
     if (gl < groups_valid) {
       const int64_t e = elem_base + (int64_t)gl * kGs + lane * 8;
-      if constexpr (ROWS) raw8_load_part(data + e, part_of_row(F, e), v[q]);
-      else raw8_load_nt(data + e, v[q]); // non-temporal for 16-bit types only (one instruction per line)
+      raw8_load_nt(data + e, v[q]);      // non-temporal for 16-bit types only (one instruction per line)
       if (DET) raw8_load_nt(noise + e, nz[DET ? q : 0]);
     } else {
       raw8_zero(v[q]);
@@ -188,7 +186,7 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
     const T* __restrict__ data, const T* __restrict__ mn, const T* __restrict__ mx,
     const int32_t* __restrict__ bits, const int32_t* __restrict__ prefix, S* __restrict__ scale,
     S* __restrict__ mn_out, int32_t* __restrict__ packed, const T* __restrict__ noise, uint64_t seed,
-    uint64_t offset, int64_t F, int64_t G, int blocks_per_sample) {
+    uint64_t offset, int64_t F, int64_t G, int blocks_per_sample, const T* last) {
   constexpr int GPH = Gph<T>::kPack;
   constexpr int kGroupsPerBlock = kHalfWaves * GPH;
   __shared__ float s_mul[kGroupsPerBlock];
@@ -208,14 +206,14 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
   // picks its 32 bytes out of LDS.
   constexpr bool kViaLds = sizeof(T) == 4 && !DET;
   __shared__ __align__(16) uint8_t s_stage[kViaLds ? kGroupsPerBlock * kGs * 4 : 16];
-  u32x4 st[kViaLds && ROWS ? 2 * GPH : 1];                       // ROWS: by way of registers, at any address
-  if constexpr (kViaLds && ROWS) {
+  constexpr int kRowVectors = sizeof(T) == 4 ? 2 * GPH : GPH;
+  RowVector st[ROWS ? kRowVectors : 1];                          // ROWS: by way of registers, at any address
+  if constexpr (ROWS) {
 #pragma unroll
-    for (int i = 0; i < 2 * GPH; ++i) {
-      const int gl = (threadIdx.x >> 6) * 2 * GPH + i;
-      const int64_t at = (gb + gl) * kGs + (threadIdx.x & 63) * 4;
-      st[i] = (u32x4){0, 0, 0, 0};
-      if (gl < groups_valid) st[i] = load16_part(data + n * F + at, part_of_row(F, at));
+    for (int i = 0; i < kRowVectors; ++i) {
+      const int gl = sizeof(T) == 4 ? (threadIdx.x >> 6) * 2 * GPH + i : Tile<1, GPH>::group_of(threadIdx.x >> 5, i);
+      const int64_t at = (gb + gl) * kGs + (sizeof(T) == 4 ? (threadIdx.x & 63) * 4 : (threadIdx.x & 31) * 8);
+      st[i] = load16_row(data + n * F + at, gl < groups_valid ? part_of_row(F, at) : 0, last);
     }
   } else if constexpr (kViaLds) {
     const int wave = threadIdx.x >> 6;
@@ -227,8 +225,7 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
         load_to_lds16_nt(data + elem_base + (int64_t)gl * kGs + wl * 4, s_stage + gl * (kGs * 4));
     }
   } else {
-    if constexpr (ROWS) load_groups<T, DET, GPH, true>(data + n * F, noise, gb * kGs, F, groups_valid, v, nz);
-    else load_groups<T, DET, GPH, false>(data, noise, elem_base, F, groups_valid, v, nz);
+    load_groups<T, DET, GPH>(data, noise, elem_base, groups_valid, v, nz);
   }
 
   const int b = bits[n];
@@ -244,10 +241,14 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
     s_mul[threadIdx.x] = mul;
     s_sub[threadIdx.x] = sub;
   }
-  if constexpr (kViaLds && ROWS) {
+  if constexpr (ROWS) {
 #pragma unroll
-    for (int i = 0; i < 2 * GPH; ++i)
-      *reinterpret_cast<u32x4*>(s_stage + ((threadIdx.x >> 6) * 2 * GPH + i) * (kGs * 4) + (threadIdx.x & 63) * 16) = st[i];
+    for (int i = 0; i < kRowVectors; ++i) {
+      if constexpr (sizeof(T) == 4)
+        *reinterpret_cast<u32x4*>(s_stage + ((threadIdx.x >> 6) * 2 * GPH + i) * (kGs * 4) + (threadIdx.x & 63) * 16) = row_vector_ends<T>(st[i]);
+      else
+        v[i].a = row_vector_ends<T>(st[i]);
+    }
   }
   __syncthreads();
   if constexpr (kViaLds) {
@@ -526,9 +527,11 @@ int launch_pack_groups(const void* data, const void* mn, const void* mx, const i
   const int64_t G = (F + kGs - 1) / kGs;
   const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
   if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
+  const T* d = static_cast<const T*>(data);
   pack_mixed_kernel<T, S, DET, ROWS><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
-      static_cast<const T*>(data), static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
-      static_cast<S*>(scale), static_cast<S*>(mn_out), packed, static_cast<const T*>(noise), seed, offset, F, G, (int)bps);
+      d, static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
+      static_cast<S*>(scale), static_cast<S*>(mn_out), packed, static_cast<const T*>(noise), seed, offset, F, G, (int)bps,
+      d + N * F - 16 / sizeof(T));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 

@@ -19,6 +19,7 @@ namespace actnn {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kFewest = 8;              // elements a tensor of rows has at least: one 16-byte vector
 constexpr int kFixedGs = 256;           // group size of the one-pass kernel and of rows of any length
 
 template <typename T, bool DET>
@@ -252,14 +253,14 @@ int launch_pack_bits(int bits, const T* data, const T* mn, const T* scale, int8_
 // four, for loads in flight), a lane 8 consecutive elements of each; the lanes fold their minima and maxima,
 // each takes over the scale (a double division) of one of the samples and hands it to the others.
 // Bound by the read: minimax, scale and pack as kernels of their own took 20.7 + 3.0 + 28.9 us at 4 bits on
-// bf16 [256, 200704]; with this one, packing and unpacking took 46.5 instead of 69.6 us.
+// bf16 [256, 200704], this one 28.3 us (34.2 when held to the 64 registers of eight waves: it spills).
 // KNOWN: the ranges come from another kernel.  ROWS: rows of F elements at any address, the last group
 // padded with zeros.  S: type of the scales and minima written (mn_out may be null if KNOWN).
 template <typename T, typename S, int BITS, bool KNOWN, bool ROWS>
 __global__ __launch_bounds__(kThreads) void quantize_fixed_kernel(
     const T* __restrict__ data, const T* __restrict__ mn_in, const T* __restrict__ mx_in, S* __restrict__ scale,
     S* __restrict__ mn_out, int8_t* __restrict__ packed, uint64_t seed, uint64_t offset, int64_t N, int64_t F,
-    int64_t G, int64_t rows) {
+    int64_t G, int64_t rows, const T* last) {
   constexpr int WPT = 8 / BITS;
   constexpr int U = WPT >= 4 ? 1 : 4 / WPT;              // rows of the stream a thread handles at a time
   constexpr int SPT = U * WPT;                           // samples
@@ -269,16 +270,28 @@ __global__ __launch_bounds__(kThreads) void quantize_fixed_kernel(
   const int64_t g = (int64_t)blockIdx.x * (kThreads / 32) + (threadIdx.x >> 5);
   const bool live = g < G;                               // (lanes stay with the others: they exchange data)
   const int64_t d0 = g * kFixedGs + lane * 8;
-  const int valid = ROWS && live ? part_of_row(F, d0) : 8;
+  const int valid = live ? part_of_row(F, d0) : 0;
   for (int64_t no0 = (int64_t)blockIdx.y * U; no0 < rows; no0 += (int64_t)gridDim.y * U) {
     const int64_t n0 = no0 * WPT;
     Raw8<T> raw[SPT];
+    if constexpr (ROWS) {
+      constexpr int V = sizeof(T) == 4 ? 2 : 1;
+      RowVector st[SPT][V];
 #pragma unroll
-    for (int s = 0; s < SPT; ++s) {
-      raw8_zero(raw[s]);
-      if (live && n0 + s < N) {
-        if constexpr (ROWS) raw8_load_part(data + (n0 + s) * F + d0, valid, raw[s]);
-        else raw8_load_nt(data + (n0 + s) * F + d0, raw[s]);
+      for (int s = 0; s < SPT; ++s)
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          st[s][i] = load16_row(data + (n0 + s) * F + d0 + 4 * i, n0 + s < N ? valid - 4 * i : 0, last);
+#pragma unroll
+      for (int s = 0; s < SPT; ++s) {
+        raw[s].a = row_vector_ends<T>(st[s][0]);
+        if constexpr (V == 2) raw[s].b = row_vector_ends<T>(st[s][1]);
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SPT; ++s) {
+        raw8_zero(raw[s]);
+        if (live && n0 + s < N) raw8_load_nt(data + (n0 + s) * F + d0, raw[s]);
       }
     }
     // this lane's share of the scales: the sample lane % SPT
@@ -355,13 +368,14 @@ int launch_fixed_bits(const void* data, const void* mn_in, const void* mx_in, in
   const T* d = static_cast<const T*>(data);
   const T* lo = static_cast<const T*>(mn_in);
   const T* hi = static_cast<const T*>(mx_in);
+  const T* last = d + N * F - 16 / sizeof(T);
   S* sc = static_cast<S*>(scale);
   S* m = static_cast<S*>(mn_out);
   switch (bits) {
 #define ACTNN_CASE(B_)                                                                              \
   case B_:                                                                                          \
     quantize_fixed_kernel<T, S, B_, KNOWN, ROWS>                                                    \
-        <<<grid, blk, 0, s>>>(d, lo, hi, sc, m, packed, seed, offset, N, F, G, rows);               \
+        <<<grid, blk, 0, s>>>(d, lo, hi, sc, m, packed, seed, offset, N, F, G, rows, last);         \
     break;
     ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(4) ACTNN_CASE(8)
 #undef ACTNN_CASE
@@ -488,7 +502,7 @@ extern "C" int actnn_quantize_fixed(const void* data, const void* mn_known, cons
   if (N < 0 || F < 0) return ACTNN_EINVAL;
   if (N == 0 || F == 0) return ACTNN_OK;
   if (!data || !scale || !packed || (!mn_known != !mx_known) || (!mn_known && !mn)) return ACTNN_EINVAL;
-  if (mn_known && F % kFixedGs != 0) return ACTNN_EINVAL;
+  if ((mn_known && F % kFixedGs != 0) || N * F < kFewest) return ACTNN_EINVAL;
   if ((mn_known && !aligned16(data)) || (reinterpret_cast<uintptr_t>(packed) & 7u) != 0) return ACTNN_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == ACTNN_F32 && store_dtype == ACTNN_BF16)

@@ -92,8 +92,8 @@ def start_quantize(input, scheme, known_minmax=None):
 
 def _rows_on_device(input):
     """The activation as contiguous [N, features] rows in the order of its memory when it is one the
-    row kernels take (a GPU tensor of a supported dtype that is not empty), else None."""
-    if not (input.is_cuda and input.dtype in ext_quantization.g.DTYPE_CODE and input.dim() >= 2 and input.numel() > 0):
+    row kernels take (a GPU tensor of a supported dtype with at least 16 bytes of any of them), else None."""
+    if not (input.is_cuda and input.dtype in ext_quantization.g.DTYPE_CODE and input.dim() >= 2 and input.numel() >= 8):
         return None
     return memory_order(input).reshape(input.shape[0], -1).contiguous()
 

@@ -111,7 +111,7 @@ int actnn_unpack_single(const int8_t* packed, int bits, const void* scale, const
                         void* out, int64_t N, int64_t G, int64_t gs, int dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------
- * Rows of any length at one width: data is [N, F], contiguous, at any element address; a row is cut
+ * Rows of any length at one width: data is [N, F] (N * F >= 8), contiguous, at any element address; a row is cut
  * into G = ceil(F / 256) groups of 256, the last one padded with zeros.
  *   actnn_quantize_fixed: minimum, maximum, scale and codes of every group in one pass: the stream
  *     actnn_minimax and actnn_pack_single give for the padded rows.  mn_known / mx_known: [N * G]
@@ -287,7 +287,7 @@ int actnn_batch_norm_forward_apply_relu(const void* x, void* y, const void* work
  *       -> actnn_batch_norm_forward_apply_relu;
  *   actnn_quantize_activation = [actnn_minimax of data as rows of 256 unless minmax_known]
  *       -> actnn_allocate_bits_device -> actnn_pack_mixed (gs = 256, in-kernel Philox mode).
- *   actnn_quantize_rows = the same for [N, F] rows of any length at any element address, cut into
+ *   actnn_quantize_rows = the same for [N, F] rows (N * F >= 8) of any length at any element address, cut into
  *       G = ceil(F / 256) groups with the last one padded with zeros (minmax_known: F % 256 == 0);
  *       scale is written in store_dtype - the dtype of data, or bfloat16 for fp32 data, and then
  *       mn_stored (else unused) receives the minima in it.

@@ -11,7 +11,7 @@ from actnn_amd.cpp_extension import quantization as ext_q
 pytestmark = pytest.mark.gpu
 
 DTYPES = [torch.float32, torch.float16, torch.bfloat16]
-SHAPES = [(1, 1), (2, 7), (5, 255), (3, 256), (4, 257), (9, 2049), (2, 4093), (65, 300), (7, 512)]
+SHAPES = [(8, 1), (1, 9), (3, 3), (2, 7), (5, 255), (3, 256), (4, 257), (9, 2049), (2, 4093), (65, 300), (7, 512)]
 
 
 def _rows(N, F, dtype, shift, seed):
