@@ -292,9 +292,153 @@ __global__ __launch_bounds__(THREADS) void allocate_kernel(const float* __restri
   }
 }
 
+// Thousands of items: a thread owns the items t, t + 1024, ... and all their steps in registers, so that the
+// patterns - a double product each, what the one-block kernel is bound by - are evaluated once, the widths
+// are counts over registers, and every access to memory is coalesced (the widths change over to runs of
+// consecutive items through LDS).  A lane starts with the step its number says, so that the lanes of a
+// histogram atomic hold different steps, as above.  8192 items: 23 - 28 us, 59 - 70 with allocate_kernel
+// (both beside the other kernels of a training step).
+template <int ITEMS>
+__global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __restrict__ sens, int32_t* __restrict__ bits,
+                                                             int32_t* __restrict__ prefix, int N, int initial,
+                                                             int64_t K) {
+  constexpr int kN = 1024, kSteps = 7;
+  constexpr int kPer = kBins / kN;
+  __shared__ double factors[8];
+  __shared__ uint32_t hist[kBins];
+  __shared__ uint32_t s_wave[kN / 64];
+  __shared__ uint32_t s_digit, s_above, s_inside;
+  __shared__ __align__(16) uint8_t s_width[kN * ITEMS];
+  const int t = threadIdx.x;
+  const int L = initial - 1;
+  const bool select = K > 0 && K < (int64_t)N * L;     // otherwise nothing or everything is taken
+  uint32_t cut = 0, left = 0;
+  uint32_t key[ITEMS][kSteps];
+  if (select) {
+    float C[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) C[k] = t + k * kN < N ? sens[t + k * kN] : 0.0f;
+    if (t < L) factors[t] = kStepFactor[initial - t];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) hist[k * kN + t] = 0;
+    __syncthreads();
+    int l = t % L;
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      if (j < L) {
+        const double f = factors[l];
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) key[k][j] = step_order(C[k], f);
+      }
+      l = l + 1 == L ? 0 : l + 1;
+    }
+    left = (uint32_t)K;
+#pragma unroll 1
+    for (int pass = 0; pass < 3; ++pass) {
+      const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0, width = pass == 2 ? 10 : 11;
+      const uint32_t last = (1u << width) - 1u;
+      if (pass > 0) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) hist[k * kN + t] = 0;
+        __syncthreads();
+      }
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) {
+        if (j < L) {
+#pragma unroll
+          for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t o = key[k][j];
+            // (the dearest steps in the last bin; a shift by 32 is what pass 0 would ask for)
+            if (t + k * kN < N && (pass == 0 || (o >> (shift + width)) == cut)) atomicAdd(&hist[last - ((o >> shift) & last)], 1u);
+          }
+        }
+      }
+      __syncthreads();
+      uint32_t h[kPer], mine = 0;
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        h[k] = hist[t * kPer + k];
+        mine += h[k];
+      }
+      uint32_t all;
+      uint32_t before = block_scan<kN>(mine, s_wave, all) - mine;
+      if (before < left && left <= before + mine) {    // one thread: the step sought lies in one of its bins
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+          if (before < left && left <= before + h[k]) {
+            s_digit = last - (t * kPer + k);
+            s_above = before;
+            s_inside = h[k];
+            before = 0xffffffffu - h[k];               // found: no later bin compares
+          } else {
+            before += h[k];
+          }
+        }
+      }
+      __syncthreads();
+      cut = (cut << width) | s_digit;
+      left -= s_above;
+      if (left == s_inside) {                          // the whole bin is taken: its lower end is the cut
+        cut = (cut << shift) - 1u;                     // (no step has the pattern 0: that is a NaN's)
+        left = 0;
+        break;
+      }
+    }
+  }
+  uint32_t behind = 0;                                 // steps of the cost `cut` that items further back hold
+#pragma unroll
+  for (int k = ITEMS - 1; k >= 0; --k) {
+    int b = K <= 0 ? initial : 1;
+    if (select) {
+      uint32_t above = 0, equal = 0;
+      const bool live = t + k * kN < N;
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) {
+        if (j < L && live) {
+          above += key[k][j] > cut ? 1u : 0u;
+          equal += key[k][j] == cut ? 1u : 0u;
+        }
+      }
+      uint32_t taken = 0;
+      if (left > 0) {                                  // (the same for all threads) not all of them are taken
+        __syncthreads();
+        uint32_t all;
+        const uint32_t upto = block_scan<kN>(equal, s_wave, all);
+        const uint32_t later = behind + (all - upto);
+        const uint32_t room = left > later ? left - later : 0u;
+        taken = equal < room ? equal : room;
+        behind += all;
+      }
+      b = initial - (int)(above + taken);
+    }
+    s_width[t + k * kN] = (uint8_t)b;
+  }
+  __syncthreads();
+  // widths and their exclusive prefix, a run of ITEMS consecutive items per thread
+  int w[ITEMS];
+  uint32_t sum = 0;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    w[k] = t * ITEMS + k < N ? (int)s_width[t * ITEMS + k] : 0;
+    sum += (uint32_t)w[k];
+  }
+  uint32_t all;
+  uint32_t at = block_scan<kN>(sum, s_wave, all) - sum;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    if (t * ITEMS + k < N) {
+      bits[t * ITEMS + k] = w[k];
+      if (prefix) prefix[t * ITEMS + k] = (int32_t)at;
+      at += (uint32_t)w[k];
+    }
+  }
+  if (prefix && t == 0) prefix[N] = (int32_t)all;
+}
+
 // As many threads as have work, and their candidates in registers while they fit.  Measured (bf16, start
 // width 8): 64 items 4.2 us, 128 items 4.6 us with 256 threads; 256 items 5.2 us, 512 items 5.6 us (9.3 us
-// with 256 threads), 1100 items 7.3 us, 8192 items 44 us with 1024.  Ranking every candidate against
+// with 256 threads), 1100 items 7.3 us with 1024;
+// more items: see allocate_many_kernel, up to the 8192 whose steps fit the registers of one block.  Ranking every candidate against
 // every other by a grid of blocks, and scanning the widths in a launch of its own, took 6.5 + 2.8 us at 32
 // items, 7.7 + 5.3 us at 256, and stopped at 8192 candidates.
 int launch_allocate(const float* sens, int32_t* bits, int32_t* prefix, int64_t N, int initial, int64_t target,
@@ -302,6 +446,9 @@ int launch_allocate(const float* sens, int32_t* bits, int32_t* prefix, int64_t N
   const int64_t K = N * initial - target, candidates = N * (initial > 1 ? initial - 1 : 1);
   if (candidates <= 256 * 4) allocate_kernel<256, 4><<<dim3(1), dim3(256), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else if (candidates <= 1024 * 8) allocate_kernel<1024, 8><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
+  else if (N <= 2048) allocate_many_kernel<2><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
+  else if (N <= 4096) allocate_many_kernel<4><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
+  else if (N <= 8192) allocate_many_kernel<8><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else if (candidates <= 1024 * 64 && N <= kLdsItems) allocate_kernel<1024, 64><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else allocate_kernel<1024, 0><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   ACTNN_RETURN_LAUNCH_STATUS();

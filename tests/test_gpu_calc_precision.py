@@ -111,12 +111,13 @@ def test_allocation_in_one_call_from_dirty_buffers(N):
         assert torch.equal(bits, first)
 
 
-@pytest.mark.parametrize("N,initial", [(146, 8), (147, 8), (1024, 2), (1170, 8), (1171, 8), (9362, 8), (9363, 8), (16385, 3),
+@pytest.mark.parametrize("N,initial", [(146, 8), (147, 8), (1024, 2), (1170, 8), (1171, 8), (2048, 8), (2049, 8),
+                                       (4097, 4), (8191, 8), (8192, 8), (8193, 8), (9362, 8), (9363, 8), (16385, 3),
                                        (40000, 8)])
 @pytest.mark.parametrize("coarse", [False, True])
 def test_allocation_of_large_batches_equals_the_host_routine(N, initial, coarse):
-    """Around the switches of the allocation kernel (256 / 1024 threads, candidates in registers, items in
-    LDS); coarse sensitivities make ties of which only some are taken."""
+    """Around the switches of the allocation kernels (256 / 1024 threads, items or candidates in registers,
+    items in LDS); coarse sensitivities make ties of which only some are taken."""
     g = torch.Generator().manual_seed(N)
     mx = torch.exp(torch.randn(N, generator=g))
     if coarse:
