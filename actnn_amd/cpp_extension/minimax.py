@@ -60,3 +60,24 @@ def sample_sqnorm(x):
         check(g.lib().actnn_sample_sqnorm(x.data_ptr(), part.data_ptr(), N, F, slices,
                                           g.DTYPE_CODE[x.dtype], g.stream_ptr(x.device)), "sample_sqnorm")
     return part.sum(1) if slices > 1 else part.view(N)
+
+
+def row_column_sums(x, with_sqnorm):
+    """(sum over the rows of a [N, F] tensor in its dtype, squared norm of every row as sample_sqnorm gives it
+    or None) from one read, or None where the kernel does not apply: few elements (torch's own reduction
+    is one launch), ragged rows, rows too long for a block, and under a graph of the backward pass."""
+    if (x.dim() != 2 or x.dtype not in g.DTYPE_CODE or not x.is_cuda or not x.is_contiguous() or torch.is_grad_enabled()
+            or x.numel() < 1 << 20 or x.data_ptr() % 16 != 0):
+        return None
+    N, F = x.shape
+    elems = 16 // x.element_size()
+    if F % elems != 0 or N > 65535 or (with_sqnorm and F > 1024 * elems):
+        return None
+    columns = torch.empty(F, dtype=x.dtype, device=x.device)
+    sq = torch.empty(N, dtype=torch.float32, device=x.device) if with_sqnorm else None
+    part = torch.empty((N + 15) // 16, F, dtype=torch.float32, device=x.device)
+    with g.on_device(x.device):
+        check(g.lib().actnn_row_column_sums(x.data_ptr(), columns.data_ptr(), sq.data_ptr() if with_sqnorm else None,
+                                            part.data_ptr(), N, F, g.DTYPE_CODE[x.dtype], g.stream_ptr(x.device)),
+              "row_column_sums")
+    return columns, sq

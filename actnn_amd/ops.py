@@ -12,6 +12,7 @@ from torch.nn.modules.utils import _pair, _single, _triple
 
 from .conf import config
 from .cpp_extension import backward_func as ext_backward_func
+from .cpp_extension import minimax as ext_minimax
 from .cpp_extension import quantization as ext_quantization
 from .utils import (channels_last_format, compute_tensor_bytes, empty_cache, get_memory_usage,
                     logical_order, memory_order, swap_to_cpu, swap_to_device)
@@ -440,11 +441,16 @@ class linear(Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        if ctx.scheme:
-            ctx.scheme.set_scale(grad_output)
         quantized, weight, bias = ctx.saved
         q_input_shape = ctx.other_args
         go = grad_output.reshape(-1, grad_output.shape[-1])
+        # the bias's gradient and the norms of the samples (rows, if there is one row each) from one read
+        need_bias = bias is not None and ctx.needs_input_grad[2]
+        sums = None
+        if need_bias:
+            sums = ext_minimax.row_column_sums(go, bool(ctx.scheme) and grad_output.dim() == 2 and ctx.scheme.wants_sqnorm(grad_output))
+        if ctx.scheme:
+            ctx.scheme.set_scale(grad_output, sums[1] if sums is not None else None)
         if _fused_grad_weight_ok(quantized, q_input_shape, go):
             # the weight gradient is computed straight from the packed stream (dequantised tiles
             # only ever exist in LDS), nothing is materialised
@@ -462,7 +468,9 @@ class linear(Function):
         del quantized, ctx.saved
         empty_cache(config.empty_cache_threshold)
         grad_input = go.mm(weight).view(*q_input_shape) if ctx.needs_input_grad[0] else None
-        grad_bias = go.sum(0) if bias is not None and ctx.needs_input_grad[2] else None
+        grad_bias = None
+        if need_bias:
+            grad_bias = sums[0] if sums is not None else go.sum(0)
         if ctx.scheme:
             ctx.scheme.if_allocate_perlayer()
         return grad_input, grad_weight, grad_bias, None

@@ -263,8 +263,14 @@ class QScheme(_LazyHost):
             return torch.where(scale == 0, scale.mean() + 1e-9, scale)     # samples not seen yet
         return self.scales
 
-    def set_scale(self, grad):
-        """Squared gradient norm per sample, kept as a running value (qscheme.py:47-55)."""
+    def wants_sqnorm(self, grad):
+        """True when set_scale(grad) reads the gradient for its samples' norms."""
+        return QScheme.update_scale and (config.use_gradient or not config.share_grad_sqnorm
+                                         or ext_backward_func.known_sumsq(grad) is None)
+
+    def set_scale(self, grad, sqnorm=None):
+        """Squared gradient norm per sample, kept as a running value (qscheme.py:47-55).  `sqnorm`: what
+        sample_sqnorm gives for `grad`, from a caller that read it anyway (wants_sqnorm)."""
         if QScheme.sensitivity_pool is not None:
             QScheme.sensitivity_pool.flush()        # (called from every backward: the first one queues the transfer)
         if not QScheme.update_scale:
@@ -275,7 +281,7 @@ class QScheme(_LazyHost):
                 self.scales = total / grad.shape[0]
                 return
         # squared L2 norm per sample, accumulated in fp32 in one pass over the gradient
-        sq = ext_minimax.sample_sqnorm(grad)
+        sq = sqnorm if sqnorm is not None else ext_minimax.sample_sqnorm(grad)
         if config.use_gradient:
             assert QScheme.batch is not None
             if self.scales.device != sq.device:

@@ -239,6 +239,14 @@ int actnn_calc_precision_dp(const float* A, const float* C, int64_t N, int max_b
 int actnn_sample_sqnorm(const void* x, float* part, int64_t N, int64_t F, int slices, int dtype,
                         void* stream);
 
+/* What a linear layer's backward wants of the gradient of its output x [N, F], from one read: columns[F]
+ * in dtype, the sum over the rows (fp32 additions in a fixed order, rounded once), and, if sqnorm is
+ * not null, sqnorm[N], what actnn_sample_sqnorm leaves with one slice (F up to 8192 in 16 bits, 4096 in
+ * fp32).  part: fp32 [ceil(N / 16), F].  F in whole 16-byte vectors, x and part 16-byte aligned.
+ * Replaces grad_output.sum(0) of ops.py:386-433 and the norms of qscheme.py:47-55. */
+int actnn_row_column_sums(const void* x, void* columns, float* sqnorm, float* part, int64_t N, int64_t F, int dtype,
+                          void* stream);
+
 /* Same allocation on the DEVICE for the case every layer uses at every step: all N items start
  * at initial_bits (1..8) with weight 1 and `target` is the bit budget, so exactly
  * N * initial_bits - target widths are taken away (clamped to [0, N * (initial_bits - 1)]).

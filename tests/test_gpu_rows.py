@@ -113,3 +113,23 @@ def test_rows_at_widths_of_their_own_equal_the_padded_composition(dtype, initial
             back = ext_q.unpack_rows_mixed(packed, bits2, scale, low.view(N, G, 1), N, F, dtype)
             full = ext_q.unpack_mixed_precision(want, bits, want_scale.to(dtype), want_mn.to(dtype), N, G, 256)
             assert torch.equal(back, full.view(N, -1)[:, :F]), (N, F, shift)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,F", [(1024, 1024), (1025, 2048), (2047, 1000), (150, 8192), (16384, 72)])
+def test_row_and_column_sums_from_one_read(dtype, N, F):
+    x = _rows(N, F, dtype, 0, N)
+    with_sq = F <= 1024 * 16 // x.element_size()
+    with torch.no_grad():
+        got = ext_minimax.row_column_sums(x, with_sq)
+    assert got is not None
+    # fp32 sums of N terms in runs of 16, then 16 partial sums side by side: under 2 * (16 + N / 256 + 5) roundings
+    exact, weight = x.double().sum(0), x.double().abs().sum(0)
+    eps = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    bound = 2 * (21 + N / 256) * 2.0 ** -24 * weight + eps * exact.abs()
+    assert bool(((got[0].double() - exact).abs() <= bound).all())
+    assert got[0].dtype == dtype
+    if with_sq:
+        slices = max(1, min(64, F // 8192))
+        if slices == 1:
+            assert torch.equal(got[1], ext_minimax.sample_sqnorm(x))
