@@ -38,7 +38,9 @@ ACTNN_DEV float finish_sensitivity(float sum, float factor, const float* mult, i
   return mult ? v * mult[n * mult_stride] : v;
 }
 
-// One block per sample: few samples of many groups.
+// One block per sample: few samples of many groups.  The running sums are chains of additions, but their terms
+// are loaded kAhead at a time: with one load per turn the pass was the latency of G / 256 loads in a row
+// (2 samples of 158080 groups in fp16: 171 us, 23.6 now; 3 of 21576 in bf16: 24.5 and 6.2 us).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void range_sqr_kernel(const T* __restrict__ mn,
                                                              const T* __restrict__ mx,
@@ -48,9 +50,17 @@ __global__ __launch_bounds__(kThreads) void range_sqr_kernel(const T* __restrict
   __shared__ float s_part[kThreads];
   const int64_t n = blockIdx.x;
   float acc = 0.0f;
-  for (int64_t g = threadIdx.x; g < G; g += kThreads) {
-    const float d = range_term(mn, mx, n * G + g);
-    acc = fmaf(d, d, acc);
+  constexpr int kAhead = 16;
+  for (int64_t g0 = threadIdx.x; g0 < G; g0 += kThreads * kAhead) {
+    float d[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int64_t g = g0 + j * kThreads < G ? g0 + j * kThreads : g0;      // (a valid address; dropped below)
+      d[j] = range_term(mn, mx, n * G + g);
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j)
+      if (g0 + j * kThreads < G) acc = fmaf(d[j], d[j], acc);
   }
   s_part[threadIdx.x] = acc;
   __syncthreads();
