@@ -6,7 +6,6 @@ import torch
 from .. import _lib
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
-COMPACT = 16          # ACTNN_COMPACT: scale and minimum of an fp32 activation are bfloat16
 
 
 def lib():

@@ -113,7 +113,7 @@ def hip_batch_norm_forward(input, weight, bias, running_mean, running_var, momen
     save_invstd = torch.empty(C, dtype=torch.float32, device=input.device)
     mn = mx = None
     if minmax:
-        groups = N * ((C * HW + 255) // 256)
+        groups = N * C * HW // 256
         mn = torch.empty(groups, dtype=input.dtype, device=input.device)
         mx = torch.empty(groups, dtype=input.dtype, device=input.device)
     with _glue.on_device(input.device):
@@ -137,7 +137,7 @@ def hip_batch_norm_forward_stats(input, weight, bias, running_mean, running_var,
     save_invstd = torch.empty(C, dtype=torch.float32, device=input.device)
     mn = mx = None
     if minmax:
-        groups = N * ((C * HW + 255) // 256)
+        groups = N * C * HW // 256
         mn = torch.empty(groups, dtype=input.dtype, device=input.device)
         mx = torch.empty(groups, dtype=input.dtype, device=input.device)
     with _glue.on_device(input.device):
@@ -164,7 +164,7 @@ def hip_batch_norm_forward_apply(input, workspace, bits=None, mn=None, mx=None, 
     packed = scale = prefix = None
     seed = offset = 0
     if bits is not None:
-        G = (C * HW + 255) // 256
+        G = C * HW // 256
         total, prefix = _bits_info(bits)
         packed = torch.empty(total * G * 8, dtype=torch.int32, device=input.device)
         scale = torch.empty(N, G, 1, dtype=input.dtype, device=input.device)
@@ -222,8 +222,7 @@ def hip_batch_norm_forward_quantize(input, geo, weight, bias, running_mean, runn
     -> (output, save_mean, save_invstd, mn, mx, bits, packed, scale), what
     hip_batch_norm_forward_stats, allocate_bits_device and hip_batch_norm_forward_apply return one
     after the other.  `geo` from hip_batch_norm_quantize_geometry, `alloc` the scheme's
-    AllocationArgs (factor, mult, initial, target, total, sens_out; with a `store_dtype` of bfloat16
-    mn and scale of an fp32 input come back in it).  With `relu`
+    AllocationArgs (factor, mult, initial, target, total, sens_out).  With `relu`
     (hip_batch_norm_relu_applies) the output is relu(bn(input)) - relu(bn(input) + residual) with a
     `residual` laid out like the input - and the tuple ends with the ReLU's mask and the group
     min / max of the output."""
@@ -232,8 +231,7 @@ def hip_batch_norm_forward_quantize(input, geo, weight, bias, running_mean, runn
     dev, dtype = input.device, input.dtype
     code = _glue.DTYPE_CODE[dtype]
     ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
-    G = (C * HW + 255) // 256
-    compact = dtype == torch.float32 and alloc.store_dtype == torch.bfloat16
+    G = C * HW // 256
     f32, i32 = torch.float32, torch.int32
     ws = torch.empty(ws_bytes // 4, dtype=f32, device=dev)
     save_mean = torch.empty(C, dtype=f32, device=dev)
@@ -245,8 +243,7 @@ def hip_batch_norm_forward_quantize(input, geo, weight, bias, running_mean, runn
     bits = torch.empty(N, dtype=i32, device=dev)
     prefix = torch.empty(N + 1, dtype=i32, device=dev)
     packed = torch.empty(alloc.total * G * 8, dtype=i32, device=dev)
-    # (compact: the minima behind the scales)
-    stored = torch.empty(2 if compact else 1, N, G, 1, dtype=torch.bfloat16 if compact else dtype, device=dev)
+    scale = torch.empty(N, G, 1, dtype=dtype, device=dev)
     mask = zmn = zmx = None
     if relu:
         mask = torch.empty(mask_words(N * C * HW), dtype=i32, device=dev)
@@ -259,15 +256,11 @@ def hip_batch_norm_forward_quantize(input, geo, weight, bias, running_mean, runn
             input.data_ptr(), _ptr(weight), _ptr(bias), _ptr(running_mean), _ptr(running_var), out.data_ptr(),
             save_mean.data_ptr(), save_invstd.data_ptr(), mn.data_ptr(), mx.data_ptr(), ws.data_ptr(), ws_bytes,
             alloc.factor, mult_ptr, per_sample, sens.data_ptr(), bits.data_ptr(), prefix.data_ptr(),
-            alloc.initial, alloc.target, stored.data_ptr(), packed.data_ptr(), seed, offset, _ptr(mask), _ptr(zmn),
-            _ptr(zmx), _ptr(residual), N, C, HW, float(momentum), float(eps), code | _glue.COMPACT if compact else code,
-            int(channels_last),
+            alloc.initial, alloc.target, scale.data_ptr(), packed.data_ptr(), seed, offset, _ptr(mask), _ptr(zmn),
+            _ptr(zmx), _ptr(residual), N, C, HW, float(momentum), float(eps), code, int(channels_last),
             _glue.stream_ptr(dev)),
             "batch_norm_forward_quantize")
     attach_bits_total(bits, alloc.total, prefix)
-    scale = stored[0]
-    if compact:
-        mn = stored[1].view(-1)
     if relu:
         return out, save_mean, save_invstd, mn, mx, bits, packed, scale, mask, zmn, zmx
     return out, save_mean, save_invstd, mn, mx, bits, packed, scale
@@ -358,10 +351,11 @@ def hip_batch_norm_backward_packed(shape, quantized, grad_output, weight, save_m
     lib = _glue.lib()
     code = _glue.DTYPE_CODE[grad_output.dtype]
     total, prefix = _bits_info(q_bits)
-    if q_input.numel() < total * ((C * HW + 255) // 256) * 8:
+    if q_input.numel() < total * (C * HW // 256) * 8:
         raise RuntimeError("batch_norm_backward_packed: packed stream is too short")
-    # an fp32 activation's scale and minimum in bf16 storage are widened as they are read (ops.py:129-131)
-    packed_code = code | _glue.COMPACT if q_scale.dtype != grad_output.dtype else code
+    if q_scale.dtype != grad_output.dtype:              # fp32 activation, bf16 storage: widened as
+        q_scale = q_scale.to(grad_output.dtype)         # dequantize_activation widens it (ops.py:129-131)
+        q_min = q_min.to(grad_output.dtype)
     ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
     dev = grad_output.device
     entries = _sumsq_entries(N, C, HW, code, int(channels_last)) if sumsq else 0
@@ -383,7 +377,7 @@ def hip_batch_norm_backward_packed(shape, quantized, grad_output, weight, save_m
                 grad_output.data_ptr(), _ptr(weight), save_mean.data_ptr(), save_invstd.data_ptr(),
                 grad_input.data_ptr(), grad_weight.data_ptr(), grad_bias.data_ptr(), ws.data_ptr(), ws_bytes,
                 ws.data_ptr() + ws_bytes if entries else None, entries,
-                N, C, HW, packed_code, int(channels_last), _glue.stream_ptr(dev)), "batch_norm_backward_packed")
+                N, C, HW, code, int(channels_last), _glue.stream_ptr(dev)), "batch_norm_backward_packed")
     if entries:
         _leave_sumsq(grad_input, ws[ws_bytes // 4:])
     return grad_input, grad_weight, grad_bias

@@ -76,27 +76,19 @@ template <> struct Chunk<bf16_t> {
 // Where a thread's chunk lies: the channel of its first element, how many of its elements belong
 // to that channel (>= kElems when the chunk does not cross a boundary; the rest belong to the
 // next channel - HW >= kElems is a precondition), and whether the chunk exists at all.
-//
-// Rows that are no whole number of quantisation groups: the chunks between the row's end and that of
-// its last group are `ghosts`.  The quantiser counts them as zeros, and its lane exchanges need their
-// threads; they read a valid address, and nothing of them reaches a sum or the output.
 struct Place {
   int64_t elem;        // offset of the chunk in the row
-  int64_t load;        // where the thread reads: elem, for chunks that do not exist a valid offset
   int64_t channel;     // channel of the first element
   int head;            // elements of the chunk in `channel`, clamped to kElems
-  bool active, ghost;
+  bool active;
 };
-ACTNN_DEV int64_t padded_row(int64_t F) { return (F + 255) & ~(int64_t)255; }
 template <int E> ACTNN_DEV Place place_of(int64_t F, int64_t HW) {
   Place p;
   p.elem = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * E;
   p.active = p.elem < F;
-  p.ghost = !p.active && p.elem < padded_row(F);
-  p.load = p.active ? p.elem : (int64_t)blockIdx.x * kThreads * E;  // a valid address; results dropped
-  if (!p.active && !p.ghost) p.elem = p.load;
-  p.channel = p.load / HW;
-  const int64_t left = (p.channel + 1) * HW - p.load;
+  if (!p.active) p.elem = (int64_t)blockIdx.x * kThreads * E;       // a valid address; results dropped
+  p.channel = p.elem / HW;
+  const int64_t left = (p.channel + 1) * HW - p.elem;
   p.head = left >= E ? E : (int)left;
   return p;
 }
@@ -163,7 +155,7 @@ ACTNN_DEV void fold_block(float* s_acc, int slots, const Place& p, int64_t first
 // thread for sample n in two steps, so that the loads of several samples can be in flight before
 // the first one is used.
 template <typename T> struct PlainInput {
-  static constexpr bool kRows = false, kGroups = false;
+  static constexpr bool kRows = false;
   static constexpr int kInFlight = 4;      // samples whose loads are issued before the first is used
   const T* p;            // already offset to the thread's chunk of sample 0
   int64_t F;
@@ -183,7 +175,7 @@ template <typename T> struct PlainInput {
 // transposes its 32 words, and lane l collects the two 32-bit halves of stream lane l >> 1 from
 // lanes l >> 1 and 32 + (l >> 1) (ds_bpermute) before it takes its four codes out of them.
 template <typename T> struct PackedInput {
-  static constexpr bool kRows = false, kGroups = true;      // kGroups: the lanes of a group work together
+  static constexpr bool kRows = false;
   static constexpr int kLanes = 256 / Chunk<T>::kElems;     // lanes that own a group: 32, or 64 for fp32
   static constexpr int kInFlight = 2;      // the decode needs registers: 2 measured faster than 1 and 4
   const int32_t* words;
@@ -194,15 +186,7 @@ template <typename T> struct PackedInput {
   int64_t G, g;          // groups per sample, this thread's group
   uint32_t lane32;       // lane within the group's kLanes lanes
   bool active;
-  bool compact;          // fp32: scale and mn are kept as bfloat16
   struct Raw { uint32_t lo, hi; float sc, m; int b; };
-  // entry base + i of scale or mn (base the same for the wave)
-  ACTNN_DEV float param(const T* p, int64_t base, uint32_t i) const {
-    if constexpr (sizeof(T) == 4) {
-      if (compact) return Conv<bf16_t>::load(reinterpret_cast<const bf16_t*>(p) + base, i);
-    }
-    return Conv<T>::load(p + base, i);
-  }
   // group `grp` of sample n, whose width b and first word (prefix[n] * G * 8) the caller knows
   ACTNN_DEV Raw fetch_known(int64_t n, int64_t grp, int b, int64_t first_word) const {
     Raw r{0u, 0u, 1.0f, 0.0f, b};
@@ -210,8 +194,8 @@ template <typename T> struct PackedInput {
       const int32_t* w = words + first_word + grp * b * 8;
       if ((int)lane32 < 8 * b) r.lo = (uint32_t)w[lane32];
       if (kLanes == 32 && (int)lane32 + 32 < 8 * b) r.hi = (uint32_t)w[lane32 + 32];
-      r.sc = param(scale, n * G, (uint32_t)grp);
-      r.m = param(mn, n * G, (uint32_t)grp);
+      r.sc = Conv<T>::load(scale, n * G + grp);
+      r.m = Conv<T>::load(mn, n * G + grp);
     }
     return r;
   }
@@ -300,8 +284,6 @@ struct PackSink {
   int32_t* packed;
   uint64_t seed, offset;
   int64_t G;             // groups per sample
-  // fp32: where the scales (scale is then null) and the minima go as bfloat16, or null
-  bf16_t *scale16, *mn16;
   // backward apply only: when set, every wave leaves the sum of the squares of the gradient values
   // it wrote (as stored, i.e. rounded to T) in sumsq[(blockIdx.y * gridDim.x + blockIdx.x) * kWaves +
   // wave] - the gradient-norm statistic of the layer that receives this gradient, for free
@@ -425,14 +407,9 @@ template <typename T> struct ParamQueue {
     mul = 0.0f;
     sub = 0.0f;
     if (live) {
-      const float lo = Conv<T>::load(static_cast<const T*>(ps.mn), gi);
-      const float sc = GroupQuant<T, false>::prepare(lo, Conv<T>::load(static_cast<const T*>(ps.mx), gi), b, mul, sub);
-      if (sizeof(T) == 4 && ps.scale16) {
-        Conv<bf16_t>::store(ps.scale16, gi, sc);
-        Conv<bf16_t>::store(ps.mn16, gi, lo);
-      } else {
-        Conv<T>::store(static_cast<T*>(ps.scale), gi, sc);
-      }
+      const float sc = GroupQuant<T, false>::prepare(Conv<T>::load(static_cast<const T*>(ps.mn), gi),
+                                                     Conv<T>::load(static_cast<const T*>(ps.mx), gi), b, mul, sub);
+      Conv<T>::store(static_cast<T*>(ps.scale), gi, sc);
     }
   }
   // (the lanes that own a group: a half-wave, or the whole wave for fp32)
@@ -547,11 +524,11 @@ ACTNN_DEV void pack_chunk(const u32x4& ux, const uint32_t (&rw)[Noise<T>::kWords
   }
 }
 
-template <typename T> ACTNN_DEV void bind_input(PlainInput<T>& xs, const Place& p) { xs.p += p.load; }
+template <typename T> ACTNN_DEV void bind_input(PlainInput<T>& xs, const Place& p) { xs.p += p.elem; }
 template <typename T> ACTNN_DEV void bind_input(PackedInput<T>& xs, const Place& p) {
   xs.g = p.elem >> 8;
   xs.lane32 = threadIdx.x & (PackedInput<T>::kLanes - 1);
-  xs.active = p.active || p.ghost;
+  xs.active = p.active;
 }
 
 // Pass 1 of either direction.  Forward: per-channel sum(x) and sum(x*x) (+ per-group min/max of
@@ -593,17 +570,16 @@ __global__ __launch_bounds__(kThreads, 6) void bn_reduce_kernel(
       for (int j = 0; j < 4; ++j) Chunk<T>::widen(w[j], v + j * PD);
       float lo, hi;
       minmax_of<E>(v, lo, hi);
-      if (p.ghost) lo = hi = 0.0f;
       lanes_minmax<LPG / 16>(lo, hi);
-      if ((threadIdx.x & (LPG - 1)) == LPG - 1 && (p.active || p.ghost)) {
-        const int64_t g = n * ((F + 255) >> 8) + (p.elem >> 8);
+      if ((threadIdx.x & (LPG - 1)) == LPG - 1 && p.active) {
+        const int64_t g = n * (F >> 8) + (p.elem >> 8);
         Conv<T>::store(mn, g, lo);
         Conv<T>::store(mx, g, hi);
       }
     }
   };
 
-  const T* pd = BWD ? dy + p.load : nullptr;
+  const T* pd = BWD ? dy + p.elem : nullptr;
   int64_t n = n0;
   for (; n + kUnroll <= n1; n += kUnroll) {
     typename XS::Raw rx[kUnroll];
@@ -805,9 +781,8 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
   static_assert(!(PACK && BWD), "the packed copy is made by the forward pass");
   const Place p = place_of<E>(F, HW);
   float sumsq = 0.0f;
-  const bool taking_part = p.active || ((PACK || XS::kGroups) && p.ghost);
-  if (!BWD && !taking_part) return;    // whole quantisation groups (32 lanes) leave together
-  if (taking_part) {                    // (backward: the lanes meet again for the wave's sum below)
+  if (!BWD && !p.active) return;       // whole quantisation groups (32 lanes) leave together
+  if (p.active) {                      // (backward: the lanes meet again for the wave's sum below)
   bind_input(xs, p);
   float k0[NC], k1[NC];
 #pragma unroll
@@ -846,15 +821,8 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
     return u32x4{r[0], r[1], r[2], r[3]};
   };
 
-  const T* pd = BWD ? dy + p.load : nullptr;
-  T* po = out + p.load;
-  auto store = [&](T* at, const u32x4& v) {
-    if (!(PACK || XS::kGroups) || p.active) store_out(at, v);
-  };
-  // PACK: what the quantiser sees of the row (zeros behind its end) and where its octets are counted
-  const uint32_t keep = p.ghost ? 0u : 0xffffffffu;
-  auto padded = [&](const u32x4& v) -> u32x4 { return PACK ? v & keep : v; };
-  const int64_t Fp = PACK ? ps.G << 8 : F;
+  const T* pd = BWD ? dy + p.elem : nullptr;
+  T* po = out + p.elem;
   if constexpr (PACK && sizeof(T) == 4) {
     // fp32: 64 samples at a time (the wave's 64 lanes own the group), packed two by two
     const int lane = threadIdx.x & 63;
@@ -865,7 +833,7 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
       queue.get(jq, q.mul, q.sub);
       q.b = ps.bits[n];
       q.dst = ps.packed + (int64_t)ps.prefix[n] * ps.G * 8 + grp * q.b * 8;
-      q.octet = (uint64_t)((n * Fp + p.elem) >> 3);
+      q.octet = (uint64_t)((n * F + p.elem) >> 3);
       return q;
     };
     for (int64_t nb = n0; nb < n1; nb += 64) {
@@ -878,14 +846,14 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
       int64_t n = nb;
       for (; n + 2 <= ne; n += 2) {
         const typename XS::Raw rx0 = xs.fetch(n), rx1 = xs.fetch(n + 1);
-        const u32x4 ux0 = padded(xs.decode(rx0)), ux1 = padded(xs.decode(rx1));
-        store(po + n * F, apply(ux0, ux0));
-        store(po + (n + 1) * F, apply(ux1, ux1));
+        const u32x4 ux0 = xs.decode(rx0), ux1 = xs.decode(rx1);
+        store_out(po + n * F, apply(ux0, ux0));
+        store_out(po + (n + 1) * F, apply(ux1, ux1));
         pack_chunk_pair_f32(ps, ux0, params(n, (int)(n - nb)), ux1, params(n + 1, (int)(n + 1 - nb)), true);
       }
       if (n < ne) {
-        const u32x4 ux = padded(xs.decode(xs.fetch(n)));
-        store(po + n * F, apply(ux, ux));
+        const u32x4 ux = xs.decode(xs.fetch(n));
+        store_out(po + n * F, apply(ux, ux));
         const ChunkParams q = params(n, (int)(n - nb));
         pack_chunk_pair_f32(ps, ux, q, ux, q, false);
       }
@@ -910,12 +878,12 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
 #pragma unroll
         for (int u = 0; u < 2; ++u) rx[u] = xs.fetch(n + u);
         uint32_t rw[2][Noise<T>::kWords];
-        const uint64_t o = (uint64_t)((n * Fp + p.elem) >> 3);
-        noise_pair<T>(ps, o, o + (uint64_t)(Fp >> 3), rw[0], rw[1], true);
+        const uint64_t o = (uint64_t)((n * F + p.elem) >> 3);
+        noise_pair<T>(ps, o, o + (uint64_t)(F >> 3), rw[0], rw[1], true);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const u32x4 ux = padded(xs.decode(rx[u]));
-          store(po + (n + u) * F, apply(ux, ux));
+          const u32x4 ux = xs.decode(rx[u]);
+          store_out(po + (n + u) * F, apply(ux, ux));
           float mul, sub;
           queue.get((int)(n + u - nb), mul, sub);
           const int b = ps.bits[n + u];
@@ -924,10 +892,10 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
       }
       for (; n < ne; ++n) {
         const typename XS::Raw rx = xs.fetch(n);
-        const u32x4 ux = padded(xs.decode(rx));
-        store(po + n * F, apply(ux, ux));
+        const u32x4 ux = xs.decode(rx);
+        store_out(po + n * F, apply(ux, ux));
         uint32_t rw[Noise<T>::kWords];
-        Noise<T>::octet((uint64_t)((n * Fp + p.elem) >> 3), ps.seed, ps.offset, rw);
+        Noise<T>::octet((uint64_t)((n * F + p.elem) >> 3), ps.seed, ps.offset, rw);
         float mul, sub;
         queue.get((int)(n - nb), mul, sub);
         const int b = ps.bits[n];
@@ -947,17 +915,17 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const u32x4 ux = xs.decode(rx[u]);
-      store(po + (n + u) * F, apply(ux, BWD ? ud[u] : ux));
+      store_out(po + (n + u) * F, apply(ux, BWD ? ud[u] : ux));
     }
   }
   for (; n < n1; ++n) {
     const typename XS::Raw rx = xs.fetch(n);
     const u32x4 ux = xs.decode(rx);
-    store(po + n * F, apply(ux, BWD ? load_last(pd + n * F) : ux));
+    store_out(po + n * F, apply(ux, BWD ? load_last(pd + n * F) : ux));
   }
   }
   }
-  if (BWD && ps.sumsq) leave_wave_sum(ps.sumsq, p.active ? sumsq : 0.0f);
+  if (BWD && ps.sumsq) leave_wave_sum(ps.sumsq, sumsq);
 }
 
 // ------------------------------------------------------------------ channels-last tensors
@@ -1030,8 +998,8 @@ template <typename T> struct PackedRows {
     Raw raw{0u, 0u, 1.0f, 0.0f, cur_b};
     if ((int)in.lane32 < 8 * cur_b) raw.lo = (uint32_t)cur_words[at];
     if (PackedInput<T>::kLanes == 32 && (int)in.lane32 + 32 < 8 * cur_b) raw.hi = (uint32_t)cur_words[at + 32];
-    raw.sc = in.param(in.scale, block_group, lane_group);
-    raw.m = in.param(in.mn, block_group, lane_group);
+    raw.sc = Conv<T>::load(in.scale + block_group, lane_group);
+    raw.m = Conv<T>::load(in.mn + block_group, lane_group);
     return raw;
   }
   ACTNN_DEV u32x4 decode(const Raw& r) const {
@@ -1623,7 +1591,7 @@ bool make_plan(int64_t N, int64_t C, int64_t HW, int dtype, Plan& pl) {
   pl.slots = (int)slots;
   pl.split = HW % pl.elems != 0;
   pl.part_floats = pl.spans * nsplit * slots * 2;
-  pl.groups_align = true;                                 // (the last group of a row may be a part of one)
+  pl.groups_align = pl.F % 256 == 0;
   pl.big = N * pl.F * (dtype == ACTNN_F32 ? 4 : 2) > kLastLevelCacheBytes;
   return true;
 }
@@ -1897,9 +1865,9 @@ int backward_packed(const Plan& pl, const int32_t* packed, const int32_t* bits, 
                     const void* scale, const void* mn, const void* dy, const float* weight,
                     const float* save_mean, const float* save_invstd, void* dx, float* dweight,
                     float* dbias, float* ws, int64_t N, int64_t C, int64_t HW, float* sumsq, hipStream_t s,
-                    const int32_t* relu_mask = nullptr, void* masked = nullptr, bool compact = false) {
+                    const int32_t* relu_mask = nullptr, void* masked = nullptr) {
   const PackedInput<T> in{packed, bits, prefix, static_cast<const T*>(scale), static_cast<const T*>(mn),
-                          (pl.F + 255) / 256, 0, 0u, false, compact};
+                          pl.F / 256, 0, 0u, false};
   if (pl.channels_last) {
     // (32-bit positions inside a sample and over the tensor's groups)
     if (C * HW >= ((int64_t)1 << 32) || N * (pl.F / 256) >= 0x7fffffffLL) return ACTNN_EINVAL;
@@ -1965,19 +1933,13 @@ extern "C" int actnn_batch_norm_forward_apply(const void* x, void* y, const void
                                               int64_t N, int64_t C, int64_t HW, int dtype, int channels_last,
                                               void* stream) {
   using namespace actnn;
-  const bool compact = dtype == (ACTNN_F32 | ACTNN_COMPACT);
-  if (compact) dtype = ACTNN_F32;
   if (dtype < 0 || dtype > 2) return ACTNN_EDTYPE;
   Plan pl;
   if (!make_plan(N, C, HW, dtype, channels_last, pl)) return ACTNN_EINVAL;
   if (!x || !y || !workspace) return ACTNN_EINVAL;
   if (workspace_bytes < workspace_floats(pl, C) * (int64_t)sizeof(float)) return ACTNN_EINVAL;
   if ((!pl.any_shape && (!aligned16(x) || !aligned16(y))) || !aligned16(workspace)) return ACTNN_EALIGN;
-  PackSink sink{bits, prefix, mn, mx, scale, packed, seed, offset, (pl.F + 255) / 256};
-  if (compact) {                     // the scales, then the minima
-    sink.scale16 = static_cast<bf16_t*>(scale);
-    sink.mn16 = sink.scale16 + N * sink.G;
-  }
+  PackSink sink{bits, prefix, mn, mx, scale, packed, seed, offset, pl.F / 256};
   const bool pack = bits != nullptr;
   if (pack) {
     if (!pl.groups_align || !prefix || !mn || !mx || !scale || !packed) return ACTNN_EINVAL;
@@ -2016,8 +1978,8 @@ extern "C" int actnn_batch_norm_forward_apply_relu(const void* x, void* y, const
   // a wave's step is one 512-element block of the mask or the same half of two, every step of every block is whole
   if (!pl.groups_align || !relu_mask_shape(pl, C)) return ACTNN_EINVAL;
   if (pl.P > 0x7fffffffLL || C * HW >= ((int64_t)1 << 32) || N * (pl.F / 256) >= 0x7fffffffLL) return ACTNN_EINVAL;
-  PackSink sink{bits, prefix, mn, mx, scale, packed, seed, offset, pl.F / 256, nullptr, nullptr, nullptr, relu_mask, relu_mn,
-                relu_mx, residual};
+  PackSink sink{bits, prefix, mn, mx, scale, packed, seed, offset, pl.F / 256, nullptr, relu_mask, relu_mn, relu_mx,
+                residual};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float* ws = static_cast<const float*>(workspace);
   if (dtype == ACTNN_F16) return forward_apply_t<__half>(pl, x, y, ws, &sink, N, C, HW, s);
@@ -2190,8 +2152,6 @@ extern "C" int actnn_batch_norm_backward_packed(const int32_t* packed, const int
                                                 int64_t HW, int dtype, int channels_last,
                                                 void* stream) {
   using namespace actnn;
-  const bool compact = dtype == (ACTNN_F32 | ACTNN_COMPACT);
-  if (compact) dtype = ACTNN_F32;
   if (dtype != ACTNN_F16 && dtype != ACTNN_BF16 && dtype != ACTNN_F32) return ACTNN_EDTYPE;
   Plan pl;
   if (!make_plan(N, C, HW, dtype, channels_last, pl) || !pl.groups_align) return ACTNN_EINVAL;
@@ -2205,7 +2165,7 @@ extern "C" int actnn_batch_norm_backward_packed(const int32_t* packed, const int
   if (dtype == ACTNN_F16)
     return backward_packed<__half>(pl, packed, bits, prefix, scale, mn, dy, weight, save_mean, save_invstd, dx, dweight, dbias, ws, N, C, HW, sumsq, s);
   if (dtype == ACTNN_F32)
-    return backward_packed<float>(pl, packed, bits, prefix, scale, mn, dy, weight, save_mean, save_invstd, dx, dweight, dbias, ws, N, C, HW, sumsq, s, nullptr, nullptr, compact);
+    return backward_packed<float>(pl, packed, bits, prefix, scale, mn, dy, weight, save_mean, save_invstd, dx, dweight, dbias, ws, N, C, HW, sumsq, s);
   return backward_packed<bf16_t>(pl, packed, bits, prefix, scale, mn, dy, weight, save_mean, save_invstd, dx, dweight, dbias, ws, N, C, HW, sumsq, s);
 }
 

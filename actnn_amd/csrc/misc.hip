@@ -130,10 +130,7 @@ extern "C" int actnn_batch_norm_forward_quantize(
     int32_t* relu_mask, void* relu_mn, void* relu_mx, const void* residual, int64_t N, int64_t C, int64_t HW,
     double momentum, double eps, int dtype, int channels_last, void* stream) {
   if (!mn || !mx || !bits || !prefix || !scale || !packed || !sensitivity || !y) return ACTNN_EINVAL;
-  const bool compact = dtype == (ACTNN_F32 | ACTNN_COMPACT);
-  const int apply_dtype = dtype;
-  if (compact) dtype = ACTNN_F32;
-  if (N <= 0 || C <= 0 || HW <= 0 || (channels_last && (C * HW) % 256 != 0)) return ACTNN_EINVAL;
+  if (N <= 0 || C <= 0 || HW <= 0 || (C * HW) % 256 != 0) return ACTNN_EINVAL;
   const bool relu = relu_mask || relu_mn || relu_mx;
   if (relu && (!relu_mask || !relu_mn || !relu_mx)) return ACTNN_EINVAL;
   if (residual && !relu) return ACTNN_EINVAL;
@@ -147,14 +144,14 @@ extern "C" int actnn_batch_norm_forward_quantize(
                                           channels_last, stream);
   if (rc != ACTNN_OK) return rc;
   rc = actnn_allocate_bits_device(mn, mx, factor, mult, mult_per_sample, sensitivity, bits, prefix, N,
-                                  (C * HW + 255) / 256, initial_bits, target, dtype, stream);
+                                  C * HW / 256, initial_bits, target, dtype, stream);
   if (rc != ACTNN_OK) return rc;
   if (relu)
     return actnn_batch_norm_forward_apply_relu(x, y, workspace, workspace_bytes, bits, prefix, mn, mx, scale,
                                                packed, seed, offset, relu_mask, relu_mn, relu_mx, residual, N, C, HW,
                                                dtype, channels_last, stream);
   return actnn_batch_norm_forward_apply(x, y, workspace, workspace_bytes, bits, prefix, mn, mx, scale, packed,
-                                        seed, offset, N, C, HW, apply_dtype, channels_last, stream);
+                                        seed, offset, N, C, HW, dtype, channels_last, stream);
 }
 
 namespace actnn {

@@ -576,15 +576,17 @@ class batch_norm(Function):
         geo = _bn_quantize_geometry(input, running_mean, running_var, weight, bias, training, scheme)
         alloc = scheme.allocation_arguments(geo[0], geo[2], input.device) if geo is not None else None
         if alloc is not None:
-            alloc.store_dtype = _stored_dtype(input.dtype)
             fused = ext_backward_func.hip_batch_norm_forward_quantize(
                 input, geo, weight, bias, running_mean, running_var, exponential_average_factor, eps, alloc)
         if fused is not None:
             output, save_mean, save_var, mn, mx, q_bits, q_input, q_scale = fused
             N = geo[0]
             scheme.adopt_device_bits(q_bits, input.numel() // N, alloc)
+            q_min = mn.view(N, -1, 1)
+            if input.dtype == torch.float32:
+                q_scale, q_min = q_scale.to(torch.bfloat16), q_min.to(torch.bfloat16)
             reserve = None
-            started = ("done", _mark_saved(_Quantized((q_input, q_bits, q_scale, mn.view(N, -1, 1))), input))
+            started = ("done", _mark_saved(_Quantized((q_input, q_bits, q_scale, q_min)), input))
         elif ((scheme or fixed_width) and config.fused_bn_pack and config.stochastic
                 and _bn_shares_min_max(input, weight, bias, running_mean, running_var, training)
                 and ext_backward_func.hip_batch_norm_pack_applies(input, weight, bias, running_mean, running_var)):

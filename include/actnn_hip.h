@@ -23,9 +23,6 @@ extern "C" {
 #endif
 
 enum { ACTNN_F32 = 0, ACTNN_F16 = 1, ACTNN_BF16 = 2 };
-/* ACTNN_F32 | ACTNN_COMPACT, where a function says so: the scales and minima of fp32 data are kept as
- * bfloat16 (actnn/actnn/ops.py:115-116). */
-enum { ACTNN_COMPACT = 16 };
 
 enum {
   ACTNN_OK = 0,
@@ -296,9 +293,6 @@ int actnn_batch_norm_forward_apply_relu(const void* x, void* y, const void* work
  *       -> actnn_allocate_bits_device (G = C * HW / 256) -> actnn_batch_norm_forward_apply (with bits),
  *       or, with relu_mask / relu_mn / relu_mx given (all three; `residual` optional),
  *       -> actnn_batch_norm_forward_apply_relu;
- *       dtype ACTNN_F32 | ACTNN_COMPACT (also of actnn_batch_norm_forward_apply): scale receives N * G
- *       bfloat16 scales and, behind them, the N * G minima; G = ceil(C * HW / 256), in the default
- *       layout with the last group of a sample padded with zeros.
  *   actnn_quantize_activation = [actnn_minimax of data as rows of 256 unless minmax_known]
  *       -> actnn_allocate_bits_device -> actnn_pack_mixed (gs = 256, in-kernel Philox mode).
  *   actnn_quantize_rows = the same for [N, F] rows (N * F >= 8) of any length at any element address, cut into
@@ -467,8 +461,7 @@ int actnn_batch_norm_forward_apply(const void* x, void* y, const void* workspace
  * in that dtype; bits / prefix / scale / mn as for actnn_unpack_mixed):
  * both passes rebuild x in registers, bit for bit what actnn_unpack_mixed would write, so the
  * full-precision copy of x that ops.py:478 (dequantize_activation before
- * cudnn_batch_norm_backward) materialises never exists.
- * dtype ACTNN_F32 | ACTNN_COMPACT: scale and mn are bfloat16. */
+ * cudnn_batch_norm_backward) materialises never exists. */
 int actnn_batch_norm_backward_packed(const int32_t* packed, const int32_t* bits,
                                      const int32_t* prefix, const void* scale, const void* mn,
                                      const void* dy, const float* weight, const float* save_mean,

@@ -133,44 +133,3 @@ def test_row_and_column_sums_from_one_read(dtype, N, F):
         slices = max(1, min(64, F // 8192))
         if slices == 1:
             assert torch.equal(got[1], ext_minimax.sample_sqnorm(x))
-
-
-@pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("shape", [(3, 16, 5, 4), (65, 24, 9, 11), (33, 96, 27, 27), (2, 8, 64, 36), (130, 40, 3, 5), (1, 32, 4, 2)])
-def test_batch_norm_passes_on_ragged_rows(dtype, shape):
-    """Planes whose rows are no whole number of groups through the passes that share their reads with
-    the quantiser: output, statistics, saved stream and gradients are those of the separate steps."""
-    from actnn_amd import layers
-    from actnn_amd.cpp_extension import backward_func as bf
-    from actnn_amd.qbnscheme import QBNScheme
-    from actnn_amd.qscheme import QScheme
-
-    def run(fused):
-        config.reset(); QScheme.reset(); QBNScheme.reset()
-        config.fused_bn_pack = config.fused_bn_backward = fused
-        torch.manual_seed(3)
-        bn = layers.QBatchNorm2d(shape[1]).to("cuda").train()
-        with torch.no_grad():
-            bn.weight.uniform_(-1.0, 1.5)
-            bn.bias.normal_()
-        g = torch.Generator(device="cuda").manual_seed(1)
-        x = (torch.randn(shape, device="cuda", generator=g) * 2 + 0.3).to(dtype).requires_grad_()
-        go = torch.randn(shape, device="cuda", generator=g).to(dtype)
-        torch.cuda.manual_seed(9)
-        y = bn(x)
-        saved = y.grad_fn.saved[0]
-        kept = [saved[0].clone(), saved[1].clone(), saved[2].clone(), saved[3].clone()]
-        y.backward(go)
-        return [y.detach(), x.grad, bn.weight.grad, bn.bias.grad, bn.running_mean, bn.running_var] + kept
-
-    calls = []
-    real = bf.hip_batch_norm_forward_quantize
-    bf.hip_batch_norm_forward_quantize = lambda *a, **k: calls.append(1) or real(*a, **k)
-    try:
-        apart, together = run(False), run(True)
-    finally:
-        bf.hip_batch_norm_forward_quantize = real
-        config.reset(); QScheme.reset(); QBNScheme.reset()
-    assert len(calls) == 1
-    for i, (u, v) in enumerate(zip(apart, together)):
-        assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v), i
