@@ -240,7 +240,7 @@ __global__ __launch_bounds__(THREADS) void allocate_kernel(const float* __restri
             s_digit = last - (threadIdx.x * kPer + k);
             s_above = before;
             s_inside = h[k];
-            before = 0xffffffffu - h[k];               // found: no later bin compares
+            before = left;                             // found: it only grows from here, so no later bin compares
           } else {
             before += h[k];
           }
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
             s_digit = last - (t * kPer + k);
             s_above = before;
             s_inside = h[k];
-            before = 0xffffffffu - h[k];               // found: no later bin compares
+            before = left;                             // found: it only grows from here, so no later bin compares
           } else {
             before += h[k];
           }

@@ -130,6 +130,27 @@ def test_allocation_of_large_batches_equals_the_host_routine(N, initial, coarse)
         assert torch.equal(prefix[1:], torch.cumsum(bits, 0).to(torch.int32)) and int(prefix[0]) == 0
 
 
+@pytest.mark.parametrize("initial", [2, 3, 4, 8])
+@pytest.mark.parametrize("spread", [0.05, 0.3, 1.0, 3.0])
+def test_allocation_over_the_whole_range_of_budgets(initial, spread):
+    """Small batches (several bins of a pass to a thread) and larger ones, at mean widths from 1 to the start
+    width: the bins behind the one that is sought may hold more steps than it does."""
+    most = 1024 // (initial - 1)
+    g = torch.Generator().manual_seed(initial)
+    for N in (1, 2, 3, 4, 5, 9, 17, 33, 64, 100, most // 2, most - 1, most, most + 1, 2 * most, 6 * most):
+        C = torch.exp(spread * torch.randn(N, generator=g))
+        if N % 3 == 0:
+            C = C.round(decimals=1)                                   # ties
+        root = C.sqrt().to(DEV)                                       # (the sensitivity is the range's square)
+        whole = N * (initial - 1)
+        for taken in sorted({1, 2, 3, whole // 60, whole // 24, whole // 8, whole // 4, whole // 2, whole - whole // 8, whole - 1}):
+            target = N * initial - taken
+            sens, bits, prefix = ext_cp.allocate_bits_device(torch.zeros_like(root), root, N, 1.0, None, initial, target)
+            exp = _host(sens.cpu(), initial, target)
+            assert np.array_equal(bits.cpu().numpy(), exp.numpy()), (N, taken)
+            assert int(prefix[-1]) == int(exp.sum()) and int(prefix[0]) == 0
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("known", [False, True])
 def test_quantise_an_activation_in_one_call_equals_the_three_calls(dtype, known):
