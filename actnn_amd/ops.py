@@ -72,8 +72,12 @@ def no_scheme_compute_quantization_bits(input, known_minmax=None):
 
 def quantize_activation(input, scheme):
     """-> (q_input, q_bits, q_scale, q_min); for fp32 activations scale and min are kept as
-    bfloat16 (ops.py:99-118)."""
-    return finish_quantize(start_quantize(input, scheme))
+    bfloat16 (ops.py:99-118).  bfloat16 scales are widened when the tuple is restored, whatever the
+    activation's dtype was (quantize_saved restores a bfloat16 activation in its own); a
+    channels-last activation comes back in its layout."""
+    q = _Quantized(finish_quantize(start_quantize(input, scheme)))
+    q.memory_format = channels_last_format(input)
+    return q
 
 
 def start_quantize(input, scheme, known_minmax=None):

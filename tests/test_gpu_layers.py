@@ -7,7 +7,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 import actnn_amd
-from actnn_amd import QBNScheme, QModule, QScheme, config, set_optimization_level
+from actnn_amd import QBNScheme, QModule, QScheme, config, ops, set_optimization_level
 from actnn_amd.ops import dequantize_activation, quantize_saved
 from actnn_amd.resnet import resnet50
 from _util import DEV
@@ -506,6 +506,36 @@ def test_channels_last_saved_activation_round_trip():
     q2 = quantize_saved(x.permute(0, 2, 3, 1).contiguous(), None)       # same memory, default layout
     # (the fixed-width stream ends in one spare byte that no kernel writes, .cu:268)
     assert torch.equal(q[0][:-1], q2[0][:-1]) and torch.equal(q[2], q2[2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("level", ["L3", "L2"])
+@pytest.mark.parametrize("channels_last", [False, True])
+@pytest.mark.parametrize("shape", [(6, 8, 16, 16), (6, 5, 7, 9)])
+def test_quantize_activation_restores_alike_on_every_path(dtype, level, channels_last, shape):
+    """Scales and minima of either 32-bit or bfloat16 activations are widened, so the restored tensor
+    holds the codes' values in fp32 (fp16 stays fp16), with or without a scheme, in both layouts."""
+    scheme = None
+    if level == "L3":
+        scheme = QScheme(nn.Module(), num_locations=9)
+        scheme.set_scale(torch.randn(shape[0], 64, device=DEV))
+    else:
+        config.activation_compression_bits = [4]
+    x = torch.randn(shape, device=DEV).to(dtype)
+    if channels_last:
+        x = x.contiguous(memory_format=torch.channels_last)
+    q = ops.quantize_activation(x, scheme)
+    assert len(q) == 4 and isinstance(q, tuple)
+    back = dequantize_activation(q, x.shape)
+    wide = torch.float16 if dtype == torch.float16 else torch.float32
+    assert back.dtype == wide and back.shape == x.shape
+    codes, bits, scale, mn = q
+    want = ops.dequantize_and_unpack(codes, x.shape, bits, scale.to(wide), mn.to(wide))
+    want = want.view(shape[0], -1)[:, :x[0].numel()]
+    rows = x.permute(0, 2, 3, 1) if channels_last else x                   # in the order of memory
+    assert torch.equal((back.permute(0, 2, 3, 1) if channels_last else back).reshape(shape[0], -1), want)
+    step = (1 / scale.float()).amax() * (1 + 2 ** -7) + 2 ** -7 * x.float().abs().max()
+    assert (want.float() - rows.reshape(shape[0], -1).float()).abs().max() <= step
 
 
 def test_resnet50_channels_last_step_runs():
