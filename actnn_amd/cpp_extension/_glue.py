@@ -74,6 +74,15 @@ def aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def has_storage(t):
+    """False for tensors that only stand for others (a vmap over the backward pass hands such to it)."""
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 def philox_args(device, increment=4):
     """(seed, offset) of the device's default generator, advancing the offset - the
     counterpart of CUDAGeneratorImpl::philox_engine_inputs under the generator mutex

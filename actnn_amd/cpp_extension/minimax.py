@@ -65,9 +65,10 @@ def sample_sqnorm(x):
 def row_column_sums(x, with_sqnorm):
     """(sum over the rows of a [N, F] tensor in its dtype, squared norm of every row as sample_sqnorm gives it
     or None) from one read, or None where the kernel does not apply: few elements (torch's own reduction
-    is one launch), ragged rows, rows too long for a block, and under a graph of the backward pass."""
+    is one launch), ragged rows, rows too long for a block, under a graph of the backward pass, and for a
+    batch of gradients at once (torch.autograd.grad with is_grads_batched), which has no memory to read."""
     if (x.dim() != 2 or x.dtype not in g.DTYPE_CODE or not x.is_cuda or not x.is_contiguous() or torch.is_grad_enabled()
-            or x.numel() < 1 << 20 or x.data_ptr() % 16 != 0):
+            or x.numel() < 1 << 20 or not g.has_storage(x) or x.data_ptr() % 16 != 0):
         return None
     N, F = x.shape
     elems = 16 // x.element_size()

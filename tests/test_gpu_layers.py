@@ -538,6 +538,25 @@ def test_quantize_activation_restores_alike_on_every_path(dtype, level, channels
     assert (want.float() - rows.reshape(shape[0], -1).float()).abs().max() <= step
 
 
+def test_linear_backward_of_a_batch_of_gradients():
+    """is_grads_batched hands the backward pass a tensor without memory: as large as the one-read column
+    sums take, the gradients are those of one backward pass after the other."""
+    config.activation_compression_bits = [4]
+    config.adaptive_conv_scheme = config.adaptive_bn_scheme = False
+    torch.manual_seed(0)
+    layer = actnn_amd.QLinear(256, 1024).to(DEV)
+    x = torch.randn(1024, 256, device=DEV, requires_grad=True)
+    grads = torch.randn(3, 1024, 1024, device=DEV)
+    wanted = [x, layer.weight, layer.bias]
+    torch.manual_seed(1)
+    got = torch.autograd.grad(layer(x), wanted, grads, is_grads_batched=True)
+    for i in range(3):
+        torch.manual_seed(1)
+        for a, b in zip(got, torch.autograd.grad(layer(x), wanted, grads[i])):
+            # the same products summed in another order: 1024 terms, at most 1024 * 2^-24 of their 2-norm
+            assert (a[i] - b).norm() <= 1024 * 2.0 ** -24 * b.norm()
+
+
 def test_resnet50_channels_last_step_runs():
     torch.manual_seed(0)
     model = _cl(QModule(resnet50()))
