@@ -19,6 +19,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "../../include/actnn_hip.h"
@@ -123,12 +124,22 @@ extern "C" int actnn_calc_precision(int32_t* b, const float* C, const int32_t* w
   }
   // (sums of whole numbers below 2^53 are exact in any order)
   if (ordinary && whole < 9007199254740992.0 && !std::isnan(target)) {
-    take_steps(b, C, w, N, whole, target);
-    return ACTNN_OK;
+    try {
+      std::vector<int32_t> widths(b, b + N);
+      take_steps(widths.data(), C, w, N, whole, target);
+      std::copy(widths.begin(), widths.end(), b);
+      return ACTNN_OK;
+    } catch (const std::bad_alloc&) {
+      // all steps at once are up to 128 bytes an item; the heap below makes do with 16
+    }
   }
 
   std::vector<Cand> heap;
-  heap.reserve((size_t)N);
+  try {
+    heap.reserve((size_t)N);                                  // (never holds more)
+  } catch (const std::bad_alloc&) {
+    return ACTNN_ETOOBIG;
+  }
   double b_sum = 0.0;
   for (int64_t i = 0; i < N; ++i) {
     heap.push_back(Cand{step_delta(C[i], b[i], w[i]), i});

@@ -30,7 +30,7 @@ enum {
   ACTNN_EDTYPE = -2,   /* unknown dtype */
   ACTNN_EBITS = -3,    /* bit width outside what the operator supports */
   ACTNN_EALIGN = -4,   /* pointer not aligned as the kernel requires (16 bytes) */
-  ACTNN_ETOOBIG = -5   /* problem needs more scratch memory than the library's fixed buffer holds */
+  ACTNN_ETOOBIG = -5   /* problem needs more scratch memory than there is */
 };
 
 /* Human-readable text for a return code of this library (static storage). */
@@ -220,6 +220,7 @@ int actnn_max_pool2d_backward_cl_nibble(const void* grad_out, const uint8_t* idx
 
 /* ---------------------------------------------------------------------------------
  * calc_precision (HOST pointers): greedy bit allocation, mutates b in place.
+ * ACTNN_ETOOBIG (b unchanged) where there is no memory for 16 bytes an item.
  * Replaces calc_precision(b, C, w, target): calc_precision.cc:9-50.
  * ------------------------------------------------------------------------------- */
 int actnn_calc_precision(int32_t* b, const float* C, const int32_t* w, int64_t N, double target);

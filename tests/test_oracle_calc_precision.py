@@ -1,5 +1,7 @@
 """Greedy bit allocation: oracle pins, and the library's host entry point against the oracle."""
 import ctypes
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -75,6 +77,31 @@ def test_library_selection_and_heap_match_oracle(lib, kind):
     full = float((b0.astype(np.float64) * w).sum())
     for share in (0.9, 0.5, 0.3) if kind != "over_budget" else (1.0, 1.5):
         assert np.array_equal(_lib_calc(lib, b0, C, w, share * full), cp.calc_precision(b0, C, w, share * full))
+
+
+def test_library_without_memory_for_all_steps_takes_the_heap():
+    """In a process that may not have the memory of all candidate steps at once the widths are the same;
+    without memory for a heap of the items either, the call returns an error instead of ending the process."""
+    code = """
+import ctypes, resource, sys
+import numpy as np
+lib = ctypes.CDLL(sys.argv[1])
+lib.actnn_calc_precision.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int64, ctypes.c_double]
+N = 1 << 21
+C = np.random.default_rng(0).lognormal(0, 2, N).astype(np.float32)
+w = np.ones(N, np.int32)
+b = [np.full(N, 30, np.int32) for _ in range(3)]
+run = lambda b: lib.actnn_calc_precision(b.ctypes.data, C.ctypes.data, w.ctypes.data, N, float(30 * N - 2000))
+assert run(b[0]) == 0
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (96 << 20), -1))        # all steps: 243 MB, the heap: 34 MB
+assert run(b[1]) == 0 and np.array_equal(b[0], b[1]) and int(b[0].sum()) == 30 * N - 2000
+resource.setrlimit(resource.RLIMIT_AS, (used + (8 << 20), -1))
+assert run(b[2]) == -5 and int(b[2].min()) == 30
+"""
+    from actnn_amd import _lib
+    done = subprocess.run([sys.executable, "-c", code, str(_lib.LIB_PATH)], capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, done.stderr
 
 
 def test_library_known_answer_and_errors(lib):
