@@ -950,7 +950,9 @@ int launch_bwd(const void* gout, const int8_t* idx, void* gin, int64_t total, co
   const int preset = preset_of(g);
   DirectGeom q;
   const bool s1 = preset == 3;                           // threads: kStrip pixels of a column, or 2x2 pixels
-  if (preset != 0 && (!s1 || (g.Ho == g.H && g.Wo == g.W)) && total <= 0x7fffffffLL && planes * g.Ho * g.Wo <= 0x7fffffffLL &&
+  // (a window outside reads the plane's first one instead: there must be one)
+  if (preset != 0 && g.Ho > 0 && g.Wo > 0 && (!s1 || (g.Ho == g.H && g.Wo == g.W)) && total <= 0x7fffffffLL &&
+      planes * g.Ho * g.Wo <= 0x7fffffffLL &&
       direct_geometry(planes, s1 ? (g.H + kStrip - 1) / kStrip : (g.H + 1) / 2, s1 ? g.W : (g.W + 1) / 2, q)) {
     const dim3 grid = direct_grid(q), blk(kThreads);
     const T* go = static_cast<const T*>(gout);

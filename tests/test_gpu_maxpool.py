@@ -251,3 +251,20 @@ def test_large_results_are_streamed_and_equal(k, s, p):
     for i in range(0, 48, 16):
         part = ext_q.max_pool2d_backward(g[i:i + 16], idx[i:i + 16], x[i:i + 16].shape, k, s, p)
         assert torch.equal(part, whole[i:i + 16])
+
+
+@pytest.mark.parametrize("k,s,p", [(3, 2, 1), (3, 2, 0), (2, 2, 0), (3, 1, 1)])
+@pytest.mark.parametrize("nibble", [False, True])
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_backward_without_any_window_is_zero(k, s, p, nibble, channels_last):
+    """No output rows (a plane smaller than a window without padding): the gradient is zero."""
+    from actnn_amd import _lib
+    lib = _lib.load()
+    gin = torch.full((2, 8, 1, 5), float("nan"), device=DEV)
+    some = torch.full((64,), float("nan"), device=DEV)
+    idx = torch.zeros(64, dtype=torch.uint8, device=DEV)
+    name = "actnn_max_pool2d_backward" + ("_cl" if channels_last else "") + ("_nibble" if nibble else "")
+    rc = getattr(lib, name)(some.data_ptr(), idx.data_ptr(), gin.data_ptr(), 2, 8, 1, 5, 0, 2, k, k, s, s, p, p, 0,
+                            torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(gin, torch.zeros_like(gin))
