@@ -1198,7 +1198,7 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_kernel(
 // input pixel where the general kernel needs 2.25 (3x3).  Every pixel adds its windows in the
 // general kernel's order (rows, then columns), hence the same bits.  grad_in is written once and
 // not read: streamed stores (measured 0.104 -> 0.079 ms on f16 [256,64,112,112]).
-template <typename T, int K, int P, bool NIB, bool EVEN>
+template <typename T, int K, int P, bool NIB, bool EVEN, bool NT>
 __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
     const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, ClGeom q, PoolGeom g) {
   constexpr int E = PoolChunk<T>::kElems;
@@ -1208,8 +1208,9 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
   const ClAt at = cl_at(q);                            // rows and columns of windows
   if (!at.live) return;
   const uint32_t C = q.cpp * E;
-  const int64_t image_o = (int64_t)at.n * g.Ho * g.Wo * C;
-  const uint32_t lane_o = (at.row * (uint32_t)g.Wo + at.col) * C + at.chunk * E;   // window (row, col) of this chunk in the image
+  constexpr bool kFlat = EVEN && NIB;
+  const int64_t image_o = kFlat ? (int64_t)at.n * q.per_image * E : (int64_t)at.n * g.Ho * g.Wo * C;
+  const uint32_t lane_o = kFlat ? at.i * E : (at.row * (uint32_t)g.Wo + at.col) * C + at.chunk * E;   // window (row, col) of this chunk in the image
   const T* gimg = gout + image_o;
   const int8_t* iimg = idx + IndexFields<NIB>::byte_of(image_o);
   u32x4 raw[NWIN][NWIN];
@@ -1258,8 +1259,11 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
   for (int rr = 0; rr < 2; ++rr)
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc)
-      if (EVEN || (2 * at.row + rr < (uint32_t)g.H && 2 * at.col + cc < (uint32_t)g.W))
-        narrow_chunk_nt<T, E>(out + ((int64_t)rr * g.W + cc) * C + lane_in, acc[rr][cc]);
+      if (EVEN || (2 * at.row + rr < (uint32_t)g.H && 2 * at.col + cc < (uint32_t)g.W)) {
+        T* pixel = out + ((int64_t)rr * g.W + cc) * C + lane_in;
+        if (NT) narrow_chunk_nt<T, E>(pixel, acc[rr][cc]);
+        else narrow_chunk<T, E>(pixel, acc[rr][cc]);
+      }
 }
 
 // Backward for 3x3 stride 1 pad 1: one pixel per thread, the loads of its nine windows issued together.
@@ -1356,11 +1360,16 @@ int launch_cl(bool forward, const void* a, const int8_t* idx_in, int8_t* idx_out
     const T* go = static_cast<const T*>(a);
     T* gi = static_cast<T*>(out);
     const bool even = g.H == 2 * g.Ho && g.W == 2 * g.Wo;
-    if (p == 1 && even) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, true><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
-    else if (p == 1) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
-    else if (p == 2 && even) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, true><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
-    else if (p == 2) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
-    else max_pool2d_backward_cl_s2_kernel<T, 3, 0, NIB, false><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    auto launch = [&](auto nt) {
+      constexpr bool NT = decltype(nt)::value;
+      if (p == 1 && even) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, true, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+      else if (p == 1) max_pool2d_backward_cl_s2_kernel<T, 3, 1, NIB, false, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+      else if (p == 2 && even) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, true, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+      else if (p == 2) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, false, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+      else max_pool2d_backward_cl_s2_kernel<T, 3, 0, NIB, false, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
+    };
+    if (C * (int64_t)sizeof(T) % 64 == 0) launch(std::true_type());
+    else launch(std::false_type());
   } else {
     max_pool2d_backward_cl_kernel<T, NIB><<<dim3(xcd_grid(blocks)), dim3(kThreads), 0, s>>>(
         static_cast<const T*>(a), idx_in, static_cast<T*>(out), chunks, cpp, C, g);
