@@ -246,13 +246,13 @@ inline int preset_of(const PoolGeom& g) {
   return 0;
 }
 
-template <typename T, bool NIB>                  // NIB: Wo even, so the two outputs of a byte sit in one row
+template <typename T, int PRESET, bool NIB>      // NIB: Wo even, so the two outputs of a byte sit in one row
 __global__ __launch_bounds__(kThreads) void max_pool2d_forward_lds_kernel(
     const T* __restrict__ x, T* __restrict__ y, int8_t* __restrict__ idx, int64_t total_in,
     PoolGeom g, int rows_per_band, int bands) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* s_in = reinterpret_cast<T*>(smem);
-  const Win<0> k(g);
+  const Win<PRESET> k(g);
   const int64_t nc = blockIdx.x / bands;
   const int ho0 = (int)(blockIdx.x % bands) * rows_per_band;
   const int rows_out = g.Ho - ho0 < rows_per_band ? g.Ho - ho0 : rows_per_band;
@@ -652,11 +652,10 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_forward_direct_s1_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Stride-2 fast path, forward of the 16-bit types and backward of all (3x3 pad 1 and 2x2 pad 0 with W % 8 == 0, Wo == W / 2,
-// Ho == H / 2): the shapes of every stem / VGG-style pooling layer.  (bf16 [64,64,112,112], 3x3: forward
-// 28 us, backward 26 us, against 59 and 38 us of the direct kernels on [64,64,114,114].  For fp32, whose
-// elements are loads of a whole dword, the direct forward is the faster one - 67 against 69 us, 2x2 40
-// against 63 us - and the backward pass keeps this one: 46 against 69 us.)  A thread produces 4 adjacent outputs from three
+// Stride-2 fast path (3x3 pad 1 and 2x2 pad 0 with W % 8 == 0, Wo == W / 2, Ho == H / 2; which of them take it
+// forward is said in launch_fwd): the shapes of every stem / VGG-style pooling layer.  (bf16 [64,64,112,112],
+// 3x3: forward 28 us, backward 26 us, against 59 and 38 us of the direct kernels on [64,64,114,114]; fp32
+// backward 46 against 69 us.)  A thread produces 4 adjacent outputs from three
 // 16-byte LDS reads (forward) or 8 adjacent inputs of two rows from a handful of LDS reads
 // (backward), compares against compile-time window positions, and writes 8/16-byte pieces that are
 // contiguous across the wave.  Padding is handled by data, not by branches: the row above the
@@ -845,11 +844,11 @@ template <typename F> int pick_rows(int rows_total, int row_elems, int want, F b
 // are cut into bands of equal height; a block of `threads` walks its band in passes of `threads` items.  Picks
 // the height with the fewest idle thread slots among those that fit the LDS budget and need at
 // most `max_passes` passes, preferring taller bands (fewer halo rows) on ties.  0 if nothing fits.
-template <typename F> int pick_band(int units, int per_unit, int threads, int max_passes, F bytes) {
+template <typename F> int pick_band(int units, int per_unit, int threads, int max_passes, F bytes, size_t budget = kLdsBudget) {
   int best = 0;
   double best_eff = 0.0;
   for (int rows = 1; rows <= units; ++rows) {
-    if (bytes(rows) > (size_t)kLdsBudget) break;
+    if (bytes(rows) > budget) break;
     const int passes = (rows * per_unit + threads - 1) / threads;
     if (passes > max_passes && best > 0) break;
     const int full = units / rows, rest = units % rows;
@@ -868,19 +867,47 @@ template <typename T, bool NIB>
 int launch_fwd(const void* x, void* y, int8_t* idx, int64_t total, const PoolGeom& g, hipStream_t s) {
   const int64_t planes = total / ((int64_t)g.Ho * g.Wo);
   auto need = [&](int rows) { return ((size_t)((rows - 1) * g.SH + g.KH) * g.W + 16) * sizeof(T); };
-  if (const int k = sizeof(T) == 2 ? s2_kernel_of(g) : 0; k != 0 && aligned16(x) && aligned16(y) && aligned16(idx)) {
-    const int rb = pick_band(g.Ho, g.Wo / 4, kFwdS2Threads, kFwdS2Passes, need);
-    const int bands = rb > 0 ? (g.Ho + rb - 1) / rb : 0;
-    if (rb > 0 && planes * bands <= 0x7fffffffLL) {
+  // fp32 takes the stride-2 kernel for 3x3 windows only: 2x2 windows share no pixel and the direct kernel is the
+  // faster one at every size ([199,16,112,112] 31 against 51 us).  Its bands take at most 27 KB, so that six
+  // blocks share a CU's LDS: with the 48 KB of the 16-bit types [199,16,112,112] took 55.9 us and
+  // [797,16,56,56] 33.5, with 27 KB 34.2 and 33.5; the direct kernel 47.1 and 56.4.  Rows below 24 pixels give
+  // a block next to nothing to do (16 pixels: 111 against 76 us), and with fewer than two blocks for
+  // every CU the many small ones of the direct kernel are done first (64 planes of 56x56: 2.7 against 2.2 us).
+  constexpr bool k16Bit = sizeof(T) == 2;
+  if (const int k = s2_kernel_of(g); (k16Bit ? k != 0 : k == 3 && g.W >= 24) && aligned16(x) && aligned16(y) && aligned16(idx)) {
+    const int rb = pick_band(g.Ho, g.Wo / 4, kFwdS2Threads, kFwdS2Passes, need, k16Bit ? kLdsBudget : 27 * 1024);
+    const int64_t bands = rb > 0 ? (g.Ho + rb - 1) / rb : 0;
+    if (rb > 0 && planes * bands <= 0x7fffffffLL && (k16Bit || planes * bands >= 512)) {
       const dim3 grid((unsigned)(planes * bands)), blk(kFwdS2Threads);
       const T* xi = static_cast<const T*>(x);
       T* yo = static_cast<T*>(y);
-      if (k == 3) max_pool2d_forward_s2_kernel<T, 3, 1, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, g, rb, bands);
-      else max_pool2d_forward_s2_kernel<T, 2, 0, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, g, rb, bands);
+      if constexpr (k16Bit) {
+        if (k == 2) {
+          max_pool2d_forward_s2_kernel<T, 2, 0, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, g, rb, (int)bands);
+          ACTNN_RETURN_LAUNCH_STATUS();
+        }
+      }
+      max_pool2d_forward_s2_kernel<T, 3, 1, NIB><<<grid, blk, need(rb), s>>>(xi, yo, idx, g, rb, (int)bands);
       ACTNN_RETURN_LAUNCH_STATUS();
     }
   }
   const int preset = preset_of(g);
+  // 3x3 stride 2 pad 1 over rows that are no multiple of 8 pixels: the LDS kernel, a row of outputs to a wave, is
+  // the faster one where at least two thirds of the lanes have an output and there are several rounds of
+  // blocks; bands of about 1024 outputs, of equal height (bf16, one index per byte: [49,16,225,225] 36 against
+  // 43 us of the direct kernel, [192,16,114,114] 35 and 45, [37,16,258,258], 67 % of the lanes, 40 and 42;
+  // [371,16,82,82], 64 %, 46 and 43; 1024 planes of 99x99, 2048 blocks, 13.6 and 13.3).
+  if (preset == 1 && aligned16(x) && (!NIB || g.Wo % 2 == 0) && 3 * (int64_t)g.Wo >= 2 * (((int64_t)g.Wo + 63) / 64 * 64)) {
+    const int64_t parts = ((int64_t)g.Ho * g.Wo + 512) / 1024;
+    int rb = parts > 1 ? (int)((g.Ho + parts - 1) / parts) : g.Ho;
+    while (rb > 1 && need(rb) > (size_t)kLdsBudget) --rb;
+    const int64_t bands = (g.Ho + rb - 1) / rb;
+    if (need(rb) <= (size_t)kLdsBudget && planes * bands >= 4096 && planes * bands <= 0x7fffffffLL) {
+      max_pool2d_forward_lds_kernel<T, 1, NIB><<<dim3((unsigned)(planes * bands)), dim3(kThreads), need(rb), s>>>(
+          static_cast<const T*>(x), static_cast<T*>(y), idx, planes * g.H * g.W, g, rb, (int)bands);
+      ACTNN_RETURN_LAUNCH_STATUS();
+    }
+  }
   // (without padding the direct kernel looks at no bounds: every window must lie inside the plane)
   const bool whole = g.PH > 0 || ((g.Ho - 1) * (int64_t)g.SH + g.KH <= g.H && (g.Wo - 1) * (int64_t)g.SW + g.KW <= g.W);
   DirectGeom q;
@@ -907,7 +934,7 @@ int launch_fwd(const void* x, void* y, int8_t* idx, int64_t total, const PoolGeo
     const int bands = (g.Ho + rb - 1) / rb;
     if (planes * bands <= 0x7fffffffLL) {
       const dim3 grid((unsigned)(planes * bands)), blk(kThreads);
-      max_pool2d_forward_lds_kernel<T, NIB><<<grid, blk, need(rb), s>>>(
+      max_pool2d_forward_lds_kernel<T, 0, NIB><<<grid, blk, need(rb), s>>>(
           static_cast<const T*>(x), static_cast<T*>(y), idx, planes * g.H * g.W, g, rb, bands);
       ACTNN_RETURN_LAUNCH_STATUS();
     }

@@ -268,3 +268,25 @@ def test_backward_without_any_window_is_zero(k, s, p, nibble, channels_last):
                             torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     assert torch.equal(gin, torch.zeros_like(gin))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nibble", [False, True])
+@pytest.mark.parametrize("shape", [(32, 16, 24, 24), (32, 16, 40, 56), (64, 8, 112, 112), (16, 128, 92, 92), (512, 4, 20, 367),
+                                   (16, 256, 25, 99)])
+def test_forward_of_many_planes_equals_that_of_few(dtype, nibble, shape):
+    """3x3 stride 2 pad 1: from some number of blocks on other kernels take it (staged rows of whole vectors in
+    fp32, staged rows of any width); small values with many ties, the last bands of a plane shorter."""
+    x = torch.randint(-2, 3, shape, generator=torch.Generator().manual_seed(sum(shape))).to(dtype)
+    xd = x.to(DEV)
+    y, idx = ext_q.max_pool2d_forward(xd, (3, 3), (2, 2), (1, 1), (1, 1), nibble)
+    assert torch.equal(y.cpu(), torch.nn.functional.max_pool2d(x.float(), 3, 2, 1).to(dtype))
+    n = max(1, shape[0] // 16)
+    for i in range(0, shape[0], n):
+        y1, idx1 = ext_q.max_pool2d_forward(xd[i:i + n], (3, 3), (2, 2), (1, 1), (1, 1), nibble)
+        assert torch.equal(y1, y[i:i + n])
+        if nibble:
+            per = idx.numel() // shape[0]                  # (whole bytes a sample)
+            assert torch.equal(idx1, idx[i * per:(i + n) * per])
+        else:
+            assert torch.equal(idx1, idx[i:i + n])
