@@ -62,17 +62,33 @@ def sample_sqnorm(x):
     return part.sum(1) if slices > 1 else part.view(N)
 
 
+def _sums_pay(N, F, size, with_sqnorm):
+    """Where row_column_sums is the faster way (us, its two kernels / torch's sum over the rows, and with the
+    norms / the sum and sample_sqnorm; f16 unless said).  From 2^20 elements on, where it was first 5 us ahead
+    ([1024,1024] 5.7 / 10.3).  Its second kernel walks N / 16 partial rows for a column, so tall and
+    narrow tensors lose: [32768,64] 19.0 / 11.6, [65535,256] 34.7 / 31.4, but [16384,256] 12.4 / 24.2,
+    [8192,64] 8.1 / 9.7; beyond 128 MB torch reads as fast: f32 [16384,4096] 49.2 / 46.9, [16384,2048]
+    28.5 / 31.6, f32 [4096,16384] 46 / 169.  The norms cost it little: [65535,64] 40.4 / 52.4, [65535,32]
+    48.8 / 47.3."""
+    if N * F < 1 << 20 or N > 65535:
+        return False
+    if with_sqnorm:
+        return F >= 64
+    return 128 <= N <= 32768 and F >= N / 128 and (N <= 4096 or N * F * size <= 1 << 27)
+
+
 def row_column_sums(x, with_sqnorm):
     """(sum over the rows of a [N, F] tensor in its dtype, squared norm of every row as sample_sqnorm gives it
-    or None) from one read, or None where the kernel does not apply: few elements (torch's own reduction
-    is one launch), ragged rows, rows too long for a block, under a graph of the backward pass, and for a
-    batch of gradients at once (torch.autograd.grad with is_grads_batched), which has no memory to read."""
+    or None) from one read, or None where the kernel does not apply or does not pay: ragged rows, rows too long
+    for a block, under a graph of the backward pass, and for a batch of gradients at once
+    (torch.autograd.grad with is_grads_batched), which has no memory to read."""
     if (x.dim() != 2 or x.dtype not in g.DTYPE_CODE or not x.is_cuda or not x.is_contiguous() or torch.is_grad_enabled()
-            or x.numel() < 1 << 20 or not g.has_storage(x) or x.data_ptr() % 16 != 0):
+            or not _sums_pay(x.shape[0], x.shape[1], x.element_size(), with_sqnorm)
+            or not g.has_storage(x) or x.data_ptr() % 16 != 0):
         return None
     N, F = x.shape
     elems = 16 // x.element_size()
-    if F % elems != 0 or N > 65535 or (with_sqnorm and F > 1024 * elems):
+    if F % elems != 0 or (with_sqnorm and F > 1024 * elems):
         return None
     columns = torch.empty(F, dtype=x.dtype, device=x.device)
     sq = torch.empty(N, dtype=torch.float32, device=x.device) if with_sqnorm else None
