@@ -142,7 +142,9 @@ ACTNN_DEV void mask_backward_rest(const T* __restrict__ gout, const int32_t* __r
 // elements of a mask row came back to its line four times in fp32).  What is left of the tensor (< 2048
 // elements) is the last block's, in the same launch.  Bound by memory: fp32 [256, 100352] 34 us forward and
 // 34 us backward (6 TB/s; 54 and 54 us with a lane per mask row), bf16 [362, 122467] 31 + 30 us (37 + 36 us with
-// the remainder in a launch of its own).
+// the remainder in a launch of its own).  fp32 results are stored through the caches, 16-bit ones past them.  For fp32 that
+// depends on who reads next (ReLU of 256 MB alone 79 us, 87 past the caches; forward and backward in turn
+// 183 and 173; 120 MB 79 and 84; 16 MB 13.7 and 10.5; 512 MB 375 and 346).
 constexpr int kTileElems = 4 * kMaskBlock;        // elements per wave
 constexpr int kTilesPerBlock = kThreads / 64;
 
@@ -266,15 +268,10 @@ ACTNN_DEV void word_to_nibbles(uint32_t w, uint32_t lane, uint32_t (&nib)[8]) {
   for (int i = 0; i < 8; ++i) nib[i] = (quad[2 * (i & 1) + (i >> 2)] >> (16 * ((i >> 1) & 1) + sh)) & 0xfu;
 }
 
-ACTNN_DEV void store_result(float* p, u32x4 v, bool stream) {
-  if (stream) store16_nt(p, v);
-  else store16(p, v);
-}
-
 template <Op OP, bool ADD>
 ACTNN_DEV void mask_forward_tile32(const float* __restrict__ x, float* __restrict__ y, int32_t* __restrict__ mask,
                                    int64_t tile, uint32_t thr, float keep_div, uint64_t seed, uint64_t offset,
-                                   const float* __restrict__ add, bool stream) {
+                                   const float* __restrict__ add) {
   const uint32_t lane = threadIdx.x & 63;
   const int64_t e0 = tile * kTileElems + lane * 4;
   u32x4 v[8];
@@ -323,7 +320,7 @@ ACTNN_DEV void mask_forward_tile32(const float* __restrict__ x, float* __restric
     }
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) store_result(y + e0 + i * 256, v[i], stream);
+  for (int i = 0; i < 8; ++i) store16(y + e0 + i * 256, v[i]);
   mask[tile * 64 + quads_word_at(lane)] = (int32_t)nibbles_to_word(nib, lane);
 }
 
@@ -331,7 +328,7 @@ template <typename T, Op OP, bool MINMAX = false, bool ADD = false>
 __global__ __launch_bounds__(kThreads) void mask_forward_kernel(const T* __restrict__ x, T* __restrict__ y,
                                                                 int32_t* __restrict__ mask, RestArgs part,
                                                                 uint32_t thr, float keep_div, uint64_t seed,
-                                                                uint64_t offset, bool stream,
+                                                                uint64_t offset,
                                                                 T* __restrict__ mn = nullptr,
                                                                 T* __restrict__ mx = nullptr,
                                                                 const T* __restrict__ add = nullptr) {
@@ -343,7 +340,7 @@ __global__ __launch_bounds__(kThreads) void mask_forward_kernel(const T* __restr
   }
   const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
   if (tile >= part.tiles) return;                  // whole waves leave together
-  if constexpr (sizeof(T) == 4) mask_forward_tile32<OP, ADD>(x, y, mask, tile, thr, keep_div, seed, offset, add, stream);
+  if constexpr (sizeof(T) == 4) mask_forward_tile32<OP, ADD>(x, y, mask, tile, thr, keep_div, seed, offset, add);
   else mask_forward_tile<T, OP, MINMAX, ADD>(x, y, mask, tile, thr, keep_div, seed, offset, mn, mx, add);
 }
 
@@ -380,7 +377,7 @@ ACTNN_DEV void mask_backward_tile(const T* __restrict__ gout, const int32_t* __r
 template <bool ACC>
 ACTNN_DEV void mask_backward_tile32(const float* __restrict__ gout, const int32_t* __restrict__ mask,
                                     float* __restrict__ gin, int64_t tile, float keep_div, bool divide,
-                                    const float* __restrict__ acc, bool stream) {
+                                    const float* __restrict__ acc) {
   const uint32_t lane = threadIdx.x & 63;
   const int64_t e0 = tile * kTileElems + lane * 4;
   const uint32_t word = (uint32_t)mask[tile * 64 + quads_word_at(lane)];
@@ -402,7 +399,7 @@ ACTNN_DEV void mask_backward_tile32(const float* __restrict__ gout, const int32_
       const float g = keep ? (divide ? f / keep_div : f) : 0.0f;
       v[i][k] = as_uint(ACC ? as_float(a[ACC ? i : 0][k]) + g : g);
     }
-    store_result(gin + e0 + i * 256, v[i], stream);
+    store16(gin + e0 + i * 256, v[i]);
   }
 }
 
@@ -410,7 +407,7 @@ template <typename T, bool ACC = false>
 __global__ __launch_bounds__(kThreads) void mask_backward_kernel(const T* __restrict__ gout,
                                                                  const int32_t* __restrict__ mask,
                                                                  T* __restrict__ gin, RestArgs part,
-                                                                 float keep_div, bool divide, bool stream,
+                                                                 float keep_div, bool divide,
                                                                  const T* __restrict__ acc = nullptr) {
   if ((int64_t)blockIdx.x >= part.tile_blocks) {
     const int64_t done = part.tiles * kTileElems;
@@ -420,7 +417,7 @@ __global__ __launch_bounds__(kThreads) void mask_backward_kernel(const T* __rest
   }
   const int64_t tile = (int64_t)blockIdx.x * kTilesPerBlock + (threadIdx.x >> 6);
   if (tile >= part.tiles) return;
-  if constexpr (sizeof(T) == 4) mask_backward_tile32<ACC>(gout, mask, gin, tile, keep_div, divide, acc, stream);
+  if constexpr (sizeof(T) == 4) mask_backward_tile32<ACC>(gout, mask, gin, tile, keep_div, divide, acc);
   else mask_backward_tile<T, ACC>(gout, mask, gin, tile, keep_div, divide, acc);
 }
 
@@ -442,13 +439,12 @@ int launch_forward(const void* x, void* y, int32_t* mask, int64_t n, uint32_t th
   RestArgs part;
   const int64_t blocks = split_tensor(n, part);
   if (blocks == 0) return ACTNN_EINVAL;
-  const bool stream = stream_results(n * (int64_t)sizeof(T));
   const dim3 grid((unsigned)blocks), blk(kThreads);
   if (OP == Op::kRelu && ai)
     mask_forward_kernel<T, Op::kRelu, false, true><<<grid, blk, 0, s>>>(xi, yo, mask, part, thr, keep_div, seed, offset,
-                                                                        stream, nullptr, nullptr, ai);
+                                                                        nullptr, nullptr, ai);
   else
-    mask_forward_kernel<T, OP><<<grid, blk, 0, s>>>(xi, yo, mask, part, thr, keep_div, seed, offset, stream);
+    mask_forward_kernel<T, OP><<<grid, blk, 0, s>>>(xi, yo, mask, part, thr, keep_div, seed, offset);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -461,10 +457,9 @@ int launch_backward(const void* gout, const int32_t* mask, void* gin, int64_t n,
   RestArgs part;
   const int64_t blocks = split_tensor(n, part);
   if (blocks == 0) return ACTNN_EINVAL;
-  const bool stream = stream_results(n * (int64_t)sizeof(T));
   const dim3 grid((unsigned)blocks), blk(kThreads);
-  if (ac) mask_backward_kernel<T, true><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide, stream, ac);
-  else mask_backward_kernel<T><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide, stream);
+  if (ac) mask_backward_kernel<T, true><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide, ac);
+  else mask_backward_kernel<T><<<grid, blk, 0, s>>>(go, mask, gi, part, keep_div, divide);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -529,11 +524,11 @@ extern "C" int actnn_relu_forward_minmax(const void* x, void* y, int32_t* mask, 
   const dim3 grid((unsigned)blocks), blk(kThreads);
   if (dtype == ACTNN_F16)
     mask_forward_kernel<__half, Op::kRelu, true><<<grid, blk, 0, s>>>(
-        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0, true,
+        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0,
         static_cast<__half*>(mn), static_cast<__half*>(mx));
   else
     mask_forward_kernel<bf16_t, Op::kRelu, true><<<grid, blk, 0, s>>>(
-        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0, true,
+        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0,
         static_cast<bf16_t*>(mn), static_cast<bf16_t*>(mx));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
@@ -556,11 +551,11 @@ extern "C" int actnn_relu_add_forward(const void* x, const void* residual, void*
   const dim3 grid((unsigned)blocks), blk(kThreads);
   if (dtype == ACTNN_F16)
     mask_forward_kernel<__half, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
-        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0, true,
+        static_cast<const __half*>(x), static_cast<__half*>(y), mask, part, 0u, 1.0f, 0, 0,
         static_cast<__half*>(mn), static_cast<__half*>(mx), static_cast<const __half*>(residual));
   else
     mask_forward_kernel<bf16_t, Op::kRelu, true, true><<<grid, blk, 0, s>>>(
-        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0, true,
+        static_cast<const bf16_t*>(x), static_cast<bf16_t*>(y), mask, part, 0u, 1.0f, 0, 0,
         static_cast<bf16_t*>(mn), static_cast<bf16_t*>(mx), static_cast<const bf16_t*>(residual));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
