@@ -163,14 +163,14 @@ template <int THREADS> ACTNN_DEV uint32_t block_scan(uint32_t v, uint32_t* s_wav
   return before + v;
 }
 
-// KEYS > 0: the patterns of a thread's candidates (at most KEYS) stay in registers over the passes (and
-// the items fit in LDS); 0: evaluated anew in each.
+// KEYS > 0: the patterns of a thread's candidates (at most KEYS) stay in registers over the passes; 0:
+// evaluated anew in each.
 template <int THREADS, int KEYS>
 __global__ __launch_bounds__(THREADS) void allocate_kernel(const float* __restrict__ sens, int32_t* __restrict__ bits,
                                                            int32_t* __restrict__ prefix, int N, int initial,
                                                            int64_t K) {
   constexpr int kPer = kBins / THREADS;                // bins a thread scans
-  constexpr int kItems = KEYS > 0 ? (THREADS * KEYS < kLdsItems ? THREADS * KEYS : kLdsItems) : kLdsItems;
+  constexpr int kItems = KEYS > 0 ? THREADS * KEYS : kLdsItems;
   __shared__ double factors[8];
   __shared__ float C_s[kItems];
   __shared__ uint32_t hist[kBins];
@@ -447,10 +447,13 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
 
 // As many threads as have work, and their candidates in registers while they fit.  Measured (bf16, start
 // width 8): 64 items 4.2 us, 128 items 4.6 us with 256 threads; 256 items 5.2 us, 512 items 5.6 us (9.3 us
-// with 256 threads), 1100 items 7.3 us with 1024;
-// more items: see allocate_many_kernel, up to the 8192 whose steps fit the registers of one block.  Ranking every candidate against
-// every other by a grid of blocks, and scanning the widths in a launch of its own, took 6.5 + 2.8 us at 32
-// items, 7.7 + 5.3 us at 256, and stopped at 8192 candidates.
+// with 256 threads), 1100 items 7.3 us with 1024; more items: see allocate_many_kernel, up to the 8192 whose
+// steps fit the registers of one block.  Beyond those the patterns are evaluated anew in each pass: with the
+// sensitivities' pass in front 9362 items take 35.7 us (47.2 with 64 patterns a thread in registers,
+// which spill), 16384 items 66 us, from memory 131072 items 694 us; the host routine needs 143, 230 and
+// 1610 us and the GPU waits for it.  Ranking every candidate against every other by a grid of blocks, and
+// scanning the widths in a launch of its own, took 6.5 + 2.8 us at 32 items, 7.7 + 5.3 us at 256, and
+// stopped at 8192 candidates.
 int launch_allocate(const float* sens, int32_t* bits, int32_t* prefix, int64_t N, int initial, int64_t target,
                     hipStream_t s) {
   const int64_t K = N * initial - target, candidates = N * (initial > 1 ? initial - 1 : 1);
@@ -459,7 +462,6 @@ int launch_allocate(const float* sens, int32_t* bits, int32_t* prefix, int64_t N
   else if (N <= 2048) allocate_many_kernel<2><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else if (N <= 4096) allocate_many_kernel<4><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else if (N <= 8192) allocate_many_kernel<8><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
-  else if (candidates <= 1024 * 64 && N <= kLdsItems) allocate_kernel<1024, 64><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   else allocate_kernel<1024, 0><<<dim3(1), dim3(1024), 0, s>>>(sens, bits, prefix, (int)N, initial, K);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
