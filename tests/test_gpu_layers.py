@@ -1082,6 +1082,38 @@ def test_closing_step_of_a_residual_block_in_the_batch_norm_pass(dtype, channels
         assert torch.equal(u, v), i
 
 
+def test_closing_step_of_a_tensor_beyond_the_last_level_cache():
+    """Above 256 MB the backward's first pass writes the masked gradient past the caches: the gradients of a closing step on
+    such a tensor against the batch norm, the addition and the ReLU one after the other."""
+    from actnn_amd.layers import QAddReLU, QBatchNorm2d, bn_add_relu
+    shape = (164, 256, 57, 57)
+    res = []
+    for fold in (False, True):
+        config.reset(); QScheme.reset(); QBNScheme.reset()
+        set_optimization_level("L3")
+        config.fused_bn_relu = fold
+        torch.manual_seed(4)
+        bn, close = QBatchNorm2d(shape[1]).to(DEV).train(), QAddReLU()
+        g = torch.Generator(device=DEV).manual_seed(10)
+        x, identity, go = (torch.randn(shape, device=DEV, generator=g, dtype=torch.bfloat16)
+                           .contiguous(memory_format=torch.channels_last) for _ in range(3))
+        assert x.numel() * 2 > 256 << 20
+        x.requires_grad_(); identity.requires_grad_()
+        torch.cuda.manual_seed(22)
+        out = bn_add_relu(bn, close, x, identity)
+        res.append((out.detach(),) + torch.autograd.grad(out, [identity, x, bn.weight, bn.bias], go))
+    two, one = res
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])          # output, masked gradient
+    # the sums run over the same 532836 terms a channel in another order: a thread adds some hundreds of them,
+    # then the partial sums of at most 2048 blocks
+    terms = one[1].float().abs().sum((0, 2, 3))                                  # |xhat| is below 6 here
+    assert bool(((one[4] - two[4]).abs() <= 2500 * 2.0 ** -24 * terms).all())
+    assert bool(((one[3] - two[3]).abs() <= 2500 * 2.0 ** -24 * 6 * terms).all())
+    # and through them move the gradient of x by no more than a bfloat16 rounding
+    a, b = one[2].float(), two[2].float()
+    assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-3 * b.square().mean().sqrt()).all())
+
+
 @pytest.mark.parametrize("level", ["L3", "L2"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("identity_from", ["input", "batch_norm"])

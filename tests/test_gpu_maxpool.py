@@ -240,17 +240,20 @@ def test_preset_windows_on_planes_of_any_size(dtype, k, s, p, shape, channels_la
     assert np.array_equal(gin.float().cpu().numpy(), gin_o)
 
 
-@pytest.mark.parametrize("k,s,p", [((3, 3), (2, 2), (0, 0)), ((3, 3), (1, 1), (1, 1))])
-def test_large_results_are_streamed_and_equal(k, s, p):
-    # above 128 MB the backward pass stores past the caches: the same values as in pieces below that
-    x = torch.randn(48, 64, 105, 105, device=DEV)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k,s,p", [((3, 3), (2, 2), (0, 0)), ((3, 3), (1, 1), (1, 1)), ((2, 2), (2, 2), (0, 0))])
+def test_large_results_are_streamed_and_equal(k, s, p, dtype):
+    # above 128 MB the backward pass stores past the caches, rows of odd width one element at a time at their
+    # ends: the same values as in pieces below that
+    N = 48 if dtype == torch.float32 else 96
+    x = torch.randn(N, 64, 105, 105, device=DEV).to(dtype)
     y, idx = ext_q.max_pool2d_forward(x, k, s, p, (1, 1))
     g = torch.randn_like(y)
     whole = ext_q.max_pool2d_backward(g, idx, x.shape, k, s, p)
-    assert whole.numel() * 4 > 128 << 20
-    for i in range(0, 48, 16):
-        part = ext_q.max_pool2d_backward(g[i:i + 16], idx[i:i + 16], x[i:i + 16].shape, k, s, p)
-        assert torch.equal(part, whole[i:i + 16])
+    assert whole.numel() * whole.element_size() > 128 << 20
+    for i in range(0, N, N // 3):
+        part = slice(i, i + N // 3)
+        assert torch.equal(ext_q.max_pool2d_backward(g[part], idx[part], x[part].shape, k, s, p), whole[part])
 
 
 @pytest.mark.parametrize("k,s,p", [(3, 2, 1), (3, 2, 0), (2, 2, 0), (3, 1, 1)])

@@ -11,7 +11,9 @@ from actnn_amd.cpp_extension import quantization as ext_q
 pytestmark = pytest.mark.gpu
 
 DTYPES = [torch.float32, torch.float16, torch.bfloat16]
-SHAPES = [(8, 1), (1, 9), (3, 3), (2, 7), (5, 255), (3, 256), (4, 257), (9, 2049), (2, 4093), (65, 300), (7, 512)]
+# (a block packs 4096 elements of a row in fp32, 8192 in 16 bits: the longest rows take several, the last one ragged)
+SHAPES = [(8, 1), (1, 9), (3, 3), (2, 7), (5, 255), (3, 256), (4, 257), (9, 2049), (2, 4093), (65, 300), (7, 512),
+          (3, 4097), (2, 8193), (3, 20001)]
 
 
 def _rows(N, F, dtype, shift, seed):
