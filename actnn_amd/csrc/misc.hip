@@ -85,23 +85,14 @@ extern "C" int actnn_stream_copy(const void* src, void* dst, int64_t bytes, void
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
-// The three allocation steps of a layer in one call (one crossing of the language boundary instead
-// of three): sensitivities, greedy widths on the device, exclusive prefix of the widths.
-extern "C" int actnn_range_sqr(const void* mn, const void* mx, float* out, int64_t N, int64_t G, float factor,
-                               const float* mult, int mult_per_sample, int dtype, void* stream);
-extern "C" int actnn_calc_precision_device(const float* C, int32_t* bits, int64_t N, int initial_bits,
-                                           int64_t target, void* stream);
-extern "C" int actnn_bits_prefix(const int32_t* bits, int32_t* prefix, int64_t N, void* stream);
-
-extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
-                                          int mult_per_sample, float* sensitivity, int32_t* bits,
-                                          int32_t* prefix, int64_t N, int64_t G, int initial_bits,
-                                          int64_t target, int dtype, void* stream);
-
 // One crossing of the language boundary for a layer's whole forward-side sequence: the calls below
 // on one stream, arguments as theirs.  Nothing is launched unless the arguments of the first step
 // pass; a later step that refuses its arguments leaves the earlier ones launched (their outputs are
 // then simply unused).
+extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
+                                          int mult_per_sample, float* sensitivity, int32_t* bits,
+                                          int32_t* prefix, int64_t N, int64_t G, int initial_bits,
+                                          int64_t target, int dtype, void* stream);
 extern "C" int actnn_batch_norm_forward_stats(const void* x, const float* weight, const float* bias,
                                               float* running_mean, float* running_var, float* save_mean,
                                               float* save_invstd, void* mn, void* mx, void* workspace,

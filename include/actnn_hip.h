@@ -259,8 +259,7 @@ int actnn_calc_precision_device(const float* C, int32_t* bits, int64_t N, int in
 
 /* actnn_range_sqr, actnn_calc_precision_device and actnn_bits_prefix back to back on `stream`, for
  * the per-layer allocation of qscheme.py:76-94 in one call: sensitivity[N] (fp32), bits[N],
- * prefix[N + 1].  Arguments as for the three calls; N and N * (initial_bits - 1) <= 2^20.  Two kernels, or one
- * where the ranges are few. */
+ * prefix[N + 1].  Arguments as for the three calls; N and N * (initial_bits - 1) <= 2^20.  Two kernels. */
 int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
                                int mult_per_sample, float* sensitivity, int32_t* bits,
                                int32_t* prefix, int64_t N, int64_t G, int initial_bits,
