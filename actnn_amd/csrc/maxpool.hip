@@ -1224,7 +1224,8 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_kernel(
 // windows that reach the block are 2x2 of them (3x3) or one (2x2): one (gradient, index) load per
 // input pixel where the general kernel needs 2.25 (3x3).  Every pixel adds its windows in the
 // general kernel's order (rows, then columns), hence the same bits.  grad_in is written once and
-// not read: streamed stores (measured 0.104 -> 0.079 ms on f16 [256,64,112,112]).
+// not read: streamed stores, NT, where they make whole pieces of memory lines (measured 0.104 -> 0.079 ms on
+// f16 [256,64,112,112]).
 template <typename T, int K, int P, bool NIB, bool EVEN, bool NT>
 __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
     const T* __restrict__ gout, const int8_t* __restrict__ idx, T* __restrict__ gin, ClGeom q, PoolGeom g) {
@@ -1235,6 +1236,8 @@ __global__ __launch_bounds__(kThreads) void max_pool2d_backward_cl_s2_kernel(
   const ClAt at = cl_at(q);                            // rows and columns of windows
   if (!at.live) return;
   const uint32_t C = q.cpp * E;
+  // (windows and cells of even planes have the same numbers; with two indices per byte the flat one measured 6 % faster,
+  // bf16 [9,64,224,224] 12.1 -> 11.5 us, with one per byte 1 - 3 % slower)
   constexpr bool kFlat = EVEN && NIB;
   const int64_t image_o = kFlat ? (int64_t)at.n * q.per_image * E : (int64_t)at.n * g.Ho * g.Wo * C;
   const uint32_t lane_o = kFlat ? at.i * E : (at.row * (uint32_t)g.Wo + at.col) * C + at.chunk * E;   // window (row, col) of this chunk in the image
@@ -1395,6 +1398,10 @@ int launch_cl(bool forward, const void* a, const int8_t* idx_in, int8_t* idx_out
       else if (p == 2) max_pool2d_backward_cl_s2_kernel<T, 2, 0, NIB, false, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
       else max_pool2d_backward_cl_s2_kernel<T, 3, 0, NIB, false, NT><<<grid, blk, 0, s>>>(go, idx_in, gi, q, g);
     };
+    // A thread's chunks lie two pixels apart.  Streamed, they make whole 64-byte pieces of memory lines only where a
+    // pixel is a multiple of that; other pixels take ordinary stores, which meet their neighbours in the
+    // cache (bf16 [37,16,225,225] 2x2 37.9 us streamed, 15.9 so; [37,16,224,224] 3x3 29.0 and 18.3; f32
+    // [24,24,225,225] 2x2 51.3 and 23.3; whole 64 bytes the other way round: bf16 [9,64,224,224] 3x3 11.5 us streamed).
     if (C * (int64_t)sizeof(T) % 64 == 0) launch(std::true_type());
     else launch(std::false_type());
   } else {
