@@ -10,11 +10,11 @@
 // elements (one 16-byte load for 16-bit types, two for f32), quantises them and
 // concatenates the 8 codes into 8*b bits of a register (several groups share a register
 // when 8*b <= 16).  One 32x32 bit transpose per register (5 exchange stages) then leaves
-// word p in lane p, which is stored coalesced.  A 256-thread block handles 16 groups of one
-// sample (2 per half-wave); the element loads are issued first, the block's scales are
-// computed by the first threads and shared through LDS while the loads are in flight.
-// unpack mirrors this; its fp32 stores go through LDS so that each store instruction of a
-// wave writes one whole 1 KiB group.
+// word p in lane p, which is stored coalesced.  A wave handles a unit of consecutive groups of
+// one sample (4 for f32, 8 for 16-bit types), a 256-thread block four units that follow each
+// other; the element loads are issued first, the block's scales are computed by the first
+// threads and shared through LDS while the loads are in flight.  unpack mirrors this; its fp32
+// stores go through LDS so that each store instruction of a wave writes one whole 1 KiB group.
 //
 // Other group sizes (multiples of 32 up to 1024) take a simple LDS-staged kernel.
 #include "quant_math.h"
@@ -22,7 +22,7 @@
 namespace actnn {
 namespace {
 
-// Groups per half-wave and block.  fp32: 2 measured best (16 KiB of input per block).
+// Groups per half-wave.  fp32: 2 measured best (16 KiB of input per block).
 // 16-bit types: a block with 8 KiB of data is dominated by its own latency chain (widths ->
 // scales -> data), so they take 4.
 template <typename T> struct Gph {
@@ -31,7 +31,6 @@ template <typename T> struct Gph {
 };
 
 constexpr int kThreads = 256;
-constexpr int kHalfWaves = kThreads / 32;
 constexpr int kGs = 256;
 
 template <int BITS, int GPH> struct Tile {
@@ -40,10 +39,32 @@ template <int BITS, int GPH> struct Tile {
   static constexpr int kFit = BITS == 1 ? 4 : BITS == 2 ? 2 : 1;
   static constexpr int kGroupsPerReg = kFit < GPH ? kFit : GPH;
   static constexpr bool kTwoRegs = BITS > 4;                                  // 8*BITS > 32
-  // Group (within the block) that half-wave hw handles in its q-th slot: GPH consecutive groups
-  // per half-wave, whatever the bit width, so that loads can be issued before the width is known.
-  static __device__ __forceinline__ int group_of(int hw, int q) { return hw * GPH + q; }
+  // Group (within the wave's unit) that a half of the wave handles in its q-th slot: GPH consecutive
+  // groups per half, whatever the bit width, so that loads can be issued before the width is known.
+  static __device__ __forceinline__ int group_of(int half, int q) { return half * GPH + q; }
 };
+
+// The unit of a wave: `valid` groups of sample n from group gb on (0 behind the last sample, where n
+// is a sample that exists all the same).  The units of a sample follow each other and a block takes the
+// next four whatever samples they belong to: with whole blocks per sample, short rows left most of a
+// block idle (f16 [8192, 4096], 16 groups a row: pack 26.1 and unpack 22.6 us with blocks of 32 groups, 20.3
+// and 16.5 us now; fp32 [256, 3136 groups] pack 149 and 145 us).
+struct Unit {
+  int64_t n, gb;
+  int valid;
+};
+template <int GROUPS> ACTNN_DEV Unit unit_of(uint32_t unit, const FastDiv& per_sample, int64_t N, int64_t G) {
+  Unit u;
+  const uint32_t n = per_sample.div(unit);
+  u.gb = (int64_t)(unit - n * per_sample.d) * GROUPS;
+  const int64_t left = G - u.gb;
+  u.valid = n >= N ? 0 : left < GROUPS ? (int)left : GROUPS;
+  u.n = n >= N ? N - 1 : n;
+  return u;
+}
+constexpr int kWaves = kThreads / 64;
+// the wave's number in its block, as a scalar
+ACTNN_DEV uint32_t wave_of_block() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 // fp32 output of unpack: a lane owns 32 contiguous bytes, which as direct stores would be two
 // half-used 16-byte accesses per cache line.  Instead lanes park their 8 values in the wave's
@@ -53,11 +74,10 @@ template <int BITS, int GPH> struct Tile {
 // complete in order.  (The same staging for the fp32 loads of pack was measured slower.)
 // ROWS: `out` is a row of F elements at any address and elem_base an offset in it; its lines are shared with
 // other waves, so the stores go through the cache.
-template <int GPH, typename TL, bool ROWS>
+template <int GPH, bool ROWS>
 ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t F, int groups_valid,
                              u32x4* __restrict__ slab, const float (&v)[GPH][8]) {
   const int wl = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
   const int h = (threadIdx.x >> 5) & 1;
   const uint32_t lane = threadIdx.x & 31;
 #pragma unroll
@@ -76,9 +96,8 @@ ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int i = 0; i < 2 * GPH; ++i) {
-    const int gl = TL::group_of(2 * w + i / GPH, i % GPH);
-    if (gl < groups_valid) {
-      const int64_t at = elem_base + (int64_t)gl * kGs + wl * 4;
+    if (i < groups_valid) {
+      const int64_t at = elem_base + (int64_t)i * kGs + wl * 4;
       if constexpr (ROWS) store16_part(out + at, slab[i * 64 + wl], part_of_row(F, at));
       else store16_nt(out + at, slab[i * 64 + wl]);
     }
@@ -99,10 +118,10 @@ ACTNN_DEV void load_groups(const T* __restrict__ data, const T* __restrict__ noi
                            int groups_valid, Raw8<T> (&v)[GPH], Raw8<T> (&nz)[DET ? GPH : 1]) {
   using TL = Tile<1, GPH>;
   const uint32_t lane = threadIdx.x & 31;
-  const int hw = threadIdx.x >> 5;
+  const int half = (threadIdx.x >> 5) & 1;
 #pragma unroll
   for (int q = 0; q < GPH; ++q) {
-    const int gl = TL::group_of(hw, q);
+    const int gl = TL::group_of(half, q);
     if (gl < groups_valid) {
       const int64_t e = elem_base + (int64_t)gl * kGs + lane * 8;
       raw8_load_nt(data + e, v[q]);      // non-temporal for 16-bit types only (one instruction per line)
@@ -125,7 +144,7 @@ ACTNN_DEV void pack_groups(const Raw8<T> (&raw)[Gph<T>::kPack], const Raw8<T> (&
   constexpr int WPG = TL::kWordsPerGroup;
   constexpr float Bf = (float)((1 << BITS) - 1);
   const uint32_t lane = threadIdx.x & 31;
-  const int hw = threadIdx.x >> 5;
+  const int half = (threadIdx.x >> 5) & 1;
   static_assert(kGroupsPerHalf % 2 == 0, "the noise of the groups is drawn in pairs");
   constexpr int NB = R > 2 ? R : 2;                    // groups whose noise is drawn together
   constexpr float kUnit = (float)(1u << (32 - BITS - Noise<T>::kBits));
@@ -140,14 +159,14 @@ ACTNN_DEV void pack_groups(const Raw8<T> (&raw)[Gph<T>::kPack], const Raw8<T> (&
       // their neighbours (elem_base is a multiple of 256, so octet and lane parity agree)
 #pragma unroll
       for (int p = 0; p < NB; p += 2) {
-        const uint64_t o = (uint64_t)(elem_base >> 3) + (uint64_t)TL::group_of(hw, q0 + p) * 32 + lane;
+        const uint64_t o = (uint64_t)(elem_base >> 3) + (uint64_t)TL::group_of(half, q0 + p) * 32 + lane;
         Noise<T>::octets(o, o + 32, seed, offset, rw[p], rw[p + 1]);
       }
     }
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {                 // last group first: see CodeShifter
       const int q = q0 + r;
-      const int gl = TL::group_of(hw, q);
+      const int gl = TL::group_of(half, q);
       const float mul = s_mul[gl];
       const float sub = s_sub[gl];
       float v[8], nz[8];
@@ -160,7 +179,7 @@ ACTNN_DEV void pack_groups(const Raw8<T> (&raw)[Gph<T>::kPack], const Raw8<T> (&
       }
     }
     if (!DET) acc = ((uint64_t)sh.hi << 32) | sh.lo;
-    const int glt = TL::group_of(hw, q0);            // first group of this register tile
+    const int glt = TL::group_of(half, q0);            // first group of this register tile
     const int64_t tile_words = word_base + (int64_t)glt * WPG;
     const uint32_t lo = transpose32((uint32_t)acc, lane);
     // each half-wave stores its own 4-byte words (whole 128-byte lines), non-temporally: 3 % faster
@@ -186,14 +205,15 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
     const T* __restrict__ data, const T* __restrict__ mn, const T* __restrict__ mx,
     const int32_t* __restrict__ bits, const int32_t* __restrict__ prefix, S* __restrict__ scale,
     S* __restrict__ mn_out, int32_t* __restrict__ packed, const T* __restrict__ noise, uint64_t seed,
-    uint64_t offset, int64_t F, int64_t G, int blocks_per_sample, const T* last) {
+    uint64_t offset, int64_t N, int64_t F, int64_t G, FastDiv per_sample, const T* last) {
   constexpr int GPH = Gph<T>::kPack;
-  constexpr int kGroupsPerBlock = kHalfWaves * GPH;
-  __shared__ float s_mul[kGroupsPerBlock];
-  __shared__ float s_sub[kGroupsPerBlock];
-  const int64_t n = blockIdx.x / blocks_per_sample;
-  const int64_t gb = (int64_t)(blockIdx.x % blocks_per_sample) * kGroupsPerBlock;
-  const int groups_valid = (int)((G - gb) < kGroupsPerBlock ? (G - gb) : kGroupsPerBlock);
+  constexpr int kUnit = 2 * GPH;                                 // groups of a wave
+  __shared__ float s_mul[kWaves * kUnit];
+  __shared__ float s_sub[kWaves * kUnit];
+  const uint32_t wave = wave_of_block();
+  const Unit u = unit_of<kUnit>(blockIdx.x * kWaves + wave, per_sample, N, G);
+  const int64_t n = u.n, gb = u.gb;
+  const int groups_valid = u.valid;
   const int64_t elem_base = (n * G + gb) * kGs;
 
   // The element loads do not depend on the bit width or the scales: get them in flight first,
@@ -205,36 +225,38 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
   // straight into LDS, one whole 1 KiB group per instruction and no registers, and each lane then
   // picks its 32 bytes out of LDS.
   constexpr bool kViaLds = sizeof(T) == 4 && !DET;
-  __shared__ __align__(16) uint8_t s_stage[kViaLds ? kGroupsPerBlock * kGs * 4 : 16];
+  __shared__ __align__(16) uint8_t s_stage[kViaLds ? kWaves * kUnit * kGs * 4 : 16];
+  uint8_t* stage = s_stage + (kViaLds ? wave * (kUnit * kGs * 4) : 0);
   constexpr int kRowVectors = sizeof(T) == 4 ? 2 * GPH : GPH;
   RowVector st[ROWS ? kRowVectors : 1];                          // ROWS: by way of registers, at any address
   if constexpr (ROWS) {
 #pragma unroll
     for (int i = 0; i < kRowVectors; ++i) {
-      const int gl = sizeof(T) == 4 ? (threadIdx.x >> 6) * 2 * GPH + i : Tile<1, GPH>::group_of(threadIdx.x >> 5, i);
+      const int gl = sizeof(T) == 4 ? i : Tile<1, GPH>::group_of((threadIdx.x >> 5) & 1, i);
       const int64_t at = (gb + gl) * kGs + (sizeof(T) == 4 ? (threadIdx.x & 63) * 4 : (threadIdx.x & 31) * 8);
       st[i] = load16_row(data + n * F + at, gl < groups_valid ? part_of_row(F, at) : 0, last);
     }
   } else if constexpr (kViaLds) {
-    const int wave = threadIdx.x >> 6;
     const uint32_t wl = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < 2 * GPH; ++i) {
-      const int gl = wave * 2 * GPH + i;                       // the wave's two half-waves own these groups
-      if (gl < groups_valid)
-        load_to_lds16_nt(data + elem_base + (int64_t)gl * kGs + wl * 4, s_stage + gl * (kGs * 4));
+    for (int i = 0; i < kUnit; ++i) {
+      if (i < groups_valid)
+        load_to_lds16_nt(data + elem_base + (int64_t)i * kGs + wl * 4, stage + i * (kGs * 4));
     }
   } else {
     load_groups<T, DET, GPH>(data, noise, elem_base, groups_valid, v, nz);
   }
 
   const int b = bits[n];
-  if (threadIdx.x < kGroupsPerBlock) {
+  if (threadIdx.x < kWaves * kUnit) {
     float mul = 0.0f, sub = 0.0f;
-    if ((int)threadIdx.x < groups_valid) {
-      const int64_t gi = n * G + gb + threadIdx.x;
+    // thread t: group t % kUnit of wave t / kUnit, which may belong to another sample than this wave's
+    const Unit ut = unit_of<kUnit>(blockIdx.x * kWaves + threadIdx.x / kUnit, per_sample, N, G);
+    const int gt = (int)threadIdx.x % kUnit;
+    if (gt < ut.valid) {
+      const int64_t gi = ut.n * G + ut.gb + gt;
       const float lo = Conv<T>::load(mn, gi);
-      const float sc = GroupQuant<T, DET>::prepare(lo, Conv<T>::load(mx, gi), b, mul, sub);
+      const float sc = GroupQuant<T, DET>::prepare(lo, Conv<T>::load(mx, gi), bits[ut.n], mul, sub);
       Conv<S>::store(scale, gi, sc);
       if constexpr (sizeof(S) != sizeof(T)) Conv<S>::store(mn_out, gi, lo);
     }
@@ -245,7 +267,7 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
 #pragma unroll
     for (int i = 0; i < kRowVectors; ++i) {
       if constexpr (sizeof(T) == 4)
-        *reinterpret_cast<u32x4*>(s_stage + ((threadIdx.x >> 6) * 2 * GPH + i) * (kGs * 4) + (threadIdx.x & 63) * 16) = row_vector_ends<T>(st[i]);
+        *reinterpret_cast<u32x4*>(stage + i * (kGs * 4) + (threadIdx.x & 63) * 16) = row_vector_ends<T>(st[i]);
       else
         v[i].a = row_vector_ends<T>(st[i]);
     }
@@ -254,13 +276,13 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
   if constexpr (kViaLds) {
     if constexpr (!ROWS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's own groups have landed
     const uint32_t lane = threadIdx.x & 31;
-    const int hw = threadIdx.x >> 5;
+    const int half = (threadIdx.x >> 5) & 1;
 #pragma unroll
     for (int q = 0; q < GPH; ++q) {
-      const int gl = Tile<1, GPH>::group_of(hw, q);
+      const int gl = Tile<1, GPH>::group_of(half, q);
       raw8_zero(v[q]);
       if (gl < groups_valid) {
-        const u32x4* src = reinterpret_cast<const u32x4*>(s_stage + gl * (kGs * 4) + lane * 32);
+        const u32x4* src = reinterpret_cast<const u32x4*>(stage + gl * (kGs * 4) + lane * 32);
         v[q].a = src[0];
         v[q].b = src[1];
       }
@@ -271,8 +293,8 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
   switch (b) {
 #define ACTNN_CASE(B_)                                                                          \
   case B_:                                                                                      \
-    pack_groups<T, B_, DET>(v, nz, packed, elem_base, word_base, groups_valid, s_mul, s_sub,    \
-                            seed, offset);                                                      \
+    pack_groups<T, B_, DET>(v, nz, packed, elem_base, word_base, groups_valid,                  \
+                            s_mul + wave * kUnit, s_sub + wave * kUnit, seed, offset);          \
     break;
     ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(3) ACTNN_CASE(4)
     ACTNN_CASE(5) ACTNN_CASE(6) ACTNN_CASE(7) ACTNN_CASE(8)
@@ -295,12 +317,12 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
   constexpr int WPG = TL::kWordsPerGroup;
   constexpr uint32_t kMask = (1u << BITS) - 1u;
   const uint32_t lane = threadIdx.x & 31;
-  const int hw = threadIdx.x >> 5;
+  const int half = (threadIdx.x >> 5) & 1;
 
   uint32_t wlo[kGroupsPerHalf / R], whi[kGroupsPerHalf / R];
 #pragma unroll
   for (int t = 0; t < kGroupsPerHalf / R; ++t) {
-    const int glt = TL::group_of(hw, t * R);
+    const int glt = TL::group_of(half, t * R);
     const int64_t tile_words = word_base + (int64_t)glt * WPG;
     wlo[t] = 0;
     whi[t] = 0;
@@ -314,13 +336,15 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
         wlo[t] = (uint32_t)packed[tile_words + lane];
     }
   }
-  // the block's scales and minima go to LDS only now, after the word loads have been issued, so
-  // that the two global round trips overlap
-  if ((int)threadIdx.x < groups_valid) {
-    s_scale[threadIdx.x] = my_scale;
-    s_min[threadIdx.x] = my_min;
+  // the wave's scales and minima go to LDS only now, after the word loads have been issued, so
+  // that the two global round trips overlap; only lanes of the wave read them
+  if ((int)(threadIdx.x & 63) < groups_valid) {
+    s_scale[threadIdx.x & 63] = my_scale;
+    s_min[threadIdx.x & 63] = my_min;
   }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int t = 0; t < kGroupsPerHalf / R; ++t) {
     const int q0 = t * R;
@@ -328,7 +352,7 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
     if (TL::kTwoRegs) acc |= (uint64_t)transpose32(whi[t], lane) << 32;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int gl = TL::group_of(hw, q0 + r);
+      const int gl = TL::group_of(half, q0 + r);
       if (gl < groups_valid) {
         const Dequant<T> dq(s_scale[gl], s_min[gl]);
         if constexpr (sizeof(T) == 2 && BITS <= 2) {
@@ -374,7 +398,7 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
     }
   }
   if constexpr (kStage)
-    stage_out_f32<kGroupsPerHalf, TL, ROWS>(reinterpret_cast<float*>(out), elem_base, F, groups_valid, slab, vs);
+    stage_out_f32<kGroupsPerHalf, ROWS>(reinterpret_cast<float*>(out), elem_base, F, groups_valid, slab, vs);
 }
 
 // S: the type the scales and minima are stored in.
@@ -382,20 +406,21 @@ template <typename T, typename S, bool ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
     const int32_t* __restrict__ packed, const int32_t* __restrict__ bits,
     const int32_t* __restrict__ prefix, const S* __restrict__ scale, const S* __restrict__ mn,
-    T* __restrict__ out, int64_t F, int64_t G, int blocks_per_sample) {
-  constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kUnpack;
-  __shared__ float s_scale[kGroupsPerBlock];
-  __shared__ float s_min[kGroupsPerBlock];
+    T* __restrict__ out, int64_t N, int64_t F, int64_t G, FastDiv per_sample) {
+  constexpr int kUnit = 2 * Gph<T>::kUnpack;                     // groups of a wave
+  __shared__ float s_scale[kWaves * kUnit];
+  __shared__ float s_min[kWaves * kUnit];
   constexpr bool kStage = IsF32<T>::value;
-  __shared__ u32x4 s_slab[kStage ? kGroupsPerBlock * 64 : 1];
-  u32x4* slab = s_slab + (kStage ? (threadIdx.x >> 6) * (2 * Gph<T>::kUnpack * 64) : 0);
-  const int64_t n = blockIdx.x / blocks_per_sample;
-  const int64_t gb = (int64_t)(blockIdx.x % blocks_per_sample) * kGroupsPerBlock;
+  __shared__ u32x4 s_slab[kStage ? kWaves * kUnit * 64 : 1];
+  const uint32_t wave = wave_of_block();
+  u32x4* slab = s_slab + (kStage ? wave * (kUnit * 64) : 0);
+  const Unit u = unit_of<kUnit>(blockIdx.x * kWaves + wave, per_sample, N, G);
+  const int64_t n = u.n, gb = u.gb;
   const int b = bits[n];
-  const int groups_valid = (int)((G - gb) < kGroupsPerBlock ? (G - gb) : kGroupsPerBlock);
+  const int groups_valid = u.valid;
   float my_scale = 0.0f, my_min = 0.0f;
-  if ((int)threadIdx.x < groups_valid) {
-    const int64_t gi = n * G + gb + threadIdx.x;
+  if ((int)(threadIdx.x & 63) < groups_valid) {
+    const int64_t gi = n * G + gb + (threadIdx.x & 63);
     my_scale = Conv<S>::load(scale, gi);
     my_min = Conv<S>::load(mn, gi);
   }
@@ -405,8 +430,9 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   switch (b) {
 #define ACTNN_CASE(B_)                                                                          \
   case B_:                                                                                      \
-    unpack_groups<T, B_, ROWS>(packed, out, elem_base, F, word_base, groups_valid, s_scale,     \
-                               s_min, my_scale, my_min, slab);                                  \
+    unpack_groups<T, B_, ROWS>(packed, out, elem_base, F, word_base, groups_valid,              \
+                               s_scale + wave * kUnit, s_min + wave * kUnit, my_scale, my_min,  \
+                               slab);                                                           \
     break;
     ACTNN_CASE(1) ACTNN_CASE(2) ACTNN_CASE(3) ACTNN_CASE(4)
     ACTNN_CASE(5) ACTNN_CASE(6) ACTNN_CASE(7) ACTNN_CASE(8)
@@ -519,31 +545,39 @@ __global__ __launch_bounds__(1024) void bits_prefix_kernel(const int32_t* __rest
   }
 }
 
+// Units of `groups` groups per sample and the blocks of four that cover them all.  Numbers of units stay
+// below 2^31 (a unit holds at least a group, so that the tensor would be 1 TiB of 16-bit values).
+bool unit_grid(int64_t N, int64_t G, int groups, int64_t& per_sample, int64_t& blocks) {
+  per_sample = (G + groups - 1) / groups;
+  if (per_sample > 0x7fffffffLL / N) return false;
+  blocks = (N * per_sample + kWaves - 1) / kWaves;
+  return true;
+}
+
 template <typename T, typename S, bool DET, bool ROWS>
 int launch_pack_groups(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
                        void* scale, void* mn_out, int32_t* packed, const void* noise, uint64_t seed, uint64_t offset,
                        int64_t N, int64_t F, hipStream_t s) {
-  constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kPack;
   const int64_t G = (F + kGs - 1) / kGs;
-  const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
-  if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
+  int64_t per_sample, blocks;
+  if (!unit_grid(N, G, 2 * Gph<T>::kPack, per_sample, blocks)) return ACTNN_EINVAL;
   const T* d = static_cast<const T*>(data);
-  pack_mixed_kernel<T, S, DET, ROWS><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
+  pack_mixed_kernel<T, S, DET, ROWS><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
       d, static_cast<const T*>(mn), static_cast<const T*>(mx), bits, prefix,
-      static_cast<S*>(scale), static_cast<S*>(mn_out), packed, static_cast<const T*>(noise), seed, offset, F, G, (int)bps,
-      d + N * F - 16 / sizeof(T));
+      static_cast<S*>(scale), static_cast<S*>(mn_out), packed, static_cast<const T*>(noise), seed, offset, N, F, G,
+      FastDiv((uint32_t)per_sample), d + N * F - 16 / sizeof(T));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
 template <typename T, typename S, bool ROWS>
 int launch_unpack_groups(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
                          const void* mn, void* out, int64_t N, int64_t F, hipStream_t s) {
-  constexpr int kGroupsPerBlock = kHalfWaves * Gph<T>::kUnpack;
   const int64_t G = (F + kGs - 1) / kGs;
-  const int64_t bps = (G + kGroupsPerBlock - 1) / kGroupsPerBlock;
-  if (N * bps > 0x7fffffffLL) return ACTNN_EINVAL;
-  unpack_mixed_kernel<T, S, ROWS><<<dim3((unsigned)(N * bps)), dim3(kThreads), 0, s>>>(
-      packed, bits, prefix, static_cast<const S*>(scale), static_cast<const S*>(mn), static_cast<T*>(out), F, G, (int)bps);
+  int64_t per_sample, blocks;
+  if (!unit_grid(N, G, 2 * Gph<T>::kUnpack, per_sample, blocks)) return ACTNN_EINVAL;
+  unpack_mixed_kernel<T, S, ROWS><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
+      packed, bits, prefix, static_cast<const S*>(scale), static_cast<const S*>(mn), static_cast<T*>(out), N, F, G,
+      FastDiv((uint32_t)per_sample));
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 

@@ -110,6 +110,23 @@ def test_rng_mode_matches_kernel_model(dtype, gs):
     assert np.array_equal(np_bits(out), np_bits(deq))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("G", [1, 3, 4, 5, 7, 8, 9, 16, 17])
+def test_blocks_that_hold_several_short_samples(dtype, G):
+    # a wave takes 4 (fp32) or 8 groups of one sample and a block four such units: samples of less than a
+    # unit, of whole units and of one group more, with numbers of samples that leave the last block ragged
+    for N in (1, 2, 9, 11):
+        bits = [(5 * n) % 8 + 1 for n in range(N)]
+        x, noise = make_groups(N, G, 256, dtype, 100 * N + G, "chan")
+        out, deq = _det_case(x, noise, bits)
+        assert np.array_equal(np_bits(out), np_bits(deq)), N
+        xd, mn, mx, bits_dev, bits_host, packed, scale, seed, offset = _rng_pack(x, bits, 77 + N)
+        scale_o = kernel_mode.kernel_scale(mn.cpu(), mx.cpu(), bits_host.numpy())
+        codes = kernel_mode.rng_codes(x, mn.cpu(), scale_o, bits_host.numpy(), seed, offset)
+        assert np.array_equal(np_bits(scale), np_bits(scale_o)), N
+        assert np.array_equal(packed.cpu().numpy(), layouts.pack_mixed(codes, bits_host.numpy())), N
+
+
 @pytest.mark.parametrize("bits", [1, 2, 4])
 def test_rng_mode_unbiased_with_closed_form_variance(bits):
     # 10^4 independent roundings of the same 4 groups: replicate them as 10^4 samples
