@@ -41,6 +41,7 @@ SIGNATURES = {
                           c_i64, c_i64, c_i64, c_i32, c_vp],
     "actnn_unpack_single": [c_vp, c_i32, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32, c_vp],
     "actnn_unpack_mixed_rows": [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i32, c_i32, c_vp],
+    "actnn_unpack_mixed_rows_transposed": [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32, c_vp],
     "actnn_quantize_rows": [c_vp, c_vp, c_vp, c_i32, ctypes.c_float, c_vp, c_i32, c_vp, c_vp, c_vp, c_i32, c_i64, c_vp,
                             c_vp, c_vp, c_u64, c_u64, c_i64, c_i64, c_i32, c_i32, c_vp],
     "actnn_quantize_fixed": [c_vp, c_vp, c_vp, c_i32, c_vp, c_vp, c_vp, c_u64, c_u64, c_i64, c_i64, c_i32, c_i32, c_vp],

@@ -161,6 +161,30 @@ def unpack_rows_mixed(packed, bits, scale, mn, N, F, dtype):
     return out
 
 
+def unpack_rows_mixed_transposed(packed, bits, scale, mn, N, F):
+    """The [N, F] rows of quantize_activation_device in the 16-bit dtype of `scale`, their samples contiguous in
+    memory (strides 1 and N rounded up to 64)."""
+    g.check_typed(packed, "data", torch.int32, 1)
+    g.check_typed(bits, "bits", torch.int32, 1)
+    g.check_float(scale, "scale", 3)
+    g.check_float(mn, "min", 3)
+    G = (F + 255) // 256
+    if mn.dtype != scale.dtype or scale.element_size() != 2:
+        raise RuntimeError("The type of min is not correct!")
+    if scale.numel() != N * G or mn.numel() != N * G or bits.numel() != N:
+        raise RuntimeError("unpack_mixed_precision: shape mismatch")
+    total, prefix = _bits_info(bits)
+    if packed.numel() < total * G * 8:
+        raise RuntimeError("unpack_mixed_precision: packed stream is too short")
+    ld = (N + 63) // 64 * 64
+    out = torch.empty(F, ld, dtype=scale.dtype, device=packed.device)
+    with g.on_device(packed.device):
+        check(g.lib().actnn_unpack_mixed_rows_transposed(
+            packed.data_ptr(), bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(), mn.data_ptr(), out.data_ptr(),
+            N, F, ld, g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)), "unpack_mixed_precision")
+    return out[:, :N].t()
+
+
 def unpack_mixed_precision(data, bits, scale, min, N, num_groups, group_size):
     g.check_typed(data, "data", torch.int32, 1)
     g.check_typed(bits, "bits", torch.int32, 1)

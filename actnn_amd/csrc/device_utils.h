@@ -600,6 +600,40 @@ template <typename T> struct Noise {
   }
 };
 
+// ------------------------------------------------------------------ transposed tiles of 16-bit values
+// A block of 256 threads holds 64 samples of 256 features: half-wave h the samples 8h .. 8h + 7, its lane j the
+// features 8j .. 8j + 7 of each, two to a word as they lie in memory (w[sample][feature / 2]).  It leaves them
+// with the samples contiguous: out[feature * ld + sample].  Two words of neighbouring samples make two words
+// of neighbouring features' rows (one byte permute each), so a lane has 16 bytes of 8 rows; through LDS the
+// eight half-waves' pieces become whole 128-byte lines of a row.  The pieces of a row are permuted in LDS by
+// the lane that wrote them, which spreads both the writes (rows 8 apart) and the reads over all banks.
+// ld is a multiple of 8 and out 16-byte aligned; rows from `features` on and samples from ld on do not exist.
+constexpr int kTileSamples = 64;
+template <typename T>
+ACTNN_DEV void store_transposed_tile(const uint32_t (&w)[8][4], u32x4* s_tile, T* out, int64_t feature0,
+                                     int64_t features, int64_t sample0, int64_t ld) {
+  static_assert(sizeof(T) == 2, "two values to a word");
+  const uint32_t lane = threadIdx.x & 31u, half = threadIdx.x >> 5;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    u32x4 even, odd;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      even[p] = __builtin_amdgcn_perm(w[2 * p + 1][j], w[2 * p][j], 0x05040100u);
+      odd[p] = __builtin_amdgcn_perm(w[2 * p + 1][j], w[2 * p][j], 0x07060302u);
+    }
+    s_tile[(8 * lane + 2 * j) * 8 + (half ^ (lane & 7u))] = even;
+    s_tile[(8 * lane + 2 * j + 1) * 8 + (half ^ (lane & 7u))] = odd;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t piece = i * 256 + threadIdx.x, f = piece >> 3, c = piece & 7u;
+    if (feature0 + f < features && sample0 + 8 * c < ld)
+      store16(out + (feature0 + f) * ld + sample0 + 8 * c, s_tile[f * 8 + (c ^ ((f >> 3) & 7u))]);
+  }
+}
+
 // ------------------------------------------------------------------ host-side helpers
 // Whether a kernel's results should pass the caches by: a tensor of at most half the chip's last-level
 // cache (256 MB) is still there when the next kernel reads it, one that is larger only displaces others

@@ -441,6 +441,82 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------- unpack, transposed
+// The rows of a linear layer's input with the samples contiguous, out[feature * ld + sample], as the matrix
+// product of its weight gradient reads them fastest: that product sums over the samples, and with both factors
+// stored sample by sample its loads run across the rows (bf16, go [N, O] and x [N, F], us with x as rows / with
+// x like this: [8192, 4096] x [8192, 4096] 260 / 202, [8192, 1024] x [8192, 1024] 54.5 / 39.0,
+// [2048, 1024] x [2048, 1024] 17.5 / 14.4, [256, 1024] x [256, 1024] 6.7 / 6.3).
+// Bound by the write, as unpack: the values are unpack's bit for bit.  A half-wave takes 8 samples of one group (a
+// block 64), whose words are loaded before the first is decoded.  The widths of the two halves of a wave
+// differ, so the decoders take them at run time: the table of four levels where neither exceeds 2 bits.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void unpack_mixed_transposed_kernel(
+    const int32_t* __restrict__ packed, const int32_t* __restrict__ bits, const int32_t* __restrict__ prefix,
+    const T* __restrict__ scale, const T* __restrict__ mn, T* __restrict__ out, int64_t N, int64_t F, int64_t G,
+    int64_t ld, int64_t blocks, FastDiv by_groups) {
+  __shared__ u32x4 s_tile[kGs * kTileSamples / 8];
+  // (the groups of a tile of samples on one XCD: at 2 bits two neighbouring groups share a line of the stream)
+  const int64_t block = xcd_block();
+  if (block >= blocks) return;
+  const uint32_t tile = by_groups.div((uint32_t)block), g = (uint32_t)block - tile * by_groups.d;
+  const uint32_t lane = threadIdx.x & 31u, half = threadIdx.x >> 5;
+  const int64_t sample0 = (int64_t)tile * kTileSamples, n0 = sample0 + 8 * half;
+  // lane l looks up sample l & 7 of the half-wave's eight
+  const int64_t nl = n0 + (lane & 7u) < N ? n0 + (lane & 7u) : N - 1;
+  const int width = bits[nl];
+  const int my_bits = width < 1 ? 1 : width > 8 ? 8 : width;
+  const int my_prefix = prefix[nl];
+  const float my_scale = Conv<T>::load(scale, nl * G + g), my_min = Conv<T>::load(mn, nl * G + g);
+  uint32_t lo[8], hi[8];
+  int b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    b[i] = __shfl(my_bits, i, 32);
+    const int32_t* words = packed + (int64_t)__shfl(my_prefix, i, 32) * G * 8 + (int64_t)g * b[i] * 8;
+    lo[i] = (int)lane < 8 * b[i] ? (uint32_t)words[lane] : 0u;
+    hi[i] = (int)lane + 32 < 8 * b[i] ? (uint32_t)words[lane + 32] : 0u;
+  }
+  uint32_t w[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const Dequant<T> dq(__shfl(my_scale, i, 32), __shfl(my_min, i, 32));
+    const uint32_t acc = transpose32(lo[i], lane);
+    if (__builtin_amdgcn_ballot_w64(b[i] > 2) == 0) {
+      // (as unpack_groups: lane l evaluates level l & 3, a byte permute picks the two values of a word)
+      const float mine = dq(lane & 3u);
+      const int h = (int)(IsBf16<T>::value ? float_to_bf16_bits(mine) : float_to_half_bits(mine));
+      const uint32_t l0 = (uint32_t)__builtin_amdgcn_update_dpp(0, h, 0x00, 0xF, 0xF, true);
+      const uint32_t l1 = (uint32_t)__builtin_amdgcn_update_dpp(0, h, 0x55, 0xF, 0xF, true);
+      const uint32_t l2 = (uint32_t)__builtin_amdgcn_update_dpp(0, h, 0xAA, 0xF, 0xF, true);
+      const uint32_t l3 = (uint32_t)__builtin_amdgcn_update_dpp(0, h, 0xFF, 0xF, 0xF, true);
+      const uint32_t lut_lo = l0 | (l1 << 16), lut_hi = l2 | (l3 << 16);
+      const uint32_t pair = ((1u << b[i]) - 1u) * 0x00010001u;
+      const uint32_t a = acc & 0xffffu, both = a | (a << (16 - b[i]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t sel = __umul24((both >> (2 * j * b[i])) & pair, 0x0202u) + 0x01000100u;
+        w[i][j] = __builtin_amdgcn_perm(lut_hi, lut_lo, sel);
+      }
+    } else {
+      uint64_t codes = acc;
+      if (__builtin_amdgcn_ballot_w64(b[i] > 4) != 0) codes |= (uint64_t)transpose32(hi[i], lane) << 32;
+      const uint32_t mask = (1u << b[i]) - 1u;
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = dq((uint32_t)(codes >> (k * b[i])) & mask);
+      const u32x4 packed8 = words_of8(out, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i][j] = packed8[j];
+    }
+    if (n0 + i >= N) {                                 // the row's end up to ld
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i][j] = 0u;
+    }
+  }
+  store_transposed_tile(w, s_tile, out, (int64_t)g * kGs, F, sample0, ld);
+}
+
 // ---------------------------------------------------------------------------- generic group size
 // One block per (sample, group); codes staged as bytes in LDS, then thread w assembles word w.
 template <typename T, bool DET>
@@ -581,6 +657,17 @@ int launch_unpack_groups(const int32_t* packed, const int32_t* bits, const int32
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
+template <typename T>
+int launch_unpack_transposed(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
+                             const void* mn, void* out, int64_t N, int64_t F, int64_t ld, hipStream_t s) {
+  const int64_t G = (F + kGs - 1) / kGs, tiles = (N + kTileSamples - 1) / kTileSamples;
+  if (tiles > (0x7fffffffLL - kXcds) / G) return ACTNN_EINVAL;
+  unpack_mixed_transposed_kernel<T><<<dim3(xcd_grid(tiles * G)), dim3(kThreads), 0, s>>>(
+      packed, bits, prefix, static_cast<const T*>(scale), static_cast<const T*>(mn), static_cast<T*>(out), N, F, G, ld,
+      tiles * G, FastDiv((uint32_t)G));
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
 // whole groups at an aligned address take the kernels without the row ends
 template <typename T, typename S>
 int launch_pack_rows(const void* data, const void* mn, const void* mx, const int32_t* bits, const int32_t* prefix,
@@ -674,6 +761,22 @@ extern "C" int actnn_unpack_mixed_rows(const int32_t* packed, const int32_t* bit
     case ACTNN_F32: return launch_unpack_rows<float, float>(packed, bits, prefix, scale, mn, out, N, F, s);
     case ACTNN_F16: return launch_unpack_rows<__half, __half>(packed, bits, prefix, scale, mn, out, N, F, s);
     case ACTNN_BF16: return launch_unpack_rows<bf16_t, bf16_t>(packed, bits, prefix, scale, mn, out, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
+extern "C" int actnn_unpack_mixed_rows_transposed(const int32_t* packed, const int32_t* bits, const int32_t* prefix,
+                                                  const void* scale, const void* mn, void* out, int64_t N, int64_t F,
+                                                  int64_t ld, int dtype, void* stream) {
+  using namespace actnn;
+  if (N < 0 || F < 0 || ld < N || ld % 8 != 0 || ld > (N + kTileSamples - 1) / kTileSamples * kTileSamples) return ACTNN_EINVAL;
+  if (N == 0 || F == 0) return ACTNN_OK;
+  if (!packed || !bits || !prefix || !scale || !mn || !out) return ACTNN_EINVAL;
+  if (!aligned16(out)) return ACTNN_EALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case ACTNN_F16: return launch_unpack_transposed<__half>(packed, bits, prefix, scale, mn, out, N, F, ld, s);
+    case ACTNN_BF16: return launch_unpack_transposed<bf16_t>(packed, bits, prefix, scale, mn, out, N, F, ld, s);
     default: return ACTNN_EDTYPE;
   }
 }

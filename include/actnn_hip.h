@@ -93,6 +93,12 @@ int actnn_unpack_mixed(const int32_t* packed, const int32_t* bits, const int32_t
 int actnn_unpack_mixed_rows(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
                             const void* mn, void* out, int64_t N, int64_t F, int dtype, int store_dtype,
                             void* stream);
+/* The same rows in a 16-bit dtype (store_dtype the dtype) with the samples contiguous: out [F, ld], sample n of
+ * feature f at f * ld + n, the columns N .. ld - 1 zero.  ld a multiple of 8, at least N and at most N
+ * rounded up to 64; out 16-byte aligned.  What the weight gradient of ops.py:386-433 multiplies. */
+int actnn_unpack_mixed_rows_transposed(const int32_t* packed, const int32_t* bits, const int32_t* prefix,
+                                       const void* scale, const void* mn, void* out, int64_t N, int64_t F,
+                                       int64_t ld, int dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------
  * pack_single_precision: one bit width (1, 2, 4 or 8) for the whole tensor; 8/bits

@@ -117,6 +117,22 @@ def test_rows_at_widths_of_their_own_equal_the_padded_composition(dtype, initial
             assert torch.equal(back, full.view(N, -1)[:, :F]), (N, F, shift)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,F", [(1, 256), (7, 300), (63, 512), (64, 257), (65, 4096), (130, 1000), (2050, 264)])
+@pytest.mark.parametrize("avg", [2, 5])
+def test_rows_with_the_samples_contiguous(dtype, N, F, avg):
+    # (both widths of a wave's halves up to 2, up to 4 and above; ragged last tiles of 64 samples and 256 features)
+    x = _rows(N, F, dtype, 0, N + F) * torch.exp(torch.randn(N, 1, device="cuda", generator=torch.Generator("cuda").manual_seed(F))).to(dtype)
+    alloc = qscheme.AllocationArgs(N, 256 / F, None, 8, avg)
+    alloc.store_dtype = dtype
+    packed, bits, scale, low = ext_q.quantize_activation_device(x, N, None, alloc)
+    low = low.view(N, -1, 1)
+    want = ext_q.unpack_rows_mixed(packed, bits, scale, low, N, F, dtype)
+    got = ext_q.unpack_rows_mixed_transposed(packed, bits, scale, low, N, F)
+    assert got.shape == want.shape and got.stride(0) == 1 and torch.equal(got, want)
+    assert not got._base[:, N:].any()                        # the columns behind the last sample are zero
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("N,F", [(1024, 1024), (1025, 2048), (2047, 1000), (150, 8192), (16384, 72)])
 def test_row_and_column_sums_from_one_read(dtype, N, F):
