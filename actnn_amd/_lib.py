@@ -31,6 +31,7 @@ SIGNATURES = {
     "actnn_range_sqr": [c_vp, c_vp, c_vp, c_i64, c_i64, ctypes.c_float, c_vp, c_i32, c_i32, c_vp],
     "actnn_sample_sqnorm": [c_vp, c_vp, c_i64, c_i64, c_i32, c_i32, c_vp],
     "actnn_row_column_sums": [c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i32, c_vp],
+    "actnn_row_column_sums_transposed": [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32, c_vp],
     "actnn_allocate_bits_device": [c_vp, c_vp, ctypes.c_float, c_vp, c_i32, c_vp, c_vp, c_vp, c_i64, c_i64, c_i32,
                                    c_i64, c_i32, c_vp],
     "actnn_bits_prefix": [c_vp, c_vp, c_i64, c_vp],

@@ -98,3 +98,26 @@ def row_column_sums(x, with_sqnorm):
                                             part.data_ptr(), N, F, g.DTYPE_CODE[x.dtype], g.stream_ptr(x.device)),
               "row_column_sums")
     return columns, sq
+
+
+def row_column_sums_transposed(x, with_columns, with_sqnorm):
+    """(sum over the rows or None, squared norm of every row or None, the rows turned over: [F, N rounded up to 64],
+    zero behind row N) of a 16-bit [N, F] tensor from one read, or None where row_column_sums says None for the
+    tensor's form.  The sums' order is another one than row_column_sums'."""
+    if (x.dim() != 2 or x.dtype not in (torch.float16, torch.bfloat16) or not x.is_cuda or not x.is_contiguous()
+            or torch.is_grad_enabled() or x.shape[1] % 8 != 0 or x.numel() == 0
+            or not g.has_storage(x) or x.data_ptr() % 16 != 0):
+        return None
+    N, F = x.shape
+    ld = (N + 63) // 64 * 64
+    out = torch.empty(F, ld, dtype=x.dtype, device=x.device)
+    columns = torch.empty(F, dtype=x.dtype, device=x.device) if with_columns else None
+    sq = torch.empty(N, dtype=torch.float32, device=x.device) if with_sqnorm else None
+    part = torch.empty(ld // 64, F, dtype=torch.float32, device=x.device) if with_columns else None
+    sq_part = torch.empty((F + 255) // 256, N, dtype=torch.float32, device=x.device) if with_sqnorm else None
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    with g.on_device(x.device):
+        check(g.lib().actnn_row_column_sums_transposed(
+            x.data_ptr(), ptr(columns), ptr(sq), out.data_ptr(), ptr(part), ptr(sq_part), N, F, ld, g.DTYPE_CODE[x.dtype],
+            g.stream_ptr(x.device)), "row_column_sums_transposed")
+    return columns, sq, out

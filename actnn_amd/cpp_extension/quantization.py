@@ -162,8 +162,8 @@ def unpack_rows_mixed(packed, bits, scale, mn, N, F, dtype):
 
 
 def unpack_rows_mixed_transposed(packed, bits, scale, mn, N, F):
-    """The [N, F] rows of quantize_activation_device in the 16-bit dtype of `scale`, their samples contiguous in
-    memory (strides 1 and N rounded up to 64)."""
+    """The [N, F] rows of quantize_activation_device in the 16-bit dtype of `scale` turned over, their samples
+    contiguous: [F, N rounded up to 64], zero behind sample N."""
     g.check_typed(packed, "data", torch.int32, 1)
     g.check_typed(bits, "bits", torch.int32, 1)
     g.check_float(scale, "scale", 3)
@@ -182,7 +182,7 @@ def unpack_rows_mixed_transposed(packed, bits, scale, mn, N, F):
         check(g.lib().actnn_unpack_mixed_rows_transposed(
             packed.data_ptr(), bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(), mn.data_ptr(), out.data_ptr(),
             N, F, ld, g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)), "unpack_mixed_precision")
-    return out[:, :N].t()
+    return out
 
 
 def unpack_mixed_precision(data, bits, scale, min, N, num_groups, group_size):

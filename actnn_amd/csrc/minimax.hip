@@ -337,12 +337,89 @@ __global__ __launch_bounds__(kThreads) void row_column_sums_kernel(const T* __re
   }
 }
 
+// The same sums of 16-bit rows, and the rows turned over on the way: out[column * ld + row], rows up to ld zero, as
+// the product of the weight gradient reads its left factor fastest.  A block takes 64 rows of 256 columns
+// (store_transposed_tile), sums its columns (part[block row][F]) and the squares of its rows' pieces
+// (sq_part[column tile][N]); the second kernel adds both up in a fixed order.  Bound by reading and writing the
+// tensor once.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void row_column_sums_transposed_kernel(
+    const T* __restrict__ x, T* __restrict__ out, float* __restrict__ part, float* __restrict__ sq_part, int64_t N,
+    int64_t F, int64_t ld, int64_t blocks, FastDiv by_tiles) {
+  __shared__ u32x4 s_tile[256 * kTileSamples / 8];
+  __shared__ float s_sum[kThreads / 64][256];
+  const int64_t block = xcd_block();
+  if (block >= blocks) return;
+  const uint32_t row = by_tiles.div((uint32_t)block), tile = (uint32_t)block - row * by_tiles.d;
+  const uint32_t lane = threadIdx.x & 31u, half = threadIdx.x >> 5;
+  const int64_t c = (int64_t)tile * 256 + 8 * lane, n0 = (int64_t)row * kTileSamples + 8 * half;
+  uint32_t w[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    u32x4 u = {0, 0, 0, 0};
+    if (c < F && n0 + i < N) u = load16(x + (n0 + i) * F + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[i][j] = u[j];
+  }
+  if (part) {
+    constexpr bool kBf16 = !__is_same(T, __half);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float a = 0.0f, b = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        a += kBf16 ? as_float(w[i][j] << 16) : half_bits_to_float(w[i][j] & 0xffffu);
+        b += kBf16 ? as_float(w[i][j] & 0xffff0000u) : half_bits_to_float(w[i][j] >> 16);
+      }
+      a += __shfl_xor(a, 32);
+      b += __shfl_xor(b, 32);
+      if ((threadIdx.x & 32u) == 0) {
+        s_sum[threadIdx.x >> 6][8 * lane + 2 * j] = a;
+        s_sum[threadIdx.x >> 6][8 * lane + 2 * j + 1] = b;
+      }
+    }
+  }
+  if (sq_part) {
+    // eight sums over 32 lanes: each exchange halves the sums a lane still carries, so that lane l ends with
+    // that of row l >> 2
+    float q[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = square_sum16<T>((u32x4){w[i][0], w[i][1], w[i][2], w[i][3]});
+    float h[4], g[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = ((lane & 16u) ? q[i + 4] : q[i]) + __shfl_xor((lane & 16u) ? q[i] : q[i + 4], 16);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) g[i] = ((lane & 8u) ? h[i + 2] : h[i]) + __shfl_xor((lane & 8u) ? h[i] : h[i + 2], 8);
+    float v = ((lane & 4u) ? g[1] : g[0]) + __shfl_xor((lane & 4u) ? g[0] : g[1], 4);
+    v += __shfl_xor(v, 2);
+    v += __shfl_xor(v, 1);
+    const int64_t n = n0 + (lane >> 2);
+    if ((lane & 3u) == 0 && n < N) sq_part[(int64_t)tile * N + n] = v;
+  }
+  store_transposed_tile(w, s_tile, out, (int64_t)tile * 256, F, (int64_t)row * kTileSamples, ld);
+  const int64_t column = (int64_t)tile * 256 + threadIdx.x;
+  if (part && column < F)                              // (the barrier inside store_transposed_tile lies between)
+    part[(int64_t)row * F + column] = (s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x]) + (s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x]);
+}
+
 // out[c] = sum of part[b][c] over the block rows b: 16 threads per vector of four columns, each every 16th
-// block row, then folded in halves.
+// block row, then folded in halves.  Blocks from column_blocks on: sq[n] = sum of sq_part[t][n] over the tiles t.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void fold_columns_kernel(const float* __restrict__ part, T* __restrict__ out,
-                                                               int64_t F, int64_t B) {
+                                                               int64_t F, int64_t B, unsigned column_blocks,
+                                                               const float* __restrict__ sq_part, float* __restrict__ sq,
+                                                               int64_t N, int tiles) {
   __shared__ float s[16][16][4];
+  if (blockIdx.x >= column_blocks) {
+    const int64_t n = (int64_t)(blockIdx.x - column_blocks) * kThreads + threadIdx.x;
+    if (n < N) {
+      float v = 0.0f;
+#pragma unroll 4
+      for (int t = 0; t < tiles; ++t) v += sq_part[(int64_t)t * N + n];
+      sq[n] = v;
+    }
+    return;
+  }
   const int v = threadIdx.x & 15, y = threadIdx.x >> 4;
   const int64_t c = ((int64_t)blockIdx.x * 16 + v) * 4;
   float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -387,7 +464,25 @@ int launch_sums(const void* x, void* columns, float* sq, float* part, int64_t N,
   } else {
     row_column_sums_kernel<T, 1, false><<<dim3((unsigned)per, (unsigned)B), blk, 0, s>>>(d, part, nullptr, N, F);
   }
-  fold_columns_kernel<T><<<dim3((unsigned)((F / 4 + 15) / 16)), blk, 0, s>>>(part, static_cast<T*>(columns), F, B);
+  const unsigned column_blocks = (unsigned)((F / 4 + 15) / 16);
+  fold_columns_kernel<T><<<dim3(column_blocks), blk, 0, s>>>(part, static_cast<T*>(columns), F, B, column_blocks, nullptr, nullptr, 0, 0);
+  ACTNN_RETURN_LAUNCH_STATUS();
+}
+
+template <typename T>
+int launch_sums_transposed(const void* x, void* columns, float* sq, void* out, float* part, float* sq_part, int64_t N,
+                           int64_t F, int64_t ld, hipStream_t s) {
+  const int64_t rows = (N + kTileSamples - 1) / kTileSamples, tiles = (F + 255) / 256;
+  if (rows > (0x7fffffffLL - kXcds) / tiles) return ACTNN_EINVAL;
+  const dim3 blk(kThreads);
+  row_column_sums_transposed_kernel<T><<<dim3(xcd_grid(rows * tiles)), blk, 0, s>>>(
+      static_cast<const T*>(x), static_cast<T*>(out), columns ? part : nullptr, sq ? sq_part : nullptr, N, F, ld,
+      rows * tiles, FastDiv((uint32_t)tiles));
+  const unsigned column_blocks = columns ? (unsigned)((F / 4 + 15) / 16) : 0;
+  const unsigned row_blocks = sq ? (unsigned)((N + kThreads - 1) / kThreads) : 0;
+  if (column_blocks + row_blocks)
+    fold_columns_kernel<T><<<dim3(column_blocks + row_blocks), blk, 0, s>>>(part, static_cast<T*>(columns), F, rows, column_blocks,
+                                                                           sq_part, sq, N, (int)tiles);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -455,6 +550,21 @@ extern "C" int actnn_row_column_sums(const void* x, void* columns, float* sqnorm
     case ACTNN_F32: return launch_sums<float>(x, columns, sqnorm, part, N, F, s);
     case ACTNN_F16: return launch_sums<__half>(x, columns, sqnorm, part, N, F, s);
     case ACTNN_BF16: return launch_sums<bf16_t>(x, columns, sqnorm, part, N, F, s);
+    default: return ACTNN_EDTYPE;
+  }
+}
+
+extern "C" int actnn_row_column_sums_transposed(const void* x, void* columns, float* sqnorm, void* transposed, float* part,
+                                                float* sq_part, int64_t N, int64_t F, int64_t ld, int dtype, void* stream) {
+  using namespace actnn;
+  if (N <= 0 || F <= 0 || F % 8 != 0 || N > 0x7fffffffLL || F > 0x7fffffffLL) return ACTNN_EINVAL;
+  if (ld < N || ld % 8 != 0 || ld > (N + kTileSamples - 1) / kTileSamples * kTileSamples) return ACTNN_EINVAL;
+  if (!x || !transposed || (columns && !part) || (sqnorm && !sq_part)) return ACTNN_EINVAL;
+  if (!aligned16(x) || !aligned16(transposed) || !aligned16(part)) return ACTNN_EALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case ACTNN_F16: return launch_sums_transposed<__half>(x, columns, sqnorm, transposed, part, sq_part, N, F, ld, s);
+    case ACTNN_BF16: return launch_sums_transposed<bf16_t>(x, columns, sqnorm, transposed, part, sq_part, N, F, ld, s);
     default: return ACTNN_EDTYPE;
   }
 }

@@ -431,20 +431,30 @@ def _fused_grad_weight_ok(quantized, shape, go):
             and isinstance(q_input, torch.Tensor) and q_input.is_cuda)
 
 
-def _input_by_sample(quantized, shape):
-    """The input of a linear layer's weight gradient, [N, F] with the samples contiguous in memory, or None where
-    the rows of dequantize_activation are as good: fp32, streams of one width, fewer than 2048 samples.  The
-    product of the gradient takes less time with it and its unpack a few us more (bf16, unpack + product as
-    rows / like this, us: [2048, 1024] x [2048, 1024] 25.0 / 24.3, [2047, 4096] x [2047, 4096] 83.8 / 81.4,
-    [8192, 1024] x [8192, 1024] 74.4 / 52.7, [8192, 4096] x [8192, 4096] 268 / 227; [1024, 1024] x [1024, 1024]
-    18.6 / 18.1, but [1021, 4096] x [1021, 4096] 54.8 / 57.3 and [512, 1024] x [512, 1024] 14.8 / 15.6)."""
+def _by_sample(quantized, shape):
+    """Whether the factors of the weight gradient's product can be had with the samples contiguous in memory: it
+    sums over them and takes less time like that.  Turning the input over costs its unpack 3 to 8 us more, and
+    the gradient, turned over by the pass that sums it, next to nothing (one read in place of two for short
+    ones).  Unpack, sums and product, us (bf16, [N, F] and [N, O]), as rows / the input turned over / both:
+      N, F, O           rows   input   both            N, F, O           rows   input   both
+      8192, 4096, 4096  281.9  263.9  245.4            1024, 4096, 4096   60.7   58.9   53.3
+      8191, 4096, 4096  289.6  274.3  232.1            1024, 1024, 1024   26.7   26.7   25.1
+      8192, 1024, 1024   84.4   62.1   53.6            512, 1024, 1024    25.6   27.6   21.7
+      2048, 4096, 4096   90.2   83.2   76.0            200, 1024, 1024    23.1   25.4   20.6
+      2048, 1024, 1024   34.6   33.8   31.3            100, 1024, 1024    19.4   21.6   18.4
+      2047, 4096, 4096   96.5   97.6   79.8            64, 1024, 1024     17.0   19.6   17.2
+      2048, 256, 100     36.2   31.2    -              1024, 256, 100     32.7   32.0    -
+    So both from _BOTH_BY_SAMPLE samples on, the input alone (a gradient row_column_sums_transposed does not
+    take) from _INPUT_BY_SAMPLE.  The turned gradient is one more tensor of the gradient's size until the
+    product has been queued.  Not for fp32 and streams of one width, which have no such unpack."""
     if not config.compress_activation or config.simulate or config.swap or config.group_size != 256:
-        return None
-    q_input, q_bits, q_scale, q_min = quantized
-    if not (len(shape) == 2 and shape[0] >= 2048 and isinstance(q_bits, torch.Tensor)
-            and (q_scale.dtype == torch.float16 or q_scale.dtype == torch.bfloat16 and not _stored_as_bf16(shape, quantized))):
-        return None
-    return ext_quantization.unpack_rows_mixed_transposed(q_input, q_bits, q_scale, q_min, *shape)
+        return False
+    _, q_bits, q_scale, _ = quantized
+    return (len(shape) == 2 and shape[0] >= _BOTH_BY_SAMPLE and isinstance(q_bits, torch.Tensor)
+            and (q_scale.dtype == torch.float16 or q_scale.dtype == torch.bfloat16 and not _stored_as_bf16(shape, quantized)))
+
+
+_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE = 128, 2048
 
 
 class linear(Function):
@@ -466,12 +476,20 @@ class linear(Function):
         go = grad_output.reshape(-1, grad_output.shape[-1])
         # the bias's gradient and the norms of the samples (rows, if there is one row each) from one read
         need_bias = bias is not None and ctx.needs_input_grad[2]
-        sums = None
-        if need_bias:
-            sums = ext_minimax.row_column_sums(go, bool(ctx.scheme) and grad_output.dim() == 2 and ctx.scheme.wants_sqnorm(grad_output))
+        fused = _fused_grad_weight_ok(quantized, q_input_shape, go)
+        by_sample = not fused and ctx.needs_input_grad[1] and _by_sample(quantized, q_input_shape)
+        want_sq = bool(ctx.scheme) and grad_output.dim() == 2 and ctx.scheme.wants_sqnorm(grad_output)
+        sums = go_turned = None
+        if by_sample:
+            sums = ext_minimax.row_column_sums_transposed(go, need_bias, want_sq)
+            go_turned = sums[2] if sums is not None else None
+            # (a batch of gradients at once keeps the product it had)
+            by_sample = go_turned is not None or q_input_shape[0] >= _INPUT_BY_SAMPLE and ext_quantization.g.has_storage(go)
+        if sums is None and need_bias:
+            sums = ext_minimax.row_column_sums(go, want_sq)
         if ctx.scheme:
             ctx.scheme.set_scale(grad_output, sums[1] if sums is not None else None)
-        if _fused_grad_weight_ok(quantized, q_input_shape, go):
+        if fused:
             # the weight gradient is computed straight from the packed stream (dequantised tiles
             # only ever exist in LDS), nothing is materialised
             q_input, q_bits, q_scale, q_min = quantized
@@ -481,12 +499,14 @@ class linear(Function):
                 go, q_input, q_bits, q_scale, q_min, q_input_shape[-1], weight.dtype) \
                 if ctx.needs_input_grad[1] else None
         else:
-            x = _input_by_sample(quantized, q_input_shape)
-            if x is None:
+            if by_sample:
+                x = ext_quantization.unpack_rows_mixed_transposed(*quantized, *q_input_shape)
+                # (both are zero behind the last sample: the product may as well run over whole tiles)
+                grad_weight = go_turned.mm(x.t()) if go_turned is not None else go.t().mm(x[:, :go.shape[0]].t())
+            else:
                 x = dequantize_activation(quantized, q_input_shape)
-                x = x.reshape(-1, x.shape[-1])
-            grad_weight = go.t().mm(x) if ctx.needs_input_grad[1] else None
-            del x
+                grad_weight = go.t().mm(x.reshape(-1, x.shape[-1])) if ctx.needs_input_grad[1] else None
+            del x, go_turned
         del quantized, ctx.saved
         empty_cache(config.empty_cache_threshold)
         grad_input = go.mm(weight).view(*q_input_shape) if ctx.needs_input_grad[0] else None

@@ -253,6 +253,12 @@ int actnn_sample_sqnorm(const void* x, float* part, int64_t N, int64_t F, int sl
  * Replaces grad_output.sum(0) of ops.py:386-433 and the norms of qscheme.py:47-55. */
 int actnn_row_column_sums(const void* x, void* columns, float* sqnorm, float* part, int64_t N, int64_t F, int dtype,
                           void* stream);
+/* The same of 16-bit rows, with the rows turned over from the same read: transposed [F, ld], row n of column f at
+ * f * ld + n, n from N to ld - 1 zero; ld a multiple of 8, at least N and at most N rounded up to 64.  columns and
+ * sqnorm may be null; the sums are in fp32 in a fixed order, another one than above.  part: fp32 [ceil(N / 64), F],
+ * sq_part: fp32 [ceil(F / 256), N].  F a multiple of 8; x, transposed and part 16-byte aligned. */
+int actnn_row_column_sums_transposed(const void* x, void* columns, float* sqnorm, void* transposed, float* part,
+                                     float* sq_part, int64_t N, int64_t F, int64_t ld, int dtype, void* stream);
 
 /* Same allocation on the DEVICE for the case every layer uses at every step: all N items start
  * at initial_bits (1..8) with weight 1 and `target` is the bit budget, so exactly

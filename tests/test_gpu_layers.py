@@ -1,6 +1,8 @@
 """Layer-level behaviour on the GPU: the compressed autograd functions against stock torch layers
 (the reference checks the same things in tests/test_act_quantized_ops.py:318-447 and
 tests/test_linear.py)."""
+import math
+
 import pytest
 import torch
 import torch.nn as nn
@@ -555,6 +557,31 @@ def test_linear_backward_of_a_batch_of_gradients():
         for a, b in zip(got, torch.autograd.grad(layer(x), wanted, grads[i])):
             # the same products summed in another order: 1024 terms, at most 1024 * 2^-24 of their 2-norm
             assert (a[i] - b).norm() <= 1024 * 2.0 ** -24 * b.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,F,O,bias", [(128, 256, 8, True), (130, 300, 1000, True), (2050, 264, 100, True), (300, 512, 512, False)])
+def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias, monkeypatch):
+    """The factors of the weight gradient turned over (the input alone where the gradient's rows are no whole
+    16-byte vectors): the gradients are those of the product over rows, in another order of addition."""
+    torch.manual_seed(0)
+    layer = actnn_amd.QLinear(F, O, bias=bias).to(DEV, dtype)
+    x = torch.randn(N, F, device=DEV).to(dtype).requires_grad_()
+    grad = torch.randn(N, O, device=DEV).to(dtype)
+    layer.scheme.set_scale(grad)
+    wanted = [x, layer.weight] + ([layer.bias] if bias else [])
+    got = []
+    for limits in ((128, 2048), (1 << 30, 1 << 30)):
+        monkeypatch.setattr(ops, "_BOTH_BY_SAMPLE", limits[0])
+        monkeypatch.setattr(ops, "_INPUT_BY_SAMPLE", limits[1])
+        torch.manual_seed(1)
+        got.append(torch.autograd.grad(layer(x), wanted, grad, retain_graph=False) + (layer.scheme.scales,))
+    eps = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    assert torch.equal(got[0][0], got[1][0])
+    for a, b in zip(got[0][1:], got[1][1:]):
+        # N terms added in another order: at most 2 N 2^-24 of their 2-norms, then one rounding each
+        bound = eps * b.double().norm() + 2 * N * 2.0 ** -24 * b.double().norm() * math.sqrt(N)
+        assert (a.double() - b.double()).norm() <= bound
 
 
 def test_resnet50_channels_last_step_runs():

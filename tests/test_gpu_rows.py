@@ -129,8 +129,8 @@ def test_rows_with_the_samples_contiguous(dtype, N, F, avg):
     low = low.view(N, -1, 1)
     want = ext_q.unpack_rows_mixed(packed, bits, scale, low, N, F, dtype)
     got = ext_q.unpack_rows_mixed_transposed(packed, bits, scale, low, N, F)
-    assert got.shape == want.shape and got.stride(0) == 1 and torch.equal(got, want)
-    assert not got._base[:, N:].any()                        # the columns behind the last sample are zero
+    assert got.shape == (F, (N + 63) // 64 * 64) and torch.equal(got[:, :N].t(), want)
+    assert not got[:, N:].any()                              # the columns behind the last sample are zero
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -151,3 +151,22 @@ def test_row_and_column_sums_from_one_read(dtype, N, F):
         slices = max(1, min(64, F // 8192))
         if slices == 1:
             assert torch.equal(got[1], ext_minimax.sample_sqnorm(x))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,F", [(1, 8), (63, 248), (64, 256), (65, 264), (2050, 1000), (4096, 512)])
+def test_sums_and_the_rows_turned_over_from_one_read(dtype, N, F):
+    x = _rows(N, F, dtype, 0, N + F)
+    with torch.no_grad():
+        columns, sq, turned = ext_minimax.row_column_sums_transposed(x, True, True)
+        none = ext_minimax.row_column_sums_transposed(x, False, False)
+    assert turned.shape == (F, (N + 63) // 64 * 64) and torch.equal(turned[:, :N].t(), x) and not turned[:, N:].any()
+    assert none[0] is None and none[1] is None and torch.equal(none[2], turned)
+    # columns: 8 rows, 8 of those, then tiles of 64 rows 16 side by side; squares: 8 products in a lane, 32
+    # lanes, then tiles of 256 columns one after the other
+    exact, weight = x.double().sum(0), x.double().abs().sum(0)
+    eps = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    bound = (8 + 3 + N / 1024 + 5) * 2.0 ** -24 * weight + eps * exact.abs()
+    assert columns.dtype == dtype and bool(((columns.double() - exact).abs() <= bound).all())
+    exact = x.double().square().sum(1)
+    assert bool(((sq.double() - exact).abs() <= (8 + 5 + F / 256 + 1) * 2.0 ** -24 * exact).all())
