@@ -1691,12 +1691,33 @@ int launch_cl_reduce(const Plan& pl, const XS& xs, const void* dy, float* part, 
       pl.tiles, rows.nsplit, relu);
   return rows.nsplit;
 }
+// Rows per block of the closing step's forward pass, relu(bn(x) + residual) with the packed copy, which streams
+// 3.7 times the bytes of its input and holds four waves per SIMD, i.e. 1024 blocks.  A block costs its steps and
+// about three more (coefficients, the group parameters of its steps), and a last round that is nearly empty costs
+// as much as a full one: of 8, 12, 16 and 20 steps the one with the least rounds * (steps + 3).  Forward of the
+// layer, bf16 [n, 512, 28, 28], us with the plan's 8 steps / with these: n = 256 195.2 / 183.1 (20), 370
+// 278.2 / 266.6 (12), 215 169.3 / 164.3 (16), 160 135.4 / 129.5 (16), 100 97.9 / 94.4 (20);
+// [128, 256, 56, 56] 188.9 / 178.4 (20); [256, 64, 56, 56] 112.6 / 113.6 (16).  Below two rounds the plan's blocks
+// stay (bf16 [256, 16, 64, 64]: 54.9 with 8 steps, 57.7 with 16).  The passes without the residual have less to
+// stream and gain nothing ([256, 64, 56, 56] bn + ReLU 97.7 with 8 steps, 99.7 with 16; bn alone 72.5, 76.1).
+int64_t closing_rows(const Plan& pl) {
+  constexpr int64_t slots = (int64_t)kCUs * 4;
+  if ((int64_t)pl.tiles * pl.nsplit_apply < 2 * slots) return pl.ppb_apply;
+  int64_t best = pl.ppb_apply, least = INT64_MAX;
+  for (int steps = 8; steps <= 20; steps += 4) {
+    const int64_t rows = (int64_t)steps * pl.R, blocks = (pl.P + rows - 1) / rows * pl.tiles;
+    const int64_t cost = (blocks + slots - 1) / slots * (steps + 3);
+    if (rows >= pl.ppb_apply && cost < least) { least = cost; best = rows; }
+  }
+  return best;
+}
 template <typename T, bool BWD, bool PACK, typename XS, int RELU = 0>
 void launch_cl_apply(const Plan& pl, const XS& xs, const void* dy, const float* coef, void* out, int64_t C,
                      const PackSink& ps, hipStream_t s, const ReluRows& relu = ReluRows{}) {
-  const dim3 grid((unsigned)pl.tiles, (unsigned)pl.nsplit_apply), blk(kThreads);
+  const int64_t rows = RELU == 2 ? closing_rows(pl) : pl.ppb_apply;
+  const dim3 grid((unsigned)pl.tiles, (unsigned)((pl.P + rows - 1) / rows)), blk(kThreads);
   bn_cl_apply_kernel<T, BWD, PACK, XS, RELU><<<grid, blk, 0, s>>>(
-      xs, static_cast<const T*>(dy), coef, static_cast<T*>(out), pl.P, C, pl.tpr, pl.R, pl.ppb_apply, ps,
+      xs, static_cast<const T*>(dy), coef, static_cast<T*>(out), pl.P, C, pl.tpr, pl.R, rows, ps,
       FastDiv((uint32_t)(pl.F / C)), relu);
 }
 

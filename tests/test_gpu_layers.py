@@ -1109,6 +1109,31 @@ def test_closing_step_of_a_residual_block_in_the_batch_norm_pass(dtype, channels
         assert torch.equal(u, v), i
 
 
+@pytest.mark.parametrize("n", [200, 215, 270])
+def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
+    """Forward passes of more than two rounds of blocks choose how many rows a block takes: 20, 12 and 16 steps of 8 rows
+    here, the last block ragged.  Output and saved stream are those of the batch norm, the addition and the ReLU."""
+    from actnn_amd.layers import QAddReLU, QBatchNorm2d, bn_add_relu, known_group_minmax
+    res = []
+    for fold in (False, True):
+        config.reset(); QScheme.reset(); QBNScheme.reset()
+        set_optimization_level("L3")
+        config.fused_bn_relu = fold
+        torch.manual_seed(4)
+        bn, close = QBatchNorm2d(256).to(DEV).train(), QAddReLU()
+        g = torch.Generator(device=DEV).manual_seed(n)
+        x, identity = (torch.randn(n, 256, 28, 28, device=DEV, generator=g, dtype=torch.bfloat16)
+                       .contiguous(memory_format=torch.channels_last) for _ in range(2))
+        torch.cuda.manual_seed(22)
+        out = bn_add_relu(bn, close, x.requires_grad_(), identity)
+        node = out.grad_fn                                     # the closing step, or the batch norm some nodes behind
+        while not (type(getattr(node, "saved", None)) is tuple and len(node.saved) == 9):
+            node = node.next_functions[0][0]
+        res.append((out.detach(), *node.saved[0], *known_group_minmax(out)))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 def test_closing_step_of_a_tensor_beyond_the_last_level_cache():
     """Above 256 MB the backward's first pass writes the masked gradient past the caches: the gradients of a closing step on
     such a tensor against the batch norm, the addition and the ReLU one after the other."""
