@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/actnn_hip.h"
 
@@ -219,6 +220,45 @@ template <typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
       else reinterpret_cast<uint16_t*>(p)[k] = (uint16_t)(w[k / 2] >> (16 * (k & 1)));
     }
   }
+}
+// A wave's `count` consecutive elements, which lie in `slab` (LDS, 16-byte aligned, up to 4 KiB and a dword that
+// may be read behind them), to `dst`, any element address: whole lines by whole instructions, what lies
+// before the first and behind the last vector element by element, all of it past the caches.  Stored from
+// the lanes that own them, 16 bytes each at the tensor's own alignment and through the caches, the lines of odd
+// rows were written by two instructions and left dirty, which the end of the kernel and the next one paid
+// for: minimax + pack + unpack of fp32 [400, 290400] 322.9 us, 265.4 like this; fp32 [128, 309123] 114.8 and 98.3; bf16
+// [300, 145200] 78.9 and 68.8; unpack of fp32 [32, 309123] alone 11.3 and 9.8 (10.6 with the lanes' own stores past the
+// caches; 9.6 for [32, 307200]).
+template <typename T> ACTNN_DEV void store_unit_any(T* dst, const uint32_t* slab, int count) {
+  constexpr int S = sizeof(T);
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t bytes = (uint32_t)(count > 0 ? count : 0) * S;
+  uint32_t head = (0u - (uint32_t)(uintptr_t)dst) & 127u;
+  if (head > bytes) head = bytes;
+  const uint32_t vectors = (bytes - head) >> 4;
+  char* body = reinterpret_cast<char*>(dst) + head;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t v = i * 64 + lane;
+    if (v < vectors) {
+      const uint32_t* p = slab + ((head + 16 * v) >> 2);
+      u32x4 w = {p[0], p[1], p[2], p[3]};
+      if constexpr (S == 2) {
+        if (head & 2u) {
+          const uint32_t next = p[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_alignbit(k < 3 ? w[k < 3 ? k + 1 : 3] : next, w[k], 16);
+        }
+      }
+      store16_nt(body + 16 * v, w);
+    }
+  }
+  typedef typename std::conditional<S == 2, uint16_t, uint32_t>::type Word;
+  const Word* values = reinterpret_cast<const Word*>(slab);
+  Word* to = reinterpret_cast<Word*>(dst);
+  const uint32_t before = head / S, first = (head + 16 * vectors) / S;
+  if (lane < before) __builtin_nontemporal_store(values[lane], to + lane);
+  if (first + lane < bytes / S) __builtin_nontemporal_store(values[first + lane], to + first + lane);
 }
 // how many elements of a row of F lie at `at` and behind (capped: only small counts matter)
 ACTNN_DEV int part_of_row(int64_t F, int64_t at) { return F - at < 1024 ? (int)(F - at) : 1024; }

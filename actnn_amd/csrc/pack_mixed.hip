@@ -66,14 +66,19 @@ constexpr int kWaves = kThreads / 64;
 // the wave's number in its block, as a scalar
 ACTNN_DEV uint32_t wave_of_block() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
+// elements of a unit of `groups` groups from element `at` of a row of F on
+ACTNN_DEV int unit_count(int64_t F, int64_t at, int groups) {
+  const int64_t left = F - at, all = (int64_t)groups * kGs;
+  return (int)(left < all ? left : all);
+}
+
 // fp32 output of unpack: a lane owns 32 contiguous bytes, which as direct stores would be two
 // half-used 16-byte accesses per cache line.  Instead lanes park their 8 values in the wave's
 // private LDS slab and the wave stores whole 1 KiB groups with one non-temporal instruction each
 // (measured 6.9 instead of 5.3 TB/s, and no dirty lines are left for the next kernel to wait on).
 // Only lanes of one wave exchange data, so no block barrier is needed: LDS operations of a wave
 // complete in order.  (The same staging for the fp32 loads of pack was measured slower.)
-// ROWS: `out` is a row of F elements at any address and elem_base an offset in it; its lines are shared with
-// other waves, so the stores go through the cache.
+// ROWS: `out` is a row of F elements at any address and elem_base an offset in it.
 template <int GPH, bool ROWS>
 ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t F, int groups_valid,
                              u32x4* __restrict__ slab, const float (&v)[GPH][8]) {
@@ -94,13 +99,12 @@ ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if constexpr (ROWS) {
+    store_unit_any(out + elem_base, reinterpret_cast<const uint32_t*>(slab), unit_count(F, elem_base, groups_valid));
+  } else {
 #pragma unroll
-  for (int i = 0; i < 2 * GPH; ++i) {
-    if (i < groups_valid) {
-      const int64_t at = elem_base + (int64_t)i * kGs + wl * 4;
-      if constexpr (ROWS) store16_part(out + at, slab[i * 64 + wl], part_of_row(F, at));
-      else store16_nt(out + at, slab[i * 64 + wl]);
-    }
+    for (int i = 0; i < 2 * GPH; ++i)
+      if (i < groups_valid) store16_nt(out + elem_base + (int64_t)i * kGs + wl * 4, slab[i * 64 + wl]);
   }
 }
 
@@ -377,9 +381,8 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
             const uint32_t sel = (c0 * 0x0202u + 0x0100u) | ((c1 * 0x0202u + 0x0100u) << 16);
             outw[j] = __builtin_amdgcn_perm(lut_hi, lut_lo, sel);
           }
-          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
-          if constexpr (ROWS) store16_part(out + at, outw, part_of_row(F, at));
-          else store16_nt(out + at, outw);
+          if constexpr (ROWS) slab[gl * 32 + lane] = outw;
+          else store16_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, outw);
           continue;
         }
         float v[8];
@@ -389,16 +392,21 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
 #pragma unroll
           for (int k = 0; k < 8; ++k) vs[kStage ? q0 + r : 0][k] = v[k];
         } else if constexpr (ROWS) {
-          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
-          store16_part(out + at, words_of8(out, v), part_of_row(F, at));
+          slab[gl * 32 + lane] = words_of8(out, v);
         } else {
           store8_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, v);
         }
       }
     }
   }
-  if constexpr (kStage)
+  if constexpr (kStage) {
     stage_out_f32<kGroupsPerHalf, ROWS>(reinterpret_cast<float*>(out), elem_base, F, groups_valid, slab, vs);
+  } else if constexpr (ROWS) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    store_unit_any(out + elem_base, reinterpret_cast<const uint32_t*>(slab), unit_count(F, elem_base, groups_valid));
+  }
 }
 
 // S: the type the scales and minima are stored in.
@@ -410,10 +418,11 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   constexpr int kUnit = 2 * Gph<T>::kUnpack;                     // groups of a wave
   __shared__ float s_scale[kWaves * kUnit];
   __shared__ float s_min[kWaves * kUnit];
-  constexpr bool kStage = IsF32<T>::value;
-  __shared__ u32x4 s_slab[kStage ? kWaves * kUnit * 64 : 1];
+  constexpr bool kStage = IsF32<T>::value || ROWS;
+  constexpr int kSlab = kUnit * kGs * (int)sizeof(T) / 16;       // (and a dword behind the last: see store_unit_any)
+  __shared__ u32x4 s_slab[kStage ? kWaves * kSlab + 1 : 1];
   const uint32_t wave = wave_of_block();
-  u32x4* slab = s_slab + (kStage ? wave * (kUnit * 64) : 0);
+  u32x4* slab = s_slab + (kStage ? wave * kSlab : 0);
   const Unit u = unit_of<kUnit>(blockIdx.x * kWaves + wave, per_sample, N, G);
   const int64_t n = u.n, gb = u.gb;
   const int b = bits[n];

@@ -117,6 +117,32 @@ def test_rows_at_widths_of_their_own_equal_the_padded_composition(dtype, initial
             assert torch.equal(back, full.view(N, -1)[:, :F]), (N, F, shift)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_end_at_every_place_in_a_line(dtype):
+    # the restored rows start anywhere in a line of 128 bytes (odd lengths) and end within, at and behind units of
+    # a wave (1024 elements in fp32, 2048 in 16 bits); what lies behind the last row stays as it was
+    for F in (1, 2, 31, 63, 64, 65, 1023, 1024, 1025, 1057, 2047, 2049, 2081, 3001):
+        N = 67
+        x = _rows(N, F, dtype, 0, F)
+        if x.numel() < 8:
+            continue
+        alloc = qscheme.AllocationArgs(N, 256 / F, None, 8, 3)
+        alloc.store_dtype = store = ops._stored_dtype(dtype)
+        packed, bits, scale, low = ext_q.quantize_activation_device(x, N, None, alloc)
+        low = low.view(N, -1, 1)
+        G = (F + 255) // 256
+        want = ext_q.unpack_mixed_precision(packed, bits, scale.to(dtype), low.to(dtype), N, G, 256).view(N, -1)[:, :F]
+        room = torch.full((N * F + 256,), 7.0, dtype=dtype, device="cuda")
+        prefix = ext_q._bits_info(bits)[1]
+        code = ext_q.g.DTYPE_CODE
+        rc = ext_q.g.lib().actnn_unpack_mixed_rows(packed.data_ptr(), bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(),
+                                                   low.data_ptr(), room.data_ptr(), N, F, code[dtype], code[store],
+                                                   torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert torch.equal(room[:N * F].view(N, F), want), F
+        assert bool((room[N * F:] == 7).all()), F
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,F", [(1, 256), (7, 300), (63, 512), (64, 257), (65, 4096), (130, 1000), (2050, 264)])
 @pytest.mark.parametrize("avg", [2, 5])
