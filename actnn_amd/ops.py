@@ -431,7 +431,7 @@ def _fused_grad_weight_ok(quantized, shape, go):
             and isinstance(q_input, torch.Tensor) and q_input.is_cuda)
 
 
-def _by_sample(quantized, shape):
+def _by_sample(quantized, shape, outputs):
     """Whether the factors of the weight gradient's product can be had with the samples contiguous in memory: it
     sums over them and takes less time like that.  Turning the input over costs its unpack 3 to 8 us more, and
     the gradient, turned over by the pass that sums it, next to nothing (one read in place of two for short
@@ -444,17 +444,21 @@ def _by_sample(quantized, shape):
       2048, 1024, 1024   34.6   33.8   31.3            100, 1024, 1024    19.4   21.6   18.4
       2047, 4096, 4096   96.5   97.6   79.8            64, 1024, 1024     17.0   19.6   17.2
       2048, 256, 100     36.2   31.2    -              1024, 256, 100     32.7   32.0    -
-    So both from _BOTH_BY_SAMPLE samples on, the input alone (a gradient row_column_sums_transposed does not
+    A layer by itself is bound by the host up to some 2^35 products, and the host has a little more to do like
+    this (forward and backward, us: bf16 [300, 1024] -> 1024 434 / 440, f16 [1000, 768] -> 3072 430 / 450, bf16 [4001, 1000] -> 100
+    497 / 528; but f16 [8192, 4096] -> 4096 789 / 723): smaller ones keep the rows (_PRODUCT_BY_SAMPLE).
+    Of the others both from _BOTH_BY_SAMPLE samples on, the input alone (a gradient row_column_sums_transposed does not
     take) from _INPUT_BY_SAMPLE.  The turned gradient is one more tensor of the gradient's size until the
     product has been queued.  Not for fp32 and streams of one width, which have no such unpack."""
     if not config.compress_activation or config.simulate or config.swap or config.group_size != 256:
         return False
     _, q_bits, q_scale, _ = quantized
-    return (len(shape) == 2 and shape[0] >= _BOTH_BY_SAMPLE and isinstance(q_bits, torch.Tensor)
+    return (len(shape) == 2 and shape[0] >= _BOTH_BY_SAMPLE and shape[0] * shape[1] * outputs >= _PRODUCT_BY_SAMPLE
+            and isinstance(q_bits, torch.Tensor)
             and (q_scale.dtype == torch.float16 or q_scale.dtype == torch.bfloat16 and not _stored_as_bf16(shape, quantized)))
 
 
-_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE = 128, 2048
+_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE, _PRODUCT_BY_SAMPLE = 128, 2048, 1 << 35
 
 
 class linear(Function):
@@ -477,7 +481,7 @@ class linear(Function):
         # the bias's gradient and the norms of the samples (rows, if there is one row each) from one read
         need_bias = bias is not None and ctx.needs_input_grad[2]
         fused = _fused_grad_weight_ok(quantized, q_input_shape, go)
-        by_sample = not fused and ctx.needs_input_grad[1] and _by_sample(quantized, q_input_shape)
+        by_sample = not fused and ctx.needs_input_grad[1] and _by_sample(quantized, q_input_shape, go.shape[1])
         want_sq = bool(ctx.scheme) and grad_output.dim() == 2 and ctx.scheme.wants_sqnorm(grad_output)
         sums = go_turned = None
         if by_sample:

@@ -570,6 +570,7 @@ def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias
     grad = torch.randn(N, O, device=DEV).to(dtype)
     layer.scheme.set_scale(grad)
     wanted = [x, layer.weight] + ([layer.bias] if bias else [])
+    monkeypatch.setattr(ops, "_PRODUCT_BY_SAMPLE", 0)
     got = []
     for limits in ((128, 2048), (1 << 30, 1 << 30)):
         monkeypatch.setattr(ops, "_BOTH_BY_SAMPLE", limits[0])
