@@ -444,9 +444,9 @@ def _by_sample(quantized, shape, outputs):
       2048, 1024, 1024   34.6   33.8   31.3            100, 1024, 1024    19.4   21.6   18.4
       2047, 4096, 4096   96.5   97.6   79.8            64, 1024, 1024     17.0   19.6   17.2
       2048, 256, 100     36.2   31.2    -              1024, 256, 100     32.7   32.0    -
-    A layer by itself is bound by the host up to some 2^35 products, and the host has a little more to do like
-    this (forward and backward, us: bf16 [300, 1024] -> 1024 434 / 440, f16 [1000, 768] -> 3072 430 / 450, bf16 [4001, 1000] -> 100
-    497 / 528; but f16 [8192, 4096] -> 4096 789 / 723): smaller ones keep the rows (_PRODUCT_BY_SAMPLE).
+    A layer by itself is bound by the host up to some 2^36 products, and the host has a little more to do like
+    this (forward and backward, us: bf16 [300, 1024] -> 1024 434 / 440, f16 [1000, 768] -> 3072 430 / 450, bf16 [8192, 1024] -> 4096
+    409 / 530; but bf16 [6001, 3072] -> 4096 547 / 523, f16 [8192, 4096] -> 4096 789 / 723): smaller ones keep the rows (_PRODUCT_BY_SAMPLE).
     Of the others both from _BOTH_BY_SAMPLE samples on, the input alone (a gradient row_column_sums_transposed does not
     take) from _INPUT_BY_SAMPLE.  The turned gradient is one more tensor of the gradient's size until the
     product has been queued.  Not for fp32 and streams of one width, which have no such unpack."""
@@ -458,7 +458,7 @@ def _by_sample(quantized, shape, outputs):
             and (q_scale.dtype == torch.float16 or q_scale.dtype == torch.bfloat16 and not _stored_as_bf16(shape, quantized)))
 
 
-_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE, _PRODUCT_BY_SAMPLE = 128, 2048, 1 << 35
+_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE, _PRODUCT_BY_SAMPLE = 128, 2048, 1 << 36
 
 
 class linear(Function):
