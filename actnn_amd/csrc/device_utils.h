@@ -169,12 +169,20 @@ typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 ACTNN_DEV u32x4 load16_any(const float* p) { return *reinterpret_cast<const u32x4_a4*>(p); }
 ACTNN_DEV u32x4 load16_any(const __half* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
 ACTNN_DEV u32x4 load16_any(const bf16_t* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
-// (past the caches: ordinary stores leave lines behind that the kernel's end and the next one wait for; quantize +
-// unpack at one width, ordinary / like this: fp32 [400, 290400] 4 bits 233 / 185 us, bf16 [300, 145200] 4 bits 47.5 / 41.9,
-// [650, 145200] 8 bits 120.6 / 101.0, f16 [300, 145200] 2 bits 45.3 / 40.7)
-ACTNN_DEV void store16_any(float* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a4*>(p)); }
-ACTNN_DEV void store16_any(__half* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2*>(p)); }
-ACTNN_DEV void store16_any(bf16_t* p, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2*>(p)); }
+// PAST: past the caches, for what is too large to be there when the next kernel reads it (stream_rows)
+template <bool PAST> ACTNN_DEV void store16_any(float* p, u32x4 v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a4*>(p));
+  else *reinterpret_cast<u32x4_a4*>(p) = v;
+}
+template <bool PAST, typename T> ACTNN_DEV void store16_any(T* p, u32x4 v) {
+  static_assert(sizeof(T) == 2, "16-bit types");
+  if constexpr (PAST) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2*>(p));
+  else *reinterpret_cast<u32x4_a2*>(p) = v;
+}
+template <bool PAST, typename W> ACTNN_DEV void store_one(W* p, W v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
 // One 16-byte vector of a row, of which only the first `valid` elements lie in it (the others count as 0).  The
 // load is never guarded: it reads what follows the row, or ends with the tensor (`last`: its last 16
 // bytes; a tensor holds at least that much), and row_vector_ends() drops what does not belong.  With guarded
@@ -210,28 +218,26 @@ template <typename T> ACTNN_DEV u32x4 row_vector_ends(const RowVector& r) {
   }
   return (u32x4){w[0], w[1], w[2], w[3]};
 }
-template <typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
+template <bool PAST, typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int valid) {
   constexpr int E = 16 / sizeof(T);
   if (valid >= E) {
-    store16_any(p, v);
+    store16_any<PAST>(p, v);
   } else if (valid > 0) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int k = 0; k < E - 1; ++k) {
       if (k >= valid) continue;
-      if constexpr (sizeof(T) == 4) __builtin_nontemporal_store(w[k], reinterpret_cast<uint32_t*>(p) + k);
-      else __builtin_nontemporal_store((uint16_t)(w[k / 2] >> (16 * (k & 1))), reinterpret_cast<uint16_t*>(p) + k);
+      if constexpr (sizeof(T) == 4) store_one<PAST>(reinterpret_cast<uint32_t*>(p) + k, w[k]);
+      else store_one<PAST>(reinterpret_cast<uint16_t*>(p) + k, (uint16_t)(w[k / 2] >> (16 * (k & 1))));
     }
   }
 }
 // A wave's `count` consecutive elements, which lie in `slab` (LDS, 16-byte aligned, up to 4 KiB and a dword that
 // may be read behind them), to `dst`, any element address: whole lines by whole instructions, what lies
-// before the first and behind the last vector element by element, all of it past the caches.  Stored from
-// the lanes that own them, 16 bytes each at the tensor's own alignment and through the caches, the lines of odd
-// rows were written by two instructions and left dirty, which the end of the kernel and the next one paid
-// for: minimax + pack + unpack of fp32 [400, 290400] 322.9 us, 265.4 like this; fp32 [128, 309123] 114.8 and 98.3; bf16
-// [300, 145200] 78.9 and 68.8; unpack of fp32 [32, 309123] alone 11.3 and 9.8 (10.6 with the lanes' own stores past the
-// caches; 9.6 for [32, 307200]).
+// before the first and behind the last vector element by element, all of it past the caches.  For tensors that
+// stream_rows sends there: stored from the lanes that own them, 16 bytes each at the tensor's own alignment and through
+// the caches, the lines of odd rows were written by two instructions and left dirty (minimax + pack + unpack
+// of fp32 [400, 290400] 322.9 us, 265.4 like this; fp32 [128, 309123] 114.8 and 98.3).
 template <typename T> ACTNN_DEV void store_unit_any(T* dst, const uint32_t* slab, int count) {
   constexpr int S = sizeof(T);
   const uint32_t lane = threadIdx.x & 63u;
@@ -683,6 +689,18 @@ ACTNN_DEV void store_transposed_tile(const uint32_t (&w)[8][4], u32x4* s_tile, T
 // (max-pool's backward pass, which writes 8 or 4 bytes per lane: f32 [128,128,28,28], 51 MB, 15 us with plain
 // stores, 24 us with non-temporal ones; [32,64,225,225], 415 MB, 148 and 84 us; the two meet at 100 - 150 MB).
 inline bool stream_results(int64_t bytes) { return bytes > (int64_t(128) << 20); }
+
+// How the unpack kernels store restored rows of odd length: up to 96 MiB through the caches, as the layer's own product
+// reads the rows next; larger ones past them, since ordinary stores leave lines behind that the kernel's end and the
+// next one wait for.  Compress + restore + the sum of the result, us, through / past: one width (4 bits) f32
+// [128, 81921] (40 MiB) 42.8 / 44.4, [128, 178177] (87 MiB) 62.6 / 69.9, bf16 [128, 356353] 74.2 / 81.5, and with a product
+// of 64 columns in the sum's place f32 [300, 76021] 95.3 / 116.5; per-sample widths f32 [128, 178177] 88.6 / 95.8, bf16
+// [300, 152043] 97.5 / 107.6; restore + sum of f32 [64, 1001] 16.6 / 21.5.  Without a reader the two are even up to there
+// (one width 38.4 / 38.8 and 48.8 / 47.5, per sample 65.4 / 65.8 and 73.0 / 73.7); larger ones lose by the caches (one width
+// f32 [128, 245761] 57.6 / 52.1, [128, 327681] 90.2 / 67.5, per sample 116.0 / 106.0, f32 [128, 614401] 85.6 / 63.5
+// for the restore alone).
+enum Rows { kWholeRows = 0, kRowsCached = 1, kRowsPast = 2 };
+inline bool stream_rows(int64_t bytes) { return bytes > (int64_t(96) << 20); }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -78,8 +78,8 @@ ACTNN_DEV int unit_count(int64_t F, int64_t at, int groups) {
 // (measured 6.9 instead of 5.3 TB/s, and no dirty lines are left for the next kernel to wait on).
 // Only lanes of one wave exchange data, so no block barrier is needed: LDS operations of a wave
 // complete in order.  (The same staging for the fp32 loads of pack was measured slower.)
-// ROWS: `out` is a row of F elements at any address and elem_base an offset in it.
-template <int GPH, bool ROWS>
+// ROWS: `out` is a row of F elements at any address and elem_base an offset in it; its ends share lines with other rows.
+template <int GPH, int ROWS>
 ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t F, int groups_valid,
                              u32x4* __restrict__ slab, const float (&v)[GPH][8]) {
   const int wl = threadIdx.x & 63;
@@ -99,12 +99,17 @@ ACTNN_DEV void stage_out_f32(float* __restrict__ out, int64_t elem_base, int64_t
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if constexpr (ROWS) {
+  if constexpr (ROWS == kRowsPast) {
     store_unit_any(out + elem_base, reinterpret_cast<const uint32_t*>(slab), unit_count(F, elem_base, groups_valid));
   } else {
 #pragma unroll
-    for (int i = 0; i < 2 * GPH; ++i)
-      if (i < groups_valid) store16_nt(out + elem_base + (int64_t)i * kGs + wl * 4, slab[i * 64 + wl]);
+    for (int i = 0; i < 2 * GPH; ++i) {
+      if (i < groups_valid) {
+        const int64_t at = elem_base + (int64_t)i * kGs + wl * 4;
+        if constexpr (ROWS == kRowsCached) store16_part<false>(out + at, slab[i * 64 + wl], part_of_row(F, at));
+        else store16_nt(out + at, slab[i * 64 + wl]);
+      }
+    }
   }
 }
 
@@ -309,7 +314,7 @@ __global__ __launch_bounds__(kThreads, DET ? 1 : 8) void pack_mixed_kernel(
 
 // ---------------------------------------------------------------------------- unpack (gs = 256)
 // ROWS: `out` is a row of F elements at any address and elem_base an offset in it.
-template <typename T, int BITS, bool ROWS>
+template <typename T, int BITS, int ROWS>
 ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__ out,
                              int64_t elem_base, int64_t F, int64_t word_base, int groups_valid,
                              float* s_scale, float* s_min, float my_scale, float my_min, u32x4* slab) {
@@ -381,8 +386,10 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
             const uint32_t sel = (c0 * 0x0202u + 0x0100u) | ((c1 * 0x0202u + 0x0100u) << 16);
             outw[j] = __builtin_amdgcn_perm(lut_hi, lut_lo, sel);
           }
-          if constexpr (ROWS) slab[gl * 32 + lane] = outw;
-          else store16_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, outw);
+          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
+          if constexpr (ROWS == kRowsPast) slab[gl * 32 + lane] = outw;
+          else if constexpr (ROWS == kRowsCached) store16_part<false>(out + at, outw, part_of_row(F, at));
+          else store16_nt(out + at, outw);
           continue;
         }
         float v[8];
@@ -391,8 +398,11 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
         if constexpr (kStage) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) vs[kStage ? q0 + r : 0][k] = v[k];
-        } else if constexpr (ROWS) {
+        } else if constexpr (ROWS == kRowsPast) {
           slab[gl * 32 + lane] = words_of8(out, v);
+        } else if constexpr (ROWS == kRowsCached) {
+          const int64_t at = elem_base + (int64_t)gl * kGs + lane * 8;
+          store16_part<false>(out + at, words_of8(out, v), part_of_row(F, at));
         } else {
           store8_nt(out + elem_base + (int64_t)gl * kGs + lane * 8, v);
         }
@@ -401,7 +411,7 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
   }
   if constexpr (kStage) {
     stage_out_f32<kGroupsPerHalf, ROWS>(reinterpret_cast<float*>(out), elem_base, F, groups_valid, slab, vs);
-  } else if constexpr (ROWS) {
+  } else if constexpr (ROWS == kRowsPast) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -410,7 +420,7 @@ ACTNN_DEV void unpack_groups(const int32_t* __restrict__ packed, T* __restrict__
 }
 
 // S: the type the scales and minima are stored in.
-template <typename T, typename S, bool ROWS>
+template <typename T, typename S, int ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
     const int32_t* __restrict__ packed, const int32_t* __restrict__ bits,
     const int32_t* __restrict__ prefix, const S* __restrict__ scale, const S* __restrict__ mn,
@@ -418,7 +428,7 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   constexpr int kUnit = 2 * Gph<T>::kUnpack;                     // groups of a wave
   __shared__ float s_scale[kWaves * kUnit];
   __shared__ float s_min[kWaves * kUnit];
-  constexpr bool kStage = IsF32<T>::value || ROWS;
+  constexpr bool kStage = IsF32<T>::value || ROWS == kRowsPast;
   constexpr int kSlab = kUnit * kGs * (int)sizeof(T) / 16;       // (and a dword behind the last: see store_unit_any)
   __shared__ u32x4 s_slab[kStage ? kWaves * kSlab + 1 : 1];
   const uint32_t wave = wave_of_block();
@@ -654,7 +664,7 @@ int launch_pack_groups(const void* data, const void* mn, const void* mx, const i
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
-template <typename T, typename S, bool ROWS>
+template <typename T, typename S, int ROWS>
 int launch_unpack_groups(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
                          const void* mn, void* out, int64_t N, int64_t F, hipStream_t s) {
   const int64_t G = (F + kGs - 1) / kGs;
@@ -690,8 +700,10 @@ int launch_pack_rows(const void* data, const void* mn, const void* mx, const int
 template <typename T, typename S>
 int launch_unpack_rows(const int32_t* packed, const int32_t* bits, const int32_t* prefix, const void* scale,
                        const void* mn, void* out, int64_t N, int64_t F, hipStream_t s) {
-  if (F % kGs == 0) return launch_unpack_groups<T, S, false>(packed, bits, prefix, scale, mn, out, N, F, s);
-  return launch_unpack_groups<T, S, true>(packed, bits, prefix, scale, mn, out, N, F, s);
+  if (F % kGs == 0) return launch_unpack_groups<T, S, kWholeRows>(packed, bits, prefix, scale, mn, out, N, F, s);
+  if (stream_rows(N * F * (int64_t)sizeof(T)))
+    return launch_unpack_groups<T, S, kRowsPast>(packed, bits, prefix, scale, mn, out, N, F, s);
+  return launch_unpack_groups<T, S, kRowsCached>(packed, bits, prefix, scale, mn, out, N, F, s);
 }
 
 template <typename T>
@@ -724,7 +736,7 @@ int launch_unpack(const int32_t* packed, const int32_t* bits, const int32_t* pre
                   const void* scale, const void* mn, void* out, int64_t N, int64_t G, int64_t gs,
                   hipStream_t s) {
   if (gs == kGs) {
-    return launch_unpack_groups<T, T, false>(packed, bits, prefix, scale, mn, out, N, G * kGs, s);
+    return launch_unpack_groups<T, T, kWholeRows>(packed, bits, prefix, scale, mn, out, N, G * kGs, s);
   } else {
     if (N * G > 0x7fffffffLL) return ACTNN_EINVAL;
     unpack_mixed_generic_kernel<T><<<dim3((unsigned)(N * G)), dim3(kThreads), 0, s>>>(

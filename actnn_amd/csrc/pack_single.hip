@@ -143,9 +143,9 @@ __global__ __launch_bounds__(kThreads) void pack_single_kernel(
   }
 }
 
-// ROWS: rows of any length at any address (the elements past a row's end are not written); their lines are
-// shared between waves, so the stores go through the cache.
-template <typename T, int BITS, bool ROWS>
+// ROWS: rows of any length at any address (the elements past a row's end are not written), stored through the caches or
+// past them (stream_rows).
+template <typename T, int BITS, int ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_single_kernel(
     const int8_t* __restrict__ packed, const T* __restrict__ scale, const T* __restrict__ mn,
     T* __restrict__ out, SingleGeom q) {
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kThreads) void unpack_single_kernel(
           const uint32_t word = k < 4 ? w.x : w.y;
           v[k] = dq((word >> (8 * (k & 3) + ni * BITS)) & kMask);
         }
-        if constexpr (ROWS) store16_part(out + n * q.F + g * gs + d0, words_of8(out, v), part_of_row(q.F, g * gs + d0));
+        if constexpr (ROWS) store16_part<ROWS == kRowsPast>(out + n * q.F + g * gs + d0, words_of8(out, v), part_of_row(q.F, g * gs + d0));
         else store8_nt(out + gi * gs + d0, v);
       }
     }
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kThreads) void unpack_single_kernel(
 
 // ---------------------------------------------------------------------------- fp32 unpack: 4 elements per lane
 // S: the type the scales and minima are stored in (bfloat16 in the compact form of an fp32 activation).
-template <typename S, int BITS, bool ROWS>
+template <typename S, int BITS, int ROWS>
 __global__ __launch_bounds__(kThreads) void unpack_single_f32_kernel(
     const int8_t* __restrict__ packed, const S* __restrict__ scale, const S* __restrict__ mn,
     float* __restrict__ out, SingleGeom q) {
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kThreads) void unpack_single_f32_kernel(
         u32x4 v;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = as_uint(dq((w >> (8 * k + ni * BITS)) & kMask));
-        if constexpr (ROWS) store16_part(out + n * q.F + g * gs + d0, v, part_of_row(q.F, g * gs + d0));
+        if constexpr (ROWS) store16_part<ROWS == kRowsPast>(out + n * q.F + g * gs + d0, v, part_of_row(q.F, g * gs + d0));
         else store16_nt(out + gi * gs + d0, v);
       }
     }
@@ -417,7 +417,7 @@ int launch_pack(const void* data, const void* mn, const void* mx, int bits, void
 }
 
 // F: elements a row of `out` has; below G * gs (or with `out` not 16-byte aligned) the ROWS kernels.
-template <typename T, typename S, bool ROWS>
+template <typename T, typename S, int ROWS>
 int launch_unpack(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
                   int64_t N, int64_t G, int64_t gs, int64_t F, hipStream_t s) {
   SingleGeom q;
@@ -446,8 +446,9 @@ template <typename T, typename S>
 int launch_unpack_rows(const int8_t* packed, int bits, const void* scale, const void* mn, void* out,
                        int64_t N, int64_t F, hipStream_t s) {
   const int64_t G = (F + kFixedGs - 1) / kFixedGs;
-  if (F == G * kFixedGs) return launch_unpack<T, S, false>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
-  return launch_unpack<T, S, true>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
+  if (F == G * kFixedGs) return launch_unpack<T, S, kWholeRows>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
+  if (stream_rows(N * F * (int64_t)sizeof(T))) return launch_unpack<T, S, kRowsPast>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
+  return launch_unpack<T, S, kRowsCached>(packed, bits, scale, mn, out, N, G, kFixedGs, F, s);
 }
 
 inline bool single_bits_ok(int bits) { return bits == 1 || bits == 2 || bits == 4 || bits == 8; }
@@ -487,9 +488,9 @@ extern "C" int actnn_unpack_single(const int8_t* packed, int bits, const void* s
   if (!aligned16(out) || (reinterpret_cast<uintptr_t>(packed) & 7u) != 0) return ACTNN_EALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
-    case ACTNN_F32: return launch_unpack<float, float, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
-    case ACTNN_F16: return launch_unpack<__half, __half, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
-    case ACTNN_BF16: return launch_unpack<bf16_t, bf16_t, false>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    case ACTNN_F32: return launch_unpack<float, float, kWholeRows>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    case ACTNN_F16: return launch_unpack<__half, __half, kWholeRows>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
+    case ACTNN_BF16: return launch_unpack<bf16_t, bf16_t, kWholeRows>(packed, bits, scale, mn, out, N, G, gs, G * gs, s);
     default: return ACTNN_EDTYPE;
   }
 }

@@ -143,6 +143,39 @@ def test_rows_end_at_every_place_in_a_line(dtype):
         assert bool((room[N * F:] == 7).all()), F
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("F", [257, 1001, 2049, 8193])
+def test_odd_rows_on_both_sides_of_the_line_between_the_stores(dtype, F):
+    # up to 96 MiB restored rows are stored through the caches, larger ones past them, from LDS at per-sample widths:
+    # the same values either way, and nothing behind the last row
+    size = torch.empty(0, dtype=dtype).element_size()
+    at_most = (96 << 20) // (F * size)
+    code = ext_q.g.DTYPE_CODE
+    store = ops._stored_dtype(dtype)
+    for N in (at_most, at_most + 1):
+        x = _rows(N, F, dtype, 0, F)
+        G = (F + 255) // 256
+        room = torch.full((N * F + 256,), 7.0, dtype=dtype, device="cuda")
+        stream = torch.cuda.current_stream().cuda_stream
+        bits = 1 + torch.arange(N, dtype=torch.int32) % 8
+        dev_bits = ext_q.attach_bits_host(bits.cuda(), bits)
+        padded = _padded(x)
+        mn, mx = ext_minimax.minimax(padded.view(-1, 256))
+        mn, mx = mn.view(N, G, 1), mx.view(N, G, 1)
+        packed, scale = ext_q.pack_mixed_precision(padded, mn, mx, dev_bits, True)
+        prefix = ext_q._bits_info(dev_bits)[1]
+        want = ext_q.unpack_mixed_precision(packed, dev_bits, scale, mn, N, G, 256).view(N, -1)[:, :F]
+        assert ext_q.g.lib().actnn_unpack_mixed_rows(packed.data_ptr(), dev_bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(),
+                                                     mn.data_ptr(), room.data_ptr(), N, F, code[dtype], code[dtype], stream) == 0
+        assert torch.equal(room[:N * F].view(N, F), want) and bool((room[N * F:] == 7).all()), N
+        packed, scale, low = ext_q.quantize_rows_fixed(x, 4, None, store)
+        want = ext_q.unpack_single_precision(packed, 4, scale.to(dtype), low.to(dtype), N, G, 256).view(N, -1)[:, :F]
+        room.fill_(7.0)
+        assert ext_q.g.lib().actnn_unpack_single_rows(packed.data_ptr(), 4, scale.data_ptr(), low.data_ptr(), room.data_ptr(),
+                                                      N, F, code[dtype], code[store], stream) == 0
+        assert torch.equal(room[:N * F].view(N, F), want) and bool((room[N * F:] == 7).all()), N
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,F", [(1, 256), (7, 300), (63, 512), (64, 257), (65, 4096), (130, 1000), (2050, 264)])
 @pytest.mark.parametrize("avg", [2, 5])
