@@ -485,8 +485,10 @@ class linear(Function):
         want_sq = bool(ctx.scheme) and grad_output.dim() == 2 and ctx.scheme.wants_sqnorm(grad_output)
         sums = go_turned = None
         if by_sample:
-            sums = ext_minimax.row_column_sums_transposed(go, need_bias, want_sq)
-            go_turned = sums[2] if sums is not None else None
+            turned = ext_minimax.row_column_sums_transposed(go, need_bias, want_sq)
+            if turned is not None:
+                sums, go_turned = turned[:2], turned[2]
+            del turned                       # (the turned gradient is to go with its product: one name holds it)
             # (a batch of gradients at once keeps the product it had)
             by_sample = go_turned is not None or q_input_shape[0] >= _INPUT_BY_SAMPLE and ext_quantization.g.has_storage(go)
         if sums is None and need_bias:

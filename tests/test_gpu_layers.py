@@ -585,6 +585,28 @@ def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias
         assert (a.double() - b.double()).norm() <= bound
 
 
+@pytest.mark.parametrize("bias", [True, False])
+def test_linear_turned_gradient_is_gone_before_the_input_gradient(bias, monkeypatch):
+    """The turned gradient lives until its product has been queued: the input's gradient finds its memory free."""
+    import weakref
+    torch.manual_seed(0)
+    layer = actnn_amd.QLinear(256, 512, bias=bias).to(DEV, torch.bfloat16)
+    x = torch.randn(512, 256, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    monkeypatch.setattr(ops, "_PRODUCT_BY_SAMPLE", 0)
+    taken, alive = [], []
+    turn = ops.ext_minimax.row_column_sums_transposed
+
+    def watched(*args):
+        out = turn(*args)
+        taken.append(weakref.ref(out[2]))
+        return out
+    y = layer(x)
+    monkeypatch.setattr(ops.ext_minimax, "row_column_sums_transposed", watched)
+    monkeypatch.setattr(ops, "empty_cache", lambda *_: alive.extend(r() is not None for r in taken))
+    y.backward(torch.randn_like(y))
+    assert len(taken) == 1 and alive == [False]
+
+
 def test_resnet50_channels_last_step_runs():
     torch.manual_seed(0)
     model = _cl(QModule(resnet50()))
