@@ -435,30 +435,49 @@ def _by_sample(quantized, shape, outputs):
     """Whether the factors of the weight gradient's product can be had with the samples contiguous in memory: it
     sums over them and takes less time like that.  Turning the input over costs its unpack 3 to 8 us more, and
     the gradient, turned over by the pass that sums it, next to nothing (one read in place of two for short
-    ones).  Unpack, sums and product, us (bf16, [N, F] and [N, O]), as rows / the input turned over / both:
-      N, F, O           rows   input   both            N, F, O           rows   input   both
-      8192, 4096, 4096  281.9  263.9  245.4            1024, 4096, 4096   60.7   58.9   53.3
-      8191, 4096, 4096  289.6  274.3  232.1            1024, 1024, 1024   26.7   26.7   25.1
-      8192, 1024, 1024   84.4   62.1   53.6            512, 1024, 1024    25.6   27.6   21.7
-      2048, 4096, 4096   90.2   83.2   76.0            200, 1024, 1024    23.1   25.4   20.6
-      2048, 1024, 1024   34.6   33.8   31.3            100, 1024, 1024    19.4   21.6   18.4
-      2047, 4096, 4096   96.5   97.6   79.8            64, 1024, 1024     17.0   19.6   17.2
-      2048, 256, 100     36.2   31.2    -              1024, 256, 100     32.7   32.0    -
-    A layer by itself is bound by the host up to some 2^36 products, and the host has a little more to do like
-    this (forward and backward, us: bf16 [300, 1024] -> 1024 434 / 440, f16 [1000, 768] -> 3072 430 / 450, bf16 [8192, 1024] -> 4096
-    409 / 530; but bf16 [6001, 3072] -> 4096 547 / 523, f16 [8192, 4096] -> 4096 789 / 723): smaller ones keep the rows (_PRODUCT_BY_SAMPLE).
-    Of the others both from _BOTH_BY_SAMPLE samples on, the input alone (a gradient row_column_sums_transposed does not
-    take) from _INPUT_BY_SAMPLE.  The turned gradient is one more tensor of the gradient's size until the
-    product has been queued.  Not for fp32 and streams of one width, which have no such unpack."""
-    if not config.compress_activation or config.simulate or config.swap or config.group_size != 256:
+    ones).  Device time of a layer's forward and backward, us (bf16, [N, F] and [N, O]), as rows / the input turned
+    over / both:
+      N, F, O            rows   input   both            N, F, O            rows   input   both
+      8192, 4096, 4096   772.6  726.4  711.6            512, 8192, 16384   543.2  543.0  510.7
+      8192, 4096, 4095   937.5  898.0    -              65536, 1024, 1024  1191   1144   1108
+      6001, 3072, 4096   550.4  540.3  528.4            16384, 4096, 1024  616.6    -    568.6
+      4096, 4096, 4096   406.5  382.2  366.1            8192, 1024, 4096   326.5  308.8  302.3
+      2048, 8192, 4096   419.3  400.5  382.6            8192, 1024, 1024   205.2  188.3  172.8
+      1024, 8192, 8192   450.0  434.0  400.3            2048, 1024, 1024    94.9   95.4   89.9
+    The turned gradient is one more tensor of the gradient's size until the product has been queued (a backward pass's
+    peak above its start for [8192, 4096] -> 4096: 160 MB, 96 as rows).
+
+    The lines (backward alone, as rows / both unless said):
+      _PRODUCT_BY_SAMPLE   smaller products keep the rows.  They would gain on the device too, as the last three lines
+                           above show, and not lose by themselves, where the host is the slower one ([8192, 1024] -> 4096 561 / 546 us
+                           a pass, [2048, 1024] -> 1024 470 / 476): there the memory stays as it was.
+      _ELEMENTS_BY_SAMPLE  factors of at most 128 MB.  Larger ones are turned over at memory speed, for products that are
+                           narrow or near the library's best as they are: [16384, 16384] -> 256 593 / 717, -> 1024 1127 / 1237,
+                           [131072, 2048] -> 2048 2405 / 2814, [2^20, 1024] -> 1024 7903 / 11236, [16384, 256] -> 16384 675 / 755.
+                           (With 2^36 products neither width is below 1024 then.)
+      _LONG_SUM, _FEW_TILES  sums of more than 16384 samples for results of up to 3 * 2^20 values only: for more the library splits
+                           the sum over the chip as rows and not like this ([33000, 2000] -> 2040 745 / 841; products alone,
+                           2048 x 2048 over 28032 samples 235 / 333, 2304 x 2304 over 26048 286 / 351, but 1792 x 1792
+                           over 32768 314 / 255, 1024 x 1024 over 65536 326 / 262).
+      _BOTH_BY_SAMPLE      512 samples: of 97 products of fewer, sizes at random, six lost 3 % or more, and so did layers
+                           ([256, 2048] -> 151936 888 / 901, [128, 1024] -> 524288 1535 / 1630, [128, 4096] -> 131072 857 / 857).
+                           Of 315 with 512 to 16384 samples six did; half of them take a quarter less time or better.
+      _INPUT_BY_SAMPLE     the input alone, for a gradient row_column_sums_transposed does not take: from 2048 samples (the product
+                           alone takes 17 % less on average; a quarter of those with 512 to 2048 samples lost).
+    Not for fp32 and streams of one width, which have no such unpack."""
+    if not config.compress_activation or config.simulate or config.swap or config.group_size != 256 or len(shape) != 2:
+        return False
+    N, F = shape
+    if (N < _BOTH_BY_SAMPLE or N * F * outputs < _PRODUCT_BY_SAMPLE or N * max(F, outputs) > _ELEMENTS_BY_SAMPLE
+            or N > _LONG_SUM and F * outputs > _FEW_TILES):
         return False
     _, q_bits, q_scale, _ = quantized
-    return (len(shape) == 2 and shape[0] >= _BOTH_BY_SAMPLE and shape[0] * shape[1] * outputs >= _PRODUCT_BY_SAMPLE
-            and isinstance(q_bits, torch.Tensor)
+    return (isinstance(q_bits, torch.Tensor)
             and (q_scale.dtype == torch.float16 or q_scale.dtype == torch.bfloat16 and not _stored_as_bf16(shape, quantized)))
 
 
-_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE, _PRODUCT_BY_SAMPLE = 128, 2048, 1 << 36
+_BOTH_BY_SAMPLE, _INPUT_BY_SAMPLE, _PRODUCT_BY_SAMPLE = 512, 2048, 1 << 36
+_ELEMENTS_BY_SAMPLE, _LONG_SUM, _FEW_TILES = 1 << 26, 16384, 3 << 20
 
 
 class linear(Function):

@@ -264,3 +264,30 @@ def test_skip_connection_hand_over_and_ordinary_accumulation():
     main, identity = ops.skip_connection.apply(x, ops.SkipGradient())
     (identity * 3.0).sum().backward()                                # only one of the two used
     assert torch.equal(x.grad, torch.full_like(x, 3.0))
+
+
+@pytest.mark.parametrize("N,F,O,taken", [
+    (8192, 4096, 4096, True), (4096, 4096, 4096, True), (4096, 4096, 4095, False),              # 2^36 products
+    (512, 16384, 8192, True), (511, 32768, 8192, False),                                        # few samples
+    (65536, 1024, 1024, True), (65536, 1025, 1024, False), (16384, 16384, 256, False), (16384, 256, 16384, False),   # 128 MB
+    (16384, 4096, 4096, True), (16385, 2048, 2048, False), (32768, 2048, 1536, True), (32768, 2048, 1537, False),    # long sums
+    (131072, 2048, 2048, False), (1 << 20, 1024, 1024, False)])
+def test_where_linear_reads_its_factors_by_sample(N, F, O, taken):
+    from actnn_amd import ops
+
+    def saved(bits, dtype, native_bf16=False):
+        q = ops._Quantized((None, bits, torch.empty(1, 1, 1, dtype=dtype), None))
+        q.native_bf16 = native_bf16
+        return q
+    widths = torch.ones(1, dtype=torch.int32)
+    assert ops._by_sample(saved(widths, torch.float16), (N, F), O) == taken
+    assert ops._by_sample(saved(widths, torch.bfloat16, True), (N, F), O) == taken
+    # one width for all, fp32 (its scales kept as bfloat16 or not), more than two dimensions, other streams: as rows
+    assert not ops._by_sample(saved(2, torch.float16), (N, F), O)
+    assert not ops._by_sample(saved(widths, torch.bfloat16), (N, F), O)
+    assert not ops._by_sample(saved(widths, torch.float32), (N, F), O)
+    assert not ops._by_sample(saved(widths, torch.float16), (N, 1, F), O)
+    for name, value in (("compress_activation", False), ("simulate", True), ("swap", True), ("group_size", 128)):
+        config.reset()
+        setattr(config, name, value)
+        assert not ops._by_sample(saved(widths, torch.float16), (N, F), O)
