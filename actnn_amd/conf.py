@@ -49,6 +49,10 @@ class QuantizationConfig:
         # against 0.25 ms on [8192,4096] x [8192,4096] for the 4-bit and the mixed-width stream);
         # False - never
         self.fused_linear_grad_weight = True
+        # the factors of a large 16-bit QLinear's weight gradient (2^36 products and more, per-sample widths) turned over
+        # before the library multiplies them: 6-10 % less time for the layer, at one more tensor of the output
+        # gradient's size (at most 128 MB) while the product runs.  False keeps the backward's peak where it is without
+        self.linear_factors_by_sample = True
         self.pool_index_nibbles = True                 # max-pool keeps its arg-max indices two per byte
         # memory management (conf.py:54-58)
         self.empty_cache_threshold = None

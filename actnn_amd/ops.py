@@ -445,7 +445,7 @@ def _by_sample(quantized, shape, outputs):
       2048, 8192, 4096   419.3  400.5  382.6            8192, 1024, 1024   205.2  188.3  172.8
       1024, 8192, 8192   450.0  434.0  400.3            2048, 1024, 1024    94.9   95.4   89.9
     The turned gradient is one more tensor of the gradient's size until the product has been queued (a backward pass's
-    peak above its start for [8192, 4096] -> 4096: 160 MB, 96 as rows).
+    peak above its start for [8192, 4096] -> 4096: 160 MB, 96 as rows; config.linear_factors_by_sample).
 
     The lines (backward alone, as rows / both unless said):
       _PRODUCT_BY_SAMPLE   smaller products keep the rows.  They would gain on the device too, as the last three lines
@@ -465,7 +465,8 @@ def _by_sample(quantized, shape, outputs):
       _INPUT_BY_SAMPLE     the input alone, for a gradient row_column_sums_transposed does not take: from 2048 samples (the product
                            alone takes 17 % less on average; a quarter of those with 512 to 2048 samples lost).
     Not for fp32 and streams of one width, which have no such unpack."""
-    if not config.compress_activation or config.simulate or config.swap or config.group_size != 256 or len(shape) != 2:
+    if (not config.linear_factors_by_sample or not config.compress_activation or config.simulate or config.swap
+            or config.group_size != 256 or len(shape) != 2):
         return False
     N, F = shape
     if (N < _BOTH_BY_SAMPLE or N * F * outputs < _PRODUCT_BY_SAMPLE or N * max(F, outputs) > _ELEMENTS_BY_SAMPLE

@@ -287,7 +287,7 @@ def test_where_linear_reads_its_factors_by_sample(N, F, O, taken):
     assert not ops._by_sample(saved(widths, torch.bfloat16), (N, F), O)
     assert not ops._by_sample(saved(widths, torch.float32), (N, F), O)
     assert not ops._by_sample(saved(widths, torch.float16), (N, 1, F), O)
-    for name, value in (("compress_activation", False), ("simulate", True), ("swap", True), ("group_size", 128)):
+    for name, value in (("linear_factors_by_sample", False), ("compress_activation", False), ("simulate", True), ("swap", True), ("group_size", 128)):
         config.reset()
         setattr(config, name, value)
         assert not ops._by_sample(saved(widths, torch.float16), (N, F), O)
