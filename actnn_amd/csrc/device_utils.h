@@ -232,8 +232,8 @@ template <bool PAST, typename T> ACTNN_DEV void store16_part(T* p, u32x4 v, int 
     }
   }
 }
-// A wave's `count` consecutive elements, which lie in `slab` (LDS, 16-byte aligned, up to 4 KiB and a dword that
-// may be read behind them), to `dst`, any element address: whole lines by whole instructions, what lies
+// A wave's `count` consecutive elements, which lie in `slab` (LDS, 16-byte aligned, up to 4 KiB), to `dst`, any
+// element address: whole lines by whole instructions, what lies
 // before the first and behind the last vector element by element, all of it past the caches.  For tensors that
 // stream_rows sends there: stored from the lanes that own them, 16 bytes each at the tensor's own alignment and through
 // the caches, the lines of odd rows were written by two instructions and left dirty (minimax + pack + unpack
@@ -254,7 +254,7 @@ template <typename T> ACTNN_DEV void store_unit_any(T* dst, const uint32_t* slab
       u32x4 w = {p[0], p[1], p[2], p[3]};
       if constexpr (S == 2) {
         if (head & 2u) {
-          const uint32_t next = p[4];
+          const uint32_t next = p[4];                  // (holds the vector's last element: head is 2 more than p)
 #pragma unroll
           for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_alignbit(k < 3 ? w[k < 3 ? k + 1 : 3] : next, w[k], 16);
         }

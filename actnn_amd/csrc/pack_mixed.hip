@@ -429,8 +429,8 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
   __shared__ float s_scale[kWaves * kUnit];
   __shared__ float s_min[kWaves * kUnit];
   constexpr bool kStage = IsF32<T>::value || ROWS == kRowsPast;
-  constexpr int kSlab = kUnit * kGs * (int)sizeof(T) / 16;       // (and a dword behind the last: see store_unit_any)
-  __shared__ u32x4 s_slab[kStage ? kWaves * kSlab + 1 : 1];
+  constexpr int kSlab = kUnit * kGs * (int)sizeof(T) / 16;
+  __shared__ u32x4 s_slab[kStage ? kWaves * kSlab : 1];
   const uint32_t wave = wave_of_block();
   u32x4* slab = s_slab + (kStage ? wave * kSlab : 0);
   const Unit u = unit_of<kUnit>(blockIdx.x * kWaves + wave, per_sample, N, G);
