@@ -463,9 +463,9 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_kernel(
 // ---------------------------------------------------------------------------- unpack, transposed
 // The rows of a linear layer's input with the samples contiguous, out[feature * ld + sample], as the matrix
 // product of its weight gradient reads them fastest: that product sums over the samples, and with both factors
-// stored sample by sample its loads run across the rows (bf16, go [N, O] and x [N, F], us with x as rows / with
-// x like this: [8192, 4096] x [8192, 4096] 260 / 202, [8192, 1024] x [8192, 1024] 54.5 / 39.0,
-// [2048, 1024] x [2048, 1024] 17.5 / 14.4, [256, 1024] x [256, 1024] 6.7 / 6.3).
+// stored sample by sample its loads run across the rows (the product alone, bf16, go [N, O] and x [N, F], us with x as
+// rows / with x like this / with go turned over as well: [8192, 4096] x [8192, 4096] 250 / 198 / 171, [4096, 4096] x
+// [4096, 4096] 128 / 103 / 90, [2048, 4096] x [2048, 8192] 137 / 112 / 96, [65536, 1024] x [65536, 1024] 321 / 281 / 258).
 // Bound by the write, as unpack: the values are unpack's bit for bit.  A half-wave takes 8 samples of one group (a
 // block 64), whose words are loaded before the first is decoded.  The widths of the two halves of a wave
 // differ, so the decoders take them at run time: the table of four levels where neither exceeds 2 bits.
@@ -641,7 +641,8 @@ __global__ __launch_bounds__(1024) void bits_prefix_kernel(const int32_t* __rest
 }
 
 // Units of `groups` groups per sample and the blocks of four that cover them all.  Numbers of units stay
-// below 2^31 (a unit holds at least a group, so that the tensor would be 1 TiB of 16-bit values).
+// below 2^31: a sample of several units holds more than 1024 elements (fp32; 2048 in 16 bits), so that only a tensor
+// of 4 TiB has as many, and one of shorter rows has a unit to a row, as it had a block before.
 bool unit_grid(int64_t N, int64_t G, int groups, int64_t& per_sample, int64_t& blocks) {
   per_sample = (G + groups - 1) / groups;
   if (per_sample > 0x7fffffffLL / N) return false;
