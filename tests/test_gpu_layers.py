@@ -559,9 +559,28 @@ def test_linear_backward_of_a_batch_of_gradients():
             assert (a[i] - b).norm() <= 1024 * 2.0 ** -24 * b.norm()
 
 
+@pytest.fixture
+def by_sample(monkeypatch):
+    """Sizes of any kind may take linear's product by sample -> {"gradient", "input": how often each was turned over}."""
+    monkeypatch.setattr(ops, "_PRODUCT_BY_SAMPLE", 0)
+    calls = {"gradient": 0, "input": 0}
+
+    def counted(module, name, kind):
+        plain = getattr(module, name)
+
+        def call(*args):
+            out = plain(*args)
+            calls[kind] += out is not None
+            return out
+        monkeypatch.setattr(module, name, call)
+    counted(ops.ext_minimax, "row_column_sums_transposed", "gradient")
+    counted(ops.ext_quantization, "unpack_rows_mixed_transposed", "input")
+    return calls
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,F,O,bias", [(128, 256, 8, True), (130, 300, 1000, True), (2050, 264, 100, True), (300, 512, 512, False)])
-def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias, monkeypatch):
+def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias, monkeypatch, by_sample):
     """The factors of the weight gradient turned over (the input alone where the gradient's rows are no whole
     16-byte vectors): the gradients are those of the product over rows, in another order of addition."""
     torch.manual_seed(0)
@@ -570,19 +589,70 @@ def test_linear_weight_gradient_with_the_samples_contiguous(dtype, N, F, O, bias
     grad = torch.randn(N, O, device=DEV).to(dtype)
     layer.scheme.set_scale(grad)
     wanted = [x, layer.weight] + ([layer.bias] if bias else [])
-    monkeypatch.setattr(ops, "_PRODUCT_BY_SAMPLE", 0)
     got = []
     for limits in ((128, 2048), (1 << 30, 1 << 30)):
         monkeypatch.setattr(ops, "_BOTH_BY_SAMPLE", limits[0])
         monkeypatch.setattr(ops, "_INPUT_BY_SAMPLE", limits[1])
         torch.manual_seed(1)
         got.append(torch.autograd.grad(layer(x), wanted, grad, retain_graph=False) + (layer.scheme.scales,))
+        assert by_sample == {"gradient": int(O % 8 == 0), "input": 1}          # (by rows: none added)
     eps = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
     assert torch.equal(got[0][0], got[1][0])
     for a, b in zip(got[0][1:], got[1][1:]):
         # N terms added in another order: at most 2 N 2^-24 of their 2-norms, then one rounding each
         bound = eps * b.double().norm() + 2 * N * 2.0 ** -24 * b.double().norm() * math.sqrt(N)
         assert (a.double() - b.double()).norm() <= bound
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_by_sample_under_a_graph_of_the_backward(dtype, monkeypatch, by_sample):
+    """create_graph: the gradient stays as it is (its sums have to be differentiable), the input is turned over; first
+    and second derivatives are those of the product over rows."""
+    N, F, O = 2050, 264, 96
+    torch.manual_seed(0)
+    layer = actnn_amd.QLinear(F, O).to(DEV, dtype)
+    x = torch.randn(N, F, device=DEV).to(dtype).requires_grad_()
+    grad = torch.randn(N, O, device=DEV).to(dtype).requires_grad_()
+    along = torch.randn(O, F, device=DEV).to(dtype)
+    layer.scheme.set_scale(grad.detach())
+    scale = layer.scheme.scales
+    got = []
+    for limit in (2048, 1 << 30):
+        monkeypatch.setattr(ops, "_INPUT_BY_SAMPLE", limit)
+        layer.scheme.scales = scale                        # the same widths for both
+        torch.manual_seed(1)
+        first = torch.autograd.grad(layer(x), [x, layer.weight, layer.bias], grad, create_graph=True)
+        got.append((*first, *torch.autograd.grad(first[1], grad, along)))
+        assert by_sample == {"gradient": 0, "input": 1}
+    eps = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    for a, b in zip(*got):
+        # up to N terms added in another order (2 N 2^-24 of their 2-norms), then one rounding each
+        a, b = a.detach().double(), b.detach().double()
+        assert (a - b).norm() <= (eps + 2 * N * 2.0 ** -24 * math.sqrt(N)) * b.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_by_sample_leaves_a_batch_of_gradients_alone(dtype, monkeypatch, by_sample):
+    """is_grads_batched at per-sample widths (which needs the gradient statistics frozen): no memory to turn over, and
+    the gradients are those of one backward pass after the other."""
+    N, F, O = 2048, 256, 64
+    torch.manual_seed(0)
+    layer = actnn_amd.QLinear(F, O).to(DEV, dtype)
+    x = torch.randn(N, F, device=DEV).to(dtype).requires_grad_()
+    grads = torch.randn(3, N, O, device=DEV).to(dtype)
+    wanted = [x, layer.weight, layer.bias]
+    layer.scheme.set_scale(grads[0])
+    monkeypatch.setattr(QScheme, "update_scale", False)
+    torch.manual_seed(1)
+    got = torch.autograd.grad(layer(x), wanted, grads, is_grads_batched=True)
+    assert by_sample == {"gradient": 0, "input": 0}
+    eps = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    for i in range(3):
+        torch.manual_seed(1)
+        for a, b in zip(got, torch.autograd.grad(layer(x), wanted, grads[i])):
+            a, b = a[i].double(), b.double()
+            assert (a - b).norm() <= (eps + 2 * N * 2.0 ** -24 * math.sqrt(N)) * b.norm()
+    assert by_sample == {"gradient": 3, "input": 3}
 
 
 @pytest.mark.parametrize("bias", [True, False])
@@ -1132,10 +1202,10 @@ def test_closing_step_of_a_residual_block_in_the_batch_norm_pass(dtype, channels
         assert torch.equal(u, v), i
 
 
-@pytest.mark.parametrize("n", [200, 215, 270])
+@pytest.mark.parametrize("n", [200, 201, 215, 270])
 def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
-    """Forward passes of more than two rounds of blocks choose how many rows a block takes: 20, 12 and 16 steps of 8 rows
-    here, the last block ragged.  Output and saved stream are those of the batch norm, the addition and the ReLU."""
+    """Forward passes of more than two rounds of blocks choose how many rows a block takes: 20, 20, 12 and 16 steps of 8
+    rows here, the last block whole (n = 200) and ragged.  Output and saved stream are those of the batch norm, the addition and the ReLU."""
     from actnn_amd.layers import QAddReLU, QBatchNorm2d, bn_add_relu, known_group_minmax
     res = []
     for fold in (False, True):
