@@ -1697,12 +1697,14 @@ int launch_cl_reduce(const Plan& pl, const XS& xs, const void* dy, float* part, 
 // as much as a full one: of 8, 12, 16 and 20 steps the one with the least rounds * (steps + 3).  Forward of the
 // layer, bf16 [n, 512, 28, 28], us with the plan's 8 steps / with these: n = 256 195.2 / 183.1 (20), 370
 // 278.2 / 266.6 (12), 215 169.3 / 164.3 (16), 160 135.4 / 129.5 (16), 100 97.9 / 94.4 (20);
-// [128, 256, 56, 56] 188.9 / 178.4 (20); [256, 64, 56, 56] 112.6 / 113.6 (16).  Below two rounds the plan's blocks
-// stay (bf16 [256, 16, 64, 64]: 54.9 with 8 steps, 57.7 with 16).  The passes without the residual have less to
+// [128, 256, 56, 56] 188.9 / 178.4 (20); [256, 64, 56, 56] 112.6 / 113.6 (16).  Below two rounds and a quarter the plan's
+// blocks stay (bf16 [256, 16, 64, 64]: 54.9 with 8 steps, 57.7 with 16): just above two the choice is one round of 20 steps
+// that leaves up to a fifth of the slots empty (f16 n = 84 90.7 / 94.8, 92 93.4 / 95.8, but 96 98.7 / 96.2; bf16
+// 93.3 / 96.1, 94.1 / 94.5, 98.7 / 94.6).  The passes without the residual have less to
 // stream and gain nothing ([256, 64, 56, 56] bn + ReLU 97.7 with 8 steps, 99.7 with 16; bn alone 72.5, 76.1).
 int64_t closing_rows(const Plan& pl) {
   constexpr int64_t slots = (int64_t)kCUs * 4;
-  if ((int64_t)pl.tiles * pl.nsplit_apply < 2 * slots) return pl.ppb_apply;
+  if ((int64_t)pl.tiles * pl.nsplit_apply < 2 * slots + slots / 4) return pl.ppb_apply;
   int64_t best = pl.ppb_apply, least = INT64_MAX;
   for (int steps = 8; steps <= 20; steps += 4) {
     const int64_t rows = (int64_t)steps * pl.R, blocks = (pl.P + rows - 1) / rows * pl.tiles;
