@@ -484,7 +484,7 @@ __global__ __launch_bounds__(kThreads) void unpack_mixed_transposed_kernel(
   // lane l looks up sample l & 7 of the half-wave's eight
   const int64_t nl = n0 + (lane & 7u) < N ? n0 + (lane & 7u) : N - 1;
   const int width = bits[nl];
-  const int my_bits = width < 1 ? 1 : width > 8 ? 8 : width;
+  const int my_bits = width < 1 || width > 8 ? 0 : width;      // (a width that there is not has no words to read)
   const int my_prefix = prefix[nl];
   const float my_scale = Conv<T>::load(scale, nl * G + g), my_min = Conv<T>::load(mn, nl * G + g);
   uint32_t lo[8], hi[8];
