@@ -1,4 +1,5 @@
-"""Build and load ``libactnn_hip.so`` - the C-ABI library of gfx950 kernels (include/actnn_hip.h).
+"""Build and load ``libactnn_hip.so`` - the C-ABI library of gfx950 kernels (include/actnn_hip.h) - and ``_host.so``, the
+native calls of a training step on top of it (csrc/host_calls.cpp).
 
 The library is compiled in-tree with hipcc and loaded with ctypes; there is no CPU fallback:
 if the library is missing, ``load()`` raises.
@@ -6,6 +7,7 @@ if the library is missing, ``load()`` raises.
 import ctypes
 import os
 import subprocess
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
@@ -18,6 +20,9 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",   # no packed-FP32 codegen
     "-Wno-unused-command-line-argument",
 ]
+
+HOST_PATH = os.path.join(_HERE, "_host.so")
+HOST_SOURCE = "host_calls.cpp"
 
 c_i64, c_i32, c_u64, c_vp = ctypes.c_int64, ctypes.c_int, ctypes.c_uint64, ctypes.c_void_p
 
@@ -121,28 +126,49 @@ _RESTYPES = {"actnn_strerror": ctypes.c_char_p, "actnn_version": ctypes.c_char_p
              "actnn_batch_norm_forward_static_limit": ctypes.c_int64,
              "actnn_batch_norm_backward_sumsq_entries": ctypes.c_int64}
 
-_lib = None
+_lib = _host = None
 
 
 def build(verbose=False):
     """Compile every source under csrc/ into libactnn_hip.so (always recompiles)."""
     srcs = [os.path.join(CSRC, s) for s in SOURCES]
     tmp = LIB_PATH + ".tmp"
-    cmd = ["hipcc", *HIPCC_FLAGS, *srcs, "-o", tmp]
+    out = _run(["hipcc", *HIPCC_FLAGS, *srcs, "-o", tmp], verbose)
+    # the host pass does not know the device-only target feature and says so once per file
+    noise = "'-packed-fp32-ops' is not a recognized feature for this target"
+    out = "\n".join(l for l in out.splitlines() if noise not in l)
+    if out.strip():
+        print(out, flush=True)
+    os.replace(tmp, LIB_PATH)
+    _build_host(verbose)
+    global _lib, _host
+    _lib = _host = None
+    return LIB_PATH
+
+
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    # the host pass does not know the device-only target feature and says so once per file
-    noise = "'-packed-fp32-ops' is not a recognized feature for this target"
-    out = "\n".join(l for l in proc.stdout.splitlines() if noise not in l)
-    if out.strip():
-        print(out, flush=True)
     if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed with exit code {proc.returncode}")
-    os.replace(tmp, LIB_PATH)
-    global _lib
-    _lib = None
-    return LIB_PATH
+        print(proc.stdout, flush=True)
+        raise RuntimeError(f"{cmd[0]} failed with exit code {proc.returncode}")
+    return proc.stdout
+
+
+def _build_host(verbose):
+    """Compile the native calls against torch and the library beside them."""
+    import torch
+    home = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    tmp = HOST_PATH + ".tmp"
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in includes),
+          os.path.join(CSRC, HOST_SOURCE), "-o", tmp, "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch_cpu",
+          "-lc10", "-lc10_hip", "-L" + _HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(tmp, HOST_PATH)
 
 
 def load():
@@ -162,6 +188,21 @@ def load():
         fn.restype = _RESTYPES.get(name, ctypes.c_int)
     _lib = lib
     return lib
+
+
+def load_host():
+    """The module of native calls (once).  Raises if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(
+                f"{HOST_PATH} is missing: the native calls are not built. Run "
+                "`python -c 'import __graft_entry__ as g; g.build()'`.")
+        import torch  # noqa: F401  (the module links against it)
+        from . import _host as module
+        _host = module
+    return _host
 
 
 def check(rc, what):

@@ -12,6 +12,11 @@ def lib():
     return _lib.load()
 
 
+def host():
+    """The module of native calls (csrc/host_calls.cpp), the C library loaded under it."""
+    return _lib.load_host()
+
+
 def _name_check(cond, msg):
     if not cond:
         raise RuntimeError(msg)

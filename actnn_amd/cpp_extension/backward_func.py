@@ -12,14 +12,13 @@ import functools
 import torch
 
 from . import _glue
-from ..utils import channels_last_format
 
 _aten = torch.ops.aten
 
 
 def _shape_geometry(shape, dtype, channels_last):
     """(N, C, HW) when the library's batch-norm kernels take a tensor of this shape, else None."""
-    return _geometry_of(tuple(int(d) for d in shape), dtype, bool(channels_last))
+    return _geometry_of(tuple(map(int, shape)), dtype, bool(channels_last))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -62,13 +61,7 @@ def known_sumsq(grad):
 
 def _bn_geometry(input):
     """(N, C, HW, channels_last) of a dense tensor in the default or the channels-last layout."""
-    if not (isinstance(input, torch.Tensor) and input.is_cuda):
-        return None
-    channels_last = channels_last_format(input) is not None
-    if not channels_last and not input.is_contiguous():
-        return None
-    geo = _shape_geometry(input.shape, input.dtype, channels_last)
-    return None if geo is None else geo + (channels_last,)
+    return _glue.host().batch_norm_geometry(input)
 
 
 def _f32_or_none(t):
@@ -76,8 +69,7 @@ def _f32_or_none(t):
 
 
 def hip_batch_norm_applies(input, weight, bias, running_mean, running_var):
-    return (_bn_geometry(input) is not None and input.data_ptr() % 16 == 0
-            and all(_f32_or_none(t) for t in (weight, bias, running_mean, running_var)))
+    return _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var) is not None
 
 
 @functools.lru_cache(maxsize=4096)
@@ -89,9 +81,10 @@ def _groups_align(N, C, HW, code, channels_last):
 
 def hip_batch_norm_minmax_applies(input, weight, bias, running_mean, running_var):
     """True when the forward pass can also return the quantiser's per-group min/max."""
-    if not hip_batch_norm_applies(input, weight, bias, running_mean, running_var):
+    geo = _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var)
+    if geo is None:
         return False
-    N, C, HW, channels_last = _bn_geometry(input)
+    N, C, HW, channels_last = geo
     return _groups_align(N, C, HW, _glue.DTYPE_CODE[input.dtype], channels_last)
 
 
@@ -103,26 +96,8 @@ def hip_batch_norm_forward(input, weight, bias, running_mean, running_var, momen
     """-> (output, save_mean, save_invstd, mn, mx): training-mode batch norm; with `minmax` the
     minimum and maximum of every group of 256 elements of a sample that are consecutive in memory
     come out of the same pass over the input (None, None otherwise)."""
-    N, C, HW, channels_last = _bn_geometry(input)
-    lib = _glue.lib()
-    code = _glue.DTYPE_CODE[input.dtype]
-    ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
-    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=input.device)
-    out = torch.empty_like(input)                       # same strides as the input
-    save_mean = torch.empty(C, dtype=torch.float32, device=input.device)
-    save_invstd = torch.empty(C, dtype=torch.float32, device=input.device)
-    mn = mx = None
-    if minmax:
-        groups = N * C * HW // 256
-        mn = torch.empty(groups, dtype=input.dtype, device=input.device)
-        mx = torch.empty(groups, dtype=input.dtype, device=input.device)
-    with _glue.on_device(input.device):
-        _glue._lib.check(lib.actnn_batch_norm_forward(
-            input.data_ptr(), _ptr(weight), _ptr(bias), _ptr(running_mean), _ptr(running_var),
-            out.data_ptr(), save_mean.data_ptr(), save_invstd.data_ptr(), _ptr(mn), _ptr(mx),
-            ws.data_ptr(), ws_bytes, N, C, HW, float(momentum), float(eps), code, int(channels_last),
-            _glue.stream_ptr(input.device)), "batch_norm_forward")
-    return out, save_mean, save_invstd, mn, mx
+    return _glue.host().batch_norm_forward(input, *_bn_geometry(input), weight, bias, running_mean, running_var, momentum, eps,
+                                           minmax)
 
 
 def hip_batch_norm_forward_stats(input, weight, bias, running_mean, running_var, momentum, eps, minmax=True):
@@ -194,10 +169,8 @@ def hip_batch_norm_quantize_geometry(input, weight, bias, running_mean, running_
     """(N, C, HW, channels_last) when statistics, group min/max and the packed copy can all come from
     the fused passes (what hip_batch_norm_minmax_applies and hip_batch_norm_pack_applies ask, looked
     up once), else None."""
-    geo = _bn_geometry(input)
-    if geo is None or input.data_ptr() % 16 != 0:
-        return None
-    if not (_f32_or_none(weight) and _f32_or_none(bias) and _f32_or_none(running_mean) and _f32_or_none(running_var)):
+    geo = _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var)
+    if geo is None:
         return None
     N, C, HW, channels_last = geo
     if not _groups_align(N, C, HW, _glue.DTYPE_CODE[input.dtype], channels_last):
@@ -226,56 +199,14 @@ def hip_batch_norm_forward_quantize(input, geo, weight, bias, running_mean, runn
     (hip_batch_norm_relu_applies) the output is relu(bn(input)) - relu(bn(input) + residual) with a
     `residual` laid out like the input - and the tuple ends with the ReLU's mask and the group
     min / max of the output."""
-    from .quantization import attach_bits_total, mask_words
-    N, C, HW, channels_last = geo
-    dev, dtype = input.device, input.dtype
-    code = _glue.DTYPE_CODE[dtype]
-    ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
-    G = C * HW // 256
-    f32, i32 = torch.float32, torch.int32
-    ws = torch.empty(ws_bytes // 4, dtype=f32, device=dev)
-    save_mean = torch.empty(C, dtype=f32, device=dev)
-    save_invstd = torch.empty(C, dtype=f32, device=dev)
-    mn = torch.empty(N * G, dtype=dtype, device=dev)
-    mx = torch.empty(N * G, dtype=dtype, device=dev)
-    out = torch.empty_like(input)
-    sens = alloc.sens_out if alloc.sens_out is not None else torch.empty(N, dtype=f32, device=dev)
-    bits = torch.empty(N, dtype=i32, device=dev)
-    prefix = torch.empty(N + 1, dtype=i32, device=dev)
-    packed = torch.empty(alloc.total * G * 8, dtype=i32, device=dev)
-    scale = torch.empty(N, G, 1, dtype=dtype, device=dev)
-    mask = zmn = zmx = None
-    if relu:
-        mask = torch.empty(mask_words(N * C * HW), dtype=i32, device=dev)
-        zmn = torch.empty(N * G, dtype=dtype, device=dev)
-        zmx = torch.empty(N * G, dtype=dtype, device=dev)
-    mult, mult_ptr, per_sample = _mult_args(alloc.mult, N, dev)          # (`mult` held until the launch)
-    seed, offset = _glue.philox_args(dev)
-    with _glue.on_device(dev):
-        _glue._lib.check(_glue.lib().actnn_batch_norm_forward_quantize(
-            input.data_ptr(), _ptr(weight), _ptr(bias), _ptr(running_mean), _ptr(running_var), out.data_ptr(),
-            save_mean.data_ptr(), save_invstd.data_ptr(), mn.data_ptr(), mx.data_ptr(), ws.data_ptr(), ws_bytes,
-            alloc.factor, mult_ptr, per_sample, sens.data_ptr(), bits.data_ptr(), prefix.data_ptr(),
-            alloc.initial, alloc.target, scale.data_ptr(), packed.data_ptr(), seed, offset, _ptr(mask), _ptr(zmn),
-            _ptr(zmx), _ptr(residual), N, C, HW, float(momentum), float(eps), code, int(channels_last),
-            _glue.stream_ptr(dev)),
-            "batch_norm_forward_quantize")
+    from .quantization import attach_bits_total
+    out, save_mean, save_invstd, mn, mx, bits, packed, scale, prefix, mask, zmn, zmx = _glue.host().batch_norm_forward_quantize(
+        input, *geo, weight, bias, running_mean, running_var, momentum, eps, alloc.factor, alloc.mult, alloc.initial,
+        alloc.target, alloc.total, alloc.sens_out, relu, residual)
     attach_bits_total(bits, alloc.total, prefix)
     if relu:
         return out, save_mean, save_invstd, mn, mx, bits, packed, scale, mask, zmn, zmx
     return out, save_mean, save_invstd, mn, mx, bits, packed, scale
-
-
-def _mult_args(mult, N, dev):
-    """(tensor, pointer, per-sample flag) of the sensitivity's multiplier: nothing, one device scalar
-    or one value per sample (fp32 on `dev`), as allocate_bits_device takes it."""
-    if mult is None:
-        return None, None, 0
-    if mult.dtype != torch.float32 or mult.device != dev or mult.numel() not in (1, N):
-        raise RuntimeError("the sensitivity's multiplier must be fp32 on the same device with 1 or N values")
-    if not mult.is_contiguous():
-        mult = mult.contiguous()
-    return mult, mult.data_ptr(), int(mult.numel() == N and N != 1)
 
 
 def hip_batch_norm_pack_applies(input, weight, bias, running_mean, running_var):
@@ -292,23 +223,10 @@ def hip_batch_norm_backward(input, grad_output, weight, save_mean, save_invstd, 
     """-> (grad_input, grad_weight, grad_bias) of training-mode batch norm; `grad_output` has the
     strides of `input`.  With `sumsq` the pass also leaves the partial sums of grad_input^2 on
     grad_input (see known_sumsq)."""
-    N, C, HW, channels_last = _bn_geometry(input)
-    lib = _glue.lib()
-    code = _glue.DTYPE_CODE[input.dtype]
-    ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
-    entries = _sumsq_entries(N, C, HW, code, int(channels_last)) if sumsq else 0
-    ws = torch.empty(ws_bytes // 4 + entries, dtype=torch.float32, device=input.device)
-    grad_input = torch.empty_like(input)
-    grad_weight = torch.empty(C, dtype=torch.float32, device=input.device)
-    grad_bias = torch.empty(C, dtype=torch.float32, device=input.device)
-    with _glue.on_device(input.device):
-        _glue._lib.check(lib.actnn_batch_norm_backward(
-            input.data_ptr(), grad_output.data_ptr(), _ptr(weight), save_mean.data_ptr(),
-            save_invstd.data_ptr(), grad_input.data_ptr(), grad_weight.data_ptr(), grad_bias.data_ptr(),
-            ws.data_ptr(), ws_bytes, ws.data_ptr() + ws_bytes if entries else None, entries,
-            N, C, HW, code, int(channels_last), _glue.stream_ptr(input.device)), "batch_norm_backward")
-    if entries:
-        _leave_sumsq(grad_input, ws[ws_bytes // 4:])
+    grad_input, grad_weight, grad_bias, squares = _glue.host().batch_norm_backward(
+        input, grad_output, *_bn_geometry(input), weight, save_mean, save_invstd, sumsq)
+    if squares is not None:
+        _leave_sumsq(grad_input, squares)
     return grad_input, grad_weight, grad_bias
 
 
@@ -348,38 +266,17 @@ def hip_batch_norm_backward_packed(shape, quantized, grad_output, weight, save_m
     q_input, q_bits, q_scale, q_min = quantized
     channels_last = getattr(quantized, "memory_format", None) is not None
     N, C, HW = _shape_geometry(shape, grad_output.dtype, channels_last)
-    lib = _glue.lib()
-    code = _glue.DTYPE_CODE[grad_output.dtype]
     total, prefix = _bits_info(q_bits)
     if q_input.numel() < total * (C * HW // 256) * 8:
         raise RuntimeError("batch_norm_backward_packed: packed stream is too short")
     if q_scale.dtype != grad_output.dtype:              # fp32 activation, bf16 storage: widened as
         q_scale = q_scale.to(grad_output.dtype)         # dequantize_activation widens it (ops.py:129-131)
         q_min = q_min.to(grad_output.dtype)
-    ws_bytes = _workspace_bytes(N, C, HW, code, int(channels_last))
-    dev = grad_output.device
-    entries = _sumsq_entries(N, C, HW, code, int(channels_last)) if sumsq else 0
-    ws = torch.empty(ws_bytes // 4 + entries, dtype=torch.float32, device=dev)
-    grad_input = torch.empty_like(grad_output)
-    grad_weight = torch.empty(C, dtype=torch.float32, device=dev)
-    grad_bias = torch.empty(C, dtype=torch.float32, device=dev)
-    with _glue.on_device(dev):
-        if relu_mask is not None:
-            _glue._lib.check(lib.actnn_batch_norm_backward_packed_add_relu(
-                q_input.data_ptr(), q_bits.data_ptr(), prefix.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(),
-                grad_output.data_ptr(), relu_mask.data_ptr(), _ptr(masked), _ptr(weight), save_mean.data_ptr(),
-                save_invstd.data_ptr(), grad_input.data_ptr(), grad_weight.data_ptr(), grad_bias.data_ptr(),
-                ws.data_ptr(), ws_bytes, ws.data_ptr() + ws_bytes if entries else None, entries,
-                N, C, HW, code, int(channels_last), _glue.stream_ptr(dev)), "batch_norm_backward_packed_relu")
-        else:
-            _glue._lib.check(lib.actnn_batch_norm_backward_packed(
-                q_input.data_ptr(), q_bits.data_ptr(), prefix.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(),
-                grad_output.data_ptr(), _ptr(weight), save_mean.data_ptr(), save_invstd.data_ptr(),
-                grad_input.data_ptr(), grad_weight.data_ptr(), grad_bias.data_ptr(), ws.data_ptr(), ws_bytes,
-                ws.data_ptr() + ws_bytes if entries else None, entries,
-                N, C, HW, code, int(channels_last), _glue.stream_ptr(dev)), "batch_norm_backward_packed")
-    if entries:
-        _leave_sumsq(grad_input, ws[ws_bytes // 4:])
+    grad_input, grad_weight, grad_bias, squares = _glue.host().batch_norm_backward_packed(
+        q_input, q_bits, prefix, q_scale, q_min, grad_output, N, C, HW, channels_last, weight, save_mean, save_invstd, sumsq,
+        relu_mask, masked)
+    if squares is not None:
+        _leave_sumsq(grad_input, squares)
     return grad_input, grad_weight, grad_bias
 
 

@@ -110,36 +110,31 @@ def quantize_activation_device(rows, N, known_minmax, alloc):
     of whole groups in the rows' dtype when another kernel has produced them, else None.  `alloc`: the
     scheme's AllocationArgs, whose `store_dtype` says what scale and mn come back in.
     -> (packed, bits with sum and prefix attached, scale [N, G, 1], mn [N * G])."""
-    from .backward_func import _mult_args
-    dev, dtype = rows.device, rows.dtype
-    store_dtype = alloc.store_dtype or dtype
-    F = rows.numel() // N
-    G = (F + 255) // 256
-    if known_minmax is None:
-        mn = torch.empty(N * G, dtype=dtype, device=dev)
-        mx = torch.empty(N * G, dtype=dtype, device=dev)
-    else:
-        mn, mx = known_minmax
-    stored = mn if store_dtype == dtype else torch.empty(N * G, dtype=store_dtype, device=dev)
-    sens = alloc.sens_out if alloc.sens_out is not None else torch.empty(N, dtype=torch.float32, device=dev)
-    bits = torch.empty(N, dtype=torch.int32, device=dev)
-    prefix = torch.empty(N + 1, dtype=torch.int32, device=dev)
-    packed = torch.empty(alloc.total * G * 8, dtype=torch.int32, device=dev)
-    scale = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
-    mult, mult_ptr, per_sample = _mult_args(alloc.mult, N, dev)           # (`mult` held until the launch)
-    seed, offset = g.philox_args(dev)
-    with g.on_device(dev):
-        check(g.lib().actnn_quantize_rows(
-            rows.data_ptr(), mn.data_ptr(), mx.data_ptr(), int(known_minmax is not None), alloc.factor, mult_ptr,
-            per_sample, sens.data_ptr(), bits.data_ptr(), prefix.data_ptr(), alloc.initial, alloc.target,
-            scale.data_ptr(), stored.data_ptr(), packed.data_ptr(), seed, offset, N, F, g.DTYPE_CODE[dtype],
-            g.DTYPE_CODE[store_dtype], g.stream_ptr(dev)), "quantize_activation")
+    mn, mx = known_minmax if known_minmax is not None else (None, None)
+    packed, bits, scale, stored, prefix = g.host().quantize_rows(
+        rows, N, mn, mx, alloc.factor, alloc.mult, alloc.initial, alloc.target, alloc.total, alloc.sens_out,
+        g.DTYPE_CODE[alloc.store_dtype or rows.dtype])
     attach_bits_total(bits, alloc.total, prefix)
     return packed, bits, scale, stored
 
 
 def unpack_rows_mixed(packed, bits, scale, mn, N, F, dtype):
     """The [N, F] rows of quantize_activation_device in `dtype`, nothing materialised for the padding."""
+    info = _fresh(bits, "_actnn_info")
+    if info is None:
+        g.check_typed(packed, "data", torch.int32, 1)
+        g.check_typed(bits, "bits", torch.int32, 1)
+        info = _bits_info(bits)
+    out = g.host().unpack_rows_mixed(packed, bits, info[1], info[0], scale, mn, N, F, g.DTYPE_CODE[dtype])
+    if out is None:                                    # something does not fit: say what
+        _check_rows(packed, bits, scale, mn, N, F)
+        raise RuntimeError("unpack_mixed_precision: the arguments do not fit together")
+    return out
+
+
+def _check_rows(packed, bits, scale, mn, N, F):
+    """Raises for arguments of unpack_rows_mixed that do not fit together, with what is wrong; -> the widths' sum
+    and prefix."""
     g.check_typed(packed, "data", torch.int32, 1)
     g.check_typed(bits, "bits", torch.int32, 1)
     g.check_float(scale, "scale", 3)
@@ -152,30 +147,15 @@ def unpack_rows_mixed(packed, bits, scale, mn, N, F, dtype):
     total, prefix = _bits_info(bits)
     if packed.numel() < total * G * 8:
         raise RuntimeError("unpack_mixed_precision: packed stream is too short")
-    out = torch.empty(N, F, dtype=dtype, device=packed.device)
-    with g.on_device(packed.device):
-        check(g.lib().actnn_unpack_mixed_rows(
-            packed.data_ptr(), bits.data_ptr(), prefix.data_ptr(), scale.data_ptr(), mn.data_ptr(), out.data_ptr(),
-            N, F, g.DTYPE_CODE[dtype], g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)),
-            "unpack_mixed_precision")
-    return out
+    return total, prefix
 
 
 def unpack_rows_mixed_transposed(packed, bits, scale, mn, N, F):
     """The [N, F] rows of quantize_activation_device in the 16-bit dtype of `scale` turned over, their samples
     contiguous: [F, N rounded up to 64], zero behind sample N."""
-    g.check_typed(packed, "data", torch.int32, 1)
-    g.check_typed(bits, "bits", torch.int32, 1)
-    g.check_float(scale, "scale", 3)
-    g.check_float(mn, "min", 3)
-    G = (F + 255) // 256
-    if mn.dtype != scale.dtype or scale.element_size() != 2:
+    _, prefix = _check_rows(packed, bits, scale, mn, N, F)
+    if scale.element_size() != 2:
         raise RuntimeError("The type of min is not correct!")
-    if scale.numel() != N * G or mn.numel() != N * G or bits.numel() != N:
-        raise RuntimeError("unpack_mixed_precision: shape mismatch")
-    total, prefix = _bits_info(bits)
-    if packed.numel() < total * G * 8:
-        raise RuntimeError("unpack_mixed_precision: packed stream is too short")
     ld = (N + 63) // 64 * 64
     out = torch.empty(F, ld, dtype=scale.dtype, device=packed.device)
     with g.on_device(packed.device):
@@ -281,48 +261,27 @@ def quantize_rows_fixed(rows, bits, known_minmax, store_dtype):
     """Contiguous [N, F] -> (packed, scale, mn), scale and mn [N, G, 1] in `store_dtype` (the rows' dtype, or
     bfloat16 for fp32 rows): group_min_max and pack_single_precision of the zero-padded rows, and the
     compact storage, from one read of the rows.  `known_minmax`: (mn, mx) [N * G] of whole groups."""
-    N, F = rows.shape
-    G = (F + 255) // 256
-    dev = rows.device
-    packed = torch.empty(single_packed_bytes(N, G, 256, bits), dtype=torch.int8, device=dev)
-    scale = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
-    mn_ptr = mx_ptr = None
-    if known_minmax is None:
-        mn = torch.empty(N, G, 1, dtype=store_dtype, device=dev)
-    else:
+    mn, mx = known_minmax if known_minmax is not None else (None, None)
+    if known_minmax is not None:
         rows = g.aligned(rows)
-        known_mn, known_mx = known_minmax
-        mn_ptr, mx_ptr = known_mn.data_ptr(), known_mx.data_ptr()
-        mn = known_mn.view(N, G, 1) if store_dtype == known_mn.dtype \
-            else torch.empty(N, G, 1, dtype=store_dtype, device=dev)
-    seed, offset = g.philox_args(dev)
-    with g.on_device(dev):
-        check(g.lib().actnn_quantize_fixed(
-            rows.data_ptr(), mn_ptr, mx_ptr, bits, scale.data_ptr(),
-            None if mn_ptr is not None and mn.data_ptr() == mn_ptr else mn.data_ptr(), packed.data_ptr(), seed, offset,
-            N, F, g.DTYPE_CODE[rows.dtype], g.DTYPE_CODE[store_dtype], g.stream_ptr(dev)), "quantize_fixed")
-    return packed, scale, mn
+    return g.host().quantize_rows_fixed(rows, bits, mn, mx, g.DTYPE_CODE[store_dtype])
 
 
 def unpack_rows_fixed(packed, bits, scale, mn, N, F, dtype):
     """Inverse of quantize_rows_fixed: [N, F] of `dtype`, nothing materialised for the padding."""
-    g.check_typed(packed, "data", torch.int8, 1)
-    g.check_float(scale, "scale", 3)
-    g.check_float(mn, "min", 3)
-    if 8 % bits != 0:
-        raise RuntimeError("unpack_single_precision: 8 % bits must be 0")          # .cu:375
-    if mn.dtype != scale.dtype:
-        raise RuntimeError("The type of min is not correct!")
-    G = (F + 255) // 256
-    if scale.numel() != N * G or mn.numel() != N * G:
-        raise RuntimeError("unpack_single_precision: shape mismatch")
-    if packed.numel() < single_packed_bytes(N, G, 256, bits) - 1:
+    out = g.host().unpack_rows_fixed(packed, bits, scale, mn, N, F, g.DTYPE_CODE[dtype])
+    if out is None:                                    # something does not fit: say what
+        g.check_typed(packed, "data", torch.int8, 1)
+        g.check_float(scale, "scale", 3)
+        g.check_float(mn, "min", 3)
+        if 8 % bits != 0:
+            raise RuntimeError("unpack_single_precision: 8 % bits must be 0")      # .cu:375
+        if mn.dtype != scale.dtype:
+            raise RuntimeError("The type of min is not correct!")
+        G = (F + 255) // 256
+        if scale.numel() != N * G or mn.numel() != N * G:
+            raise RuntimeError("unpack_single_precision: shape mismatch")
         raise RuntimeError("unpack_single_precision: packed stream is too short")
-    out = torch.empty(N, F, dtype=dtype, device=packed.device)
-    with g.on_device(packed.device):
-        check(g.lib().actnn_unpack_single_rows(
-            packed.data_ptr(), bits, scale.data_ptr(), mn.data_ptr(), out.data_ptr(), N, F, g.DTYPE_CODE[dtype],
-            g.DTYPE_CODE[scale.dtype], g.stream_ptr(packed.device)), "unpack_single_precision")
     return out
 
 
@@ -398,14 +357,7 @@ def mask_words(n):
 
 
 def relu_forward(x):
-    x = g.aligned(x)
-    n = x.numel()
-    y = torch.empty_like(x)
-    mask = torch.empty(mask_words(n), dtype=torch.int32, device=x.device)
-    with g.on_device(x.device):
-        check(g.lib().actnn_relu_forward(x.data_ptr(), y.data_ptr(), mask.data_ptr(), n,
-                                         g.DTYPE_CODE[x.dtype], g.stream_ptr(x.device)), "relu_forward")
-    return y, mask
+    return g.host().relu_forward(x)
 
 
 def relu_forward_minmax(x):
@@ -429,13 +381,7 @@ def relu_minmax_applies(x):
 
 
 def relu_backward(grad_output, mask):
-    grad_output = g.aligned(grad_output.contiguous())
-    gin = torch.empty_like(grad_output)
-    with g.on_device(gin.device):
-        check(g.lib().actnn_relu_backward(grad_output.data_ptr(), mask.data_ptr(), gin.data_ptr(),
-                                          gin.numel(), g.DTYPE_CODE[gin.dtype],
-                                          g.stream_ptr(gin.device)), "relu_backward")
-    return gin
+    return g.host().relu_backward(grad_output, mask)
 
 
 def relu_backward_add(grad_output, mask, other):
@@ -553,26 +499,11 @@ def act_quantized_relu(input):
 
 
 def dropout_forward(x, p):
-    x = g.aligned(x)
-    n = x.numel()
-    y = torch.empty_like(x)
-    mask = torch.empty(mask_words(n), dtype=torch.int32, device=x.device)
-    seed, offset = g.philox_args(x.device)
-    with g.on_device(x.device):
-        check(g.lib().actnn_dropout_forward(x.data_ptr(), y.data_ptr(), mask.data_ptr(), n, float(p),
-                                            seed, offset, g.DTYPE_CODE[x.dtype],
-                                            g.stream_ptr(x.device)), "dropout_forward")
-    return y, mask
+    return g.host().dropout_forward(x, p)
 
 
 def dropout_backward(grad_output, mask, p):
-    grad_output = g.aligned(grad_output.contiguous())
-    gin = torch.empty_like(grad_output)
-    with g.on_device(gin.device):
-        check(g.lib().actnn_dropout_backward(grad_output.data_ptr(), mask.data_ptr(), gin.data_ptr(),
-                                             gin.numel(), float(p), g.DTYPE_CODE[gin.dtype],
-                                             g.stream_ptr(gin.device)), "dropout_backward")
-    return gin
+    return g.host().dropout_backward(grad_output, mask, p)
 
 
 class ActQuantizedDropout(Function):
@@ -616,27 +547,10 @@ def max_pool2d_forward(x, kernel_size, stride, padding, dilation, nibble_indices
     """-> (y, idx) in the memory format of x (default or channels-last).  idx: int8 of y's shape as in
     the reference, or with nibble_indices a flat uint8 tensor holding two indices per byte
     ((y.numel() + 1) // 2 bytes, in the order of y's memory)."""
-    N, C, H, W = x.shape
-    KH, KW = kernel_size
-    Ho = (H + 2 * padding[0] - dilation[0] * (KH - 1) - 1) // stride[0] + 1       # .cu:679
-    Wo = (W + 2 * padding[1] - dilation[1] * (KW - 1) - 1) // stride[1] + 1       # .cu:680
     channels_last = pool_takes_channels_last(x)
-    fmt = torch.channels_last if channels_last else torch.contiguous_format
     if not channels_last:
         x = x.contiguous()
-    y = torch.empty((N, C, Ho, Wo), dtype=x.dtype, device=x.device, memory_format=fmt)
-    if nibble_indices:
-        idx = torch.empty(((N * C * Ho * Wo + 1) // 2,), dtype=torch.uint8, device=x.device)
-        fn = g.lib().actnn_max_pool2d_forward_cl_nibble if channels_last else g.lib().actnn_max_pool2d_forward_nibble
-    else:
-        idx = torch.empty((N, C, Ho, Wo), dtype=torch.int8, device=x.device, memory_format=fmt)
-        fn = g.lib().actnn_max_pool2d_forward_cl if channels_last else g.lib().actnn_max_pool2d_forward
-    with g.on_device(x.device):
-        check(fn(
-            x.data_ptr(), y.data_ptr(), idx.data_ptr(), N, C, H, W, Ho, Wo, KH, KW, stride[0],
-            stride[1], padding[0], padding[1], g.DTYPE_CODE[x.dtype], g.stream_ptr(x.device)),
-            "max_pool2d_forward")
-    return y, idx
+    return g.host().max_pool2d_forward(x, channels_last, *kernel_size, *stride, *padding, *dilation, nibble_indices)
 
 
 def max_pool2d_backward(grad_output, idx, input_shape, kernel_size, stride, padding, channels_last=None):
@@ -651,21 +565,10 @@ def max_pool2d_backward(grad_output, idx, input_shape, kernel_size, stride, padd
         channels_last = channels_last_format(idx) is not None
     fmt = torch.channels_last if channels_last else torch.contiguous_format
     grad_output = grad_output.contiguous(memory_format=fmt)
-    N, C, H, W = input_shape
-    Ho, Wo = grad_output.shape[2], grad_output.shape[3]
-    gin = torch.empty((N, C, H, W), dtype=grad_output.dtype, device=grad_output.device, memory_format=fmt)
-    if nibble_indices:
-        if idx.numel() != (grad_output.numel() + 1) // 2:
-            raise RuntimeError("max_pool2d_backward: the index tensor does not match grad_output")
-        fn = g.lib().actnn_max_pool2d_backward_cl_nibble if channels_last else g.lib().actnn_max_pool2d_backward_nibble
-    else:
-        fn = g.lib().actnn_max_pool2d_backward_cl if channels_last else g.lib().actnn_max_pool2d_backward
-    with g.on_device(gin.device):
-        check(fn(
-            grad_output.data_ptr(), idx.data_ptr(), gin.data_ptr(), N, C, H, W, Ho, Wo,
-            kernel_size[0], kernel_size[1], stride[0], stride[1], padding[0], padding[1],
-            g.DTYPE_CODE[gin.dtype], g.stream_ptr(gin.device)), "max_pool2d_backward")
-    return gin
+    if nibble_indices and idx.numel() != (grad_output.numel() + 1) // 2:
+        raise RuntimeError("max_pool2d_backward: the index tensor does not match grad_output")
+    return g.host().max_pool2d_backward(grad_output, idx, channels_last, nibble_indices, *input_shape, *kernel_size, *stride,
+                                        *padding)
 
 
 class ActQuantizedMaxPool2d(Function):
