@@ -297,17 +297,17 @@ struct PackSink {
   const void* relu_add;
 };
 
-// ReLU on a word of two 16-bit values (already rounded to T, so the rule sees what a separate pass
-// over the stored tensor would see): -> the word with the non-positive halves zeroed; their keep
-// flags in bits 0 and 1 of `keep`; the two results as floats.
-template <typename T> ACTNN_DEV uint32_t relu_word(uint32_t w, uint32_t& keep, float& z0, float& z1) {
-  float v[2];
-  Chunk<T>::widen(w, v);
-  const bool k0 = v[0] > 0.0f, k1 = v[1] > 0.0f;
-  z0 = k0 ? v[0] : 0.0f;
-  z1 = k1 ? v[1] : 0.0f;
-  keep = (k0 ? 1u : 0u) | (k1 ? 2u : 0u);
-  return (k0 ? w & 0x0000ffffu : 0u) | (k1 ? w & 0xffff0000u : 0u);
+// ReLU on a word of two 16-bit values (already rounded to T, so the rule sees what a separate pass over the stored
+// tensor would see): all ones in the halves that hold a value above zero.  As integers those are 1 ... the pattern of
+// infinity: zeros, negative values and NaNs lie outside (the subtractions saturate).
+typedef short s16x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+template <typename T> ACTNN_DEV uint32_t positive_halves(uint32_t w) {
+  constexpr short kNan = __is_same(T, __half) ? 0x7c01 : 0x7f81;
+  const s16x2_t v = __builtin_bit_cast(s16x2_t, w);
+  const s16x2_t below = __builtin_elementwise_sub_sat((s16x2_t){0, 0}, v);
+  const s16x2_t finite = __builtin_elementwise_sub_sat(v, (s16x2_t){kNan, kNan});
+  return __builtin_bit_cast(uint32_t, (s16x2_t)((below & finite) >> 15));
 }
 // The other direction: a backward pass whose incoming gradient is that of a ReLU's output takes the
 // ReLU's mask along and zeroes what the ReLU's own backward pass would have zeroed, instead of reading
@@ -470,26 +470,34 @@ ACTNN_DEV void pack_chunk_pair_f32(const PackSink& ps, const u32x4& xa, const Ch
   }
 }
 
+// A uniform value the compiler works with anew in every turn of a loop.
+ACTNN_DEV uint64_t unhoisted(uint64_t v) {
+  uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  asm volatile("" : "+s"(lo), "+s"(hi));
+  return ((uint64_t)hi << 32) | lo;
+}
+
 // Noise words of two octets of this lane whose neighbours (index ^ 1) lane ^ 1 holds: the two lanes
 // share their Philox calls when octet and lane parity agree (they do wherever a block starts on an
 // even octet; the test is the same for every lane of a block).
 template <typename T>
 ACTNN_DEV void noise_pair(const PackSink& ps, uint64_t oa, uint64_t ob, uint32_t (&wa)[Noise<T>::kWords],
                           uint32_t (&wb)[Noise<T>::kWords], bool together) {
+  const uint64_t seed = unhoisted(ps.seed);
   // together: lane ^ 1 is known to make this call in the same step
   if (together && (((uint32_t)oa ^ threadIdx.x) & 1u) == 0 && (((uint32_t)ob ^ threadIdx.x) & 1u) == 0) {
-    Noise<T>::octets(oa, ob, ps.seed, ps.offset, wa, wb);
+    Noise<T>::octets(oa, ob, seed, ps.offset, wa, wb);
   } else {
-    Noise<T>::octet(oa, ps.seed, ps.offset, wa);
-    Noise<T>::octet(ob, ps.seed, ps.offset, wb);
+    Noise<T>::octet(oa, seed, ps.offset, wa);
+    Noise<T>::octet(ob, seed, ps.offset, wb);
   }
 }
 
 // b: the sample's width, dst: first word of the chunk's group in the stream (both looked up by the
 // caller, who knows how often the sample changes); (mul, sub): the group's parameters from the queue;
 // rw: the noise words of the chunk's octet.  SCALAR_B: b is known to be one number for the wave (the
-// sample comes from the block's index); otherwise the wave checks, and takes one scalar branch when
-// its lanes agree - as they do except where a wave spans two samples of different widths.
+// sample comes from the block's index); otherwise the wave takes a scalar branch for the width of its first lane,
+// and another turn where it spans two samples of different widths (the lanes of a group always agree).
 template <typename T>
 ACTNN_DEV void pack_chunk_width(const float (&v)[8], const uint32_t (&rw)[Noise<T>::kWords], float mul, float sub,
                                 uint32_t lane32, int32_t* __restrict__ dst, int b) {
@@ -518,9 +526,13 @@ ACTNN_DEV void pack_chunk(const u32x4& ux, const uint32_t (&rw)[Noise<T>::kWords
   if constexpr (SCALAR_B) {
     pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b);
   } else {
-    const int b0 = __builtin_amdgcn_readfirstlane(b);
-    if (__builtin_amdgcn_ballot_w64(b != b0) == 0) pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b0);
-    else pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b);
+    for (bool done = false; !done;) {
+      const int b0 = __builtin_amdgcn_readfirstlane(b);
+      if (b == b0) {
+        pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b0);
+        done = true;
+      }
+    }
   }
 }
 
@@ -1317,49 +1329,54 @@ __global__ __launch_bounds__(kThreads, (RELU ? 4 : 1)) void bn_cl_apply_kernel(
     // in rows of a multiple of 512 channels, the same half of two blocks (mask_place), and a half-wave's
     // 32 chunks one group of 256 outputs (the launcher takes this path only when that holds and every
     // step of a block is whole).  emit() applies the rule to the normalised chunk,
-    // stores it, leaves the group's min / max and the lane's 8 keep bits in `row`; four steps' rows
+    // stores it, leaves the group's min / max and returns the lane's 8 keep bits; four steps' rows
     // make the wave's 64 mask words (blocks 4 apart: a step of the block is 2048 elements).
     const uint32_t lane = threadIdx.x & 63u;
-    auto emit = [&](int64_t ru, const u32x4& y, uint32_t& row, const u32x4& res) __attribute__((always_inline)) {
-      if constexpr (RELU != 0) {
-        uint32_t w[4] = {y.x, y.y, y.z, y.w};
-        if constexpr (RELU == 2) {
-          // bn(x), rounded to T as its store would round it, plus the residual, rounded as the tensor
-          // addition rounds it
-          const uint32_t a[4] = {res.x, res.y, res.z, res.w};
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float u[2], v[2];
-            Chunk<T>::widen(w[k], u);
-            Chunk<T>::widen(a[k], v);
-            u[0] += v[0];
-            u[1] += v[1];
-            w[k] = Chunk<T>::narrow(u);
-          }
-        }
-        float z[8];
-        row = 0;
+    auto emit = [&](int64_t ru, const u32x4& y, const u32x4& res) __attribute__((always_inline)) -> uint32_t {
+      uint32_t w[4] = {y.x, y.y, y.z, y.w};
+      if constexpr (RELU == 2) {
+        // bn(x), rounded to T as its store would round it, plus the residual, rounded as the tensor
+        // addition rounds it
+        const uint32_t a[4] = {res.x, res.y, res.z, res.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          uint32_t keep;
-          w[k] = relu_word<T>(w[k], keep, z[2 * k], z[2 * k + 1]);
-          row |= keep << (2 * k);
+          float u[2], v[2];
+          Chunk<T>::widen(w[k], u);
+          Chunk<T>::widen(a[k], v);
+          u[0] += v[0];
+          u[1] += v[1];
+          w[k] = Chunk<T>::narrow(u);
         }
-        store_out(out_at(ru), u32x4{w[0], w[1], w[2], w[3]});
-        float lo, hi;
-        minmax_of<8>(z, lo, hi);
-        lanes_minmax<2>(lo, hi);
-        if ((lane & 31u) == 31u) {
-          const uint32_t g = (uint32_t)((ru * C) >> 8) + (lane_elems >> 8);
-          Conv<T>::store(static_cast<T*>(ps.relu_mn), g, lo);
-          Conv<T>::store(static_cast<T*>(ps.relu_mx), g, hi);
-        }
-      } else {
-        store_out(out_at(ru), y);
       }
+      uint32_t row = 0;                                // element 2k's flag in bit 2k, that of 2k + 1 in bit 16 + 2k + 1
+      u16x2_t least, most;                             // (what is left is not negative: ordered as its patterns are)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t keep = positive_halves<T>(w[k]);
+        w[k] &= keep;
+        row |= keep & (0x20001u << (2 * k));
+        const u16x2_t z = __builtin_bit_cast(u16x2_t, w[k]);
+        least = k ? __builtin_elementwise_min(least, z) : z;
+        most = k ? __builtin_elementwise_max(most, z) : z;
+      }
+      row = (row | (row >> 16)) & 0xffu;
+      store_out(out_at(ru), u32x4{w[0], w[1], w[2], w[3]});
+      float v[2];
+      Chunk<T>::widen(__builtin_bit_cast(uint32_t, least), v);
+      float lo = min_f32(v[0], v[1]);
+      Chunk<T>::widen(__builtin_bit_cast(uint32_t, most), v);
+      float hi = max_f32(v[0], v[1]);
+      lanes_minmax<2>(lo, hi);
+      if ((lane & 31u) == 31u) {
+        const uint32_t g = (uint32_t)((ru * C) >> 8) + (lane_elems >> 8);
+        Conv<T>::store(static_cast<T*>(ps.relu_mn), g, lo);
+        Conv<T>::store(static_cast<T*>(ps.relu_mx), g, hi);
+      }
+      return row;
     };
-    auto leave_mask = [&](int64_t ru_first, const uint32_t (&rows)[4], int count) __attribute__((always_inline)) {
-      const uint32_t word = rows_to_word(rows, lane);
+    // the rows of four steps (two per word), of which `count` exist
+    auto leave_mask = [&](int64_t ru_first, uint32_t rows01, uint32_t rows23, int count) __attribute__((always_inline)) {
+      const uint32_t word = row_pairs_to_word(rows01, rows23, lane);
       const int slot = 2 * (int)(lane & 1u) + (int)(lane >> 5);
       const MaskPlace at = mask_place(ru_first, C, R, blockIdx.x);
       if (slot < count) {
@@ -1378,29 +1395,6 @@ __global__ __launch_bounds__(kThreads, (RELU ? 4 : 1)) void bn_cl_apply_kernel(
       else
         return u32x4{0u, 0u, 0u, 0u};
     };
-    auto pair = [&](int64_t rb0, int j, uint32_t& row0, uint32_t& row1) __attribute__((always_inline)) {
-      const int64_t ru0 = rb0 + (int64_t)j * R, ru1 = ru0 + R;
-      const typename XS::Raw rx0 = xs.fetch(ru0), rx1 = xs.fetch(ru1);
-      const u32x4 res0 = res_at(ru0), res1 = res_at(ru1);
-      uint32_t rw[2][Noise<T>::kWords];
-      noise_pair<T>(ps, (uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), (uint64_t)((ru1 * C) >> 3) + (lane_elems >> 3),
-                    rw[0], rw[1], (tpr & 1) == 0);      // lane ^ 1 is in the same row, hence in the same steps
-      const u32x4 ux0 = xs.decode(rx0);
-      emit(ru0, apply(ux0, ux0), row0, res0);
-      pack_one(ux0, rw[0], ru0, j);
-      const u32x4 ux1 = xs.decode(rx1);
-      emit(ru1, apply(ux1, ux1), row1, res1);
-      pack_one(ux1, rw[1], ru1, j + 1);
-    };
-    auto single = [&](int64_t rb0, int j, uint32_t& row) __attribute__((always_inline)) {
-      const int64_t ru0 = rb0 + (int64_t)j * R;
-      const u32x4 res = res_at(ru0);
-      const u32x4 ux = xs.decode(xs.fetch(ru0));
-      emit(ru0, apply(ux, ux), row, res);
-      uint32_t rw[Noise<T>::kWords];
-      Noise<T>::octet((uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), ps.seed, ps.offset, rw);
-      pack_one(ux, rw, ru0, j);
-    };
     for (int64_t rb0 = p0; rb0 + t.r < p1; rb0 += (int64_t)32 * R) {
       const int64_t rb = rb0 + t.r;
       {
@@ -1411,40 +1405,63 @@ __global__ __launch_bounds__(kThreads, (RELU ? 4 : 1)) void bn_cl_apply_kernel(
       }
       int j = 0;
       if constexpr (RELU != 0) {
-        uint32_t rows[4] = {0u, 0u, 0u, 0u};
-        for (; j + 4 <= 32 && rb + (int64_t)(j + 3) * R < p1; j += 4) {
-          pair(rb0, j, rows[0], rows[1]);
-          pair(rb0, j + 2, rows[2], rows[3]);
-          leave_mask(rb0 + (int64_t)j * R, rows, 4);
+        // One copy of a step's code, gone through twice for the two rows whose noise is made together: eight widths
+        // make it long, and with a copy for each step of four, others for the rows left over, and every one of them
+        // twice (for waves of one width and of several) the kernel had 17000 instructions and too few scalar
+        // registers: a thousand moves spilled them in the middle of the steps (1400 and none now).  Bound by vector
+        // instructions and HBM alike.  Forward of the layer, us, before / now: bf16 [256, 512, 28, 28] with ReLU
+        // 159.9 / 132.8, with the residual 181.2 / 169.2; [256, 64, 56, 56] 94.7 / 79.5 and 110.0 / 96.1.  Two copies, for the
+        // two rows: 132.5 in place of 128.0 for the kernel alone; loads a step ahead 133.8; five waves per SIMD 134.8.
+        uint32_t before = 0;                           // the rows of the two steps before
+#pragma unroll 1
+        for (; j < 32 && rb0 + (int64_t)j * R < p1; j += 2) {
+          int64_t ru = rb0 + (int64_t)j * R;
+          const bool two = j + 1 < 32 && ru + R < p1;
+          const int64_t next = two ? ru + R : ru;
+          u32x4 ux = xs.decode(xs.fetch(ru)), res = res_at(ru);
+          const u32x4 ux1 = xs.decode(xs.fetch(next)), res1 = res_at(next);
+          // (a chunk's octet has the lane's parity here, and lane ^ 1 holds its partner in the same step)
+          uint32_t rw[Noise<T>::kWords], rw1[Noise<T>::kWords];
+          const uint64_t octet = (uint64_t)((ru * C) >> 3) + (lane_elems >> 3);
+          Noise<T>::octets(octet, octet + (uint64_t)(((next - ru) * C) >> 3), unhoisted(ps.seed), ps.offset, rw, rw1);
+          uint32_t rows = 0;
+#pragma unroll 1
+          for (int h = 0;; ++h) {
+            rows |= emit(ru, apply(ux, ux), res) << (16 * h);
+            pack_one(ux, rw, ru, j + h);
+            if (h == (int)two) break;
+            ux = ux1;
+            res = res1;
+            ru = next;
+#pragma unroll
+            for (int k = 0; k < Noise<T>::kWords; ++k) rw[k] = rw1[k];
+          }
+          const bool last = j + 2 >= 32 || rb0 + (int64_t)(j + 2) * R >= p1;
+          if (j & 2) leave_mask(rb0 + (int64_t)(j - 2) * R, before, rows, two ? 4 : 3);
+          else if (last) leave_mask(rb0 + (int64_t)j * R, rows, 0u, two ? 2 : 1);
+          before = rows;
         }
-        // what is left of the block's rows: up to three steps
-        const int64_t ru_first = rb0 + (int64_t)j * R;
-        int left = 0;
-        if (j < 32 && rb + (int64_t)j * R < p1) { single(rb0, j, rows[0]); ++j; ++left; }
-        if (j < 32 && rb + (int64_t)j * R < p1) { single(rb0, j, rows[1]); ++j; ++left; }
-        if (j < 32 && rb + (int64_t)j * R < p1) { single(rb0, j, rows[2]); ++j; ++left; }
-        if (left) leave_mask(ru_first, rows, left);
       } else {
-        for (; j + 2 <= 32 && rb + (int64_t)(j + 1) * R < p1; j += 2) {
-          const int64_t ru0 = rb0 + (int64_t)j * R, ru1 = ru0 + R;
-          const typename XS::Raw rx0 = xs.fetch(ru0), rx1 = xs.fetch(ru1);
-          uint32_t rw[2][Noise<T>::kWords];
-          noise_pair<T>(ps, (uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), (uint64_t)((ru1 * C) >> 3) + (lane_elems >> 3),
-                        rw[0], rw[1], (tpr & 1) == 0);      // lane ^ 1 is in the same row, hence in the same steps
-          const u32x4 ux0 = xs.decode(rx0);
-          store_out(out_at(ru0), apply(ux0, ux0));
-          pack_one(ux0, rw[0], ru0, j);
-          const u32x4 ux1 = xs.decode(rx1);
-          store_out(out_at(ru1), apply(ux1, ux1));
-          pack_one(ux1, rw[1], ru1, j + 1);
-        }
-        for (; j < 32 && rb + (int64_t)j * R < p1; ++j) {
-          const int64_t ru0 = rb0 + (int64_t)j * R;
-          const u32x4 ux = xs.decode(xs.fetch(ru0));
-          store_out(out_at(ru0), apply(ux, ux));
-          uint32_t rw[Noise<T>::kWords];
-          Noise<T>::octet((uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), ps.seed, ps.offset, rw);
-          pack_one(ux, rw, ru0, j);
+        // (as above; the rows of a step need not be there for every lane, but for all lanes of a group)
+#pragma unroll 1
+        for (; j < 32 && rb + (int64_t)j * R < p1; j += 2) {
+          int64_t ru = rb0 + (int64_t)j * R;
+          const bool two = j + 1 < 32 && rb + (int64_t)(j + 1) * R < p1;
+          u32x4 ux = xs.decode(xs.fetch(ru)), ux1 = ux;
+          if (two) ux1 = xs.decode(xs.fetch(ru + R));
+          uint32_t rw[Noise<T>::kWords], rw1[Noise<T>::kWords];
+          noise_pair<T>(ps, (uint64_t)((ru * C) >> 3) + (lane_elems >> 3), (uint64_t)(((ru + R) * C) >> 3) + (lane_elems >> 3),
+                        rw, rw1, (tpr & 1) == 0);      // lane ^ 1 is in the same row, hence in the same steps
+#pragma unroll 1
+          for (int h = 0;; ++h) {
+            store_out(out_at(ru), apply(ux, ux));
+            pack_one(ux, rw, ru, j + h);
+            if (h == 1 || !two) break;
+            ux = ux1;
+            ru += R;
+#pragma unroll
+            for (int k = 0; k < Noise<T>::kWords; ++k) rw[k] = rw1[k];
+          }
         }
       }
     }
@@ -1691,35 +1708,15 @@ int launch_cl_reduce(const Plan& pl, const XS& xs, const void* dy, float* part, 
       pl.tiles, rows.nsplit, relu);
   return rows.nsplit;
 }
-// Rows per block of the closing step's forward pass, relu(bn(x) + residual) with the packed copy, which streams
-// 3.7 times the bytes of its input and holds four waves per SIMD, i.e. 1024 blocks.  A block costs its steps and
-// about three more (coefficients, the group parameters of its steps), and a last round that is nearly empty costs
-// as much as a full one: of 8, 12, 16 and 20 steps the one with the least rounds * (steps + 3).  Forward of the
-// layer, bf16 [n, 512, 28, 28], us with the plan's 8 steps / with these: n = 256 195.2 / 183.1 (20), 370
-// 278.2 / 266.6 (12), 215 169.3 / 164.3 (16), 160 135.4 / 129.5 (16), 100 97.9 / 94.4 (20);
-// [128, 256, 56, 56] 188.9 / 178.4 (20); [256, 64, 56, 56] 112.6 / 113.6 (16).  Below two rounds and a quarter the plan's
-// blocks stay (bf16 [256, 16, 64, 64]: 54.9 with 8 steps, 57.7 with 16): just above two the choice is one round of 20 steps
-// that leaves up to a fifth of the slots empty (f16 n = 84 90.7 / 94.8, 92 93.4 / 95.8, but 96 98.7 / 96.2; bf16
-// 93.3 / 96.1, 94.1 / 94.5, 98.7 / 94.6).  The passes without the residual have less to
-// stream and gain nothing ([256, 64, 56, 56] bn + ReLU 97.7 with 8 steps, 99.7 with 16; bn alone 72.5, 76.1).
-int64_t closing_rows(const Plan& pl) {
-  constexpr int64_t slots = (int64_t)kCUs * 4;
-  if ((int64_t)pl.tiles * pl.nsplit_apply < 2 * slots + slots / 4) return pl.ppb_apply;
-  int64_t best = pl.ppb_apply, least = INT64_MAX;
-  for (int steps = 8; steps <= 20; steps += 4) {
-    const int64_t rows = (int64_t)steps * pl.R, blocks = (pl.P + rows - 1) / rows * pl.tiles;
-    const int64_t cost = (blocks + slots - 1) / slots * (steps + 3);
-    if (rows >= pl.ppb_apply && cost < least) { least = cost; best = rows; }
-  }
-  return best;
-}
+// (The plan's rows per block for every kind of pass: with the residual's stream longer blocks lose as well.  Forward of
+// relu(bn(x) + residual), bf16 [256, 512, 28, 28], with 8 (the plan's), 12, 16, 20, 24 steps a block 169.2, 170.9, 172.9, 172.3, 180.3 us;
+// [370, 512, 28, 28] 247.8, 252.9, 255.6, 262.1, 260.0; [256, 64, 56, 56] 96.1, 99.3, 99.7, 105.0, 110.1.)
 template <typename T, bool BWD, bool PACK, typename XS, int RELU = 0>
 void launch_cl_apply(const Plan& pl, const XS& xs, const void* dy, const float* coef, void* out, int64_t C,
                      const PackSink& ps, hipStream_t s, const ReluRows& relu = ReluRows{}) {
-  const int64_t rows = RELU == 2 ? closing_rows(pl) : pl.ppb_apply;
-  const dim3 grid((unsigned)pl.tiles, (unsigned)((pl.P + rows - 1) / rows)), blk(kThreads);
+  const dim3 grid((unsigned)pl.tiles, (unsigned)pl.nsplit_apply), blk(kThreads);
   bn_cl_apply_kernel<T, BWD, PACK, XS, RELU><<<grid, blk, 0, s>>>(
-      xs, static_cast<const T*>(dy), coef, static_cast<T*>(out), pl.P, C, pl.tpr, pl.R, rows, ps,
+      xs, static_cast<const T*>(dy), coef, static_cast<T*>(out), pl.P, C, pl.tpr, pl.R, pl.ppb_apply, ps,
       FastDiv((uint32_t)(pl.F / C)), relu);
 }
 

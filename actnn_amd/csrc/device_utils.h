@@ -559,13 +559,15 @@ ACTNN_DEV Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t 
 // lanes hold the rows of blocks A|B and the odd lanes those of C|D, and two interleaved 32x32 bit
 // transposes turn rows into words or back.
 // rows (per lane: 8 keep bits for each of the 4 blocks) -> this lane's mask word
-ACTNN_DEV uint32_t rows_to_word(const uint32_t (&m)[4], uint32_t lane) {
+ACTNN_DEV uint32_t row_pairs_to_word(uint32_t ab, uint32_t cd, uint32_t lane) {
   const bool odd = lane & 1u;
-  const uint32_t ab = m[0] | (m[1] << 16), cd = m[2] | (m[3] << 16);
   const uint32_t recv = lane_xor<1>(odd ? ab : cd);           // the half-row the partner computed for me
   const uint32_t mine = odd ? cd : ab;
   const uint32_t row = odd ? (recv | (mine << 8)) : (mine | (recv << 8));
   return transpose32_x2(row, lane);
+}
+ACTNN_DEV uint32_t rows_to_word(const uint32_t (&m)[4], uint32_t lane) {
+  return row_pairs_to_word(m[0] | (m[1] << 16), m[2] | (m[3] << 16), lane);
 }
 // inverse: this lane's mask word -> 8 keep bits for each of the 4 blocks
 ACTNN_DEV void word_to_rows(uint32_t w, uint32_t lane, uint32_t (&m)[4]) {

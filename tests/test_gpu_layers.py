@@ -1204,8 +1204,8 @@ def test_closing_step_of_a_residual_block_in_the_batch_norm_pass(dtype, channels
 
 @pytest.mark.parametrize("n", [200, 201, 215, 270])
 def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
-    """Forward passes of more than two rounds of blocks choose how many rows a block takes: 20, 20, 12 and 16 steps of 8
-    rows here, the last block whole (n = 200) and ragged.  Output and saved stream are those of the batch norm, the addition and the ReLU."""
+    """Forward passes of more than two rounds of blocks, the last block whole (n = 200) and ragged.  Output and saved stream
+    are those of the batch norm, the addition and the ReLU."""
     from actnn_amd.layers import QAddReLU, QBatchNorm2d, bn_add_relu, known_group_minmax
     res = []
     for fold in (False, True):
@@ -1225,6 +1225,50 @@ def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
         res.append((out.detach(), *node.saved[0], *known_group_minmax(out)))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("channels,size,n", [(64, 2, 8), (64, 2, 16), (64, 2, 24), (64, 2, 40), (64, 6, 72), (512, 2, 2), (512, 3, 8),
+                                             (512, 3, 56), (8, 8, 4)])
+@pytest.mark.parametrize("add", [False, True])
+def test_relu_in_the_batch_norm_pass_between_samples_and_at_special_values(dtype, channels, size, n, add):
+    """The folded ReLU where a wave's lanes hold samples of different widths and a block has one to three steps left over, on
+    zeros of both signs, infinities, NaNs and the smallest values (in the residual, or made by the batch norm): output,
+    mask, group ranges and saved stream are those of the separate layers."""
+    from actnn_amd.layers import QAddReLU, QBatchNorm2d, QReLU, bn_add_relu, bn_relu, known_group_minmax
+    res = []
+    for fold in (False, True):
+        config.reset(); QScheme.reset(); QBNScheme.reset()
+        config.fused_bn_relu = fold
+        torch.manual_seed(4)
+        bn = QBatchNorm2d(channels).to(DEV).train()
+        with torch.no_grad():
+            bn.weight[::4] = 0.0                               # constant channels: zeros, tiny and huge values
+            bn.bias[0::8], bn.bias[4::8] = -0.0, 1e-7
+            bn.bias[1] = float("nan")
+            bn.bias[2] = float("inf")
+        g = torch.Generator(device=DEV).manual_seed(n)
+        x = torch.randn(n, channels, size, size, device=DEV, generator=g)
+        x *= torch.exp(2 * torch.randn(n, 1, 1, 1, device=DEV, generator=g))           # widths of 1 to 8
+        x = x.to(dtype).contiguous(memory_format=torch.channels_last).requires_grad_()
+        identity = torch.randn(x.shape, device=DEV, generator=g).to(dtype)
+        special = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), 1e-7, -1e-7, 6e4], device=DEV).to(dtype)
+        identity.view(-1)[::3] = special[torch.randint(8, identity.view(-1)[::3].shape, device=DEV, generator=g)]
+        identity = identity.contiguous(memory_format=torch.channels_last).requires_grad_()
+        grad = torch.randn(x.shape, device=DEV, generator=g).to(dtype).contiguous(memory_format=torch.channels_last)
+        torch.cuda.manual_seed(22)
+        out = bn_add_relu(bn, QAddReLU(), x, identity) if add else bn_relu(bn, QReLU(), x)
+        assert (type(out.grad_fn).__name__ in ("batch_norm_add_reluBackward", "batch_norm_reluBackward")) == fold
+        known = known_group_minmax(out)
+        node = out.grad_fn
+        while not (type(getattr(node, "saved", None)) is tuple and len(node.saved) == 9):
+            node = node.next_functions[0][0]
+        saved = tuple(t.clone() for t in node.saved[0])
+        masked = torch.autograd.grad(out, identity, grad)[0] if add else torch.zeros(())
+        res.append((out.detach(), *saved, masked, *(known or ())))
+    assert not torch.isnan(res[1][0]).any()
+    for i, (a, b) in enumerate(zip(*res)):
+        assert torch.equal(a, b), i
 
 
 def test_closing_step_of_a_tensor_beyond_the_last_level_cache():
