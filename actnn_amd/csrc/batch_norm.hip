@@ -18,6 +18,7 @@
 // which saves the quantiser's own read of the tensor.
 #include <mutex>
 
+#include "bn_finalize.h"
 #include "device_utils.h"
 #include "quant_math.h"
 
@@ -617,68 +618,9 @@ __global__ __launch_bounds__(kThreads, 6) void bn_reduce_kernel(
                 SPLIT ? t0 - h0 : 0.0f, SPLIT ? t1 - h1 : 0.0f, part);
 }
 
-// Folds the table of partial sums of channel c in double precision: the wave's lanes take the
-// (span, batch split) entries of the channel in a fixed assignment and are combined by a butterfly,
-// so every lane ends with the same totals and the order of the additions is fixed.
-// (channels-last tables, slots == 0, hold nsplit consecutive values per channel and sum.)
-ACTNN_DEV void channel_totals(const float* __restrict__ part, int64_t c, int64_t HW, int64_t L,
-                              int nsplit, int slots, double& s0, double& s1) {
-  const int lane = threadIdx.x & 63;
-  s0 = 0.0;
-  s1 = 0.0;
-  if (slots == 0) {
-    const float* q0 = part + (c * 2) * (int64_t)nsplit;
-    const float* q1 = q0 + nsplit;
-#pragma unroll 8
-    for (int i = lane; i < nsplit; i += 64) {
-      s0 += (double)q0[i];
-      s1 += (double)q1[i];
-    }
-  } else {
-    const int64_t j0 = (c * HW) / L, j1 = ((c + 1) * HW - 1) / L;
-    const int64_t count = (j1 - j0 + 1) * nsplit;
-    for (int64_t i = lane; i < count; i += 64) {
-      const int64_t j = j0 + i / nsplit, y = i % nsplit;
-      const int64_t slot = c - (j * L) / HW;
-      const float* q = part + ((j * nsplit + y) * slots + slot) * 2;
-      s0 += (double)q[0];
-      s1 += (double)q[1];
-    }
-  }
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    s0 += __shfl_xor(s0, d);
-    s1 += __shfl_xor(s1, d);
-  }
-}
-
-// mean / inverse standard deviation of the batch, the running estimates (unbiased variance, as
-// torch's batch norm keeps them) and the per-channel coefficients of y = a*x + b.
-__global__ __launch_bounds__(kThreads) void bn_forward_finalize_kernel(
-    const float* __restrict__ part, const float* __restrict__ weight, const float* __restrict__ bias,
-    float* __restrict__ running_mean, float* __restrict__ running_var, float* __restrict__ save_mean,
-    float* __restrict__ save_invstd, float* __restrict__ coef, int64_t N, int64_t C, int64_t HW,
-    int64_t L, int nsplit, int slots, double momentum, double eps) {
+__global__ __launch_bounds__(kThreads) void bn_forward_finalize_kernel(BnFinalize f) {
   const int64_t c = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);     // one wave per channel
-  if (c >= C) return;
-  double S, Q;
-  channel_totals(part, c, HW, L, nsplit, slots, S, Q);
-  if ((threadIdx.x & 63) != 0) return;
-  const double M = (double)N * (double)HW;
-  const double mean = S / M;
-  double var = Q / M - mean * mean;
-  if (!(var > 0.0)) var = 0.0;
-  const double invstd = 1.0 / sqrt(var + eps);
-  save_mean[c] = (float)mean;
-  save_invstd[c] = (float)invstd;
-  if (running_mean) running_mean[c] = (float)((1.0 - momentum) * running_mean[c] + momentum * mean);
-  if (running_var) {
-    const double unbiased = M > 1.0 ? var * (M / (M - 1.0)) : var;
-    running_var[c] = (float)((1.0 - momentum) * running_var[c] + momentum * unbiased);
-  }
-  const double a = (weight ? (double)weight[c] : 1.0) * invstd;
-  coef[2 * c] = (float)a;
-  coef[2 * c + 1] = (float)((bias ? (double)bias[c] : 0.0) - mean * a);
+  if (c < f.C) bn_finalize_channel(f, c);
 }
 
 // grad_weight, grad_bias and the per-channel coefficients of dx = A*dy + B*x + K, from
@@ -1723,7 +1665,7 @@ void launch_cl_apply(const Plan& pl, const XS& xs, const void* dy, const float* 
 template <typename T>
 int forward_stats_t(const Plan& pl, const void* x, const float* weight, const float* bias, float* running_mean,
                     float* running_var, float* save_mean, float* save_invstd, void* mn, void* mx, float* ws,
-                    int64_t N, int64_t C, int64_t HW, double momentum, double eps, hipStream_t s) {
+                    int64_t N, int64_t C, int64_t HW, double momentum, double eps, BnFinalize* open, hipStream_t s) {
   float* part = ws;
   float* coef = ws + pl.part_floats;
   int nsplit = pl.nsplit;
@@ -1748,9 +1690,10 @@ int forward_stats_t(const Plan& pl, const void* x, const float* weight, const fl
     if (mn) launch_reduce<T, false, true>(pl, xs, nullptr, part, mn, mx, N, HW, s);
     else launch_reduce<T, false, false>(pl, xs, nullptr, part, nullptr, nullptr, N, HW, s);
   }
-  bn_forward_finalize_kernel<<<dim3((unsigned)((C + kWaves - 1) / kWaves)), dim3(kThreads), 0, s>>>(
-      part, weight, bias, running_mean, running_var, save_mean, save_invstd, coef, N, C, HW, pl.L, nsplit,
-      pl.slots, momentum, eps);
+  const BnFinalize fold{part, weight, bias, running_mean, running_var, save_mean, save_invstd, coef, N, C, HW, pl.L, nsplit,
+                        pl.slots, momentum, eps};
+  if (open) *open = fold;                              // (the caller launches it)
+  else bn_forward_finalize_kernel<<<dim3((unsigned)((C + kWaves - 1) / kWaves)), dim3(kThreads), 0, s>>>(fold);
   ACTNN_RETURN_LAUNCH_STATUS();
 }
 
@@ -1923,13 +1866,12 @@ extern "C" int actnn_batch_norm_groups_align(int64_t N, int64_t C, int64_t HW, i
   return pl.groups_align && !pl.any_shape ? 1 : 0;
 }
 
-extern "C" int actnn_batch_norm_forward_stats(const void* x, const float* weight, const float* bias,
-                                              float* running_mean, float* running_var, float* save_mean,
-                                              float* save_invstd, void* mn, void* mx, void* workspace,
-                                              int64_t workspace_bytes, int64_t N, int64_t C, int64_t HW,
-                                              double momentum, double eps, int dtype, int channels_last,
-                                              void* stream) {
-  using namespace actnn;
+namespace actnn {
+// actnn_batch_norm_forward_stats; with `open` the fold of the pass's sums is left to the caller.
+int batch_norm_statistics(const void* x, const float* weight, const float* bias, float* running_mean, float* running_var,
+                          float* save_mean, float* save_invstd, void* mn, void* mx, void* workspace,
+                          int64_t workspace_bytes, int64_t N, int64_t C, int64_t HW, double momentum, double eps, int dtype,
+                          int channels_last, BnFinalize* open, hipStream_t s) {
   if (dtype < 0 || dtype > 2) return ACTNN_EDTYPE;
   Plan pl;
   if (!make_plan(N, C, HW, dtype, channels_last, pl)) return ACTNN_EINVAL;
@@ -1937,13 +1879,24 @@ extern "C" int actnn_batch_norm_forward_stats(const void* x, const float* weight
   if (workspace_bytes < workspace_floats(pl, C) * (int64_t)sizeof(float)) return ACTNN_EINVAL;
   if (mn && !pl.groups_align) return ACTNN_EINVAL;
   if ((!pl.any_shape && !aligned16(x)) || !aligned16(workspace)) return ACTNN_EALIGN;
-  hipStream_t s = static_cast<hipStream_t>(stream);
   float* ws = static_cast<float*>(workspace);
   switch (dtype) {
-    case ACTNN_F32: return forward_stats_t<float>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, s);
-    case ACTNN_F16: return forward_stats_t<__half>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, s);
-    default: return forward_stats_t<bf16_t>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, s);
+    case ACTNN_F32: return forward_stats_t<float>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, open, s);
+    case ACTNN_F16: return forward_stats_t<__half>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, open, s);
+    default: return forward_stats_t<bf16_t>(pl, x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, ws, N, C, HW, momentum, eps, open, s);
   }
+}
+}  // namespace actnn
+
+extern "C" int actnn_batch_norm_forward_stats(const void* x, const float* weight, const float* bias,
+                                              float* running_mean, float* running_var, float* save_mean,
+                                              float* save_invstd, void* mn, void* mx, void* workspace,
+                                              int64_t workspace_bytes, int64_t N, int64_t C, int64_t HW,
+                                              double momentum, double eps, int dtype, int channels_last,
+                                              void* stream) {
+  return actnn::batch_norm_statistics(x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, workspace,
+                                      workspace_bytes, N, C, HW, momentum, eps, dtype, channels_last, nullptr,
+                                      static_cast<hipStream_t>(stream));
 }
 
 extern "C" int actnn_batch_norm_forward_apply(const void* x, void* y, const void* workspace,

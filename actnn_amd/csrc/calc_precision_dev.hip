@@ -16,6 +16,7 @@
 // items on, the LDS atomics of the histograms.  The candidates are walked so that the lanes of a wave
 // hold different steps of neighbouring items: the exponents of an item's steps lie two apart, so few
 // lanes of an atomic meet in one bin.
+#include "bn_finalize.h"
 #include "device_utils.h"
 
 namespace actnn {
@@ -42,13 +43,9 @@ ACTNN_DEV float finish_sensitivity(float sum, float factor, const float* mult, i
 // are loaded kAhead at a time: with one load per turn the pass was the latency of G / 256 loads in a row
 // (2 samples of 158080 groups in fp16: 171 us, 23.6 now; 3 of 21576 in bf16: 24.5 and 6.2 us).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void range_sqr_kernel(const T* __restrict__ mn,
-                                                             const T* __restrict__ mx,
-                                                             float* __restrict__ out, int64_t G,
-                                                             float factor, const float* __restrict__ mult,
-                                                             int mult_stride) {
+ACTNN_DEV void range_sqr_of_block(const T* __restrict__ mn, const T* __restrict__ mx, float* __restrict__ out, int64_t n, int64_t G,
+                                  float factor, const float* __restrict__ mult, int mult_stride) {
   __shared__ float s_part[kThreads];
-  const int64_t n = blockIdx.x;
   float acc = 0.0f;
   constexpr int kAhead = 16;
   for (int64_t g0 = threadIdx.x; g0 < G; g0 += kThreads * kAhead) {
@@ -69,6 +66,14 @@ __global__ __launch_bounds__(kThreads) void range_sqr_kernel(const T* __restrict
     __syncthreads();
   }
   if (threadIdx.x == 0) out[n] = finish_sensitivity(s_part[0], factor, mult, mult_stride, n);
+}
+template <typename T>
+__global__ __launch_bounds__(kThreads) void range_sqr_kernel(const T* __restrict__ mn,
+                                                             const T* __restrict__ mx,
+                                                             float* __restrict__ out, int64_t G,
+                                                             float factor, const float* __restrict__ mult,
+                                                             int mult_stride) {
+  range_sqr_of_block(mn, mx, out, (int64_t)blockIdx.x, G, factor, mult, mult_stride);
 }
 
 // The same sum by one wave, lane l holding the running sums l, l + 64, l + 128 and l + 192: valid in lane 0.
@@ -99,6 +104,43 @@ __global__ __launch_bounds__(kThreads) void range_sqr_wave_kernel(const T* __res
   if (n >= N) return;
   const float v = range_sqr_of_wave(mn, mx, n * G, G);
   if ((threadIdx.x & 63) == 0) out[n] = finish_sensitivity(v, factor, mult, mult_stride, n);
+}
+
+// Either kernel in the first sample_blocks blocks; the others fold batch norm's partial sums, a wave per channel.  The two do not
+// wait for each other, and each is a few microseconds of latency: bf16 [256, 512, 28, 28] 6.2 + 4.7 us one after the other,
+// 7.3 side by side (the widths could come from the same launch, made by the block that is the last to arrive: 14.6 us for the three,
+// and 9.0 for the two of bf16 [32, 64, 56, 56], where two launches take 6.6).
+template <typename T, bool WAVES>
+__global__ __launch_bounds__(kThreads) void range_sqr_and_fold_kernel(const T* __restrict__ mn, const T* __restrict__ mx,
+                                                                      float* __restrict__ out, int64_t N, int64_t G, float factor,
+                                                                      const float* __restrict__ mult, int mult_stride,
+                                                                      unsigned sample_blocks, BnFinalize fold) {
+  const int wave = threadIdx.x >> 6;
+  if (blockIdx.x >= sample_blocks) {
+    const int64_t c = (int64_t)(blockIdx.x - sample_blocks) * (kThreads / 64) + wave;
+    if (c < fold.C) bn_finalize_channel(fold, c);
+  } else if constexpr (WAVES) {
+    const int64_t n = (int64_t)blockIdx.x * (kThreads / 64) + wave;
+    if (n >= N) return;
+    const float v = range_sqr_of_wave(mn, mx, n * G, G);
+    if ((threadIdx.x & 63) == 0) out[n] = finish_sensitivity(v, factor, mult, mult_stride, n);
+  } else {
+    range_sqr_of_block(mn, mx, out, (int64_t)blockIdx.x, G, factor, mult, mult_stride);
+  }
+}
+
+template <typename T>
+int launch_range_sqr_and_fold(const void* mn, const void* mx, float* out, int64_t N, int64_t G, float factor, const float* mult,
+                              int stride, const BnFinalize& fold, hipStream_t s) {
+  const T* lo = static_cast<const T*>(mn);
+  const T* hi = static_cast<const T*>(mx);
+  const bool waves = G <= 512;                         // (as launch_range_sqr)
+  const int64_t blocks = waves ? (N + 3) / 4 : N, folds = (fold.C + kThreads / 64 - 1) / (kThreads / 64);
+  if (blocks + folds > 0x7fffffffLL) return ACTNN_EINVAL;
+  const dim3 grid((unsigned)(blocks + folds)), blk(kThreads);
+  if (waves) range_sqr_and_fold_kernel<T, true><<<grid, blk, 0, s>>>(lo, hi, out, N, G, factor, mult, stride, (unsigned)blocks, fold);
+  else range_sqr_and_fold_kernel<T, false><<<grid, blk, 0, s>>>(lo, hi, out, N, G, factor, mult, stride, (unsigned)blocks, fold);
+  ACTNN_RETURN_LAUNCH_STATUS();
 }
 
 template <typename T>
@@ -497,19 +539,32 @@ extern "C" int actnn_calc_precision_device(const float* C, int32_t* bits, int64_
   return launch_allocate(C, bits, nullptr, N, initial_bits, target, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
-                                          int mult_per_sample, float* sensitivity, int32_t* bits,
-                                          int32_t* prefix, int64_t N, int64_t G, int initial_bits,
-                                          int64_t target, int dtype, void* stream) {
-  using namespace actnn;
+namespace actnn {
+// actnn_allocate_bits_device; with `fold`, batch norm's partial sums are folded beside the sensitivities.  (N > 0 then.)
+int allocate_bits(const void* mn, const void* mx, float factor, const float* mult, int mult_per_sample, float* sensitivity, int32_t* bits,
+                  int32_t* prefix, int64_t N, int64_t G, int initial_bits, int64_t target, int dtype, const BnFinalize* fold,
+                  hipStream_t s) {
   if (N < 0 || G < 0 || (dtype != ACTNN_F32 && dtype != ACTNN_F16 && dtype != ACTNN_BF16))
     return N < 0 || G < 0 ? ACTNN_EINVAL : ACTNN_EDTYPE;
   if (initial_bits < 1 || initial_bits > 8) return ACTNN_EBITS;
   if (N > kMaxAllocated || N * (initial_bits - 1) > kMaxAllocated) return ACTNN_EINVAL;
   if (!prefix || (N > 0 && (!sensitivity || !bits || (G > 0 && (!mn || !mx))))) return ACTNN_EINVAL;
   if (N > 0) {
-    const int rc = actnn_range_sqr(mn, mx, sensitivity, N, G, factor, mult, mult_per_sample, dtype, stream);
+    const int stride = mult_per_sample ? 1 : 0;
+    const int rc = !fold ? actnn_range_sqr(mn, mx, sensitivity, N, G, factor, mult, mult_per_sample, dtype, s)
+                   : dtype == ACTNN_F32 ? launch_range_sqr_and_fold<float>(mn, mx, sensitivity, N, G, factor, mult, stride, *fold, s)
+                   : dtype == ACTNN_F16 ? launch_range_sqr_and_fold<__half>(mn, mx, sensitivity, N, G, factor, mult, stride, *fold, s)
+                                        : launch_range_sqr_and_fold<bf16_t>(mn, mx, sensitivity, N, G, factor, mult, stride, *fold, s);
     if (rc != ACTNN_OK) return rc;
   }
-  return launch_allocate(sensitivity, bits, prefix, N, initial_bits, target, static_cast<hipStream_t>(stream));
+  return launch_allocate(sensitivity, bits, prefix, N, initial_bits, target, s);
+}
+}  // namespace actnn
+
+extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float factor, const float* mult,
+                                          int mult_per_sample, float* sensitivity, int32_t* bits,
+                                          int32_t* prefix, int64_t N, int64_t G, int initial_bits,
+                                          int64_t target, int dtype, void* stream) {
+  return actnn::allocate_bits(mn, mx, factor, mult, mult_per_sample, sensitivity, bits, prefix, N, G, initial_bits, target, dtype, nullptr,
+                              static_cast<hipStream_t>(stream));
 }

@@ -1,5 +1,6 @@
 // Library-level helpers: error strings, version, the plain streaming copy used to calibrate
 // bandwidth counters, and the matrix-pipe probe the benchmark prices the fused GEMM against.
+#include "bn_finalize.h"
 #include "device_utils.h"
 
 namespace actnn {
@@ -93,12 +94,15 @@ extern "C" int actnn_allocate_bits_device(const void* mn, const void* mx, float 
                                           int mult_per_sample, float* sensitivity, int32_t* bits,
                                           int32_t* prefix, int64_t N, int64_t G, int initial_bits,
                                           int64_t target, int dtype, void* stream);
-extern "C" int actnn_batch_norm_forward_stats(const void* x, const float* weight, const float* bias,
-                                              float* running_mean, float* running_var, float* save_mean,
-                                              float* save_invstd, void* mn, void* mx, void* workspace,
-                                              int64_t workspace_bytes, int64_t N, int64_t C, int64_t HW,
-                                              double momentum, double eps, int dtype, int channels_last,
-                                              void* stream);
+namespace actnn {
+int allocate_bits(const void* mn, const void* mx, float factor, const float* mult, int mult_per_sample, float* sensitivity, int32_t* bits,
+                  int32_t* prefix, int64_t N, int64_t G, int initial_bits, int64_t target, int dtype, const BnFinalize* fold,
+                  hipStream_t s);
+int batch_norm_statistics(const void* x, const float* weight, const float* bias, float* running_mean, float* running_var,
+                          float* save_mean, float* save_invstd, void* mn, void* mx, void* workspace,
+                          int64_t workspace_bytes, int64_t N, int64_t C, int64_t HW, double momentum, double eps, int dtype,
+                          int channels_last, BnFinalize* open, hipStream_t s);
+}  // namespace actnn
 extern "C" int actnn_batch_norm_forward_apply(const void* x, void* y, const void* workspace,
                                               int64_t workspace_bytes, const int32_t* bits,
                                               const int32_t* prefix, const void* mn, const void* mx, void* scale,
@@ -130,12 +134,14 @@ extern "C" int actnn_batch_norm_forward_quantize(
   if (relu && (!channels_last || (dtype != ACTNN_F16 && dtype != ACTNN_BF16) ||
                !((C <= 256 && 256 % C == 0) || C % 512 == 0) || (N * HW) % (2048 / (C < 256 ? C : 256)) != 0))
     return ACTNN_EINVAL;
-  int rc = actnn_batch_norm_forward_stats(x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn,
-                                          mx, workspace, workspace_bytes, N, C, HW, momentum, eps, dtype,
-                                          channels_last, stream);
+  // the fold of the statistics' sums goes with the sensitivities
+  actnn::BnFinalize fold;
+  int rc = actnn::batch_norm_statistics(x, weight, bias, running_mean, running_var, save_mean, save_invstd, mn, mx, workspace,
+                                        workspace_bytes, N, C, HW, momentum, eps, dtype, channels_last, &fold,
+                                        static_cast<hipStream_t>(stream));
   if (rc != ACTNN_OK) return rc;
-  rc = actnn_allocate_bits_device(mn, mx, factor, mult, mult_per_sample, sensitivity, bits, prefix, N,
-                                  C * HW / 256, initial_bits, target, dtype, stream);
+  rc = actnn::allocate_bits(mn, mx, factor, mult, mult_per_sample, sensitivity, bits, prefix, N, C * HW / 256, initial_bits, target,
+                            dtype, &fold, static_cast<hipStream_t>(stream));
   if (rc != ACTNN_OK) return rc;
   if (relu)
     return actnn_batch_norm_forward_apply_relu(x, y, workspace, workspace_bytes, bits, prefix, mn, mx, scale,
