@@ -348,16 +348,17 @@ __global__ __launch_bounds__(THREADS) void allocate_kernel(const float* __restri
 // patterns - a double product each, what the one-block kernel is bound by - are evaluated once, the widths
 // are counts over registers, and every access to memory is coalesced (the widths change over to runs of
 // consecutive items through LDS).  A lane starts with the step its number says, so that the lanes of a
-// histogram atomic hold different steps, as above.  8192 items: 23 - 28 us, 59 - 70 with allocate_kernel
-// (both beside the other kernels of a training step).
+// histogram atomic hold different steps, as above, and items of like sensitivities, whose steps of one kind share a
+// bin, count in kCopies histograms by their lanes.  8192 items: 23.1 us, 25.0 with one histogram, 59 - 70 with
+// allocate_kernel (all beside the other kernels of a training step).
 template <int ITEMS>
 __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __restrict__ sens, int32_t* __restrict__ bits,
                                                              int32_t* __restrict__ prefix, int N, int initial,
                                                              int64_t K) {
   constexpr int kN = 1024, kSteps = 7;
-  constexpr int kPer = kBins / kN;
+  constexpr int kPer = kBins / kN, kCopies = 4;
   __shared__ double factors[8];
-  __shared__ uint32_t hist[kBins];
+  __shared__ uint32_t hist[kCopies][kBins];
   __shared__ uint32_t s_wave[kN / 64];
   __shared__ uint32_t s_digit, s_above, s_inside;
   __shared__ __align__(16) uint8_t s_width[kN * ITEMS];
@@ -372,8 +373,9 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
     for (int k = 0; k < ITEMS; ++k) C[k] = t + k * kN < N ? sens[t + k * kN] : 0.0f;
     if (t < L) factors[t] = kStepFactor[initial - t];
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) hist[k * kN + t] = 0;
+    for (int k = 0; k < kCopies * kPer; ++k) (&hist[0][0])[k * kN + t] = 0;
     __syncthreads();
+    uint32_t* const my_hist = hist[(t >> 3) & (kCopies - 1)];      // (lanes of one step lie 7 apart)
     int l = t % L;
 #pragma unroll
     for (int j = 0; j < kSteps; ++j) {
@@ -391,7 +393,7 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
       const uint32_t last = (1u << width) - 1u;
       if (pass > 0) {
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) hist[k * kN + t] = 0;
+        for (int k = 0; k < kCopies * kPer; ++k) (&hist[0][0])[k * kN + t] = 0;
         __syncthreads();
       }
 #pragma unroll
@@ -401,7 +403,7 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
           for (int k = 0; k < ITEMS; ++k) {
             const uint32_t o = key[k][j];
             // (the dearest steps in the last bin; a shift by 32 is what pass 0 would ask for)
-            if (t + k * kN < N && (pass == 0 || (o >> (shift + width)) == cut)) atomicAdd(&hist[last - ((o >> shift) & last)], 1u);
+            if (t + k * kN < N && (pass == 0 || (o >> (shift + width)) == cut)) atomicAdd(&my_hist[last - ((o >> shift) & last)], 1u);
           }
         }
       }
@@ -409,7 +411,9 @@ __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __rest
       uint32_t h[kPer], mine = 0;
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        h[k] = hist[t * kPer + k];
+        h[k] = 0;
+#pragma unroll
+        for (int c = 0; c < kCopies; ++c) h[k] += hist[c][t * kPer + k];
         mine += h[k];
       }
       uint32_t all;
