@@ -484,21 +484,23 @@ ACTNN_DEV uint64_t unhoisted(uint64_t v) {
 template <typename T>
 ACTNN_DEV void noise_pair(const PackSink& ps, uint64_t oa, uint64_t ob, uint32_t (&wa)[Noise<T>::kWords],
                           uint32_t (&wb)[Noise<T>::kWords], bool together) {
-  const uint64_t seed = unhoisted(ps.seed);
   // together: lane ^ 1 is known to make this call in the same step
   if (together && (((uint32_t)oa ^ threadIdx.x) & 1u) == 0 && (((uint32_t)ob ^ threadIdx.x) & 1u) == 0) {
-    Noise<T>::octets(oa, ob, seed, ps.offset, wa, wb);
+    Noise<T>::octets(oa, ob, ps.seed, ps.offset, wa, wb);
   } else {
-    Noise<T>::octet(oa, seed, ps.offset, wa);
-    Noise<T>::octet(ob, seed, ps.offset, wb);
+    Noise<T>::octet(oa, ps.seed, ps.offset, wa);
+    Noise<T>::octet(ob, ps.seed, ps.offset, wb);
   }
 }
 
 // b: the sample's width, dst: first word of the chunk's group in the stream (both looked up by the
 // caller, who knows how often the sample changes); (mul, sub): the group's parameters from the queue;
 // rw: the noise words of the chunk's octet.  SCALAR_B: b is known to be one number for the wave (the
-// sample comes from the block's index); otherwise the wave takes a scalar branch for the width of its first lane,
-// and another turn where it spans two samples of different widths (the lanes of a group always agree).
+// sample comes from the block's index); otherwise the wave checks, and takes one scalar branch when
+// its lanes agree - as they do except where a wave spans two samples of different widths.  TURNS: a scalar branch for
+// the width of the first lane and another turn where there are two widths (the lanes of a group always agree), which
+// needs one copy of the packers: for the pass with the ReLU, whose code is long (the plain pass packs up to
+// 6 % slower like that: bf16 [512, 128, 56, 56] 0.159 and 0.166 ms).
 template <typename T>
 ACTNN_DEV void pack_chunk_width(const float (&v)[8], const uint32_t (&rw)[Noise<T>::kWords], float mul, float sub,
                                 uint32_t lane32, int32_t* __restrict__ dst, int b) {
@@ -514,7 +516,7 @@ ACTNN_DEV void pack_chunk_width(const float (&v)[8], const uint32_t (&rw)[Noise<
     default: break;
   }
 }
-template <typename T, bool SCALAR_B>
+template <typename T, bool SCALAR_B, bool TURNS = false>
 ACTNN_DEV void pack_chunk(const u32x4& ux, const uint32_t (&rw)[Noise<T>::kWords], float mul, float sub,
                           int32_t* __restrict__ dst, int b) {
   constexpr int PD = Chunk<T>::kPerDword;
@@ -526,6 +528,10 @@ ACTNN_DEV void pack_chunk(const u32x4& ux, const uint32_t (&rw)[Noise<T>::kWords
   for (int k = 0; k < 4; ++k) Chunk<T>::widen(w[k], v + k * PD);
   if constexpr (SCALAR_B) {
     pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b);
+  } else if constexpr (!TURNS) {
+    const int b0 = __builtin_amdgcn_readfirstlane(b);
+    if (__builtin_amdgcn_ballot_w64(b != b0) == 0) pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b0);
+    else pack_chunk_width<T>(v, rw, mul, sub, lane32, dst, b);
   } else {
     for (bool done = false; !done;) {
       const int b0 = __builtin_amdgcn_readfirstlane(b);
@@ -1265,7 +1271,7 @@ __global__ __launch_bounds__(kThreads, (RELU ? 4 : 1)) void bn_cl_apply_kernel(
       locate((uint32_t)ru + (uint32_t)t.r);
       float mul, sub;
       queue.get(j, mul, sub);
-      pack_chunk<T, false>(ux, rw, mul, sub, group_words((uint32_t)((ru * C) >> 8) + (lane_elems >> 8)), cur_b);
+      pack_chunk<T, false, (RELU != 0)>(ux, rw, mul, sub, group_words((uint32_t)((ru * C) >> 8) + (lane_elems >> 8)), cur_b);
     };
     // RELU: the wave's 64 chunks of a step are 512 consecutive elements - one block of the mask - or,
     // in rows of a multiple of 512 channels, the same half of two blocks (mask_place), and a half-wave's
@@ -1384,26 +1390,26 @@ __global__ __launch_bounds__(kThreads, (RELU ? 4 : 1)) void bn_cl_apply_kernel(
           before = rows;
         }
       } else {
-        // (as above; the rows of a step need not be there for every lane, but for all lanes of a group)
-#pragma unroll 1
-        for (; j < 32 && rb + (int64_t)j * R < p1; j += 2) {
-          int64_t ru = rb0 + (int64_t)j * R;
-          const bool two = j + 1 < 32 && rb + (int64_t)(j + 1) * R < p1;
-          u32x4 ux = xs.decode(xs.fetch(ru)), ux1 = ux;
-          if (two) ux1 = xs.decode(xs.fetch(ru + R));
-          uint32_t rw[Noise<T>::kWords], rw1[Noise<T>::kWords];
-          noise_pair<T>(ps, (uint64_t)((ru * C) >> 3) + (lane_elems >> 3), (uint64_t)(((ru + R) * C) >> 3) + (lane_elems >> 3),
-                        rw, rw1, (tpr & 1) == 0);      // lane ^ 1 is in the same row, hence in the same steps
-#pragma unroll 1
-          for (int h = 0;; ++h) {
-            store_out(out_at(ru), apply(ux, ux));
-            pack_one(ux, rw, ru, j + h);
-            if (h == 1 || !two) break;
-            ux = ux1;
-            ru += R;
-#pragma unroll
-            for (int k = 0; k < Noise<T>::kWords; ++k) rw[k] = rw1[k];
-          }
+        for (; j + 2 <= 32 && rb + (int64_t)(j + 1) * R < p1; j += 2) {
+          const int64_t ru0 = rb0 + (int64_t)j * R, ru1 = ru0 + R;
+          const typename XS::Raw rx0 = xs.fetch(ru0), rx1 = xs.fetch(ru1);
+          uint32_t rw[2][Noise<T>::kWords];
+          noise_pair<T>(ps, (uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), (uint64_t)((ru1 * C) >> 3) + (lane_elems >> 3),
+                        rw[0], rw[1], (tpr & 1) == 0);      // lane ^ 1 is in the same row, hence in the same steps
+          const u32x4 ux0 = xs.decode(rx0);
+          store_out(out_at(ru0), apply(ux0, ux0));
+          pack_one(ux0, rw[0], ru0, j);
+          const u32x4 ux1 = xs.decode(rx1);
+          store_out(out_at(ru1), apply(ux1, ux1));
+          pack_one(ux1, rw[1], ru1, j + 1);
+        }
+        for (; j < 32 && rb + (int64_t)j * R < p1; ++j) {
+          const int64_t ru0 = rb0 + (int64_t)j * R;
+          const u32x4 ux = xs.decode(xs.fetch(ru0));
+          store_out(out_at(ru0), apply(ux, ux));
+          uint32_t rw[Noise<T>::kWords];
+          Noise<T>::octet((uint64_t)((ru0 * C) >> 3) + (lane_elems >> 3), ps.seed, ps.offset, rw);
+          pack_one(ux, rw, ru0, j);
         }
       }
     }
