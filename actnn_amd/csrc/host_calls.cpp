@@ -30,11 +30,12 @@ struct Args {
   Args(PyObject* const* a, Py_ssize_t count, Py_ssize_t want) : at(a), n(count) {
     TORCH_CHECK(count == want, "expected ", want, " arguments, got ", count);
   }
-  const Tensor& tensor() {
+  PyObject* tensor_object() {
     PyObject* o = at[i++];
     TORCH_CHECK_TYPE(THPVariable_Check(o), "argument ", i, " must be a tensor");
-    return THPVariable_Unpack(o);
+    return o;
   }
+  const Tensor& tensor() { return THPVariable_Unpack(tensor_object()); }
   // whether the next `count` arguments are tensors
   bool tensors(int count) const {
     for (int k = 0; k < count; ++k)
@@ -113,20 +114,55 @@ Tensor empty(at::IntArrayRef size, const Tensor& like, at::ScalarType dtype) {
   return at::empty(size, at::TensorOptions().dtype(dtype).device(like.device()));
 }
 
-// torch.empty_like(t), through Python where t's class may have a say in it
-Tensor empty_like(PyObject* o, const Tensor& t) {
-  if (!o || THPVariable_CheckExact(o)) return at::empty_like(t);
-  PyObject* torch = PyImport_ImportModule("torch");
-  if (!torch) throw python_error();
-  PyObject* made = PyObject_CallMethod(torch, "empty_like", "O", o);
-  Py_DECREF(torch);
-  if (!made) throw python_error();
-  Tensor out;
-  if (THPVariable_Check(made)) out = THPVariable_Unpack(made);
-  Py_DECREF(made);
-  TORCH_CHECK(out.defined(), "empty_like gave no tensor");
-  return out;
-}
+// A tensor argument with the Python object it came as.  What makes a new tensor of it goes through Python where its class may
+// have a say, and the object goes along with the tensor: the next step works on the same one the kernel reads or writes.
+class Given {
+ public:
+  explicit Given(PyObject* o) : object_(o), tensor_(THPVariable_Unpack(o)) { Py_INCREF(object_); }
+  Given(const Given&) = delete;
+  Given& operator=(const Given&) = delete;
+  ~Given() { Py_DECREF(object_); }
+  const Tensor& tensor() const { return tensor_; }
+  void make_contiguous() {
+    if (plain()) tensor_ = tensor_.contiguous();
+    else replace(PyObject_CallMethod(object_, "contiguous", nullptr));
+  }
+  // (the kernels use 16-byte accesses; only views with a storage offset are not aligned)
+  void make_aligned() {
+    if (reinterpret_cast<uintptr_t>(tensor_.data_ptr()) % 16 == 0) return;
+    if (plain()) tensor_ = tensor_.clone();
+    else replace(PyObject_CallMethod(object_, "clone", nullptr));
+  }
+  Tensor empty_like() const {
+    if (plain()) return at::empty_like(tensor_);
+    PyObject* torch = PyImport_ImportModule("torch");
+    if (!torch) throw python_error();
+    PyObject* made = PyObject_CallMethod(torch, "empty_like", "O", object_);
+    Py_DECREF(torch);
+    const Tensor out = unpacked(made);
+    Py_DECREF(made);
+    return out;
+  }
+
+ private:
+  // (a plain object_ stays when its tensor is replaced: only its class counts)
+  bool plain() const { return THPVariable_CheckExact(object_); }
+  static Tensor unpacked(PyObject* made) {
+    if (!made) throw python_error();
+    if (!THPVariable_Check(made)) {
+      Py_DECREF(made);
+      TORCH_CHECK_TYPE(false, "a tensor's class made something that is no tensor");
+    }
+    return THPVariable_Unpack(made);
+  }
+  void replace(PyObject* made) {
+    tensor_ = unpacked(made);
+    Py_DECREF(object_);
+    object_ = made;
+  }
+  PyObject* object_;
+  Tensor tensor_;
+};
 
 // (seed, offset) of the device's default generator, advancing the offset by 4 under its lock
 struct Draw {
@@ -272,17 +308,16 @@ PyObject* unpack_rows_fixed(PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---------------------------------------------------------------------------- masks
-Tensor aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone(); }
-
 // x -> relu(x), mask;  x, p -> dropout(x), mask
 PyObject* mask_forward(Args& args, bool dropout) {
-  PyObject* given = args.at[0];
-  const Tensor x = aligned(args.tensor());
+  Given given(args.tensor_object());
+  given.make_aligned();
+  const Tensor& x = given.tensor();
   TORCH_CHECK(x.is_cuda(), "input must be a CUDA tensor!");
   const double p = dropout ? args.number() : 0.0;
   const int64_t count = x.numel();
   const c10::DeviceGuard guard(x.device());
-  const Tensor y = empty_like(given, x), mask = empty({mask_words(count)}, x, at::kInt);
+  const Tensor y = given.empty_like(), mask = empty({mask_words(count)}, x, at::kInt);
   const int code = code_of(x.scalar_type());
   if (dropout) {
     const Draw draw(x);
@@ -307,12 +342,15 @@ PyObject* dropout_forward(PyObject* const* a, Py_ssize_t n) {
 
 // grad, mask[, p] -> gradient of the input
 PyObject* mask_backward(Args& args, bool dropout) {
-  PyObject* given = args.at[0];
-  const Tensor grad = aligned(args.tensor().contiguous()), mask = args.tensor();
+  Given given(args.tensor_object());
+  given.make_contiguous();                             // (the order the kernel reads and writes in: before the result is made)
+  given.make_aligned();
+  const Tensor& grad = given.tensor();
+  const Tensor mask = args.tensor();
   TORCH_CHECK(grad.is_cuda() && mask.is_cuda(), "grad_output must be a CUDA tensor!");
   const double p = dropout ? args.number() : 0.0;
   const c10::DeviceGuard guard(grad.device());
-  const Tensor out = empty_like(THPVariable_CheckExact(given) ? nullptr : given, grad);
+  const Tensor out = given.empty_like();
   const int code = code_of(grad.scalar_type());
   if (dropout)
     launch("dropout_backward", [&] {
@@ -392,7 +430,7 @@ PyObject* batch_norm_forward_quantize(PyObject* const* a, Py_ssize_t n) {
   const int64_t G = g.C * g.HW / 256, ws_bytes = g.workspace();
   const c10::DeviceGuard guard(x.device());
   const Tensor ws = empty({ws_bytes / 4}, x, at::kFloat), mean = empty({g.C}, x, at::kFloat), invstd = empty({g.C}, x, at::kFloat);
-  const Tensor mn = empty({g.N * G}, x, dtype), mx = empty({g.N * G}, x, dtype), y = empty_like(a[0], x);
+  const Tensor mn = empty({g.N * G}, x, dtype), mx = empty({g.N * G}, x, dtype), y = Given(a[0]).empty_like();
   if (!sens.defined()) sens = empty({g.N}, x, at::kFloat);
   const Tensor bits = empty({g.N}, x, at::kInt), prefix = empty({g.N + 1}, x, at::kInt);
   const Tensor packed = empty({total * G * 8}, x, at::kInt), scale = empty({g.N, G, 1}, x, dtype);
@@ -424,7 +462,7 @@ PyObject* batch_norm_forward(PyObject* const* a, Py_ssize_t n) {
   const bool ranges = args.flag();
   const int64_t ws_bytes = g.workspace();
   const c10::DeviceGuard guard(x.device());
-  const Tensor ws = empty({ws_bytes / 4}, x, at::kFloat), y = empty_like(a[0], x);
+  const Tensor ws = empty({ws_bytes / 4}, x, at::kFloat), y = Given(a[0]).empty_like();
   const Tensor mean = empty({g.C}, x, at::kFloat), invstd = empty({g.C}, x, at::kFloat);
   Tensor mn, mx;
   if (ranges) {
@@ -448,7 +486,7 @@ PyObject* batch_norm_backward(PyObject* const* a, Py_ssize_t n) {
   const Tensor weight = args.optional(), mean = args.tensor(), invstd = args.tensor();
   const int64_t entries = args.flag() ? g.sumsq_entries() : 0, ws_bytes = g.workspace();
   const c10::DeviceGuard guard(x.device());
-  const Tensor ws = empty({ws_bytes / 4 + entries}, x, at::kFloat), dx = empty_like(a[0], x);
+  const Tensor ws = empty({ws_bytes / 4 + entries}, x, at::kFloat), dx = Given(a[0]).empty_like();
   const Tensor dweight = empty({g.C}, x, at::kFloat), dbias = empty({g.C}, x, at::kFloat);
   launch("batch_norm_backward", [&] {
       return actnn_batch_norm_backward(ptr(x), ptr(dy), f32(weight), f32(mean), f32(invstd), ptr(dx), f32(dweight), f32(dbias), ptr(ws),
@@ -469,7 +507,7 @@ PyObject* batch_norm_backward_packed(PyObject* const* a, Py_ssize_t n) {
   const int64_t entries = args.flag() ? g.sumsq_entries() : 0, ws_bytes = g.workspace();
   const Tensor mask = args.optional(), masked = args.optional();
   const c10::DeviceGuard guard(dy.device());
-  const Tensor ws = empty({ws_bytes / 4 + entries}, dy, at::kFloat), dx = empty_like(a[5], dy);
+  const Tensor ws = empty({ws_bytes / 4 + entries}, dy, at::kFloat), dx = Given(a[5]).empty_like();
   const Tensor dweight = empty({g.C}, dy, at::kFloat), dbias = empty({g.C}, dy, at::kFloat);
   float* squares = entries ? f32(ws) + ws_bytes / 4 : nullptr;
   if (mask.defined())

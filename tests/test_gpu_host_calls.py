@@ -50,6 +50,37 @@ def test_tensor_classes_come_back_as_empty_like_makes_them():
         assert torch.equal(y.as_subclass(torch.Tensor), torch.relu(given.detach()).as_subclass(torch.Tensor))
 
 
+class _Named(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("operator", ["relu", "dropout"])
+@pytest.mark.parametrize("order", ["transposed", "channels last", "default", "misaligned"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gradient_of_a_tensor_class_in_any_order(operator, order, dtype):
+    """A gradient that is an instance of a subclass keeps its class; its values come back in their places whatever its strides are."""
+    shape = (6, 16, 5, 7)
+    x = torch.randn(shape, device=DEV, dtype=dtype)
+    if operator == "relu":
+        y, mask = ext_q.relu_forward(x)
+        factor = (x > 0).to(dtype)
+    else:
+        factor, mask = ext_q.dropout_forward(torch.ones_like(x), 0.5)                # 0 and 2
+    values = torch.randn(shape, device=DEV, dtype=dtype)
+    grad = {"transposed": lambda: values.permute(3, 2, 1, 0).contiguous().permute(3, 2, 1, 0),
+            "channels last": lambda: values.contiguous(memory_format=torch.channels_last), "default": values.clone,
+            "misaligned": lambda: torch.cat([values.new_zeros(1), values.flatten()])[1:].view(shape)}[order]()
+    for given in (grad, grad.as_subclass(_Named)):
+        got = ext_q.relu_backward(given, mask) if operator == "relu" else ext_q.dropout_backward(given, mask, 0.5)
+        assert torch.equal(got.as_subclass(torch.Tensor), values * factor)
+        assert type(got) is type(given) and got.is_contiguous()
+    leaf = (x if operator == "relu" else torch.ones_like(x)).requires_grad_()
+    out = ext_q.act_quantized_relu(leaf) if operator == "relu" else ext_q.act_quantized_dropout(leaf, 0.5)
+    factor = factor if operator == "relu" else out.detach()
+    (got,) = torch.autograd.grad(out, leaf, grad.as_subclass(_Named))
+    assert torch.equal(got.as_subclass(torch.Tensor), values * factor)
+
+
 def test_misaligned_input_is_copied():
     x = torch.randn(4097, device=DEV)[1:]
     y, mask = ext_q.relu_forward(x)
