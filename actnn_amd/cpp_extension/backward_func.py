@@ -59,9 +59,12 @@ def known_sumsq(grad):
     return left[0].sum()
 
 
-def _bn_geometry(input):
-    """(N, C, HW, channels_last) of a dense tensor in the default or the channels-last layout."""
-    return _glue.host().batch_norm_geometry(input)
+def _bn_geometry(input, *parameters):
+    """(N, C, HW, channels_last) of a dense tensor in the default or the channels-last layout, else None (also, where
+    parameters are given, for an input that is not 16-byte aligned and parameters that are not dense fp32 ones)."""
+    if not (isinstance(input, torch.Tensor) and input.is_cuda):        # (asked of CPU tensors too, where nothing may be built)
+        return None
+    return _glue.host().batch_norm_geometry(input, *parameters)
 
 
 def _f32_or_none(t):
@@ -69,7 +72,7 @@ def _f32_or_none(t):
 
 
 def hip_batch_norm_applies(input, weight, bias, running_mean, running_var):
-    return _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var) is not None
+    return _bn_geometry(input, weight, bias, running_mean, running_var) is not None
 
 
 @functools.lru_cache(maxsize=4096)
@@ -81,7 +84,7 @@ def _groups_align(N, C, HW, code, channels_last):
 
 def hip_batch_norm_minmax_applies(input, weight, bias, running_mean, running_var):
     """True when the forward pass can also return the quantiser's per-group min/max."""
-    geo = _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var)
+    geo = _bn_geometry(input, weight, bias, running_mean, running_var)
     if geo is None:
         return False
     N, C, HW, channels_last = geo
@@ -169,7 +172,7 @@ def hip_batch_norm_quantize_geometry(input, weight, bias, running_mean, running_
     """(N, C, HW, channels_last) when statistics, group min/max and the packed copy can all come from
     the fused passes (what hip_batch_norm_minmax_applies and hip_batch_norm_pack_applies ask, looked
     up once), else None."""
-    geo = _glue.host().batch_norm_geometry(input, weight, bias, running_mean, running_var)
+    geo = _bn_geometry(input, weight, bias, running_mean, running_var)
     if geo is None:
         return None
     N, C, HW, channels_last = geo
