@@ -550,7 +550,9 @@ def max_pool2d_forward(x, kernel_size, stride, padding, dilation, nibble_indices
     channels_last = pool_takes_channels_last(x)
     if not channels_last:
         x = x.contiguous()
-    return g.host().max_pool2d_forward(x, channels_last, *kernel_size, *stride, *padding, *dilation, nibble_indices)
+    KH, KW = kernel_size
+    return g.host().max_pool2d_forward(x, channels_last, KH, KW, stride[0], stride[1], padding[0], padding[1], dilation[0],
+                                       dilation[1], nibble_indices)
 
 
 def max_pool2d_backward(grad_output, idx, input_shape, kernel_size, stride, padding, channels_last=None):
@@ -567,8 +569,9 @@ def max_pool2d_backward(grad_output, idx, input_shape, kernel_size, stride, padd
     grad_output = grad_output.contiguous(memory_format=fmt)
     if nibble_indices and idx.numel() != (grad_output.numel() + 1) // 2:
         raise RuntimeError("max_pool2d_backward: the index tensor does not match grad_output")
-    return g.host().max_pool2d_backward(grad_output, idx, channels_last, nibble_indices, *input_shape, *kernel_size, *stride,
-                                        *padding)
+    N, C, H, W = input_shape
+    return g.host().max_pool2d_backward(grad_output, idx, channels_last, nibble_indices, N, C, H, W, kernel_size[0], kernel_size[1],
+                                        stride[0], stride[1], padding[0], padding[1])
 
 
 class ActQuantizedMaxPool2d(Function):

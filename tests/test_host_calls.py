@@ -4,7 +4,9 @@ import torch
 import torch.nn.functional as F
 
 from actnn_amd import _lib
+from actnn_amd.cpp_extension import _glue
 from actnn_amd.cpp_extension import backward_func as ext_bf
+from actnn_amd.cpp_extension import quantization as ext_q
 
 
 @pytest.fixture
@@ -28,3 +30,27 @@ def test_batch_norm_of_cpu_tensors_needs_nothing_built(nothing_built):
     gi, _, _ = ext_bf.native_batch_norm_backward(torch.ones_like(x), x, one, zero, one, mean, invstd, False, 1e-5,
                                                  [True, True, True])
     assert torch.allclose(gi, torch.full_like(x, (1 + 1e-5) ** -0.5))
+
+
+class _Recorder:
+    def __getattr__(self, name):
+        return lambda *args: (name, args[2:] if name.endswith("backward") else args[1:])
+
+
+@pytest.mark.parametrize("window,stride,want", [((3, 2), (2, 1, 7), (3, 2, 2, 1, 1, 0, 1, 2)), ((3, 2, 9), (2,), None),
+                                                ((3,), (2, 1, 7, 7), None)])
+def test_pool_arguments_keep_their_places(monkeypatch, window, stride, want):
+    """The native calls count their arguments: one more in one tuple must not stand in for one that another lacks.  The window has
+    two values; of the others the first two are read, as ever."""
+    monkeypatch.setattr(_glue, "host", lambda: _Recorder())
+    x = torch.zeros(2, 4, 8, 8)
+    padding, dilation = (1, 0, 5), [1, 2, 5]
+    if want is None:
+        with pytest.raises(ValueError):
+            ext_q.max_pool2d_forward(x, window, stride, padding[:2], dilation[:2])
+        return
+    assert ext_q.max_pool2d_forward(x, window, stride, padding, dilation) == ("max_pool2d_forward", (False, *want, False))
+    got = ext_q.max_pool2d_backward(x, x.to(torch.int8), x.shape, window, stride, padding)
+    assert got == ("max_pool2d_backward", (False, False, 2, 4, 8, 8, *want[:6]))
+    with pytest.raises(ValueError):
+        ext_q.max_pool2d_backward(x, x.to(torch.int8), x.shape[1:], (3, 2, 2), (2, 1), (1, 0))
