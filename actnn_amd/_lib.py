@@ -8,6 +8,7 @@ import ctypes
 import os
 import subprocess
 import sysconfig
+import tempfile
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
@@ -130,19 +131,21 @@ _lib = _host = None
 
 
 def build(verbose=False):
-    """Compile every source under csrc/ into libactnn_hip.so (always recompiles)."""
+    """Compile every source under csrc/ into libactnn_hip.so and _host.so (always recompiles).  The two belong together:
+    neither is replaced unless both were built.  A process that has loaded them goes on with what it loaded."""
     srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = LIB_PATH + ".tmp"
-    out = _run(["hipcc", *HIPCC_FLAGS, *srcs, "-o", tmp], verbose)
-    # the host pass does not know the device-only target feature and says so once per file
-    noise = "'-packed-fp32-ops' is not a recognized feature for this target"
-    out = "\n".join(l for l in out.splitlines() if noise not in l)
-    if out.strip():
-        print(out, flush=True)
-    os.replace(tmp, LIB_PATH)
-    _build_host(verbose)
-    global _lib, _host
-    _lib = _host = None
+    with tempfile.TemporaryDirectory(dir=_HERE, prefix="build-") as made:
+        lib = os.path.join(made, os.path.basename(LIB_PATH))           # (its own name already: the module asks for it)
+        host = os.path.join(made, os.path.basename(HOST_PATH))
+        out = _run(["hipcc", *HIPCC_FLAGS, *srcs, "-o", lib], verbose)
+        # the host pass does not know the device-only target feature and says so once per file
+        noise = "'-packed-fp32-ops' is not a recognized feature for this target"
+        out = "\n".join(l for l in out.splitlines() if noise not in l)
+        if out.strip():
+            print(out, flush=True)
+        _build_host(lib, host, verbose)
+        os.replace(lib, LIB_PATH)
+        os.replace(host, HOST_PATH)
     return LIB_PATH
 
 
@@ -156,19 +159,17 @@ def _run(cmd, verbose):
     return proc.stdout
 
 
-def _build_host(verbose):
-    """Compile the native calls against torch and the library beside them."""
+def _build_host(lib, target, verbose):
+    """Compile the native calls into `target`, against torch and the library `lib` that will lie beside them."""
     import torch
     home = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     includes = [os.path.join(home, "include"), os.path.join(home, "include", "torch", "csrc", "api", "include"),
                 os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
-    tmp = HOST_PATH + ".tmp"
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + i for i in includes),
-          os.path.join(CSRC, HOST_SOURCE), "-o", tmp, "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch_cpu",
-          "-lc10", "-lc10_hip", "-L" + _HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"], verbose)
-    os.replace(tmp, HOST_PATH)
+          os.path.join(CSRC, HOST_SOURCE), "-o", target, "-L" + os.path.join(home, "lib"), "-ltorch_python", "-ltorch_cpu",
+          "-lc10", "-lc10_hip", "-L" + os.path.dirname(lib), "-l:" + os.path.basename(lib), "-Wl,-rpath,$ORIGIN"], verbose)
 
 
 def load():

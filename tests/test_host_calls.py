@@ -1,4 +1,6 @@
 """The Python side of the native calls of csrc/host_calls.cpp, as far as it shows without a GPU."""
+import os
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -54,3 +56,29 @@ def test_pool_arguments_keep_their_places(monkeypatch, window, stride, want):
     assert got == ("max_pool2d_backward", (False, False, 2, 4, 8, 8, *want[:6]))
     with pytest.raises(ValueError):
         ext_q.max_pool2d_backward(x, x.to(torch.int8), x.shape[1:], (3, 2, 2), (2, 1), (1, 0))
+
+
+@pytest.mark.parametrize("fails", [None, "hipcc", "g++"])
+def test_a_build_replaces_both_files_or_none(monkeypatch, tmp_path, fails):
+    paths = [str(tmp_path / name) for name in ("libactnn_hip.so", "_host.so")]
+    monkeypatch.setattr(_lib, "_HERE", str(tmp_path))
+    monkeypatch.setattr(_lib, "LIB_PATH", paths[0])
+    monkeypatch.setattr(_lib, "HOST_PATH", paths[1])
+    for path in paths:
+        with open(path, "w") as f:
+            f.write("old")
+
+    def compile_(cmd, verbose):
+        if cmd[0] == fails:
+            raise RuntimeError(f"{fails} failed")
+        with open(cmd[cmd.index("-o") + 1], "w") as f:
+            f.write("new")
+        return ""
+    monkeypatch.setattr(_lib, "_run", compile_)
+    if fails:
+        with pytest.raises(RuntimeError):
+            _lib.build()
+    else:
+        _lib.build()
+    assert [open(path).read() for path in paths] == ["old" if fails else "new"] * 2
+    assert sorted(os.listdir(tmp_path)) == ["_host.so", "libactnn_hip.so"]
