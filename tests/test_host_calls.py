@@ -82,3 +82,26 @@ def test_a_build_replaces_both_files_or_none(monkeypatch, tmp_path, fails):
         _lib.build()
     assert [open(path).read() for path in paths] == ["old" if fails else "new"] * 2
     assert sorted(os.listdir(tmp_path)) == ["_host.so", "libactnn_hip.so"]
+
+
+@pytest.mark.parametrize("broken", [None, "load", "load_host"])
+def test_a_build_loads_what_it_built(monkeypatch, broken):
+    import __graft_entry__
+    from oracle import build_ref
+    loaded = []
+    monkeypatch.setattr(_lib, "build", lambda verbose=False: None)
+    monkeypatch.setattr(build_ref, "build", lambda: None)
+    for name in ("load", "load_host"):
+        def load(name=name, real=getattr(_lib, name)):
+            if name == broken:
+                raise ImportError(f"{name}: undefined symbol")
+            loaded.append(name)
+            return real()
+        monkeypatch.setattr(_lib, name, load)
+    monkeypatch.setattr(_lib, "_host", None)
+    if broken:
+        with pytest.raises(ImportError):
+            __graft_entry__.build()
+    else:
+        __graft_entry__.build()
+        assert set(loaded) == {"load", "load_host"}
