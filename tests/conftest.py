@@ -10,9 +10,9 @@ if ROOT not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
-    # the C-ABI library is built in-tree beforehand; build it only if nothing is there
+    # the C-ABI library and the native calls are built in-tree beforehand; build them only if one is not there
     from actnn_amd import _lib
-    if not os.path.exists(_lib.LIB_PATH):
+    if not (os.path.exists(_lib.LIB_PATH) and os.path.exists(_lib.HOST_PATH)):
         _lib.build()
 
 

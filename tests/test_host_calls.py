@@ -105,3 +105,20 @@ def test_a_build_loads_what_it_built(monkeypatch, broken):
     else:
         __graft_entry__.build()
         assert set(loaded) == {"load", "load_host"}
+
+
+@pytest.mark.parametrize("there", [(), ("LIB_PATH",), ("HOST_PATH",), ("LIB_PATH", "HOST_PATH")])
+def test_tests_build_where_a_file_is_missing(monkeypatch, tmp_path, there):
+    import conftest
+    built = []
+    monkeypatch.setattr(_lib, "build", lambda: built.append(True))
+    for name in ("LIB_PATH", "HOST_PATH"):
+        monkeypatch.setattr(_lib, name, str(tmp_path / name))
+        if name in there:
+            (tmp_path / name).touch()
+
+    class Config:
+        def addinivalue_line(self, *line):
+            pass
+    conftest.pytest_configure(Config())
+    assert len(built) == (len(there) < 2)
