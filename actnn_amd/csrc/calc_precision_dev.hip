@@ -348,15 +348,19 @@ __global__ __launch_bounds__(THREADS) void allocate_kernel(const float* __restri
 // patterns - a double product each, what the one-block kernel is bound by - are evaluated once, the widths
 // are counts over registers, and every access to memory is coalesced (the widths change over to runs of
 // consecutive items through LDS).  A lane starts with the step its number says, so that the lanes of a
-// histogram atomic hold different steps, as above, and items of like sensitivities, whose steps of one kind share a
-// bin, count in kCopies histograms by their lanes.  8192 items: 23.1 us, 25.0 with one histogram, 59 - 70 with
-// allocate_kernel (all beside the other kernels of a training step).
+// histogram atomic hold different steps, as above.  Items of like sensitivities, whose steps of one kind share a bin, can
+// count in several histograms by their lanes, which all have to be cleared and added up: four for 4097 items and more, one for
+// fewer.  us with the sensitivities' pass in front, one / four histograms, for equal sensitivities at 1.5 bits on average, for
+// sensitivities within a few percent, and for ones e^(z/2) and e^(4 z) apart (z normal), at 2 bits: 1171 items 12.7 / 12.0,
+// 8.4 / 8.2, 9.2 / 9.4, 9.3 / 9.5; 2048 14.8 / 14.0, 9.3 / 9.3, 10.0 / 10.3, 10.0 / 10.3; 4096 24.0 / 21.8, 14.1 / 13.7, 14.9 / 15.1,
+// 14.8 / 15.2; 4097 30.1 / 27.3, 18.6 / 18.1, 20.4 / 20.6, 23.0 / 23.2; 6000 37.0 / 33.1, 22.3 / 21.6, 23.8 / 23.9, 23.5 / 23.7;
+// 8192 45.1 / 39.9, 27.3 / 25.8, 27.6 / 27.6, 27.4 / 27.6: the larger the batch, the more the like ones gain and the less the others lose.
 template <int ITEMS>
 __global__ __launch_bounds__(1024) void allocate_many_kernel(const float* __restrict__ sens, int32_t* __restrict__ bits,
                                                              int32_t* __restrict__ prefix, int N, int initial,
                                                              int64_t K) {
   constexpr int kN = 1024, kSteps = 7;
-  constexpr int kPer = kBins / kN, kCopies = 4;
+  constexpr int kPer = kBins / kN, kCopies = ITEMS > 4 ? 4 : 1;
   __shared__ double factors[8];
   __shared__ uint32_t hist[kCopies][kBins];
   __shared__ uint32_t s_wave[kN / 64];

@@ -112,7 +112,7 @@ def test_allocation_in_one_call_from_dirty_buffers(N):
 
 
 @pytest.mark.parametrize("N,initial", [(146, 8), (147, 8), (1024, 2), (1170, 8), (1171, 8), (2048, 8), (2049, 8),
-                                       (4097, 4), (8191, 8), (8192, 8), (8193, 8), (9362, 8), (9363, 8), (16385, 3),
+                                       (4096, 8), (4097, 4), (4097, 8), (8191, 8), (8192, 8), (8193, 8), (9362, 8), (9363, 8), (16385, 3),
                                        (40000, 8)])
 @pytest.mark.parametrize("coarse", [False, True])
 def test_allocation_of_large_batches_equals_the_host_routine(N, initial, coarse):
