@@ -40,11 +40,6 @@ def _workspace_bytes(N, C, HW, code, channels_last):
     return _glue.lib().actnn_batch_norm_workspace_bytes(N, C, HW, code, channels_last)
 
 
-@functools.lru_cache(maxsize=4096)
-def _sumsq_entries(N, C, HW, code, channels_last):
-    return _glue.lib().actnn_batch_norm_backward_sumsq_entries(N, C, HW, code, channels_last)
-
-
 def _leave_sumsq(grad_input, table):
     """Attach the partial sums of grad_input^2 that the backward pass left, for the layer that
     receives this gradient next (QScheme.set_scale); the version pins them to these contents."""
