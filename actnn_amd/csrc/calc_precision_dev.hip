@@ -94,6 +94,7 @@ template <typename T> ACTNN_DEV float range_sqr_of_wave(const T* __restrict__ mn
 }
 
 // One wave per sample: many samples of few groups (8192 samples of 16: 7.6 us with a block each).
+constexpr int64_t kWaveGroups = 512;
 template <typename T>
 __global__ __launch_bounds__(kThreads) void range_sqr_wave_kernel(const T* __restrict__ mn,
                                                                   const T* __restrict__ mx,
@@ -134,7 +135,7 @@ int launch_range_sqr_and_fold(const void* mn, const void* mx, float* out, int64_
                               int stride, const BnFinalize& fold, hipStream_t s) {
   const T* lo = static_cast<const T*>(mn);
   const T* hi = static_cast<const T*>(mx);
-  const bool waves = G <= 512;                         // (as launch_range_sqr)
+  const bool waves = G <= kWaveGroups;
   const int64_t blocks = waves ? (N + 3) / 4 : N, folds = (fold.C + kThreads / 64 - 1) / (kThreads / 64);
   if (blocks + folds > 0x7fffffffLL) return ACTNN_EINVAL;
   const dim3 grid((unsigned)(blocks + folds)), blk(kThreads);
@@ -148,7 +149,7 @@ int launch_range_sqr(const void* mn, const void* mx, float* out, int64_t N, int6
                      int stride, hipStream_t s) {
   const T* lo = static_cast<const T*>(mn);
   const T* hi = static_cast<const T*>(mx);
-  if (G <= 512)
+  if (G <= kWaveGroups)
     range_sqr_wave_kernel<T><<<dim3((unsigned)((N + 3) / 4)), dim3(kThreads), 0, s>>>(lo, hi, out, N, G, factor, mult, stride);
   else
     range_sqr_kernel<T><<<dim3((unsigned)N), dim3(kThreads), 0, s>>>(lo, hi, out, G, factor, mult, stride);
