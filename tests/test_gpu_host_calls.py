@@ -5,7 +5,7 @@ import torch
 
 import actnn_amd.cpp_extension.quantization as ext_q
 from actnn_amd.cpp_extension import backward_func as ext_bf
-from actnn_amd.cpp_extension import _glue
+from actnn_amd.qscheme import AllocationArgs
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -16,16 +16,89 @@ def _rows(N, F, bits=4):
     return ext_q.quantize_rows_fixed(torch.randn(N, F, device=DEV), bits, None, torch.bfloat16)
 
 
-def test_calls_run_on_the_current_stream():
-    x = torch.randn(1 << 22, device=DEV)
+def _compress(x, known):
+    rows = x.reshape(256, -1)
+    alloc = AllocationArgs(256, 1.0, None, 8, 2.0)
+    ranges = torch.aminmax(rows.reshape(-1, 256), dim=1) if known else None
+    packed, bits, scale, mn = ext_q.quantize_activation_device(rows, 256, ranges, alloc)
+    back = ext_q.unpack_rows_mixed(packed, bits, scale, mn.view(scale.shape), 256, rows.shape[1], rows.dtype)
+    return packed, bits, scale, mn, back
+
+
+def _compress_fixed(x):
+    rows = x.reshape(256, -1)
+    packed, scale, mn = ext_q.quantize_rows_fixed(rows, 4, None, rows.dtype)
+    back = ext_q.unpack_rows_fixed(packed, 4, scale, mn, 256, rows.shape[1], rows.dtype)
+    return packed[:-1], scale, mn, back                # (the last byte is spare)
+
+
+def _relu(x):
+    y, mask = ext_q.relu_forward(x)
+    return y, mask, ext_q.relu_backward(x, mask)
+
+
+def _dropout(x):
+    y, mask = ext_q.dropout_forward(x, 0.25)
+    return y, mask, ext_q.dropout_backward(x, mask, 0.25)
+
+
+def _pool(x, channels_last, nibble):
+    x = x.contiguous(memory_format=torch.channels_last) if channels_last else x
+    window = (3, 3), (2, 2), (1, 1)
+    y, idx = ext_q.max_pool2d_forward(x, *window, (1, 1), nibble)
+    return y, idx, ext_q.max_pool2d_backward(y, idx, x.shape, *window, channels_last)
+
+
+def _batch_norm(x):
+    weight, bias, mean, var = (torch.full((64,), v, device=DEV) for v in (1.0, 0.5, 0.0, 1.0))
+    y, save_mean, invstd, mn, mx = ext_bf.hip_batch_norm_forward(x, weight, bias, mean, var, 0.1, 1e-5, True)
+    return (y, save_mean, invstd, mn, mx, mean, var, *ext_bf.hip_batch_norm_backward(x, y, weight, save_mean, invstd, True))
+
+
+def _batch_norm_packed(x, relu):
+    x = x.contiguous(memory_format=torch.channels_last)
+    weight, bias, mean, var = (torch.full((64,), v, device=DEV) for v in (1.0, 0.5, 0.0, 1.0))
+    geo = ext_bf.hip_batch_norm_quantize_geometry(x, weight, bias, mean, var)
+    got = ext_bf.hip_batch_norm_forward_quantize(x, geo, weight, bias, mean, var, 0.1, 1e-5, AllocationArgs(256, 1.0, None, 8, 2.0),
+                                                 relu, x if relu else None)
+    y, save_mean, invstd, mn, mx, bits, packed, scale = got[:8]
+    stream = _Stream((packed, bits, scale, mn.view(scale.shape)))
+    stream.memory_format = torch.channels_last
+    back = ext_bf.hip_batch_norm_backward_packed(x.shape, stream, y, weight, save_mean, invstd, True, got[8] if relu else None)
+    return (*got, mean, var, *back)
+
+
+class _Stream(tuple):
+    pass
+
+
+@pytest.mark.parametrize("operator", [lambda x: _compress(x, False), lambda x: _compress(x, True), _compress_fixed, _relu, _dropout,
+                                      lambda x: _pool(x, False, False), lambda x: _pool(x, False, True), lambda x: _pool(x, True, False),
+                                      lambda x: _pool(x, True, True), _batch_norm, lambda x: _batch_norm_packed(x, False),
+                                      lambda x: _batch_norm_packed(x, True)],
+                         ids=["compress", "compress known ranges", "compress fixed", "relu", "dropout", "pool", "pool nibbles",
+                              "pool channels last", "pool channels last nibbles", "batch norm", "batch norm packed",
+                              "batch norm relu packed"])
+def test_calls_run_on_the_current_stream(operator):
+    """Forward and backward of each native call behind work that only calls on the same stream come behind."""
+    x = torch.randn(256, 64, 16, 16, device=DEV).to(torch.bfloat16)
+    ahead = torch.randn(1 << 24, device=DEV)
+    torch.cuda.manual_seed(5)
+    expected = operator(x)
+    torch.cuda.synchronize()
     side = torch.cuda.Stream()
-    side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        for _ in range(20):                            # work in front, that only calls on this stream come behind
-            x = x * 1.0009765625
-        y, mask = _glue.host().relu_forward(x)
+        late = torch.zeros_like(x)                     # what a call on another stream would read
+        side.synchronize()
+        for _ in range(40):                            # (about a millisecond)
+            ahead.mul_(1.0009765625)
+        late.copy_(x)
+        torch.cuda.manual_seed(5)
+        got = operator(late)
     side.synchronize()
-    assert torch.equal(y, torch.relu(x))
+    assert len(got) == len(expected)
+    for i, (a, b) in enumerate(zip(got, expected)):
+        assert torch.equal(a, b), i
 
 
 @pytest.mark.parametrize("draws", [1, 3])
@@ -40,18 +113,26 @@ def test_each_call_advances_the_generator_as_one_draw(draws):
     assert draws == 1 or not torch.equal(got[0], got[1])
 
 
-def test_tensor_classes_come_back_as_empty_like_makes_them():
-    class Named(torch.Tensor):
-        pass
-    x = torch.randn(2048, device=DEV)
-    for given in (x, torch.nn.Parameter(x.clone()), x.clone().as_subclass(Named)):
-        y, _ = ext_q.relu_forward(given.detach() if type(given) is torch.nn.Parameter else given)
-        assert type(y) is type(torch.empty_like(given.detach()))
-        assert torch.equal(y.as_subclass(torch.Tensor), torch.relu(given.detach()).as_subclass(torch.Tensor))
-
-
 class _Named(torch.Tensor):
     pass
+
+
+@pytest.mark.parametrize("make", [lambda x: x, lambda x: torch.nn.Parameter(x), lambda x: x.as_subclass(_Named)],
+                         ids=["tensor", "parameter", "subclass"])
+def test_tensor_classes_come_back_as_empty_like_makes_them(make):
+    x = torch.randn(2048, device=DEV)
+    given = make(x.clone())
+    with torch.no_grad():
+        y, mask = ext_q.relu_forward(given)
+        back = ext_q.relu_backward(given, mask)
+        z, kept = ext_q.dropout_forward(given, 0.5)
+        scaled = ext_q.dropout_backward(given, kept, 0.5)
+        for got in (y, back, z, scaled):
+            assert type(got) is type(torch.empty_like(given)) and not got.requires_grad
+    for got in (y, back):
+        assert torch.equal(got.as_subclass(torch.Tensor), torch.relu(x))
+    assert torch.equal(z.as_subclass(torch.Tensor), scaled.as_subclass(torch.Tensor))
+    assert torch.isin(z.as_subclass(torch.Tensor) / x, torch.tensor([0.0, 2.0], device=DEV)).all()
 
 
 @pytest.mark.parametrize("operator", ["relu", "dropout"])
