@@ -1202,10 +1202,11 @@ def test_closing_step_of_a_residual_block_in_the_batch_norm_pass(dtype, channels
         assert torch.equal(u, v), i
 
 
-@pytest.mark.parametrize("n", [200, 201, 215, 270])
-def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
-    """Forward passes of more than two rounds of blocks, the last block whole (n = 200) and ragged.  Output and saved stream
-    are those of the batch norm, the addition and the ReLU."""
+@pytest.mark.parametrize("size,n", [(28, 200), (28, 201), (28, 215), (28, 270), (27, 192), (27, 200), (27, 208), (27, 216)])
+def test_closing_step_over_several_rounds_of_blocks(size, n):
+    """Forward passes of more than two rounds of blocks of 8 steps (8 rows each), the last block whole, with one to three steps
+    (planes of 27 x 27: 0, 1, 2 and 3 left over) or with more (of 28 x 28: 0, 2, 6 and 4).  Output and saved stream are those of
+    the batch norm, the addition and the ReLU."""
     from actnn_amd.layers import QAddReLU, QBatchNorm2d, bn_add_relu, known_group_minmax
     res = []
     for fold in (False, True):
@@ -1215,7 +1216,7 @@ def test_closing_step_of_a_large_tensor_takes_longer_blocks(n):
         torch.manual_seed(4)
         bn, close = QBatchNorm2d(256).to(DEV).train(), QAddReLU()
         g = torch.Generator(device=DEV).manual_seed(n)
-        x, identity = (torch.randn(n, 256, 28, 28, device=DEV, generator=g, dtype=torch.bfloat16)
+        x, identity = (torch.randn(n, 256, size, size, device=DEV, generator=g, dtype=torch.bfloat16)
                        .contiguous(memory_format=torch.channels_last) for _ in range(2))
         torch.cuda.manual_seed(22)
         out = bn_add_relu(bn, close, x.requires_grad_(), identity)
