@@ -239,7 +239,8 @@ PyObject* quantize_rows_fixed(PyObject* const* a, Py_ssize_t n) {
   const Tensor known_mn = args.optional(), known_mx = args.optional();
   const auto dtype = rows.scalar_type();
   const auto store = type_of(args.integer());
-  TORCH_CHECK(rows.dim() == 2 && bits >= 1 && bits <= 8 && 8 % bits == 0, "quantize_rows_fixed: 8 % bits must be 0");
+  TORCH_CHECK(rows.dim() == 2, "quantize_rows_fixed: rows must have two dimensions, got ", rows.dim());
+  TORCH_CHECK(bits >= 1 && bits <= 8 && 8 % bits == 0, "quantize_rows_fixed: 8 % bits must be 0, got ", bits);
   const int64_t N = rows.size(0), F = rows.size(1), G = (F + 255) / 256;
   const c10::DeviceGuard guard(rows.device());
   const Tensor packed = empty({single_packed_bytes(N, G, bits)}, rows, at::kChar), scale = empty({N, G, 1}, rows, store);

@@ -58,6 +58,13 @@ def test_pool_arguments_keep_their_places(monkeypatch, window, stride, want):
         ext_q.max_pool2d_backward(x, x.to(torch.int8), x.shape[1:], (3, 2, 2), (2, 1), (1, 0))
 
 
+@pytest.mark.parametrize("shape,bits,what", [((4, 6, 100), 4, "two dimensions, got 3"), ((600,), 4, "two dimensions, got 1"),
+                                             ((4, 600), 3, "8 % bits must be 0, got 3"), ((4, 600), 0, "got 0"), ((4, 600), 16, "got 16")])
+def test_refusal_of_rows_at_one_width_says_what_is_wrong(shape, bits, what):
+    with pytest.raises(RuntimeError, match=what):
+        ext_q.quantize_rows_fixed(torch.zeros(shape), bits, None, torch.float32)
+
+
 @pytest.mark.parametrize("fails", [None, "hipcc", "g++"])
 def test_a_build_replaces_both_files_or_none(monkeypatch, tmp_path, fails):
     paths = [str(tmp_path / name) for name in ("libactnn_hip.so", "_host.so")]
