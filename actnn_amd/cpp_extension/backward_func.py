@@ -57,9 +57,12 @@ def known_sumsq(grad):
 def _bn_geometry(input, *parameters):
     """(N, C, HW, channels_last) of a dense tensor in the default or the channels-last layout, else None (also, where
     parameters are given, for an input that is not 16-byte aligned and parameters that are not dense fp32 ones)."""
-    if not (isinstance(input, torch.Tensor) and input.is_cuda):        # (asked of CPU tensors too, where nothing may be built)
-        return None
-    return _glue.host().batch_norm_geometry(input, *parameters)
+    host = _glue._lib._host
+    if host is None:                                    # not loaded yet: asked of CPU tensors too, where nothing may be built
+        if not (isinstance(input, torch.Tensor) and input.is_cuda):
+            return None
+        host = _glue.host()
+    return host.batch_norm_geometry(input, *parameters)
 
 
 def _f32_or_none(t):

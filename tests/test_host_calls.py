@@ -17,6 +17,8 @@ def nothing_built(monkeypatch):
         raise RuntimeError("not built")
     monkeypatch.setattr(_lib, "load", missing)
     monkeypatch.setattr(_lib, "load_host", missing)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_host", None)
 
 
 def test_batch_norm_of_cpu_tensors_needs_nothing_built(nothing_built):
